@@ -599,15 +599,16 @@ def _exact_model(case, seed):
             ws[role] = Weight(seed, key, dt, r, c, std)
         xn = rms(x, _norm(seed, "blk.%d.attn_norm" % l, d))
         q = rope(xn @ ws["q"].f64().T, H)
-        k = rope(xn @ ws["k"].f64().T, KH).half().double()
-        v = (xn @ ws["v"].f64().T).view(-1, KH, hd).half().double()
+        k = rope(xn @ ws["k"].f64().T, KH)
+        v = (xn @ ws["v"].f64().T).view(-1, KH, hd)
         att = []
         for i, (t, par, kc, vc) in enumerate(ins):
             sl = slice(i * M, (i + 1) * M)
             ks[i].append(k[sl].reshape(M, KH * hd))
             vs[i].append(v[sl].permute(1, 2, 0))
-            keys = torch.cat([kc[l].view(past, KH, hd).double(), k[sl]], 0)
-            vals = torch.cat([vc[l].view(past, KH, hd).double(), v[sl]], 0)
+            # the cache holds halves, and attention reads the cache
+            keys = torch.cat([kc[l].view(past, KH, hd), k[sl].half()], 0).double()
+            vals = torch.cat([vc[l].view(past, KH, hd), v[sl].half()], 0).double()
             heads = []
             for h in range(H):
                 sc = q[sl, h] @ keys[:, h // (H // KH)].T / math.sqrt(hd)
