@@ -546,7 +546,8 @@ struct AttnMArgs {
     int pslots = 0;      // slots per partial (set by the launcher)
     MmFragDst frag;      // frag.xh set: the fp32 combine writes this operand instead of out
 };
-bool attn_mfma_supported(int64_t hd, int kv_f16, int64_t M, int64_t n_head, int64_t n_kv);
+bool attn_mfma_supported(int64_t hd, int kv_f16, int64_t M, int64_t n_head, int64_t n_kv,
+                         int64_t cap_alloc);
 size_t attn_part_floats(int64_t M, int64_t n_head, int64_t hd, int64_t cap_alloc);
 // xq != null: the chunk combine writes the output projection's activation
 // operand (xq_dev.h layout, K = n_head * hd) instead of a.out

@@ -506,9 +506,14 @@ __device__ __forceinline__ void attn_fa_wg(const AttnMArgs& a, int grp, int kvh,
     const int64_t npast = a.npast, total = npast + a.M;
     const int64_t gslot0 = (int64_t)grp * a.pslots;
     if (gslot0 >= total) return;  // block-uniform
-    const int nck = (int)min((int64_t)(a.pslots / FA_CHK), (total - gslot0 + FA_CHK - 1) / FA_CHK);
     const int gqa = a.n_head / a.n_kv, qrows = a.M * gqa;
     const int rbase = (qsplit * FA_WAVES + w) * 16;  // the wave's first query row
+    // a node sees no draft slot past its own, so the chunks past the last
+    // node of the workgroup's rows are masked for all of them: not computed
+    // (a 256-token chain's row groups then do 62% of its draft chunks).  A
+    // group without a chunk writes an empty partial.
+    const int64_t seen = npast + (min((qsplit + 1) * FA_WAVES * 16, qrows) - 1) / gqa + 1;
+    const int nck = (int)min((int64_t)(a.pslots / FA_CHK), (seen - gslot0 + FA_CHK - 1) / FA_CHK);
     const bool wlive = rbase < qrows;                // wave-uniform
 
     // the wave's blocks b0 + i, b0 = BPW w: K blocks (st, dc0 + i) or V^T
@@ -532,7 +537,7 @@ __device__ __forceinline__ void attn_fa_wg(const AttnMArgs& a, int grp, int kvh,
             __builtin_amdgcn_global_load_lds((const void*)(src + ioff(i)),
                                              (lds_void*)(dst + i * 1024), 16, 0, 0);
     };
-    stage(gslot0, 0);
+    if (nck > 0) stage(gslot0, 0);
 
     // the rows' B operands (rows past qrows repeat the last valid row: their
     // results stay in their own O^T columns and are never stored)
@@ -898,8 +903,16 @@ bool attn_combine_xq_supported(int64_t hd, int64_t n_head) {
     return (hd == 64 || hd == 128) && K % 512 == 0 && K <= 16384;
 }
 
-bool attn_mfma_supported(int64_t hd, int kv_f16, int64_t M, int64_t n_head, int64_t n_kv) {
-    return kv_f16 && (hd == 64 || hd == 128) && M >= 1 && (M * (n_head / n_kv)) <= 32 * 16;
+// Any number of query rows: past 16 rows per kv head the many-row kernel takes
+// them 128 at a time.  Above 512 rows (256-token prefill chains) a cache of
+// more than 1024 chunks, whose weights the combine could not hold in LDS,
+// stays on the generic kernel.  Measured (256 tokens, 32 query heads on 8 kv
+// heads of 128, context 0-444): 2.05 ms per layer on the generic kernel, 14.5
+// + 8.5 us (combine) here.
+bool attn_mfma_supported(int64_t hd, int kv_f16, int64_t M, int64_t n_head, int64_t n_kv,
+                         int64_t cap_alloc) {
+    return kv_f16 && (hd == 64 || hd == 128) && M >= 1 &&
+           (M * (n_head / n_kv) <= 512 || cap_alloc / chunk_slots((int)hd) <= 1024);
 }
 
 size_t attn_part_floats(int64_t M, int64_t n_head, int64_t hd, int64_t cap_alloc) {
