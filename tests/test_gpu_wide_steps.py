@@ -29,3 +29,62 @@ def test_attention_of_more_than_512_query_rows(gctx, orc, hd, heads, kvh, M, npa
     assert rel_err_rows(got, want) < LOGIT_TOL
     for a, b in zip(kv, kvo):
         np.testing.assert_allclose(a.astype(np.float32), b.astype(np.float32), rtol=3e-3, atol=3e-3)
+
+
+# ---- the backend's single operations ----
+
+
+def weight(gctx, orc, rng, dt, rows, cols):
+    """A quantised weight on the device and its values in float64."""
+    raw = orc.quantize((rng.standard_normal((rows, cols)) * 0.02).astype(np.float32), dt)
+    values = orc.dequant(raw, dt, cols, rows=rows).reshape(rows, cols)
+    return gctx.upload(raw, dt, (cols, rows)), values.astype(np.float64)
+
+
+def close(got, want, terms):
+    """Sums of `terms` fp32 products in any order: each rounding is at most
+    2^-24 of a partial sum, which random signs keep near the result's size;
+    measured 2e-7 of the row's norm, 1e-6 is far from any misplaced operand."""
+    err = np.linalg.norm(got - want, axis=1) / np.maximum(np.linalg.norm(want, axis=1), 1e-30)
+    assert err.max() < 1e-6, (err.max(), terms)
+
+
+@pytest.mark.parametrize("dt", [P.Q4_0, P.Q8_0, P.Q4_K, P.Q6_K])
+@pytest.mark.parametrize("M,n_in,blocks", [(1, 1, 1), (3, 33, 2), (16, 257, 3), (17, 31, 5),
+                                           (33, 300, 1), (65, 96, 9), (130, 1408, 2)])
+def test_down_axpy_mfma(gctx, orc, dt, M, n_in, blocks):
+    """The column-axpy MFMA kernel at the edges of its token tiles (16, 32, 64),
+    32-row slices and 128-column groups, with one split and several; the
+    rows it adds to are kept."""
+    N = blocks * (256 if dt in (P.Q4_K, P.Q6_K) else 32)
+    rng = np.random.default_rng(dt * 1000 + M + n_in)
+    t, w = weight(gctx, orc, rng, dt, n_in, N)
+    x = rng.standard_normal((M, n_in)).astype(np.float32)
+    y0 = (rng.standard_normal((M, N)) * 0.1).astype(np.float32)
+    got = gctx.down_axpy(x, t, y0)
+    t.free()
+    close(got.astype(np.float64), y0 + x.astype(np.float64) @ w, n_in)
+
+
+@pytest.mark.parametrize("dt", [P.Q4_0, P.Q8_0, P.Q4_K, P.Q6_K])
+def test_down_axpy_special_values(gctx, orc, dt):
+    """Infinite, NaN, huge and tiny activations give what a sum of fp32
+    products gives; other tokens are untouched by them."""
+    rng = np.random.default_rng(5 + dt)
+    n_in, N = 70, 512
+    t, w = weight(gctx, orc, rng, dt, n_in, N)
+    x = rng.standard_normal((6, n_in)).astype(np.float32)
+    x[1, 40] = np.inf
+    x[2, 3], x[2, 50] = np.inf, -np.inf
+    x[3, 69] = np.nan
+    x[4] *= np.float32(1e30)
+    x[5] *= np.float32(1e-30)
+    got = gctx.down_axpy(x, t)
+    t.free()
+    w32 = w.astype(np.float32)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = (x[:, :, None] * w32[None]).astype(np.float64).sum(1)
+    for m in (0, 4, 5):
+        close(got[m:m + 1].astype(np.float64), want[m:m + 1], n_in)
+    for m in (1, 2, 3):
+        assert np.array_equal(got[m], want[m].astype(np.float32), equal_nan=True)

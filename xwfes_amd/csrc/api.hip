@@ -375,6 +375,24 @@ int ftx_matmul(ftx_ctx* ctx, const float* x, int64_t M, int64_t K, const ftx_ten
     return FTX_OK;
 }
 
+// y += x W over the stored rows: the MFMA kernel for the block types it takes,
+// else the generic one.  `part` holds down_part_floats(); the MFMA kernel's
+// splits stay within the allocation-free entry point's scratch for every
+// caller, so that both entry points sum in one order.
+static size_t down_part_floats(ftx_ctx* ctx, int dt, int64_t M, int64_t n_in, int64_t N) {
+    return axpy_supported(dt, N)
+               ? axpy_part_floats(M, n_in, N, NOALLOC_SCRATCH_FLOATS, ctx->cu_count)
+               : down_scratch_floats(M, n_in, N);
+}
+static hipError_t down(ftx_ctx* ctx, const uint8_t* W, int dt, int64_t row_bytes, int64_t n_in,
+                       int64_t N, const float* x, int64_t M, float* y, float* part,
+                       size_t part_floats) {
+    if (axpy_supported(dt, N))
+        return launch_axpy(ctx->stream, W, dt, row_bytes, n_in, N, x, n_in, M, y, N, part,
+                           part_floats, ctx->cu_count);
+    return launch_down(ctx->stream, W, dt, row_bytes, n_in, N, x, n_in, M, y, N, part);
+}
+
 int ftx_down_axpy(ftx_ctx* ctx, const float* x, int64_t M, int64_t n_in, const ftx_tensor* W,
                   float* y) {
     if (!ctx || !x || !W || !y) return ftx_fail(ctx, FTX_E_INVALID, "null argument");
@@ -384,11 +402,10 @@ int ftx_down_axpy(ftx_ctx* ctx, const float* x, int64_t M, int64_t n_in, const f
     if (M == 0) return FTX_OK;
     Staged s{};
     float* part;
-    const size_t pf = down_scratch_floats(M, n_in, N);
+    const size_t pf = down_part_floats(ctx, W->dtype, M, n_in, N);
     int rc = stage_xy(ctx, x, (size_t)(M * n_in), y, (size_t)(M * N), true, pf, s, &part);
     if (rc) return rc;
-    FTX_HIP(ctx, launch_down(ctx->stream, W->data, W->dtype, W->row_bytes, n_in, N, s.x, n_in, M,
-                             s.y, N, part));
+    FTX_HIP(ctx, down(ctx, W->data, W->dtype, W->row_bytes, n_in, N, s.x, M, s.y, part, pf));
     if (s.y_host)
         FTX_HIP(ctx, hipMemcpyAsync(y, s.y, (size_t)(M * N) * sizeof(float),
                                     hipMemcpyDeviceToHost, ctx->stream));
@@ -419,8 +436,8 @@ int ftx_down_axpy_noalloc(ftx_ctx* ctx, const float* x, int64_t M, int64_t n_in,
     if (!ctx->noalloc_scratch)
         return ftx_fail(ctx, FTX_E_DEVICE, "down_axpy_noalloc: the scratch array's address "
                                            "could not be looked up on this device");
-    FTX_HIP(ctx, launch_down(ctx->stream, W->data, W->dtype, W->row_bytes, n_in, N, x, n_in, M, y,
-                             N, ctx->noalloc_scratch));
+    FTX_HIP(ctx, down(ctx, W->data, W->dtype, W->row_bytes, n_in, N, x, M, y, ctx->noalloc_scratch,
+                      NOALLOC_SCRATCH_FLOATS));
     // results are stream-ordered: the call returns once the work is enqueued
     // (a capturing stream must not be synchronised)
     return FTX_OK;
@@ -440,7 +457,7 @@ int ftx_expert_chunk(ftx_ctx* ctx, const ftx_expert_job* j) {
     const int64_t M = j->M, K = j->K, IC = j->IC;
     Staged s{};
     float* extra;
-    const size_t pf = down_scratch_floats(M, IC, K);
+    const size_t pf = down_part_floats(ctx, j->dt, M, IC, K);
     int rc = stage_xy(ctx, j->x, (size_t)(M * K), j->out, (size_t)(M * K), true,
                       pf + (size_t)(M * IC) + 64, s, &extra);
     if (rc) return rc;
@@ -448,8 +465,7 @@ int ftx_expert_chunk(ftx_ctx* ctx, const ftx_expert_job* j) {
     float* part = extra + (((size_t)(M * IC) + 63) & ~(size_t)63);
     FTX_HIP(ctx, launch_gemv_swiglu(ctx->stream, (const uint8_t*)j->gate, (const uint8_t*)j->up,
                                     j->dt, rb, IC, s.x, K, K, M, h, IC));
-    FTX_HIP(ctx, launch_down(ctx->stream, (const uint8_t*)j->down, j->dt, rb, IC, K, h, IC, M, s.y,
-                             K, part));
+    FTX_HIP(ctx, down(ctx, (const uint8_t*)j->down, j->dt, rb, IC, K, h, M, s.y, part, pf));
     if (s.y_host)
         FTX_HIP(ctx, hipMemcpyAsync(j->out, s.y, (size_t)(M * K) * sizeof(float),
                                     hipMemcpyDeviceToHost, ctx->stream));

@@ -304,6 +304,16 @@ hipError_t launch_mm_prep_fold(hipStream_t st, float* x, int64_t ldx, const floa
                                const MmPend& fold);
 // the partials `fold` added into y rows < M (a reduce launch)
 hipError_t launch_mm_fold(hipStream_t st, const MmPend& fold, int64_t M, float* y, int64_t ldy);
+// y[m][j] += sum_i h[m][i] W[i][j] over the stored rows (k_axpy.hip: Q4_0,
+// Q8_0, Q4_K, Q6_K of whole blocks), any M and any h.  Split partials go to
+// `part` (at most part_floats) and are added into y by a reduce launch, or
+// left in *pend for y's next reader; without room for them there is one split.
+bool axpy_supported(int dt, int64_t N);
+// the partials of the best split within `cap` floats
+size_t axpy_part_floats(int64_t M, int64_t n_in, int64_t N, size_t cap, int cu_count);
+hipError_t launch_axpy(hipStream_t st, const uint8_t* W, int dt, int64_t row_bytes, int64_t n_in,
+                       int64_t N, const float* h, int64_t ldh, int64_t M, float* y, int64_t ldy,
+                       float* part, size_t part_floats, int cu_count, MmPend* pend = nullptr);
 bool mm_supported(int dt, int64_t K);
 // the one-pass GEMM's copy of Q8_0 / Q4_0 weights (per 16-row tile and
 // 256-element step, every lane's bytes contiguous): its internal dtype (or

@@ -1,0 +1,532 @@
+// k_axpy.hip -- the column-axpy form y[m, j] += sum_i h[m, i] * W[i, j]
+// (matmul_down_axpy, src/cpu_backend.cpp:60-75) on MFMA over the tensor as it
+// is stored: n_in rows of N columns, blocks along the columns, no re-tiled
+// copy, any h.
+//
+// Along the contraction i every row carries its own block scale, so the scale
+// goes into the activation operand: A = h[m, i] * d[i, block], formed in fp32
+// and split into three bf16 limbs by truncation (8 + 8 + 8 bits: the split is
+// exact and needs no range assumption), B = the block's integers, exact in
+// bf16 (q - 8, q or q - 32: at most 8 bits).  Three MFMAs per product; every
+// product is exact and the only rounding is that of the fp32 sums.
+//   Q4_0  d (q - 8)         Q8_0  d q            one A per 32 columns
+//   Q6_K  (d sc) (q - 32)                         one A per 16 columns
+//   Q4_K  (d sc) (q - 8) - (dmin m - 8 d sc)      one A per 32 columns; the min
+//         term is a product of its own, h (3 limbs) x its 3 limbs, with the
+//         four 32-column sub-blocks as B columns (centred on q = 8 the two
+//         sums are the size of the result: with q and dmin m their difference
+//         loses a bit and a half)
+//
+// The MFMA wants 8 contraction values (rows) of one column in a lane, the
+// tensor has a row's columns side by side.  A wave loads 8 rows x 4 or 8
+// bytes per lane, transposes bytes in registers (v_perm) and passes the
+// columns through its own LDS slots ([tile][kq][column] x 8 bytes, columns
+// XOR-swizzled by the tile: no bank conflict either way); no barrier until
+// the end.  A workgroup's 8 waves take a 128-column group's 32-row slices in
+// turn and are added in LDS in wave order; splits over the rows leave
+// partials for the next kernel.
+//
+// What bounds it: up to 16 tokens the arrival of the weights and the byte
+// work (about 100 VALU instructions per 32 x 32 weights), above that the limb
+// splits (52 VALU per 32 x 32 weights and 16 tokens) and MFMAs.
+// Measured, one launch (before: the generic kernel, or Q6_K's 8-token chunks):
+// Q8_0 14336 x 4096, 1 token 795 -> 25.6 us (2.4 TB/s); Q4_0, 24 tokens 2013 ->
+// 35.9 us; Q6_K, 256 tokens 531 -> 214 us (140 TFLOP/s); Q4_0 1408 x 512, 1
+// token 30.8 -> 7 us.  Error against 64 bits 1.2e-7 to 1.7e-7 where the fp32
+// sums of the generic kernel had 2.9e-7 to 5.7e-7.
+#include "ftx_internal.h"
+#include "quant_dev.h"
+
+namespace {
+
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+constexpr int AX_WAVES = 8;
+constexpr int AX_COLS = 128;  // columns per workgroup
+
+struct AxArgs {
+    const uint8_t* W;
+    int64_t row_bytes, n_in, N;
+    const float* h;
+    int64_t ldh;
+    int M;
+    int ntt;               // token tiles of 16 MS
+    int slices_per_split;  // 32-row slices
+    float* out;            // partials [split][M][ldo], or y with accum
+    int64_t ldo, split_stride;
+    int accum;
+};
+
+// loads of any alignment (the hardware takes them as they come)
+struct __attribute__((packed)) u32u { uint32_t v; };
+struct __attribute__((packed)) u64u { uint32_t v[2]; };
+struct __attribute__((packed)) u16u { uint16_t v; };
+struct __attribute__((packed)) u128u { uint32_t v[4]; };
+struct __attribute__((packed, aligned(4))) f4u { float v[4]; };
+
+__device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) {
+    return __builtin_amdgcn_perm(hi, lo, sel);
+}
+
+// rows r0..r3 of four bytes -> columns c[0..3], byte e = row e
+__device__ __forceinline__ void tr4(uint32_t r0, uint32_t r1, uint32_t r2, uint32_t r3, uint32_t* c) {
+    const uint32_t a = perm(r1, r0, 0x05010400u), b = perm(r1, r0, 0x07030602u);
+    const uint32_t d = perm(r3, r2, 0x05010400u), e = perm(r3, r2, 0x07030602u);
+    c[0] = perm(d, a, 0x05040100u);
+    c[1] = perm(d, a, 0x07060302u);
+    c[2] = perm(e, b, 0x05040100u);
+    c[3] = perm(e, b, 0x07060302u);
+}
+
+// the high halves of two floats (bf16 by truncation)
+__device__ __forceinline__ uint32_t pack_hi(float a, float b) {
+    return perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+__device__ __forceinline__ float trunc_bf(float a) {
+    return __uint_as_float(__float_as_uint(a) & 0xFFFF0000u);
+}
+
+// a = l[0] + l[1] + l[2] exactly
+__device__ __forceinline__ void split3(const float* a, v8bf* l) {
+#pragma clang fp contract(off)
+    uint32_t p[3][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float a0 = a[2 * i], a1 = a[2 * i + 1];
+        const float b0 = a0 - trunc_bf(a0), b1 = a1 - trunc_bf(a1);
+        const float c0 = b0 - trunc_bf(b0), c1 = b1 - trunc_bf(b1);
+        p[0][i] = pack_hi(a0, a1);
+        p[1][i] = pack_hi(b0, b1);
+        p[2][i] = pack_hi(c0, c1);
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const uint4 v = {p[k][0], p[k][1], p[k][2], p[k][3]};
+        l[k] = __builtin_bit_cast(v8bf, v);
+    }
+}
+
+// 8 signed bytes -> bf16, exact
+__device__ __forceinline__ v8bf sbytes(uint32_t x, uint32_t y) {
+    uint4 v;
+    v.x = pack_hi((float)(int8_t)x, (float)(int8_t)(x >> 8));
+    v.y = pack_hi((float)(int8_t)(x >> 16), (float)(int8_t)(x >> 24));
+    v.z = pack_hi((float)(int8_t)y, (float)(int8_t)(y >> 8));
+    v.w = pack_hi((float)(int8_t)(y >> 16), (float)(int8_t)(y >> 24));
+    return __builtin_bit_cast(v8bf, v);
+}
+// 4 bytes 0..127 minus `bias` (at most 120), as signed bytes
+__device__ __forceinline__ uint32_t minus4(uint32_t x, uint32_t bias) {
+    return (x + (0x80u - bias) * 0x01010101u) ^ 0x80808080u;
+}
+
+template <int DT>
+struct AxCfg {
+    // LDS tiles of 16 columns x 32 rows (nibble types hold two in one)
+    static constexpr int TILES = (DT == FTX_Q8_0 || DT == FTX_Q6_K) ? 8 : 4;
+    static constexpr int SWZ = DT == FTX_Q8_0 ? 7 : 3;
+    // scales per row: blocks, Q4_K's scales then mins, Q6_K's 16-column scales
+    static constexpr int NSC = (DT == FTX_Q4_K || DT == FTX_Q6_K) ? 8 : 4;
+    static constexpr int WORDS = (DT == FTX_Q8_0 || DT == FTX_Q6_K) ? 2 : 1;  // per lane and row
+};
+
+// a wave's raw operands of one slice: 8 rows of the lane's bytes, and the
+// scale fields of row 8 kq + c % 8 (c = lane % 16)
+template <int DT>
+struct AxRaw {
+    uint32_t w[8][AxCfg<DT>::WORDS];
+    uint32_t s[DT == FTX_Q4_K ? 4 : 2];
+};
+
+template <int DT, int MS>
+__global__ void __launch_bounds__(64 * AX_WAVES)
+    __attribute__((amdgpu_waves_per_eu(MS == 1 ? 4 : 2, MS == 1 ? 4 : 2))) k_axpy(AxArgs a) {
+    using C = AxCfg<DT>;
+    // per wave: columns, then scales; at the end the waves' sums of one
+    // 16-token tile
+    constexpr int WB = C::TILES * 512 + C::NSC * 128;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[65536];
+    static_assert(WB * AX_WAVES <= 65536, "");
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 15, kq = lane >> 4;
+    const int64_t j0 = (int64_t)(blockIdx.x / (unsigned)a.ntt) * AX_COLS;  // first column
+    const int m0 = (int)(blockIdx.x % (unsigned)a.ntt) * 16 * MS;
+    const int ks = blockIdx.z;
+    const int64_t nsl = (a.n_in + 31) / 32;
+    const int64_t I0 = (int64_t)ks * a.slices_per_split;
+    const int64_t I1 = min(I0 + (int64_t)a.slices_per_split, nsl);
+    uint2* cols = (uint2*)(lds + w * WB);
+    float* scl = (float*)(lds + w * WB + C::TILES * 512);  // [NSC][kq][8]
+
+    // the lane's byte offset in a row and its scale fields' (blocks past the
+    // row's end read the last one; their columns are not stored)
+    int64_t off, soff[2] = {0, 0}, doff = 0;
+    if constexpr (DT == FTX_Q4_0 || DT == FTX_Q8_0) {
+        constexpr int bb = DT == FTX_Q4_0 ? 18 : 34;
+        const int64_t nb = a.N / 32, b0 = j0 / 32;
+        off = min(b0 + c / 4, nb - 1) * bb + 2 + (c % 4) * (bb - 2) / 4;
+        soff[0] = min(b0 + c / 8, nb - 1) * bb;
+        soff[1] = min(b0 + 2 + c / 8, nb - 1) * bb;
+    } else if constexpr (DT == FTX_Q4_K) {
+        const int64_t sb = j0 / 256;
+        off = sb * 144 + 16 + 64 * ((j0 / 128) & 1) + 4 * c;
+        soff[0] = sb * 144;
+    } else {  // planar Q6_K rows (quant_dev.h)
+        const int64_t sb = j0 / 256, nsb = a.N / 256, half = (j0 / 128) & 1;
+        off = sb * 128 + 64 * (c >> 3) + 32 * half + 4 * (c & 7);
+        soff[0] = nsb * 128 + sb * 64 + 32 * (c >> 3) + 16 * half + 4 * (c & 3);  // QH
+        soff[1] = nsb * 192 + sb * 16 + 8 * half + 4 * (c >> 3);                   // 4 scales
+        doff = nsb * 208 + sb * 2;
+    }
+    auto load = [&](AxRaw<DT>& o, int64_t I) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const uint8_t* r = a.W + min(32 * I + 8 * kq + e, a.n_in - 1) * a.row_bytes;
+            if constexpr (DT == FTX_Q8_0) {
+                const u64u v = *(const u64u*)(r + off);
+                o.w[e][0] = v.v[0];
+                o.w[e][1] = v.v[1];
+            } else {
+                o.w[e][0] = ((const u32u*)(r + off))->v;
+                if constexpr (DT == FTX_Q6_K) o.w[e][1] = ((const u32u*)(r + soff[0]))->v;
+            }
+        }
+        const uint8_t* r = a.W + min(32 * I + 8 * kq + (c & 7), a.n_in - 1) * a.row_bytes;
+        if constexpr (DT == FTX_Q4_K) {
+            const u128u v = *(const u128u*)(r + soff[0]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o.s[i] = v.v[i];
+        } else if constexpr (DT == FTX_Q6_K) {
+            o.s[0] = ((const u32u*)(r + soff[1]))->v;
+            o.s[1] = ((const u16u*)(r + doff))->v;
+        } else {
+            o.s[0] = ((const u16u*)(r + soff[0]))->v;
+            o.s[1] = ((const u16u*)(r + soff[1]))->v;
+        }
+    };
+    // the columns of tile n into its slots: row octet kq, column col
+    auto slot = [&](int n, int col) { return (n * 4 + kq) * 16 + (col ^ (n & C::SWZ)); };
+    auto put = [&](const AxRaw<DT>& o) {
+        uint32_t lo[4], hi[4];
+        if constexpr (DT == FTX_Q8_0) {
+#pragma unroll
+            for (int hw = 0; hw < 2; ++hw) {
+                tr4(o.w[0][hw], o.w[1][hw], o.w[2][hw], o.w[3][hw], lo);
+                tr4(o.w[4][hw], o.w[5][hw], o.w[6][hw], o.w[7][hw], hi);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    cols[slot(c >> 1, 8 * (c & 1) + 4 * hw + i)] = uint2{lo[i], hi[i]};
+            }
+        } else if constexpr (DT == FTX_Q6_K) {
+            // ql byte of element 32 k + l (k = a, and 2 + a in its high
+            // nibble), l = 16 b + 8 g + t; the two high bits from the qh byte
+            const int g = c >> 3, av = (c >> 2) & 1, b = (c >> 1) & 1, t = 4 * (c & 1);
+#pragma unroll
+            for (int k2 = 0; k2 < 2; ++k2) {
+                uint32_t q[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    q[e] = minus4(((o.w[e][0] >> (4 * k2)) & 0x0F0F0F0Fu) |
+                                      (((o.w[e][1] >> (4 * k2 + 2 * av)) & 0x03030303u) << 4), 32);
+                tr4(q[0], q[1], q[2], q[3], lo);
+                tr4(q[4], q[5], q[6], q[7], hi);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    cols[slot(2 * (2 * k2 + av) + b, 8 * g + t + i)] = uint2{lo[i], hi[i]};
+            }
+        } else {
+            tr4(o.w[0][0], o.w[1][0], o.w[2][0], o.w[3][0], lo);
+            tr4(o.w[4][0], o.w[5][0], o.w[6][0], o.w[7][0], hi);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) cols[slot(c >> 2, 4 * (c & 3) + i)] = uint2{lo[i], hi[i]};
+        }
+        // scales of row 8 kq + c % 8
+        const int at = kq * 8 + (c & 7), hf = c >> 3;
+        if constexpr (DT == FTX_Q4_K) {
+            const float d = h2f((uint16_t)(o.s[0] & 0xFFFF)), dmin = h2f((uint16_t)(o.s[0] >> 16));
+            // sub-blocks 4 h .. 4 h + 3 of the row's super-block; this lane
+            // takes two of them
+            const bool up = ((j0 / 128) & 1) != 0;
+            const uint32_t sc = up ? (o.s[3] & 0x0F0F0F0Fu) | ((o.s[1] >> 2) & 0x30303030u)
+                                   : o.s[1] & 0x3F3F3F3Fu;
+            const uint32_t mn = up ? ((o.s[3] >> 4) & 0x0F0F0F0Fu) | ((o.s[2] >> 2) & 0x30303030u)
+                                   : o.s[2] & 0x3F3F3F3Fu;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int sh = 16 * hf + 8 * i;
+                const float ds = d * (float)((sc >> sh) & 0xFF);
+                scl[(2 * hf + i) * 32 + at] = ds;
+                scl[(4 + 2 * hf + i) * 32 + at] = dmin * (float)((mn >> sh) & 0xFF) - 8.f * ds;
+            }
+        } else if constexpr (DT == FTX_Q6_K) {
+            const float d = h2f((uint16_t)o.s[1]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                scl[(4 * hf + i) * 32 + at] = d * (float)(int8_t)(o.s[0] >> (8 * i));
+        } else {
+            scl[hf * 32 + at] = h2f((uint16_t)o.s[0]);
+            scl[(2 + hf) * 32 + at] = h2f((uint16_t)o.s[1]);
+        }
+    };
+    // h of the lane's token (past M: the last one's, never stored) in each
+    // 16-token tile, rows 8 kq .. + 7 of the slice (zero past n_in)
+    const float* hrow[MS];
+#pragma unroll
+    for (int ms = 0; ms < MS; ++ms)
+        hrow[ms] = a.h + (int64_t)min(m0 + 16 * ms + c, a.M - 1) * a.ldh;
+    auto load_h = [&](float (&hv)[MS][8], int64_t I) {
+        const int64_t i = 32 * I + 8 * kq;
+        if (32 * I + 32 <= a.n_in) {  // uniform
+#pragma unroll
+            for (int ms = 0; ms < MS; ++ms) {
+                const f4u u = *(const f4u*)(hrow[ms] + i), v = *(const f4u*)(hrow[ms] + i + 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    hv[ms][e] = u.v[e];
+                    hv[ms][4 + e] = v.v[e];
+                }
+            }
+        } else {
+#pragma unroll
+            for (int ms = 0; ms < MS; ++ms)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float v = hrow[ms][min(i + e, a.n_in - 1)];
+                    hv[ms][e] = i + e < a.n_in ? v : 0.f;
+                }
+        }
+    };
+    v4f acc[8][MS], accm[DT == FTX_Q4_K ? MS : 1];
+#pragma unroll
+    for (int n = 0; n < 8; ++n)
+#pragma unroll
+        for (int ms = 0; ms < MS; ++ms) acc[n][ms] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ms = 0; ms < (DT == FTX_Q4_K ? MS : 1); ++ms) accm[ms] = v4f{0.f, 0.f, 0.f, 0.f};
+    auto mfma3 = [&](const v8bf* l, const v8bf& b, v4f acc_) {
+        acc_ = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l[2], b, acc_, 0, 0, 0);
+        acc_ = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l[1], b, acc_, 0, 0, 0);
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(l[0], b, acc_, 0, 0, 0);
+    };
+    auto scales8 = [&](int s, int q, float* d) {
+        const float4 u = *(const float4*)&scl[s * 32 + q * 8], v = *(const float4*)&scl[s * 32 + q * 8 + 4];
+        d[0] = u.x; d[1] = u.y; d[2] = u.z; d[3] = u.w;
+        d[4] = v.x; d[5] = v.y; d[6] = v.z; d[7] = v.w;
+    };
+
+    if (I0 + w < I1) {
+        AxRaw<DT> raw;
+        float hv[MS][8];
+        load(raw, I0 + w);
+        for (int64_t I = I0 + w; I < I1; I += AX_WAVES) {
+            load_h(hv, I);
+            put(raw);
+            // (the last slice's load is its own again: no branch between the
+            // loads and the waits)
+            load(raw, min(I + AX_WAVES, I1 - 1));
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if constexpr (DT == FTX_Q4_K) {
+                // B column b < 4: dmin m - 8 d sc of sub-block b
+                float dm[8];
+                scales8(4 + (c & 3), kq, dm);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) dm[e] = c < 4 ? dm[e] : 0.f;
+                v8bf bm[3];
+                split3(dm, bm);
+#pragma unroll
+                for (int ms = 0; ms < MS; ++ms) {
+                    v8bf l[3];
+                    split3(hv[ms], l);
+#pragma unroll
+                    for (int p = 2; p >= 0; --p)
+#pragma unroll
+                        for (int q = p; q >= 0; --q)
+                            accm[ms] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l[q], bm[p - q], accm[ms], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {  // 32 columns
+                v8bf bw[2];
+                if constexpr (DT == FTX_Q4_0) {
+                    const uint2 v = cols[slot(b, c)];
+#pragma unroll
+                    for (int p = 0; p < 2; ++p)
+                        bw[p] = sbytes(minus4((v.x >> (4 * p)) & 0x0F0F0F0Fu, 8),
+                                       minus4((v.y >> (4 * p)) & 0x0F0F0F0Fu, 8));
+                } else if constexpr (DT == FTX_Q4_K) {
+#pragma unroll
+                    for (int p = 0; p < 2; ++p) {
+                        const uint2 v = cols[slot(2 * (b >> 1) + p, c)];
+                        bw[p] = sbytes(minus4((v.x >> (4 * (b & 1))) & 0x0F0F0F0Fu, 8),
+                                       minus4((v.y >> (4 * (b & 1))) & 0x0F0F0F0Fu, 8));
+                    }
+                } else {
+#pragma unroll
+                    for (int p = 0; p < 2; ++p) {
+                        const uint2 v = cols[slot(2 * b + p, c)];
+                        bw[p] = sbytes(v.x, v.y);
+                    }
+                }
+                float d[DT == FTX_Q6_K ? 2 : 1][8];
+#pragma unroll
+                for (int p = 0; p < (DT == FTX_Q6_K ? 2 : 1); ++p)
+                    scales8(DT == FTX_Q6_K ? 2 * b + p : b, kq, d[p]);
+#pragma unroll
+                for (int ms = 0; ms < MS; ++ms) {
+                    v8bf l[3];
+                    float t[8];
+#pragma unroll
+                    for (int p = 0; p < 2; ++p) {
+                        if (p == 0 || DT == FTX_Q6_K) {
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) t[e] = hv[ms][e] * d[DT == FTX_Q6_K ? p : 0][e];
+                            split3(t, l);
+                        }
+                        acc[2 * b + p][ms] = mfma3(l, bw[p], acc[2 * b + p][ms]);
+                    }
+                }
+            }
+            // (the reads above before the next slice's writes)
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+    }
+    if constexpr (DT == FTX_Q4_K) {
+        // the min sums: lane (c, kq) of tile n holds tokens 4 kq + r; those of
+        // sub-block n / 2 are in lane 16 kq + n / 2
+#pragma unroll
+        for (int ms = 0; ms < MS; ++ms)
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float v = __shfl(accm[ms][r], 16 * kq + b, 64);
+                    acc[2 * b][ms][r] -= v;
+                    acc[2 * b + 1][ms][r] -= v;
+                }
+    }
+    // wave w adds the eight waves' sums of tile w, in wave order, and writes
+    // them: columns 32 (w / 2) + .. of the group
+    v4f* red = (v4f*)lds;  // [wave][tile][lane]
+    const int64_t col = j0 + 32 * (w >> 1) + (DT == FTX_Q4_0 ? 2 * c + (w & 1) : 16 * (w & 1) + c);
+#pragma unroll
+    for (int ms = 0; ms < MS; ++ms) {
+        __syncthreads();
+#pragma unroll
+        for (int n = 0; n < 8; ++n) red[(w * 8 + n) * 64 + lane] = acc[n][ms];
+        __syncthreads();
+        v4f s = red[w * 64 + lane];
+#pragma unroll
+        for (int k = 1; k < AX_WAVES; ++k) s += red[(k * 8 + w) * 64 + lane];
+        if (col >= a.N) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int m = m0 + 16 * ms + 4 * kq + r;
+            if (m >= a.M) continue;
+            float v = s[r];
+            if (v != v) {
+                // an infinite or NaN operand breaks the limbs: this sum again,
+                // one product after the other
+                const float* hr = a.h + (int64_t)m * a.ldh;
+                v = 0.f;
+                for (int64_t i = 32 * I0; i < min(32 * I1, a.n_in); ++i) {
+                    float q[8], x = 0.f;
+                    dq8(a.W + i * a.row_bytes, DT, col & ~(int64_t)7, a.N, q);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) x = (int)(col & 7) == e ? q[e] : x;
+                    v += hr[i] * x;
+                }
+            }
+            float* p = a.out + (int64_t)ks * a.split_stride + (int64_t)m * a.ldo + col;
+            *p = a.accum ? *p + v : v;
+        }
+    }
+}
+
+}  // namespace
+
+// whole blocks along a row (the K types have 256-column blocks)
+bool axpy_supported(int dt, int64_t N) {
+    return N > 0 && (((dt == FTX_Q4_0 || dt == FTX_Q8_0) && N % 32 == 0) ||
+                     ((dt == FTX_Q4_K || dt == FTX_Q6_K) && N % 256 == 0));
+}
+
+// 16-token tiles per workgroup, and splits over the rows: workgroups run two
+// to a CU in rounds of 512, each as long as its waves' slices (every eighth of
+// the split's) plus about two slices of start and reduction; the fewest slice
+// times, the fewest splits on ties, within `cap` partial floats (one split
+// writes y itself)
+static int axpy_ms(int64_t M) { return M <= 16 ? 1 : (M <= 32 ? 2 : 4); }
+static int axpy_splits(int64_t M, int64_t n_in, int64_t N, size_t cap, int cu_count) {
+    const int ms = axpy_ms(M);
+    const int64_t wg = (N + AX_COLS - 1) / AX_COLS * ((M + 16 * ms - 1) / (16 * ms));
+    const int64_t nsl = (n_in + 31) / 32, slots = 2 * (cu_count > 0 ? cu_count : 256);
+    int best = 1;
+    int64_t best_cost = -1;
+    for (int64_t S = 1; S <= 32 && S <= nsl; ++S) {
+        // (the reduce has a grid row per token)
+        if (S > 1 && ((size_t)(S * M * N) > cap || M > 65535)) break;
+        const int64_t per = (nsl + S - 1) / S;
+        const int64_t cost = (wg * S + slots - 1) / slots * ((per + AX_WAVES - 1) / AX_WAVES + 2);
+        if (best_cost < 0 || cost < best_cost) {
+            best_cost = cost;
+            best = (int)S;
+        }
+    }
+    return best;
+}
+
+size_t axpy_part_floats(int64_t M, int64_t n_in, int64_t N, size_t cap, int cu_count) {
+    const int S = M > 0 ? axpy_splits(M, n_in, N, cap, cu_count) : 1;
+    return S > 1 ? (size_t)S * (size_t)(M * N) : 0;
+}
+
+hipError_t launch_axpy(hipStream_t st, const uint8_t* W, int dt, int64_t row_bytes, int64_t n_in,
+                       int64_t N, const float* h, int64_t ldh, int64_t M, float* y, int64_t ldy,
+                       float* part, size_t part_floats, int cu_count, MmPend* pend) {
+    if (pend) *pend = MmPend{};
+    if (M <= 0 || n_in <= 0) return hipSuccess;
+    if (!axpy_supported(dt, N)) return hipErrorInvalidValue;
+    int S = axpy_splits(M, n_in, N, part ? part_floats : 0, cu_count);
+    const int64_t nsl = (n_in + 31) / 32;
+    AxArgs a{};
+    a.W = W;
+    a.row_bytes = row_bytes;
+    a.n_in = n_in;
+    a.N = N;
+    a.h = h;
+    a.ldh = ldh;
+    a.M = (int)M;
+    const int ms = axpy_ms(M);
+    a.ntt = (int)((M + 16 * ms - 1) / (16 * ms));
+    a.slices_per_split = (int)((nsl + S - 1) / S);
+    S = (int)((nsl + a.slices_per_split - 1) / a.slices_per_split);
+    a.out = S > 1 ? part : y;
+    a.ldo = S > 1 ? N : ldy;
+    a.split_stride = S > 1 ? M * N : 0;
+    a.accum = S == 1;
+    using K_t = void (*)(AxArgs);
+    static const K_t kerns[4][3] = {
+        {k_axpy<FTX_Q4_0, 1>, k_axpy<FTX_Q4_0, 2>, k_axpy<FTX_Q4_0, 4>},
+        {k_axpy<FTX_Q8_0, 1>, k_axpy<FTX_Q8_0, 2>, k_axpy<FTX_Q8_0, 4>},
+        {k_axpy<FTX_Q4_K, 1>, k_axpy<FTX_Q4_K, 2>, k_axpy<FTX_Q4_K, 4>},
+        {k_axpy<FTX_Q6_K, 1>, k_axpy<FTX_Q6_K, 2>, k_axpy<FTX_Q6_K, 4>}};
+    const int di = dt == FTX_Q4_0 ? 0 : (dt == FTX_Q8_0 ? 1 : (dt == FTX_Q4_K ? 2 : 3));
+    const dim3 grid((unsigned)((N + AX_COLS - 1) / AX_COLS * a.ntt), 1, (unsigned)S);
+    ktimed_launch(kerns[di][ms == 4 ? 2 : ms - 1], grid, dim3(64 * AX_WAVES), 0, st, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || S == 1) return e;
+    MmPend p;
+    p.part = part;
+    p.split_stride = M * N;
+    p.ldp = N;
+    p.S = S;
+    p.N = N;
+    p.accum = 1;
+    if (pend) {
+        *pend = p;  // added into y by the next kernel that reads it
+        return hipSuccess;
+    }
+    return launch_mm_fold(st, p, M, y, ldy);
+}

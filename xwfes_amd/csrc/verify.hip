@@ -431,8 +431,11 @@ static int verify_large(ftx_ctx* ctx, ftx_model* m, const ftx_seq_args* sq, int6
                      launch_gemv_swiglu(st, sg->data, su->data, sg->dtype, sg->row_bytes, FS,
                                         m->xn, D, D, Mt, m->h, FS, true));
             TRACED_L(TK_DOWN, wbytes(sd) + Md * FS * f4 + 2 * Md * D * f4,
-                     launch_down(st, sd->data, sd->dtype, sd->row_bytes, FS, D, m->h, FS, Mt,
-                                 m->tmpo, D, m->part));
+                     axpy_supported(sd->dtype, D)
+                         ? launch_axpy(st, sd->data, sd->dtype, sd->row_bytes, FS, D, m->h, FS, Mt,
+                                       m->tmpo, D, m->part, m->part_floats, ctx->cu_count)
+                         : launch_down(st, sd->data, sd->dtype, sd->row_bytes, FS, D, m->h, FS, Mt,
+                                       m->tmpo, D, m->part));
             TRACED_L(TK_MOE_COMBINE, 3 * Md * D * f4, launch_add(st, m->tmpo, m->x, Mt * D));
         }
         return FTX_OK;
@@ -631,22 +634,22 @@ static int verify_large(ftx_ctx* ctx, ftx_model* m, const ftx_seq_args* sq, int6
             TRACED_L(TK_DOWN, down_b,
                      launch_mm_down(st, m->down_tiled[l], F, D, m->h, F, Mt, out1(m->x, D, 1),
                                     m->mm_part, m->mm_part_n, ctx->cu_count, &xpend));
-        } else if (m->down_tiled[l] && down_mfma_supported(dn->dtype, F, D, 8)) {
-            // the MFMA down kernel on 8-row chunks, every chunk's split
-            // partials added into x by one reduce
-            auto chunks = [&]() -> hipError_t {
+        } else if (Mt <= 8 && m->down_tiled[l] && down_mfma_supported(dn->dtype, F, D, Mt)) {
+            auto small = [&]() -> hipError_t {
                 int S = 0;
-                for (int64_t c0 = 0; c0 < Mt; c0 += 8) {
-                    const int64_t mc = Mt - c0 < 8 ? Mt - c0 : 8;
-                    float* pc = m->downpart + (S ? (c0 / 8) * (int64_t)S * 8 * D : 0);
-                    hipError_t e = launch_down_mfma(st, dn->dtype, m->down_tiled[l], F, D,
-                                                    m->h + c0 * F, F, mc, m->x + c0 * D, D, pc,
-                                                    ctx->cu_count, &S);
-                    if (e != hipSuccess) return e;
-                }
-                return launch_part_reduce(st, m->downpart, S, D, Mt, m->x, D);
+                hipError_t e = launch_down_mfma(st, dn->dtype, m->down_tiled[l], F, D, m->h, F, Mt,
+                                                m->x, D, m->downpart, ctx->cu_count, &S);
+                return e != hipSuccess ? e
+                                       : launch_part_reduce(st, m->downpart, S, D, Mt, m->x, D);
             };
-            TRACED_L(TK_DOWN, down_b, chunks());
+            TRACED_L(TK_DOWN, down_b, small());
+        } else if (axpy_supported(dn->dtype, D)) {
+            // from the stored rows; its partials added into x by the next
+            // prep where that can (rows of at most 16384 in whole blocks)
+            TRACED_L(TK_DOWN, down_b,
+                     launch_axpy(st, dn->data, dn->dtype, dn->row_bytes, F, D, m->h, F, Mt, m->x, D,
+                                 m->mm_part, m->mm_part_n, ctx->cu_count,
+                                 D % 256 == 0 && D <= 16384 ? &xpend : nullptr));
         } else {
             TRACED_L(TK_DOWN, down_b,
                      launch_down(st, dn->data, dn->dtype, dn->row_bytes, F, D, m->h, F, Mt, m->x,
@@ -860,7 +863,7 @@ int ftx_model_create(ftx_ctx* ctx, const ftx_model_desc* d, ftx_model** out) {
     if (ok && any_tiled) {
         size_t pf = 0;
         for (int dt : {FTX_Q4_K, FTX_Q6_K})
-            pf = std::max(pf, down_mfma_part_floats(dt, d->n_ff, D, Mmax, ctx->cu_count));
+            pf = std::max(pf, down_mfma_part_floats(dt, d->n_ff, D, 8, ctx->cu_count));
         ok = dalloc(&m->downpart, pf);
     }
     // row-dot projections and the LM head: tiled copies for the MFMA kernel
@@ -1494,24 +1497,11 @@ int ftx_verify_step(ftx_ctx* ctx, ftx_model* m, ftx_kv* kv, const ftx_verify_arg
             TRACED_IDEM(TK_DOWN, down_b,
                         launch_down_mfma(st, T[FTX_T_DOWN]->dtype, m->down_tiled[l], F, D, m->h,
                                          F, M, m->x, D, m->downpart, ctx->cu_count, &fold_S));
-        } else if (m->down_tiled[l] && down_mfma_supported(T[FTX_T_DOWN]->dtype, F, D, 8)) {
-            // more than 8 tokens: the MFMA down kernel on 8-row chunks, every
-            // chunk's split partials added into x by one reduce
-            auto chunks = [&]() -> hipError_t {
-                int S = 0;
-                for (int64_t c0 = 0; c0 < M; c0 += 8) {
-                    const int64_t mc = M - c0 < 8 ? M - c0 : 8;
-                    // chunk c's partials at downpart + c * S * 8 * D (S is the
-                    // same for every chunk: it depends on the shape only)
-                    float* pc = m->downpart + (S ? (c0 / 8) * (int64_t)S * 8 * D : 0);
-                    hipError_t e = launch_down_mfma(st, T[FTX_T_DOWN]->dtype, m->down_tiled[l], F,
-                                                    D, m->h + c0 * F, F, mc, m->x + c0 * D, D, pc,
-                                                    ctx->cu_count, &S);
-                    if (e != hipSuccess) return e;
-                }
-                return launch_part_reduce(st, m->downpart, S, D, M, m->x, D);
-            };
-            TRACED(TK_DOWN, down_b, chunks());
+        } else if (axpy_supported(T[FTX_T_DOWN]->dtype, D)) {
+            TRACED(TK_DOWN, down_b,
+                   launch_axpy(st, T[FTX_T_DOWN]->data, T[FTX_T_DOWN]->dtype,
+                               T[FTX_T_DOWN]->row_bytes, F, D, m->h, F, M, m->x, D, m->part,
+                               m->part_floats, ctx->cu_count));
         } else {
             TRACED(TK_DOWN, down_b,
                    launch_down(st, T[FTX_T_DOWN]->data, T[FTX_T_DOWN]->dtype,
