@@ -177,20 +177,20 @@ struct GemvSeg {
     int rpt = 0;
 };
 enum { EPI_STORE = 0, EPI_ACCUM = 1 };
-// planar Q8_0 / Q4_0 copies (scales, then quants; the generic kernels read
-// them through dq8): the internal dtype for a tensor of ncols columns, or -1
-int planar_dtype(int dt, int64_t ncols);
-hipError_t launch_planar(hipStream_t st, const uint8_t* src, int dt, int64_t nrows, int64_t ncols,
-                         uint8_t* dst);
 // fp16_range: the activations and dequantised weights lie within the fp16
-// range, so the MFMA form (fp16 hi + lo operands) may run
+// range, so the MFMA form (fp16 hi + lo operands) may run.  normw: the
+// RMSNorm (weights normw, eps) of x is part of the launch; only where
+// gemv_norm_ok says so.
+bool gemv_norm_ok(const GemvSeg* segs, int nseg, int64_t K, int64_t M);
 hipError_t launch_gemv(hipStream_t st, const GemvSeg* segs, int nseg, const float* x,
-                       int64_t ldx, int64_t K, int64_t M, int epi, bool fp16_range = false);
+                       int64_t ldx, int64_t K, int64_t M, int epi, bool fp16_range = false,
+                       const float* normw = nullptr, float eps = 0.f);
 // gate/up pair with SwiGLU epilogue: h[m*ldh + n] = silu(x.g_n) * (x.u_n)
 hipError_t launch_gemv_swiglu(hipStream_t st, const uint8_t* Wg, const uint8_t* Wu, int dt,
                               int64_t row_bytes, int64_t N, const float* x, int64_t ldx,
                               int64_t K, int64_t M, float* h, int64_t ldh,
-                              bool fp16_range = false);
+                              bool fp16_range = false, const float* normw = nullptr,
+                              float eps = 0.f);
 // y[m*ldy + j] += sum_i h[m*ldh + i] W[i, j] (W n_in rows x N cols)
 // uses `part` scratch of down_scratch_floats(...) floats
 size_t down_scratch_floats(int64_t M, int64_t n_in, int64_t N);
@@ -304,6 +304,13 @@ hipError_t launch_mm_prep_fold(hipStream_t st, float* x, int64_t ldx, const floa
                                const MmPend& fold);
 // the partials `fold` added into y rows < M (a reduce launch)
 hipError_t launch_mm_fold(hipStream_t st, const MmPend& fold, int64_t M, float* y, int64_t ldy);
+// a backend operation y[m][n] = sum_k x[m][k] W[n][k] (SwiGLU: two segments)
+// on the one-pass GEMM over rows as they are stored (segments with rpt 0 and
+// row_bytes), any fp32 x; ws of mm_op_bytes(), cols = the segments' rows
+bool mm_op_supported(int dt, int64_t M, int64_t K, int64_t N, int64_t row_bytes);
+size_t mm_op_bytes(int64_t M, int64_t K, int64_t cols, int epi, int cu_count);
+hipError_t launch_mm_op(hipStream_t st, const MmSeg* segs, int nseg, const float* x, int64_t ldx,
+                        int64_t K, int64_t M, int epi, float* y, int64_t ldy, void* ws, int cu_count);
 // y[m][j] += sum_i h[m][i] W[i][j] over the stored rows (k_axpy.hip: Q4_0,
 // Q8_0, Q4_K, Q6_K of whole blocks), any M and any h.  Split partials go to
 // `part` (at most part_floats) and are added into y by a reduce launch, or

@@ -3,9 +3,10 @@
 // Row-dot form (y = x W^T, blocks along the contraction) follows
 // CpuBackend::matmul (src/cpu_backend.cpp:90-104) with y[m*N + n] per row;
 // column-axpy form (y += h W, blocks along the output) follows
-// matmul_down_axpy (src/cpu_backend.cpp:60-75).  These are the general
-// paths for every dtype; the MFMA kernels in k_mfma.hip take over the hot
-// dtypes at small M.
+// matmul_down_axpy (src/cpu_backend.cpp:60-75).  k_rows takes up to 8 rows of
+// Q8_0 / Q4_0 / F16 / F32 weights; the others are the general paths for every
+// dtype and shape that the kernels of k_mfma.hip, k_gemm.hip and k_axpy.hip do
+// not take.
 #include "ftx_internal.h"
 #include "quant_dev.h"
 
@@ -116,6 +117,268 @@ __global__ void __launch_bounds__(256) k_gemv_swiglu(const uint8_t* __restrict__
             // src/engine.cpp:271-273: g / (1 + exp(-g)) * u
             h[(m0 + m) * ldh + n] = g / (1.f + expf(-g)) * au[m];
         }
+    }
+}
+
+// ---------------------------------------------------------------- few rows
+//
+// Row-dot form for up to 8 activation rows over the rows as they are stored
+// (Q8_0, Q4_0, F16, F32; K a whole number of blocks and of 8): a wave owns R
+// output rows (a SwiGLU pair: R gate rows and their up rows), a lane the 8
+// elements 8 g .. 8 g + 7 of the row for g = lane, lane + 64, ..: one load of
+// a lane's quants, whatever their alignment, covers 64 x 8 elements of a row
+// without a gap, and the activations are read once for all R rows.  The
+// next group's weights are in flight while one is multiplied.  With normw the
+// RMSNorm is part of it: every wave sees all of x, so it sums x^2 on the
+// way, multiplies x by the norm weights and the finished sums by 1 / rms
+// (src/engine.cpp:23-41).
+//
+// Bound by the weights' arrival; up to 8 rows the VALU (8 M multiply-adds and
+// about 20 decode instructions per 8 weights) stays below it.  Measured with
+// one token, Q8_0: gate / up 2 x 14336 x 4096 123 -> 36.9 us (3.4 TB/s; with
+// the separate norm launch before, 11.5 us more), head 32000 x 4096 104 (MFMA
+// form) -> 42.4 us (3.3 TB/s), o 4096 x 4096 37.7 -> 8.6 us.
+template <int DT>
+struct Row8 {
+    static constexpr int NQ = DT == FTX_Q8_0 ? 2 : DT == FTX_Q4_0 ? 1 : DT == FTX_F16 ? 4 : 8;
+    uint32_t q[NQ];
+    uint32_t d;
+};
+
+struct __attribute__((packed)) pk16 { uint16_t v; };
+struct __attribute__((packed)) pk32 { uint32_t v; };
+struct __attribute__((packed)) pk64 { uint32_t v[2]; };
+struct __attribute__((packed)) pk128 { uint32_t v[4]; };
+struct __attribute__((packed, aligned(4))) pkf4 { float v[4]; };
+
+template <int DT>
+__device__ __forceinline__ void row8_load(Row8<DT>& o, const uint8_t* __restrict__ row, int g) {
+    if constexpr (DT == FTX_Q8_0) {
+        const uint8_t* p = row + (uint32_t)((g >> 2) * 34);
+        o.d = ((const pk16*)p)->v;
+        const pk64 v = *(const pk64*)(p + 2 + 8 * (g & 3));
+        o.q[0] = v.v[0];
+        o.q[1] = v.v[1];
+    } else if constexpr (DT == FTX_Q4_0) {
+        const uint8_t* p = row + (uint32_t)((g >> 2) * 18);
+        o.d = ((const pk16*)p)->v;
+        o.q[0] = ((const pk32*)(p + 2 + 4 * (g & 3)))->v;
+    } else {
+        constexpr int NV = Row8<DT>::NQ / 4;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const pk128 v = *(const pk128*)(row + (uint32_t)g * 16 * NV + 16 * i);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) o.q[4 * i + k] = v.v[k];
+        }
+    }
+}
+
+// the values dq8 gives
+template <int DT>
+__device__ __forceinline__ void row8_dec(const Row8<DT>& o, float* w) {
+#pragma clang fp contract(off)
+    if constexpr (DT == FTX_Q8_0) {
+        const float d = h2f((uint16_t)o.d);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[i] = d * (float)(int8_t)(o.q[i >> 2] >> (8 * (i & 3)));
+    } else if constexpr (DT == FTX_Q4_0) {
+        const float d = h2f((uint16_t)o.d);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[i] = d * (float)((int)((o.q[0] >> (4 * i)) & 15) - 8);
+    } else if constexpr (DT == FTX_F16) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[i] = h2f((uint16_t)(o.q[i >> 1] >> (16 * (i & 1))));
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[i] = __uint_as_float(o.q[i]);
+    }
+}
+
+// v[0 .. n - 1] of every lane summed over the wave: lane l gets the sum of
+// v[l * n / 64] (n a power of two): halves exchanged until one value is left,
+// then the remaining lanes of its group
+template <int N>
+__device__ __forceinline__ float wave_sums(float* v, int lane) {
+    int o = 32;
+#pragma unroll
+    for (int n = N; n > 1; n >>= 1, o >>= 1) {
+        const bool up = (lane & o) != 0;
+#pragma unroll
+        for (int i = 0; i < n / 2; ++i) {
+            const float give = up ? v[i] : v[i + n / 2];
+            v[i] = (up ? v[i + n / 2] : v[i]) + __shfl_xor(give, o, 64);
+        }
+    }
+    float s = v[0];
+#pragma unroll
+    for (int k = 32 / N; k > 0; k >>= 1) s += __shfl_xor(s, k, 64);
+    return s;
+}
+
+template <int DT, int MC, int R, bool PAIR>
+__global__ void __launch_bounds__(256) k_rows(Segs segs, const float* __restrict__ x, int64_t ldx,
+                                              int K, int M, int epi,
+                                              const float* __restrict__ normw, float eps) {
+    constexpr int NW = PAIR ? 2 * R : R;  // weight rows
+    constexpr int U = MC == 1 ? 2 : 1;    // groups in flight together
+    const int lane = threadIdx.x & 63;
+    const int64_t m0 = (int64_t)blockIdx.y * MC;  // (more than 8 rows: chunks of 8)
+    x += m0 * ldx;
+    M = min(MC, M - (int)m0);
+    const int64_t total = PAIR ? segs.s[0].N : segs.start[segs.n];
+    const int64_t r0 = ((int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * R;
+    if (r0 >= total) return;
+    const uint8_t* wr[NW];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int64_t n = min(r0 + r, total - 1);
+        if constexpr (PAIR) {
+            wr[r] = segs.s[0].W + n * segs.s[0].row_bytes;
+            wr[R + r] = segs.s[1].W + n * segs.s[1].row_bytes;
+        } else {
+            const int si = n < segs.start[1] ? 0 : (n < segs.start[2] ? 1 : 2);
+            wr[r] = segs.s[si].W + (n - segs.start[si]) * segs.s[si].row_bytes;
+        }
+    }
+    const float* xr[MC];
+#pragma unroll
+    for (int m = 0; m < MC; ++m) xr[m] = x + (int64_t)min(m, M - 1) * ldx;
+    float acc[NW * MC], ss[MC];
+#pragma unroll
+    for (int i = 0; i < NW * MC; ++i) acc[i] = 0.f;
+#pragma unroll
+    for (int m = 0; m < MC; ++m) ss[m] = 0.f;
+    const int ng = K / 8;
+    auto mul = [&](int g, const Row8<DT>* rw) {
+        float xv[MC][8];
+#pragma unroll
+        for (int m = 0; m < MC; ++m) {
+            const pkf4 a = *(const pkf4*)(xr[m] + 8 * g), b = *(const pkf4*)(xr[m] + 8 * g + 4);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                xv[m][i] = a.v[i];
+                xv[m][4 + i] = b.v[i];
+            }
+        }
+        if (normw) {  // uniform
+            const pkf4 a = *(const pkf4*)(normw + 8 * g), b = *(const pkf4*)(normw + 8 * g + 4);
+#pragma unroll
+            for (int m = 0; m < MC; ++m)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    ss[m] += xv[m][i] * xv[m][i];
+                    xv[m][i] *= i < 4 ? a.v[i & 3] : b.v[i & 3];
+                }
+        }
+#pragma unroll
+        for (int r = 0; r < NW; ++r) {
+            float w[8];
+            row8_dec<DT>(rw[r], w);
+#pragma unroll
+            for (int m = 0; m < MC; ++m) {
+                float s = 0.f;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) s += xv[m][i] * w[i];
+                acc[r * MC + m] += s;
+            }
+        }
+    };
+    Row8<DT> rw[U][NW];
+    auto fetch = [&](int g) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int r = 0; r < NW; ++r) row8_load<DT>(rw[u][r], wr[r], min(g + 64 * u, ng - 1));
+    };
+    fetch(lane);
+    int g = lane;
+    // whole strides of all lanes, then the rest by lane
+    for (; g - lane + 64 * U <= ng; g += 64 * U) {
+        Row8<DT> cur[U][NW];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int r = 0; r < NW; ++r) cur[u][r] = rw[u][r];
+        fetch(g + 64 * U);
+#pragma unroll
+        for (int u = 0; u < U; ++u) mul(g + 64 * u, cur[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (g + 64 * u < ng) mul(g + 64 * u, rw[u]);
+    // lane l holds the sum of weight row l / (64 / NW) ..: value l * (NW MC) / 64
+    constexpr int NV = NW * MC, PER = 64 / NV;
+    const float v = wave_sums<NV>(acc, lane);
+    float sq = 0.f;
+    if (normw) {
+        sq = wave_sums<MC>(ss, lane);
+        // the lane's activation row is value index % MC
+        const int m = (lane / PER) % MC;
+        sq = __shfl(sq, m * (64 / MC), 64);
+    }
+    const int idx = lane / PER, r = idx / MC, m = idx % MC;
+    float o = normw ? v * (1.f / sqrtf(sq / (float)K + eps)) : v;
+    float up = 0.f;
+    if constexpr (PAIR) up = __shfl(o, (lane + 32) & 63, 64);  // the up rows' lanes are the upper half
+    if (lane % PER || m >= M) return;
+    if constexpr (PAIR) {
+        const int64_t n = r0 + r;
+        if (r >= R || n >= total) return;
+        // src/engine.cpp:271-273: g / (1 + exp(-g)) * u
+        segs.s[0].y[(m0 + m) * segs.s[0].ldy + n] = o / (1.f + expf(-o)) * up;
+    } else {
+        const int64_t n = r0 + r;
+        if (n >= total) return;
+        const int si = n < segs.start[1] ? 0 : (n < segs.start[2] ? 1 : 2);
+        float* yp = segs.s[si].y + (m0 + m) * segs.s[si].ldy + (n - segs.start[si]);
+        *yp = epi == EPI_ACCUM ? *yp + o : o;
+    }
+}
+
+// the stored types it takes, in whole blocks and 8-element groups
+bool rows_ok(int dt, int64_t K, int64_t M) {
+    const int64_t step = dt == FTX_Q8_0 || dt == FTX_Q4_0 ? 32 : (dt == FTX_F16 || dt == FTX_F32 ? 8 : 0);
+    return step > 0 && M >= 1 && M <= 8 * 65535 && K >= step && K % step == 0 && K < (1 << 28);
+}
+
+template <int DT, int MC>
+hipError_t rows_launch(hipStream_t st, const Segs& s, int64_t rows, bool pair, const float* x,
+                       int64_t ldx, int64_t K, int64_t M, int epi, const float* normw, float eps) {
+    // rows per wave: 4 (a pair: 2 + 2) once that leaves two waves per SIMD
+    // (2048), else one: more rows share the activations' loads, fewer leave
+    // the chip idle
+    const int R = pair ? (rows >= 4096 ? 2 : 1) : (rows >= 8192 ? 4 : 1);
+    const dim3 grid((unsigned)((rows + 4 * R - 1) / (4 * R)), (unsigned)((M + MC - 1) / MC)), block(256);
+#define ROWS_GO(RR, PP)                                                                        \
+    hipLaunchKernelGGL((k_rows<DT, MC, RR, PP>), grid, block, 0, st, s, x, ldx, (int)K, (int)M, \
+                       epi, normw, eps)
+    if (pair && R == 2) ROWS_GO(2, true);
+    else if (pair) ROWS_GO(1, true);
+    else if (R == 4) ROWS_GO(4, false);
+    else ROWS_GO(1, false);
+#undef ROWS_GO
+    return hipGetLastError();
+}
+
+template <int DT>
+hipError_t rows_launch_m(hipStream_t st, const Segs& s, int64_t rows, bool pair, const float* x,
+                         int64_t ldx, int64_t K, int64_t M, int epi, const float* normw, float eps) {
+    return M == 1   ? rows_launch<DT, 1>(st, s, rows, pair, x, ldx, K, M, epi, normw, eps)
+           : M == 2 ? rows_launch<DT, 2>(st, s, rows, pair, x, ldx, K, M, epi, normw, eps)
+           : M <= 4 ? rows_launch<DT, 4>(st, s, rows, pair, x, ldx, K, M, epi, normw, eps)
+                    : rows_launch<DT, 8>(st, s, rows, pair, x, ldx, K, M, epi, normw, eps);
+}
+
+// segments: two (gate, up) for a pair
+hipError_t launch_rows(hipStream_t st, const Segs& s, int64_t rows, bool pair, const float* x,
+                       int64_t ldx, int64_t K, int64_t M, int epi, const float* normw, float eps) {
+    switch (s.s[0].dt) {
+        case FTX_Q8_0: return rows_launch_m<FTX_Q8_0>(st, s, rows, pair, x, ldx, K, M, epi, normw, eps);
+        case FTX_Q4_0: return rows_launch_m<FTX_Q4_0>(st, s, rows, pair, x, ldx, K, M, epi, normw, eps);
+        case FTX_F16: return rows_launch_m<FTX_F16>(st, s, rows, pair, x, ldx, K, M, epi, normw, eps);
+        case FTX_F32: return rows_launch_m<FTX_F32>(st, s, rows, pair, x, ldx, K, M, epi, normw, eps);
+        default: return hipErrorInvalidValue;
     }
 }
 
@@ -375,49 +638,52 @@ bool gemm_rows_ok(const float* x, int64_t ldx, int64_t K, int64_t M, int64_t row
            (M > 8 || rows >= 16384);
 }
 
-// planar copy of Q8_0 / Q4_0 rows: thread per (row, block)
-__global__ void __launch_bounds__(256) k_planar(const uint8_t* __restrict__ src, int64_t nrows,
-                                                int64_t nb, int qb, uint8_t* __restrict__ dst) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nrows * nb) return;
-    const int64_t r = t / nb, b = t % nb;
-    const int64_t rb = nb * (2 + qb);
-    const uint8_t* s = src + r * rb + b * (2 + qb);
-    uint8_t* d = dst + r * rb;
-    d[2 * b] = s[0];
-    d[2 * b + 1] = s[1];
-    for (int i = 0; i < qb; ++i) d[2 * nb + b * qb + i] = s[2 + i];
-}
-
 }  // namespace
 
-int planar_dtype(int dt, int64_t ncols) {
-    if (ncols % 128) return -1;
-    return dt == FTX_Q8_0 ? FTX_Q8_0_PLANAR : (dt == FTX_Q4_0 ? FTX_Q4_0_PLANAR : -1);
+bool gemv_norm_ok(const GemvSeg* segs, int nseg, int64_t K, int64_t M) {
+    bool ok = M <= 8;
+    for (int i = 0; i < nseg; ++i) ok = ok && rows_ok(segs[i].dt, K, M);
+    return ok;
 }
 
-hipError_t launch_planar(hipStream_t st, const uint8_t* src, int dt, int64_t nrows, int64_t ncols,
-                         uint8_t* dst) {
-    if (planar_dtype(dt, ncols) < 0) return hipErrorInvalidValue;
-    const int64_t nb = ncols / 32, total = nrows * nb;
-    const int qb = dt == FTX_Q8_0 ? 32 : 16;
-    hipLaunchKernelGGL(k_planar, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, src,
-                       nrows, nb, qb, dst);
-    return hipGetLastError();
-}
-
+// Which kernel: the MFMA form takes more than 8 rows of the model's own
+// activations in whole 512-element steps; k_rows what it can (measured, one
+// token: Q8_0 4096 x 4096 43 us on k_gemv_rows, 8.6 us here; 8
+// tokens of 14336 x 4096 0.87 ms there, 46 us here); k_gemv_rows the
+// rest (the K types, Q4_1 and BF16 of shapes that their own kernels do not
+// take, rows that end inside a block).
 hipError_t launch_gemv(hipStream_t st, const GemvSeg* segs, int nseg, const float* x,
-                       int64_t ldx, int64_t K, int64_t M, int epi, bool fp16_range) {
+                       int64_t ldx, int64_t K, int64_t M, int epi, bool fp16_range,
+                       const float* normw, float eps) {
     if (nseg < 1 || nseg > 3) return hipErrorInvalidValue;
     Segs s{};
     s.n = nseg;
     s.start[0] = 0;
+    bool rok = true, one_dt = true;
     for (int i = 0; i < nseg; ++i) {
         s.s[i] = segs[i];
         s.start[i + 1] = s.start[i] + segs[i].N;
+        rok = rok && rows_ok(segs[i].dt, K, M);
+        one_dt = one_dt && segs[i].dt == segs[0].dt;
     }
     const int64_t rows = s.start[nseg];
     if (rows == 0 || M == 0) return hipSuccess;
+    if (M > 8 && fp16_range && !normw && gemm_rows_ok(x, ldx, K, M, rows))
+        return launch_gemm_rows<false>(st, s, rows, x, ldx, K, M, epi);
+    if (rok && one_dt) return launch_rows(st, s, rows, false, x, ldx, K, M, epi, normw, eps);
+    if (rok) {  // one launch per segment
+        for (int i = 0; i < nseg; ++i) {
+            Segs t{};
+            t.n = 1;
+            t.s[0] = segs[i];
+            t.start[1] = segs[i].N;
+            const hipError_t e =
+                segs[i].N ? launch_rows(st, t, segs[i].N, false, x, ldx, K, M, epi, normw, eps) : hipSuccess;
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
+    if (normw) return hipErrorInvalidValue;
     if (fp16_range && gemm_rows_ok(x, ldx, K, M, rows))
         return launch_gemm_rows<false>(st, s, rows, x, ldx, K, M, epi);
     dim3 grid((unsigned)((rows + 3) / 4), (unsigned)((M + MT - 1) / MT));
@@ -427,17 +693,20 @@ hipError_t launch_gemv(hipStream_t st, const GemvSeg* segs, int nseg, const floa
 
 hipError_t launch_gemv_swiglu(hipStream_t st, const uint8_t* Wg, const uint8_t* Wu, int dt,
                               int64_t row_bytes, int64_t N, const float* x, int64_t ldx,
-                              int64_t K, int64_t M, float* h, int64_t ldh, bool fp16_range) {
+                              int64_t K, int64_t M, float* h, int64_t ldh, bool fp16_range,
+                              const float* normw, float eps) {
     if (N == 0 || M == 0) return hipSuccess;
-    if (fp16_range && gemm_rows_ok(x, ldx, K, M, N)) {
-        Segs s{};
-        s.n = 2;
-        s.s[0] = GemvSeg{Wg, dt, row_bytes, N, h, ldh};
-        s.s[1] = GemvSeg{Wu, dt, row_bytes, N, nullptr, 0};
-        s.start[1] = N;
-        s.start[2] = 2 * N;
-        return launch_gemm_rows<true>(st, s, N, x, ldx, K, M, EPI_SWIGLU);
-    }
+    Segs s{};
+    s.n = 2;
+    s.s[0] = GemvSeg{Wg, dt, row_bytes, N, h, ldh};
+    s.s[1] = GemvSeg{Wu, dt, row_bytes, N, nullptr, 0};
+    s.start[1] = N;
+    s.start[2] = 2 * N;
+    const bool gemm = fp16_range && !normw && gemm_rows_ok(x, ldx, K, M, N);
+    if (M > 8 && gemm) return launch_gemm_rows<true>(st, s, N, x, ldx, K, M, EPI_SWIGLU);
+    if (rows_ok(dt, K, M)) return launch_rows(st, s, N, true, x, ldx, K, M, EPI_SWIGLU, normw, eps);
+    if (normw) return hipErrorInvalidValue;
+    if (gemm) return launch_gemm_rows<true>(st, s, N, x, ldx, K, M, EPI_SWIGLU);
     dim3 grid((unsigned)((N + 3) / 4), (unsigned)((M + MT - 1) / MT));
     hipLaunchKernelGGL(k_gemv_swiglu, grid, dim3(256), 0, st, Wg, Wu, dt, row_bytes, N, x, ldx,
                        K, M, h, ldh);

@@ -43,10 +43,6 @@ struct ftx_model {
     // tensor] and the LM head last (null where the kernel does not apply)
     std::vector<uint8_t*> mvt;
     std::vector<int> mvt_rpt;
-    // planar copies of Q8_0 / Q4_0 projections for the generic kernels (same
-    // indexing; null where they do not apply) and their internal dtypes
-    std::vector<uint8_t*> pln;
-    std::vector<int> pln_dt;
     // the one-pass GEMM's re-tiled copies of Q8_0 / Q4_0 projections (same
     // indexing; null where they do not apply) and their internal dtypes
     std::vector<uint8_t*> mmt;
@@ -149,8 +145,6 @@ static void model_release(ftx_model* m) {
     for (uint8_t* b : m->down_tiled)
         if (b) (void)hipFree(b);
     for (uint8_t* b : m->mvt)
-        if (b) (void)hipFree(b);
-    for (uint8_t* b : m->pln)
         if (b) (void)hipFree(b);
     for (uint8_t* b : m->mmt)
         if (b) (void)hipFree(b);
@@ -360,15 +354,11 @@ static int verify_large(ftx_ctx* ctx, ftx_model* m, const ftx_seq_args* sq, int6
             TRACED_L(kind, bytes, chunks());
             return FTX_OK;
         }
-        bool pl_all = true;
-        for (int i = 0; i < nseg; ++i) pl_all = pl_all && m->pln[idx[i]] != nullptr;
-        for (int i = 0; pl_all && i < nseg; ++i) {
-            gs[i].W = m->pln[idx[i]];
-            gs[i].dt = m->pln_dt[idx[i]];
-        }
+        // (the few-row kernel has the norm in it)
+        const float* nw = normw && gemv_norm_ok(gs, nseg, K, Mr) ? normw : nullptr;
         const float* src = xin;
         int64_t lds = ldx;
-        if (normw) {
+        if (normw && !nw) {
             TRACED_L(TK_RMSNORM, 2 * Mr * K * f4, launch_rmsnorm(st, xin, normw, K, Mr, eps, m->xn));
             src = m->xn;
             lds = K;
@@ -376,9 +366,9 @@ static int verify_large(ftx_ctx* ctx, ftx_model* m, const ftx_seq_args* sq, int6
         if (epi == EPI_SWIGLU)
             TRACED_L(kind, bytes,
                      launch_gemv_swiglu(st, gs[0].W, gs[1].W, gs[0].dt, gs[0].row_bytes, gs[0].N,
-                                        src, lds, K, Mr, gs[0].y, gs[0].ldy, true));
+                                        src, lds, K, Mr, gs[0].y, gs[0].ldy, true, nw, eps));
         else
-            TRACED_L(kind, bytes, launch_gemv(st, gs, nseg, src, lds, K, Mr, epi, true));
+            TRACED_L(kind, bytes, launch_gemv(st, gs, nseg, src, lds, K, Mr, epi, true, nw, eps));
         return FTX_OK;
     };
     auto seg = [](const ftx_tensor* t, float* y, int64_t ldy) {
@@ -890,28 +880,6 @@ int ftx_model_create(ftx_ctx* ctx, const ftx_model_desc* d, ftx_model** out) {
                            buf) != hipSuccess)
             ok = false;
     }
-    m->pln.assign(nmvt, nullptr);
-    m->pln_dt.assign(nmvt, -1);
-    for (size_t i = 0; ok && i < nmvt; ++i) {
-        const int t = (int)(i % FTX_LAYER_TENSORS);
-        const bool head = i + 1 == nmvt;
-        if (!head && t != FTX_T_Q && t != FTX_T_K && t != FTX_T_V && t != FTX_T_O &&
-            t != FTX_T_GATE && t != FTX_T_UP)
-            continue;
-        const ftx_tensor* w = head ? (d->output ? d->output : d->tok_embd) : d->layers[i];
-        if (!w) continue;
-        const int pdt = planar_dtype(w->dtype, w->ne[0]);
-        if (pdt < 0 || w->row_bytes * 32 != w->ne[0] * (w->dtype == FTX_Q8_0 ? 34 : 18)) continue;
-        uint8_t* buf = nullptr;
-        if (!dalloc(&buf, (size_t)(w->row_bytes * w->nrows))) {
-            ok = false;
-            break;
-        }
-        m->pln[i] = buf;
-        m->pln_dt[i] = pdt;
-        if (launch_planar(ctx->stream, w->data, w->dtype, w->nrows, w->ne[0], buf) != hipSuccess)
-            ok = false;
-    }
     m->mmt.assign(nmvt, nullptr);
     m->mmt_dt.assign(nmvt, -1);
     for (size_t i = 0; ok && i < nmvt; ++i) {
@@ -1377,16 +1345,11 @@ int ftx_verify_step(ftx_ctx* ctx, ftx_model* m, ftx_kv* kv, const ftx_verify_arg
             TRACED(kind, bytes, chunks());
             return FTX_OK;
         }
-        // the planar copies where every segment has one
-        bool pl_all = true;
-        for (int i = 0; i < nseg; ++i) pl_all = pl_all && m->pln[tix0 + tix[i]] != nullptr;
-        for (int i = 0; pl_all && i < nseg; ++i) {
-            segs[i].W = m->pln[tix0 + tix[i]];
-            segs[i].dt = m->pln_dt[tix0 + tix[i]];
-        }
+        // (the few-row kernel has the norm in it)
+        const float* nw = normw && gemv_norm_ok(segs, nseg, K, M) ? normw : nullptr;
         const float* src = xin;
         int64_t lds = ldx;
-        if (normw) {
+        if (normw && !nw) {
             TRACED(TK_RMSNORM, norm_b, launch_rmsnorm(st, xin, normw, K, M, eps, m->xn));
             src = m->xn;
             lds = K;
@@ -1394,9 +1357,9 @@ int ftx_verify_step(ftx_ctx* ctx, ftx_model* m, ftx_kv* kv, const ftx_verify_arg
         if (epi == EPI_SWIGLU)
             TRACED(kind, bytes,
                    launch_gemv_swiglu(st, segs[0].W, segs[1].W, segs[0].dt, segs[0].row_bytes,
-                                      segs[0].N, src, lds, K, M, segs[0].y, segs[0].ldy, true));
+                                      segs[0].N, src, lds, K, M, segs[0].y, segs[0].ldy, true, nw, eps));
         else
-            TRACED(kind, bytes, launch_gemv(st, segs, nseg, src, lds, K, M, epi, true));
+            TRACED(kind, bytes, launch_gemv(st, segs, nseg, src, lds, K, M, epi, true, nw, eps));
         return FTX_OK;
     };
     auto seg = [](const ftx_tensor* t, float* y, int64_t ldy) {
