@@ -1,10 +1,13 @@
 """GPU parity of the paths that long prefill chains, small steps of Q8_0 /
 Q4_0 models and the backend's single operations take, against the CPU oracle
 (models) and a float64 product (operations)."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import pyoracle as P
+from xwfes_amd import ftx
 from test_gpu_batch import LOGIT_TOL, random_tree, rel_err_rows, run_batch
 
 pytestmark = pytest.mark.gpu
@@ -41,12 +44,14 @@ def weight(gctx, orc, rng, dt, rows, cols):
     return gctx.upload(raw, dt, (cols, rows)), values.astype(np.float64)
 
 
-def close(got, want, terms):
-    """Sums of `terms` fp32 products in any order: each rounding is at most
-    2^-24 of a partial sum, which random signs keep near the result's size;
-    measured 2e-7 of the row's norm, 1e-6 is far from any misplaced operand."""
-    err = np.linalg.norm(got - want, axis=1) / np.maximum(np.linalg.norm(want, axis=1), 1e-30)
-    assert err.max() < 1e-6, (err.max(), terms)
+def close(got, want, size):
+    """|got - want| against `size`, the sum of the products' magnitudes: an
+    activation split in two fp16 halves is off by at most 2^-23 of itself
+    (three bf16 limbs: exact), and sums of blocks in fp32, in chains of some
+    20 additions at most, by 20 x 2^-24 of it at worst: 2^-19 together, 2^-20
+    asked for.  A misplaced operand moves a sum by about size / sqrt(terms)."""
+    err = np.abs(got - want) / np.maximum(size, 1e-300)
+    assert err.max() < 2.0 ** -20, err.max()
 
 
 @pytest.mark.parametrize("dt", [P.Q4_0, P.Q8_0, P.Q4_K, P.Q6_K])
@@ -63,7 +68,7 @@ def test_down_axpy_mfma(gctx, orc, dt, M, n_in, blocks):
     y0 = (rng.standard_normal((M, N)) * 0.1).astype(np.float32)
     got = gctx.down_axpy(x, t, y0)
     t.free()
-    close(got.astype(np.float64), y0 + x.astype(np.float64) @ w, n_in)
+    close(got, y0 + x.astype(np.float64) @ w, np.abs(y0) + np.abs(x.astype(np.float64)) @ np.abs(w))
 
 
 @pytest.mark.parametrize("dt", [P.Q4_0, P.Q8_0, P.Q4_K, P.Q6_K])
@@ -84,7 +89,110 @@ def test_down_axpy_special_values(gctx, orc, dt):
     w32 = w.astype(np.float32)
     with np.errstate(invalid="ignore", over="ignore"):
         want = (x[:, :, None] * w32[None]).astype(np.float64).sum(1)
-    for m in (0, 4, 5):
-        close(got[m:m + 1].astype(np.float64), want[m:m + 1], n_in)
+    keep = [0, 4, 5]
+    close(got[keep], want[keep], np.abs(x[keep].astype(np.float64)) @ np.abs(w))
     for m in (1, 2, 3):
         assert np.array_equal(got[m], want[m].astype(np.float32), equal_nan=True)
+
+
+@pytest.mark.parametrize("dt", [P.Q4_0, P.Q8_0, P.F16, P.F32])
+@pytest.mark.parametrize("M,K,N", [(1, 32, 1), (1, 544, 8195), (2, 1056, 37), (3, 512, 300),
+                                   (5, 64, 8192), (8, 2080, 66)])
+def test_matmul_few_rows(gctx, orc, dt, M, K, N):
+    """The few-row kernel: rows of part of a 64-lane stride, whole strides and
+    both; one and four output rows per wave, the last wave partly used; every
+    activation-row count it is built for and ones between."""
+    rng = np.random.default_rng(dt * 100 + M + K + N)
+    t, w = weight(gctx, orc, rng, dt, N, K)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    got = gctx.matmul(x, t)
+    t.free()
+    close(got, x.astype(np.float64) @ w.T, np.abs(x.astype(np.float64)) @ np.abs(w).T)
+
+
+@pytest.mark.parametrize("dt", [P.Q4_0, P.Q8_0, P.Q4_K, P.Q6_K, P.F16, P.F32])
+@pytest.mark.parametrize("M,K,N", [(9, 1, 1), (16, 3, 33), (17, 9, 257), (33, 8, 300), (70, 17, 64)])
+def test_matmul_many_rows(gctx, orc, dt, M, K, N):
+    """More than 8 rows (K in blocks of 32, or of 256 for the K types): the
+    edges of 16- and 32-token tiles, 32-row units and 256-element steps, one
+    split and several; rows scaled over the fp32 range keep their precision.
+    (F32 goes through the few-row kernel in chunks of 8.)"""
+    K *= 256 if dt in (P.Q4_K, P.Q6_K) else 32
+    rng = np.random.default_rng(dt * 100 + M + K + N)
+    t, w = weight(gctx, orc, rng, dt, N, K)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[1] *= np.float32(1e25)
+    x[2] *= np.float32(1e-30)
+    x[3, K // 2:] *= np.float32(1e-4)
+    x[4] = 0
+    got = gctx.matmul(x, t)
+    t.free()
+    assert not got[4].any()
+    close(got, x.astype(np.float64) @ w.T, np.abs(x.astype(np.float64)) @ np.abs(w).T)
+
+
+@pytest.mark.parametrize("dt,M", [(P.Q8_0, 4), (P.Q8_0, 12), (P.Q4_0, 12), (P.Q4_K, 12), (P.Q6_K, 12),
+                                  (P.F16, 12)])
+def test_matmul_special_values(gctx, orc, dt, M):
+    """Infinite and NaN activations give what a sum of fp32 products gives,
+    and leave the other rows alone."""
+    rng = np.random.default_rng(50 + dt)
+    K, N = 768, 70
+    t, w = weight(gctx, orc, rng, dt, N, K)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[1, 700] = np.inf
+    x[2, 3], x[2, 50] = np.inf, -np.inf
+    x[3, 69] = np.nan
+    got = gctx.matmul(x, t)
+    t.free()
+    with np.errstate(invalid="ignore"):
+        want = (x[:, None, :] * w.astype(np.float32)[None]).astype(np.float64).sum(2)
+    keep = [0] + list(range(4, M))
+    close(got[keep], want[keep], np.abs(x[keep].astype(np.float64)) @ np.abs(w).T)
+    for m in (1, 2, 3):
+        assert np.array_equal(got[m], want[m].astype(np.float32), equal_nan=True)
+
+
+@pytest.mark.parametrize("dt,M,K,IC", [(P.Q4_0, 1, 544, 70), (P.Q8_0, 3, 1024, 4100), (P.F16, 8, 64, 33),
+                                       (P.Q4_K, 2, 768, 40), (P.Q6_K, 9, 256, 70), (P.Q4_0, 40, 288, 33)])
+def test_expert_chunk_shapes(gctx, orc, dt, M, K, IC):
+    """Gate and up rows with SwiGLU through the few-row and the many-row
+    kernels, then the column-axpy of the result, added to `out`."""
+    rng = np.random.default_rng(dt + M + K + IC)
+    (g, wg), (u, wu), (d, wd) = (weight(gctx, orc, rng, dt, IC, K) for _ in range(3))
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    out = rng.standard_normal((M, K)).astype(np.float32)
+    # the rows' device size (Q6_K rows are padded to 16 bytes)
+    j = ftx.ExpertJob(x.ctypes.data, 0, g.ptr, u.ptr, d.ptr, dt, 0, M, K, IC, g.nbytes // IC, d.nbytes // IC)
+    got = out.copy()
+    j.out = got.ctypes.data
+    gctx.check(gctx.lib.ftx_expert_chunk(gctx.h, ctypes.byref(j)))
+    for t in (g, u, d):
+        t.free()
+    xg, xu = x.astype(np.float64) @ wg.T, x.astype(np.float64) @ wu.T
+    h = xg / (1 + np.exp(-xg)) * xu
+    # h itself is a product of two sums: each off by its own size
+    ax = np.abs(x.astype(np.float64))
+    ah = (ax @ np.abs(wg).T + 1) * (ax @ np.abs(wu).T)
+    close(got, out + h @ wd, np.abs(out) + ah @ np.abs(wd))
+
+
+@pytest.mark.parametrize("dts,d,ff", [("q8_0", 512, 1408), ("q4_0", 256, 544), ("f16", 128, 200),
+                                      ("mixed", 384, 512)])
+@pytest.mark.parametrize("M", [1, 3, 8])
+def test_small_steps_of_stored_types(gctx, orc, dts, d, ff, M):
+    """One to eight tokens through models whose projections run on the
+    few-row kernel with the RMSNorm in it (one type, and q / k / v of
+    different types) and whose ffn_down is Q8_0 / Q4_0 of whole and part
+    128-column groups, or F16 on the generic kernel."""
+    one = {"q8_0": P.Q8_0, "q4_0": P.Q4_0, "f16": P.F16, "mixed": P.Q8_0}[dts]
+    types = dict(tok_embd=P.F32, output=one, q=one, k=one, v=one, o=one, gate=one, up=one, down=one)
+    if dts == "mixed":
+        types.update(k=P.Q4_0, v=P.F16, o=P.Q4_0)
+    cfg = P.model_cfg(2, d, d // 64, max(d // 128, 1), 64, ff, 500, rope_theta=10000.0)
+    model = P.make_model(orc, cfg, types, seed=d + M)
+    toks = np.random.default_rng(M).integers(0, 500, M).tolist()
+    (got, want, kv, kvo), = run_batch(gctx, orc, model, [(toks, None, 21, 40)], 16)
+    assert rel_err_rows(got, want) < LOGIT_TOL
+    for a, b in zip(kv, kvo):
+        np.testing.assert_allclose(a.astype(np.float32), b.astype(np.float32), rtol=3e-3, atol=3e-3)

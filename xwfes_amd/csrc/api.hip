@@ -345,6 +345,14 @@ int ftx_dequant(ftx_ctx* ctx, const ftx_tensor* W, float* out) {
     return FTX_OK;
 }
 
+// whether a row-dot operation takes the one-pass GEMM (three launches:
+// operand, GEMM, and the sum of its splits) instead of launch_gemv's kernels
+// (one launch; up to 8 tokens they read the weights once)
+static bool op_mm(int dt, int64_t M, int64_t K, int64_t N, int64_t row_bytes) {
+    const bool few = M <= 8 && dt != FTX_Q4_K && dt != FTX_Q6_K;
+    return !few && mm_op_supported(dt, M, K, N, row_bytes);
+}
+
 int ftx_matmul(ftx_ctx* ctx, const float* x, int64_t M, int64_t K, const ftx_tensor* W,
                float* y) {
     if (!ctx || !x || !W || !y) return ftx_fail(ctx, FTX_E_INVALID, "null argument");
@@ -355,12 +363,17 @@ int ftx_matmul(ftx_ctx* ctx, const float* x, int64_t M, int64_t K, const ftx_ten
     Staged s{};
     float* extra;
     const bool mv = mv_supported(W->dtype, K, M);
+    const bool mm = !mv && op_mm(W->dtype, M, K, N, W->row_bytes);
     const size_t xqf = (xq_bytes(K) + 255) / 4;
-    const size_t mvf = mv ? xqf : 0;
-    int rc = stage_xy(ctx, x, (size_t)(M * K), y, (size_t)(M * N), false, mvf, s, &extra);
+    const size_t ef = mv ? xqf : (mm ? mm_op_bytes(M, K, N, EPI_STORE, ctx->cu_count) / 4 + 64 : 0);
+    int rc = stage_xy(ctx, x, (size_t)(M * K), y, (size_t)(M * N), false, ef, s, &extra);
     if (rc) return rc;
     GemvSeg seg{W->data, W->dtype, W->row_bytes, N, s.y, N};
-    if (mv) {
+    if (mm) {
+        const MmSeg ms{W->data, W->dtype, N, 0, W->row_bytes};
+        FTX_HIP(ctx, launch_mm_op(ctx->stream, &ms, 1, s.x, K, K, M, EPI_STORE, s.y, N, extra,
+                                  ctx->cu_count));
+    } else if (mv) {
         int8_t* xq = (int8_t*)extra;
         FTX_HIP(ctx, launch_xq_prep(ctx->stream, const_cast<float*>(s.x), K, nullptr, nullptr, 0, 0,
                                     K, M, xq));
@@ -458,13 +471,23 @@ int ftx_expert_chunk(ftx_ctx* ctx, const ftx_expert_job* j) {
     Staged s{};
     float* extra;
     const size_t pf = down_part_floats(ctx, j->dt, M, IC, K);
+    // h, then one block for the gate / up launch and after it the down one
+    const bool mm = op_mm(j->dt, M, K, 2 * IC, rb);
+    const size_t gf = mm ? mm_op_bytes(M, K, 2 * IC, EPI_SWIGLU, ctx->cu_count) / 4 + 64 : 0;
     int rc = stage_xy(ctx, j->x, (size_t)(M * K), j->out, (size_t)(M * K), true,
-                      pf + (size_t)(M * IC) + 64, s, &extra);
+                      (pf > gf ? pf : gf) + (size_t)(M * IC) + 64, s, &extra);
     if (rc) return rc;
     float* h = extra;
     float* part = extra + (((size_t)(M * IC) + 63) & ~(size_t)63);
-    FTX_HIP(ctx, launch_gemv_swiglu(ctx->stream, (const uint8_t*)j->gate, (const uint8_t*)j->up,
-                                    j->dt, rb, IC, s.x, K, K, M, h, IC));
+    if (mm) {
+        const MmSeg ms[2] = {{(const uint8_t*)j->gate, j->dt, IC, 0, rb},
+                             {(const uint8_t*)j->up, j->dt, IC, 0, rb}};
+        FTX_HIP(ctx, launch_mm_op(ctx->stream, ms, 2, s.x, K, K, M, EPI_SWIGLU, h, IC, part,
+                                  ctx->cu_count));
+    } else {
+        FTX_HIP(ctx, launch_gemv_swiglu(ctx->stream, (const uint8_t*)j->gate, (const uint8_t*)j->up,
+                                        j->dt, rb, IC, s.x, K, K, M, h, IC));
+    }
     FTX_HIP(ctx, down(ctx, (const uint8_t*)j->down, j->dt, rb, IC, K, h, M, s.y, part, pf));
     if (s.y_host)
         FTX_HIP(ctx, hipMemcpyAsync(j->out, s.y, (size_t)(M * K) * sizeof(float),

@@ -32,8 +32,8 @@
 // Measured, one launch (before: the generic kernel, or Q6_K's 8-token chunks):
 // Q8_0 14336 x 4096, 1 token 795 -> 25.6 us (2.4 TB/s); Q4_0, 24 tokens 2013 ->
 // 35.9 us; Q6_K, 256 tokens 531 -> 214 us (140 TFLOP/s); Q4_0 1408 x 512, 1
-// token 30.8 -> 7 us.  Error against 64 bits 1.2e-7 to 1.7e-7 where the fp32
-// sums of the generic kernel had 2.9e-7 to 5.7e-7.
+// token 30.8 -> 5.8 us.  Error against 64 bits 0.8e-7 to 1.4e-7 (1000 to 14336
+// rows) where the fp32 sums of the generic kernel had 1.6e-7 to 5.7e-7.
 #include "ftx_internal.h"
 #include "quant_dev.h"
 
@@ -157,6 +157,9 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
     const int64_t nsl = (a.n_in + 31) / 32;
     const int64_t I0 = (int64_t)ks * a.slices_per_split;
     const int64_t I1 = min(I0 + (int64_t)a.slices_per_split, nsl);
+    // The MFMA rounds its sums down (toward minus infinity): odd waves form
+    // theirs negated, so that the shares cancel in the waves' sum
+    const float sgn = (w & 1) ? -1.f : 1.f;
     uint2* cols = (uint2*)(lds + w * WB);
     float* scl = (float*)(lds + w * WB + C::TILES * 512);  // [NSC][kq][8]
 
@@ -245,7 +248,7 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
         // scales of row 8 kq + c % 8
         const int at = kq * 8 + (c & 7), hf = c >> 3;
         if constexpr (DT == FTX_Q4_K) {
-            const float d = h2f((uint16_t)(o.s[0] & 0xFFFF)), dmin = h2f((uint16_t)(o.s[0] >> 16));
+            const float d = sgn * h2f((uint16_t)(o.s[0] & 0xFFFF)), dmin = sgn * h2f((uint16_t)(o.s[0] >> 16));
             // sub-blocks 4 h .. 4 h + 3 of the row's super-block; this lane
             // takes two of them
             const bool up = ((j0 / 128) & 1) != 0;
@@ -261,13 +264,13 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
                 scl[(4 + 2 * hf + i) * 32 + at] = dmin * (float)((mn >> sh) & 0xFF) - 8.f * ds;
             }
         } else if constexpr (DT == FTX_Q6_K) {
-            const float d = h2f((uint16_t)o.s[1]);
+            const float d = sgn * h2f((uint16_t)o.s[1]);
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 scl[(4 * hf + i) * 32 + at] = d * (float)(int8_t)(o.s[0] >> (8 * i));
         } else {
-            scl[hf * 32 + at] = h2f((uint16_t)o.s[0]);
-            scl[(2 + hf) * 32 + at] = h2f((uint16_t)o.s[1]);
+            scl[hf * 32 + at] = sgn * h2f((uint16_t)o.s[0]);
+            scl[(2 + hf) * 32 + at] = sgn * h2f((uint16_t)o.s[1]);
         }
     };
     // h of the lane's token (past M: the last one's, never stored) in each
@@ -418,7 +421,10 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
         __syncthreads();
         v4f s = red[w * 64 + lane];
 #pragma unroll
-        for (int k = 1; k < AX_WAVES; ++k) s += red[(k * 8 + w) * 64 + lane];
+        for (int k = 1; k < AX_WAVES; ++k) {
+            const v4f v = red[(k * 8 + w) * 64 + lane];
+            s = (k & 1) ? s - v : s + v;
+        }
         if (col >= a.N) continue;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {

@@ -30,6 +30,15 @@
 // reduce launch adds in split order with the epilogue (store, accumulate,
 // SwiGLU).
 //
+// The backend's single operations (launch_mm_op: ftx_matmul, ftx_expert_chunk)
+// run the same kernel over rows as they are stored and any fp32 activations
+// (scaled per row by a power of two, k_mm_prep_op); their sums are kept
+// tighter than the steps' (64-bit additions, alternating signs against the
+// MFMA's rounding): 0.7e-7 to 0.9e-7 against 64 bits where the generic
+// kernel's fp32 sums had 0.8e-7 to 1.0e-7.  Measured (whole call): 48 tokens of
+// Q4_K 14336 x 4096 4.70 ms on the generic kernel -> 66 us; 16 tokens of Q8_0
+// 4096 x 4096 473 -> 50 us.
+//
 // Column-axpy form (ffn_down in the reference orientation, n_ff rows of
 // n_embd columns, Q4_K blocks along the output): per 32-row slice the
 // workgroup (one 256-column block) stages h*d and h*dmin of its rows as
@@ -40,6 +49,8 @@
 #include "quant_dev.h"
 
 namespace {
+
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 constexpr int MM_TOK = 64;              // tokens per workgroup tile
 constexpr int MM_MS = MM_TOK / 16;      // 16-token MFMA tiles
@@ -306,6 +317,83 @@ __global__ void __launch_bounds__(1024) k_mm_prep_row(float* __restrict__ x, int
     }
 }
 
+// The operand of a backend operation: rows of any fp32 values (rows m < M;
+// elements past K up to the contraction's padded length Kp are zeros).  Row m
+// is scaled by the power of two that brings its largest finite value into
+// [2^9, 2^10), so that the hi and lo halves carry 22 bits of every element
+// down to 2^-13 of that value (and 2^-35 of it below) and the 32-element sums
+// stay finite; rscale[m] undoes it.  Workgroup = row m.
+__global__ void __launch_bounds__(512) k_mm_prep_op(const float* __restrict__ x, int64_t ldx,
+                                                    int64_t K, int64_t Kp, int inter,
+                                                    _Float16* __restrict__ xh, _Float16* __restrict__ xl,
+                                                    v8bf* __restrict__ xs, float* __restrict__ rscale) {
+#pragma clang fp contract(off)
+    struct __attribute__((packed, aligned(4))) f4 { float v[4]; };
+    __shared__ float red[8];
+    const int m = blockIdx.x, t = threadIdx.x;
+    const float* row = x + (int64_t)m * ldx;
+    float mx = 0.f;
+    for (int64_t k = 4 * t; k < K; k += 2048) {
+        const f4 u = *(const f4*)(row + k);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float b = fabsf(u.v[i]);
+            mx = b <= 3.402823466e38f ? fmaxf(mx, b) : mx;
+        }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    if ((t & 63) == 0) red[t >> 6] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 8; ++i) mx = fmaxf(mx, red[i]);
+    // 2^e with mx 2^e in [2^9, 2^10); both factors normal
+    int e = mx > 0.f ? 9 - ilogbf(mx) : 0;
+    e = min(max(e, -118), 126);
+    const float s = ldexpf(1.f, e);
+    if (t == 0) rscale[m] = ldexpf(1.f, -e);
+    for (int64_t k = 4 * t; k < Kp; k += 2048) {
+        float o[4] = {0.f, 0.f, 0.f, 0.f};
+        if (k < K) {  // whole 32-element blocks
+            const f4 u = *(const f4*)(row + k);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = u.v[i] * s;
+        }
+        _Float16 hv[4], lv[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) split_hl(o[i], hv[i], lv[i]);
+        if (!inter) {
+            const int64_t at = frag_at(m, k, Kp, false);
+            *(v4h*)(xh + at) = v4h{hv[0], hv[1], hv[2], hv[3]};
+            *(v4h*)(xl + at) = v4h{lv[0], lv[1], lv[2], lv[3]};
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int64_t at = frag_at(m, k + i, Kp, true);
+                xh[at] = hv[i];
+                xl[at] = lv[i];
+            }
+        }
+        float q = (o[0] + o[1]) + (o[2] + o[3]);
+        q += __shfl_xor(q, 1, 64);
+        q += __shfl_xor(q, 2, 64);
+        q += __shfl_xor(q, 4, 64);
+        if (xs && (t & 7) == 0) {
+            // Q4_K's min operand: lane (token, kq) of fragment (16-token tile,
+            // super-block, MFMA), element j = sub-block j's limb
+            const int j = (int)(k / 32 % 8);
+            const float h = __uint_as_float(__float_as_uint(q) & 0xFFFF0000u), r = q - h;
+            const float md = __uint_as_float(__float_as_uint(r) & 0xFFFF0000u), l = r - md;
+            __bf16* f = (__bf16*)(xs + ((int64_t)(m >> 4) * (Kp / 256) + k / 256) * 128 + (m & 15)) + j;
+            f[0 * 128] = f[1 * 128] = (__bf16)h;
+            f[2 * 128] = f[3 * 128] = (__bf16)md;
+            f[4 * 128] = (__bf16)h;
+            f[5 * 128] = (__bf16)l;
+            f[6 * 128] = f[7 * 128] = (__bf16)0.f;
+        }
+    }
+}
+
 // ---------------------------------------------------------------- row-dot
 
 struct MmSegDev {
@@ -345,7 +433,26 @@ struct MmArgs {
     const _Float16 *xh, *xl, *sh, *sl;  // fragment-order operands (k_mm_prep)
     int M;
     MmOutDev out;
+    // the backend's single operations (null otherwise): row m of the operand
+    // is row m of x times 1 / rscale[m], a power of two; a sum that comes out
+    // as NaN is formed again from x itself (k_mm_prep_op)
+    const float* rscale;
+    const float* x;
+    int64_t ldx;
+    int nblk;  // 32-element blocks of the contraction
 };
+
+// sum_k x[m][k] W[n][k], k0 <= k < k1, one fp32 product after the other
+__device__ float mm_redo(const MmArgs& a, const uint8_t* row, int dt, int64_t m, int64_t k0, int64_t k1) {
+    const float* x = a.x + m * a.ldx;
+    float v = 0.f;
+    for (int64_t k = k0; k < k1; k += 8) {
+        float q[8];
+        dq8(row, dt, k, (int64_t)a.nblk * 32, q);
+        for (int i = 0; i < 8; ++i) v += x[k + i] * q[i];
+    }
+    return v;
+}
 
 __device__ __forceinline__ int mm_seg_of(const MmArgs& a, int64_t u) {
     int si = 0;
@@ -377,6 +484,40 @@ struct MmW<FTX_Q6_K_MMT> {
     v4i sc[MM_NT];     // its row's 16 int8 sub-block scales
     uint32_t d[MM_NT]; // its row's fp16 super-block scale
 };
+
+// rows as they are stored (the backend's single operations, which have no
+// re-tiled copy): Q8_0 and Q4_0 blocks of 34 / 18 bytes, Q4_K, planar Q6_K
+// (quant_dev.h), F16
+constexpr int FTX_Q4_K_ROWS = 212;
+template <>
+struct MmW<FTX_Q4_K_ROWS> : MmW<FTX_Q4_K> {};
+template <>
+struct MmW<FTX_Q8_0> {
+    v2i q[MM_NT][8];       // the lane's 8 quant bytes of each 32-block
+    uint32_t d[MM_NT][8];  // the fp16 block scales
+};
+template <>
+struct MmW<FTX_Q4_0> {
+    uint32_t q[MM_NT][8];
+    uint32_t d[MM_NT][8];
+};
+template <>
+struct MmW<FTX_Q6_K> : MmW<FTX_Q6_K_MMT> {};
+template <>
+struct MmW<FTX_F16> {
+    v8h b[MM_NT][8];       // the operand itself
+};
+__host__ __device__ constexpr bool mm_stored(int dt) {
+    return dt == FTX_Q8_0 || dt == FTX_Q4_0 || dt == FTX_Q6_K || dt == FTX_F16 || dt == FTX_Q4_K_ROWS;
+}
+// Q6_K operands (tiled or stored): the same registers
+__host__ __device__ constexpr bool mm_q6k(int dt) { return dt == FTX_Q6_K_MMT || dt == FTX_Q6_K; }
+
+// loads of any alignment (the hardware takes them as they come)
+struct __attribute__((packed)) mm_u16 { uint16_t v; };
+struct __attribute__((packed)) mm_u32 { uint32_t v; };
+struct __attribute__((packed)) mm_u64 { v2i v; };
+struct __attribute__((packed)) mm_u128 { v4i v; };
 
 // the re-tiled Q8_0 / Q4_0 copy (k_mm_tile): per 16-row tile and 256-element
 // step, [lane 64][bytes of the lane's 8 blocks] then [row 16][8 fp16 scales].
@@ -411,6 +552,8 @@ struct MmPtr {
     uint32_t ld[MM_NT];          // Q6_K: its row's d
     uint32_t qstep;              // bytes per 256-element step
     uint32_t cstride;            // Q4_K: bytes from one 64-element chunk to the next
+    const uint8_t* base;         // stored rows
+    int nblk, nsb;               // stored rows: 32-element blocks, 256-element super-blocks
 };
 
 // Rows past N read the last tile's padding rows (the tiled copies hold whole
@@ -418,11 +561,24 @@ struct MmPtr {
 // discarded.  Segments are below 4 GB.
 template <int DT>
 __device__ __forceinline__ void mm_ptrs(MmPtr& p, const MmSegDev& sg, int64_t rbase, int nsb,
-                                        int col, int kq) {
+                                        int col, int kq, int nblk) {
     p.rs = mm_rsrc(sg.W);
+    p.base = sg.W;
+    p.nblk = nblk;
+    p.nsb = nsb;
 #pragma unroll
     for (int t = 0; t < MM_NT; ++t) {
-        if constexpr (DT == FTX_Q4_K) {
+        if constexpr (mm_stored(DT)) {
+            const uint32_t r = (uint32_t)(min(rbase + 16 * t + col, sg.N - 1) * sg.row_bytes);
+            p.tile[t] = 0;
+            p.lh[t] = r;
+            p.ld[t] = 0;
+            p.lq[t] = r + (DT == FTX_Q8_0 ? 2 + 8 * kq
+                           : DT == FTX_Q4_0 ? 2 + 4 * kq
+                           : DT == FTX_F16  ? 16 * kq
+                           : DT == FTX_Q4_K_ROWS ? 16 + 8 * kq
+                                            : 64 * (kq & 1) + 8 * (kq >> 1));
+        } else if constexpr (DT == FTX_Q4_K) {
             // rbase is a multiple of 32: row rbase + 16 t + col is row
             // (16 t + col) % R of tile (rbase + 16 t) / R
             const int R = sg.rpt;
@@ -444,8 +600,8 @@ __device__ __forceinline__ void mm_ptrs(MmPtr& p, const MmSegDev& sg, int64_t rb
         p.qstep = (uint32_t)(sg.rpt * 144);
         p.cstride = (uint32_t)(sg.rpt * 32);
     } else {
-        p.qstep = (uint32_t)mmt_step_bytes(DT);
-        p.cstride = 0;
+        p.qstep = DT == FTX_Q4_K_ROWS ? 144 : mm_stored(DT) ? 0 : (uint32_t)mmt_step_bytes(DT);
+        p.cstride = DT == FTX_Q4_K_ROWS ? 32 : 0;
     }
 }
 
@@ -461,7 +617,43 @@ __device__ __forceinline__ void mm_load(MmW<DT>& o, const MmPtr& p, int sb) {
 #pragma unroll
     for (int t = 0; t < MM_NT; ++t) {
         const uint32_t so = p.tile[t] + (uint32_t)sb * p.qstep;  // uniform
-        if constexpr (DT == FTX_Q4_K) {
+        if constexpr (DT == FTX_Q6_K) {
+            // planes QL [nsb][128], QH [nsb][64], SC [nsb][16], D [nsb][2] of
+            // the lane's row; ql run (h, a) of the lane at 32 h + 16 a
+            const uint8_t* b = p.base + (int64_t)sb * 128;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const v2i v = ((const mm_u64*)(b + 32 * (i >> 1) + 16 * (i & 1) + p.lq[t]))->v;
+                o.q[t][i >> 1][2 * (i & 1)] = v.x;
+                o.q[t][i >> 1][2 * (i & 1) + 1] = v.y;
+            }
+            // (qh: lane offset 32 (kq & 1) + 8 (kq >> 1))
+            const uint32_t qh = p.lh[t] + 32 * ((threadIdx.x >> 4) & 1) + 8 * ((threadIdx.x >> 5) & 1);
+            const uint8_t* bh = p.base + (int64_t)p.nsb * 128 + (int64_t)sb * 64;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const v2i v = ((const mm_u64*)(bh + 16 * i + qh))->v;
+                o.q[t][2][2 * i] = v.x;
+                o.q[t][2][2 * i + 1] = v.y;
+            }
+            o.sc[t] = ((const mm_u128*)(p.base + (int64_t)p.nsb * 192 + (int64_t)sb * 16 + p.lh[t]))->v;
+            o.d[t] = ((const mm_u16*)(p.base + (int64_t)p.nsb * 208 + (int64_t)sb * 2 + p.lh[t]))->v;
+        } else if constexpr (mm_stored(DT) && DT != FTX_Q4_K_ROWS) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                // (past the row's last block: that one again, against zeros)
+                const int64_t blk = min(8 * sb + j, p.nblk - 1);  // uniform
+                if constexpr (DT == FTX_Q8_0) {
+                    o.q[t][j] = ((const mm_u64*)(p.base + blk * 34 + p.lq[t]))->v;
+                    o.d[t][j] = ((const mm_u16*)(p.base + blk * 34 + p.lh[t]))->v;
+                } else if constexpr (DT == FTX_Q4_0) {
+                    o.q[t][j] = ((const mm_u32*)(p.base + blk * 18 + p.lq[t]))->v;
+                    o.d[t][j] = ((const mm_u16*)(p.base + blk * 18 + p.lh[t]))->v;
+                } else {
+                    o.b[t][j] = __builtin_bit_cast(v8h, ((const mm_u128*)(p.base + blk * 64 + p.lq[t]))->v);
+                }
+            }
+        } else if constexpr (DT == FTX_Q4_K || DT == FTX_Q4_K_ROWS) {
 #pragma unroll
             for (int c = 0; c < 4; ++c) o.qs[t][c] = mm_ld8(p.rs, p.lq[t], so + c * p.cstride);
             o.hdr[t] = mm_ld16(p.rs, p.lh[t], so);
@@ -495,6 +687,15 @@ __device__ __forceinline__ void bytes4_h(uint32_t w, v2h& lo, v2h& hi) {
 }
 
 typedef __attribute__((address_space(3))) void lds_void;
+
+template <bool D>
+struct MmAcc {
+    typedef v4f T;
+};
+template <>
+struct MmAcc<true> {
+    typedef double T __attribute__((ext_vector_type(4)));
+};
 
 // waves per SIMD the register allocation targets: two workgroups per CU for
 // Q4_0 16-row tiles (they fit 128 registers), one otherwise (the larger
@@ -550,7 +751,7 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
     const int sb1 = min(sb0 + a.sb_per_split, a.nsb);
     const int64_t nks = a.K / 32;
     MmPtr wp;
-    mm_ptrs<DT>(wp, sg, rbase, a.nsb, col, kq);
+    mm_ptrs<DT>(wp, sg, rbase, a.nsb, col, kq, a.nblk);
 
     // the step's 16 MS fragments: block b = (hl, ms, j) = 8 (MS hl + ms) + j
     // -> LDS offset b KB; wave w copies blocks BPW w .. BPW w + BPW - 1 (one
@@ -578,11 +779,14 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
     const uint32_t soff = (uint32_t)(mt0 * a.nsb * 32 * 4 * 2);  // bytes, uniform
     const uint32_t xlane = (uint32_t)(lane & 31) * 8;
 
-    v4f acc[MM_NT][MS];
+    // (the backend's operations: in 64 bits, added to once per four blocks)
+    typename MmAcc<mm_stored(DT)>::T acc[MM_NT][MS];
 #pragma unroll
     for (int t = 0; t < MM_NT; ++t)
 #pragma unroll
-        for (int ms = 0; ms < MS; ++ms) acc[t][ms] = v4f{0.f, 0.f, 0.f, 0.f};
+        for (int ms = 0; ms < MS; ++ms)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[t][ms][r] = 0.f;
     const v4f zero4 = {0.f, 0.f, 0.f, 0.f};
 
     // one 256-element step from LDS buffer `buf` with weights `wc`; the
@@ -639,6 +843,46 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
                 for (int i = 0; i < 4; ++i) scn[t][i] = scp[t][i] * v2h{(_Float16)(-1024.f), (_Float16)(-1024.f)};
             }
         }
+        // stored Q4_K: w = d sc (q - 8) - g, g = dmin m - 8 d sc; the g of the
+        // eight sub-blocks against the 32-element sums is two MFMAs of three
+        // bf16 limbs each (K slot 8 kq + j: sub-block j; first the limb pairs
+        // hh, hm, mh, mm of kq = 0 .. 3, then hl, lh)
+        float bsk[DT == FTX_Q4_K_ROWS ? MM_NT : 1][8];
+        if constexpr (DT == FTX_Q4_K_ROWS) {
+            const v8bf* xs = (const v8bf*)a.sh;
+#pragma unroll
+            for (int t = 0; t < MM_NT; ++t) {
+                const uint32_t S0 = wc.hdr[t].y, S1 = wc.hdr[t].z, S2 = wc.hdr[t].w;
+                const float d = h2f((uint16_t)((uint32_t)wc.hdr[t].x & 0xFFFF));
+                const float dmin = h2f((uint16_t)((uint32_t)wc.hdr[t].x >> 16));
+                const uint32_t sc[2] = {S0 & 0x3F3F3F3Fu, (S2 & 0x0F0F0F0Fu) | ((S0 >> 2) & 0x30303030u)};
+                const uint32_t mn[2] = {S1 & 0x3F3F3F3Fu, ((S2 >> 4) & 0x0F0F0F0Fu) | ((S1 >> 2) & 0x30303030u)};
+                v8bf g0, g1;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int h = 8 * (j & 3);
+                    bsk[t][j] = d * (float)((sc[j >> 2] >> h) & 0xFF);
+                    const float g = dmin * (float)((mn[j >> 2] >> h) & 0xFF) - 8.f * bsk[t][j];
+                    const float gh = __uint_as_float(__float_as_uint(g) & 0xFFFF0000u), r = g - gh;
+                    const float gm = __uint_as_float(__float_as_uint(r) & 0xFFFF0000u), gl = r - gm;
+                    g0[j] = (__bf16)((kq & 1) ? gm : gh);
+                    g1[j] = (__bf16)(kq == 0 ? gl : (kq == 1 ? gh : 0.f));
+                }
+#pragma unroll
+                for (int ms = 0; ms < MS; ++ms) {
+                    const v8bf* xp = xs + ((mt0 + ms) * a.nsb + sb) * 128 + lane;
+                    v4f mt = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xp[64], g1, zero4, 0, 0, 0);
+                    mt = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xp[0], g0, mt, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[t][ms][r] -= (double)mt[r];
+                }
+            }
+        }
+        float dq6[DT == FTX_Q6_K ? MM_NT : 1];
+        if constexpr (DT == FTX_Q6_K) {
+#pragma unroll
+            for (int t = 0; t < MM_NT; ++t) dq6[t] = h2f((uint16_t)wc.d[t]);
+        }
         v4f tmp[MM_NT][MS];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {  // 32-element K-step (sub-block / block) of the step
@@ -676,11 +920,32 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
                     for (int i = 0; i < 4; ++i) q[i] = __builtin_elementwise_fma(q[i], sc, sn);
                     bw[t] = v8h{q[0][0], q[0][1], q[1][0], q[1][1], q[2][0], q[2][1], q[3][0], q[3][1]};
                     bs[t] = 0.f;
+                } else if constexpr (DT == FTX_Q4_K_ROWS) {
+                    // (the nibbles of 8 consecutive bytes: bytes4_h's pairs)
+                    const v2i wv = wc.qs[t][j >> 1];
+                    const uint32_t x0 = ((uint32_t)wv.x >> (4 * (j & 1))) & 0x0F0F0F0Fu;
+                    const uint32_t x1 = ((uint32_t)wv.y >> (4 * (j & 1))) & 0x0F0F0F0Fu;
+                    const v2h o8 = {(_Float16)(-1032.f), (_Float16)(-1032.f)};
+                    const v2h h0 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(x0, 0x64646464u, 0x00050004u)) + o8;
+                    const v2h h1 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(x0, 0x64646464u, 0x00070006u)) + o8;
+                    const v2h h2 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(x1, 0x64646464u, 0x00050004u)) + o8;
+                    const v2h h3 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(x1, 0x64646464u, 0x00070006u)) + o8;
+                    bw[t] = v8h{h0[0], h0[1], h1[0], h1[1], h2[0], h2[1], h3[0], h3[1]};
+                    bs[t] = bsk[t][j];
+                } else if constexpr (DT == FTX_Q8_0) {
+                    bw[t] = i8x8(wc.q[t][j]);
+                    bs[t] = h2f((uint16_t)wc.d[t][j]);
+                } else if constexpr (DT == FTX_Q4_0) {
+                    bw[t] = nib8(wc.q[t][j], 8.f);
+                    bs[t] = h2f((uint16_t)wc.d[t][j]);
+                } else if constexpr (DT == FTX_F16) {
+                    bw[t] = wc.b[t][j];
+                    bs[t] = 0.f;
                 } else if constexpr (DT == FTX_Q8_0_MMT) {
                     const v4i qv = wc.q[t][j >> 1];
                     bw[t] = i8x8((j & 1) ? v2i{qv[2], qv[3]} : v2i{qv[0], qv[1]});
                     bs[t] = scale8(wc.d[t], j);
-                } else if constexpr (DT == FTX_Q6_K_MMT) {
+                } else if constexpr (mm_q6k(DT)) {
                     // elements 32 j + 8 kq .. + 7: half h, 32-group g of it;
                     // low nibbles from ql run 2 h + (g & 1) (high half of
                     // the byte for g >= 2), two high bits from qh run h
@@ -720,7 +985,55 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
                     bs[t] = scale8(wc.d[t], j);
                 }
             }
-            if constexpr (DT == FTX_Q4_K || DT == FTX_Q6_K_MMT) {
+            if constexpr (mm_stored(DT)) {
+                // the backend's operations: a fresh sum per 32 elements, the lo
+                // half first (its small terms are then rounded at their own
+                // size), added in fp32 with the block scale, four blocks to one
+                // 64-bit addition.  The MFMA rounds its sums down (toward
+                // minus infinity), so every other block is formed negated and
+                // subtracted: the shares cancel instead of adding up.
+                if (j & 1) {
+#pragma unroll
+                    for (int t = 0; t < MM_NT; ++t) {
+                        bw[t] = -bw[t];
+                        if constexpr (DT == FTX_Q6_K) bw2[t] = -bw2[t];
+                    }
+                }
+                v4f p[MM_NT][MS];
+#pragma unroll
+                for (int t = 0; t < MM_NT; ++t)
+#pragma unroll
+                    for (int ms = 0; ms < MS; ++ms)
+                        p[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[ms], bw[t], zero4, 0, 0, 0);
+                if constexpr (DT == FTX_Q6_K) {
+#pragma unroll
+                    for (int t = 0; t < MM_NT; ++t)
+#pragma unroll
+                        for (int ms = 0; ms < MS; ++ms) {
+                            p[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[ms], bw2[t], p[t][ms], 0, 0, 0);
+                            p[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[ms], bw2[t], p[t][ms], 0, 0, 0);
+                        }
+                }
+#pragma unroll
+                for (int t = 0; t < MM_NT; ++t)
+#pragma unroll
+                    for (int ms = 0; ms < MS; ++ms)
+                        p[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[ms], bw[t], p[t][ms], 0, 0, 0);
+#pragma unroll
+                for (int t = 0; t < MM_NT; ++t) {
+                    const float f0 = DT == FTX_F16 ? 1.f : (DT == FTX_Q6_K ? dq6[t] : bs[t]);
+                    const float f = (j & 1) ? -f0 : f0;
+#pragma unroll
+                    for (int ms = 0; ms < MS; ++ms) {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            tmp[t][ms][r] = j % 4 == 0 ? f * p[t][ms][r] : fmaf(f, p[t][ms][r], tmp[t][ms][r]);
+                        if (j % 4 == 3)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) acc[t][ms][r] += (double)tmp[t][ms][r];
+                    }
+                }
+            } else if constexpr (DT == FTX_Q4_K || DT == FTX_Q6_K_MMT) {
                 // hi parts of every tile first, then lo: no MFMA waits on the
                 // one before it
 #pragma unroll
@@ -837,7 +1150,14 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
                 const int64_t n = rbase + 16 * t + col;
                 if (n >= sg.N) continue;
                 float* yp = yrow + sg.col0 + n;
-                *yp = o.accum ? *yp + acc[t][ms][r] : acc[t][ms][r];
+                float v = (float)acc[t][ms][r];
+                if constexpr (mm_stored(DT)) {
+                    v *= a.rscale[m];
+                    if (v != v)
+                        v = mm_redo(a, sg.W + n * sg.row_bytes, DT == FTX_Q4_K_ROWS ? FTX_Q4_K : DT, m,
+                                    (int64_t)sb0 * 256, min((int64_t)sb1 * 256, (int64_t)a.nblk * 32));
+                }
+                *yp = o.accum ? *yp + v : v;
             }
         }
 }
@@ -1168,6 +1488,7 @@ struct MmReduceArgs {
     _Float16 *fh, *fl;
     float fscale;
     int64_t fK;
+    int wide;       // the backend's operations: the splits added in 64 bits
 };
 
 __global__ void __launch_bounds__(256) k_mm_reduce(MmReduceArgs a) {
@@ -1183,9 +1504,18 @@ __global__ void __launch_bounds__(256) k_mm_reduce(MmReduceArgs a) {
     if (valid) {
         const float* p = a.part + m * a.ldp + n;
         float g = 0.f, u = 0.f;
-        for (int s = 0; s < a.S; ++s) g += p[(int64_t)s * a.split_stride];
-        if (a.swiglu)
-            for (int s = 0; s < a.S; ++s) u += p[(int64_t)s * a.split_stride + a.N];
+        if (a.wide) {
+            double gd = 0., ud = 0.;
+            for (int s = 0; s < a.S; ++s) gd += p[(int64_t)s * a.split_stride];
+            if (a.swiglu)
+                for (int s = 0; s < a.S; ++s) ud += p[(int64_t)s * a.split_stride + a.N];
+            g = (float)gd;
+            u = (float)ud;
+        } else {
+            for (int s = 0; s < a.S; ++s) g += p[(int64_t)s * a.split_stride];
+            if (a.swiglu)
+                for (int s = 0; s < a.S; ++s) u += p[(int64_t)s * a.split_stride + a.N];
+        }
         v = a.swiglu ? g / (1.f + expf(-g)) * u : g;
     }
     if (a.fh) {
@@ -1207,27 +1537,28 @@ __global__ void __launch_bounds__(256) k_mm_reduce(MmReduceArgs a) {
 // The same for dense launches (no tile table, no fragment output) with every
 // row, split and output 16-byte aligned: four columns per thread, the same
 // sums in the same order.  grid = (ceil(N / 1024), M).
+template <typename F>
+__device__ __forceinline__ float4 mm_sum4(const float* p, int S, int64_t stride) {
+    F x = 0, y = 0, z = 0, w = 0;
+    for (int s = 0; s < S; ++s) {
+        const float4 t = *(const float4*)(p + (int64_t)s * stride);
+        x += t.x;
+        y += t.y;
+        z += t.z;
+        w += t.w;
+    }
+    return float4{(float)x, (float)y, (float)z, (float)w};
+}
+
 __global__ void __launch_bounds__(256) k_mm_reduce4(MmReduceArgs a) {
     const int64_t n = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
     const int64_t m = blockIdx.y;
     if (n >= a.N) return;
     const float* p = a.part + m * a.ldp + n;
-    float4 g = {0.f, 0.f, 0.f, 0.f}, u = {0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < a.S; ++s) {
-        const float4 t = *(const float4*)(p + (int64_t)s * a.split_stride);
-        g.x += t.x;
-        g.y += t.y;
-        g.z += t.z;
-        g.w += t.w;
-    }
+    float4 g = a.wide ? mm_sum4<double>(p, a.S, a.split_stride) : mm_sum4<float>(p, a.S, a.split_stride);
     if (a.swiglu) {
-        for (int s = 0; s < a.S; ++s) {
-            const float4 t = *(const float4*)(p + (int64_t)s * a.split_stride + a.N);
-            u.x += t.x;
-            u.y += t.y;
-            u.z += t.z;
-            u.w += t.w;
-        }
+        const float4 u = a.wide ? mm_sum4<double>(p + a.N, a.S, a.split_stride)
+                                : mm_sum4<float>(p + a.N, a.S, a.split_stride);
         g.x = g.x / (1.f + expf(-g.x)) * u.x;
         g.y = g.y / (1.f + expf(-g.y)) * u.y;
         g.z = g.z / (1.f + expf(-g.z)) * u.z;
@@ -1276,7 +1607,9 @@ static hipError_t launch_prep_row(hipStream_t st, float* x, int64_t ldx, const f
               : ch == 2 ? k_mm_prep_row<2>
               : ch == 3 ? k_mm_prep_row<3>
                         : k_mm_prep_row<4>;
-    hipLaunchKernelGGL(kern, dim3((unsigned)act.Mp), dim3(1024), 0, st, x, ldx, normw, eps, act.K,
+    // dense rows past M are left as they are: each MFMA row depends on its own
+    // operand row alone, and theirs are not stored
+    hipLaunchKernelGGL(kern, dim3((unsigned)(gather ? act.Mp : M)), dim3(1024), 0, st, x, ldx, normw, eps, act.K,
                        (int)M, weight_dt == FTX_Q4_0_MMT ? 1 : 0, gather, part, split_stride, ldp,
                        S, act.xh, act.xl, act.sh, act.sl);
     return hipGetLastError();
@@ -1375,6 +1708,13 @@ bool mm_down_supported(int dt, int64_t n_in, int64_t N) {
     return dt == FTX_Q4_K && n_in % 32 == 0 && N % 256 == 0;
 }
 
+// a backend operation's launch: its operand's row scales and its activations
+struct MmOp {
+    const float* rscale;
+    const float* x;
+    int64_t ldx, K;
+};
+
 static MmOutDev out_dev(const MmOut& o) {
     MmOutDev d{};
     d.nseq = o.nseq;
@@ -1425,7 +1765,7 @@ static hipError_t mm_launch(hipStream_t st, const MmSeg* segs, int nseg, const M
                             int64_t M, int epi, const MmOut& out, float* part,
                             size_t part_floats, int cu_count, const int32_t* xtab,
                             const int64_t* plane, int64_t ntile_max, int64_t trows,
-                            const MmFragOut* fo, MmPend* pend) {
+                            const MmFragOut* fo, MmPend* pend, const MmOp* op = nullptr) {
     if (pend) *pend = MmPend{};
     if (nseg < 1 || nseg > 3 || M < 1 || M > act.Mp || out.nseq < 1 || out.nseq > FTX_MAX_SEQ)
         return hipErrorInvalidValue;
@@ -1435,14 +1775,17 @@ static hipError_t mm_launch(hipStream_t st, const MmSeg* segs, int nseg, const M
     // dense launches of at most 32 tokens take 16- or 32-token tiles: the
     // MFMAs, fragment reads and accumulator updates of the padding rows of a
     // 64-token tile are then not spent
-    const int ms = xtab ? (int)(trows / 16) : (M <= 16 ? 1 : (M <= 32 ? 2 : MM_MS));
+    // (the backend's operations: at most 32-token tiles, whose 64-bit sums
+    // fit the registers)
+    const int ms = xtab ? (int)(trows / 16) : (M <= 16 ? 1 : (M <= 32 || op ? 2 : MM_MS));
     if (fo && (!xtab || epi != EPI_SWIGLU)) return hipErrorInvalidValue;
     const int dt = segs[0].dt;
     MmArgs a{};
     a.nseg = nseg;
     int64_t units = 0, cols = 0;
     for (int i = 0; i < nseg; ++i) {
-        if (segs[i].dt != dt || !mm_supported(dt, act.K)) return hipErrorInvalidValue;
+        if (segs[i].dt != dt || act.K % 256 || (op ? !mm_stored(dt) : !mm_supported(dt, act.K)))
+            return hipErrorInvalidValue;
         if (dt == FTX_Q4_K && segs[i].rpt != 16 && segs[i].rpt != 32) return hipErrorInvalidValue;
         MmSegDev& d = a.seg[i];
         d.W = segs[i].W;
@@ -1464,23 +1807,32 @@ static hipError_t mm_launch(hipStream_t st, const MmSeg* segs, int nseg, const M
     a.sh = act.sh;
     a.sl = act.sl;
     a.M = (int)M;
+    a.nblk = (int)(act.K / 32);
+    if (op) {
+        a.rscale = op->rscale;
+        a.x = op->x;
+        a.ldx = op->ldx;
+        a.nblk = (int)(op->K / 32);
+    }
+    // rows of a split's partials
+    const int64_t prows = xtab ? act.Mp : M;
     const int64_t wg = (units + MM_WAVES - 1) / MM_WAVES,
-                  mt = xtab ? ntile_max : (ms == MM_MS ? act.Mp / MM_TOK : 1);
+                  mt = xtab ? ntile_max : (M + 16 * ms - 1) / (16 * ms);
     int S = mm_splits(wg * mt, a.nsb, cu_count, MM_SPLIT_COST);
     // SwiGLU needs the gate and up sums together: always through the reduce
     const bool via_part = S > 1 || epi == EPI_SWIGLU || xtab;
     if (via_part) {
-        if (!part || (size_t)S * (size_t)act.Mp * (size_t)cols > part_floats) {
+        if (!part || (size_t)S * (size_t)prows * (size_t)cols > part_floats) {
             S = 1;
-            if (!part || (size_t)act.Mp * (size_t)cols > part_floats) return hipErrorInvalidValue;
+            if (!part || (size_t)prows * (size_t)cols > part_floats) return hipErrorInvalidValue;
         }
         MmOutDev& o = a.out;
         o.nseq = 1;
         o.base[0] = part;
         o.row0[0] = 0;
-        o.row0[1] = act.Mp;
+        o.row0[1] = prows;
         o.ld = cols;
-        o.split_stride = act.Mp * cols;
+        o.split_stride = prows * cols;
         o.accum = 0;
     } else {
         a.out = out_dev(out);
@@ -1492,8 +1844,8 @@ static hipError_t mm_launch(hipStream_t st, const MmSeg* segs, int nseg, const M
     const size_t lds = 2 * (size_t)ms * 16384;
     using K_t = void (*)(MmArgs);
     // [dtype][dense 64 | expert 64-row tiles | expert 16-row tiles | dense
-    // 32 | dense 16] (Q6_K: dense only)
-    static const K_t kerns[4][5] = {
+    // 32 | dense 16] (Q6_K and stored rows: dense only)
+    static const K_t kerns[9][5] = {
         {k_mm<FTX_Q4_K, false, 4>, k_mm<FTX_Q4_K, true, 4>, k_mm<FTX_Q4_K, true, 1>,
          k_mm<FTX_Q4_K, false, 2>, k_mm<FTX_Q4_K, false, 1>},
         {k_mm<FTX_Q8_0_MMT, false, 4>, k_mm<FTX_Q8_0_MMT, true, 4>, k_mm<FTX_Q8_0_MMT, true, 1>,
@@ -1501,12 +1853,26 @@ static hipError_t mm_launch(hipStream_t st, const MmSeg* segs, int nseg, const M
         {k_mm<FTX_Q4_0_MMT, false, 4>, k_mm<FTX_Q4_0_MMT, true, 4>, k_mm<FTX_Q4_0_MMT, true, 1>,
          k_mm<FTX_Q4_0_MMT, false, 2>, k_mm<FTX_Q4_0_MMT, false, 1>},
         {k_mm<FTX_Q6_K_MMT, false, 4>, nullptr, nullptr, k_mm<FTX_Q6_K_MMT, false, 2>,
-         k_mm<FTX_Q6_K_MMT, false, 1>}};
-    const int di = dt == FTX_Q4_K ? 0 : (dt == FTX_Q8_0_MMT ? 1 : (dt == FTX_Q4_0_MMT ? 2 : 3));
+         k_mm<FTX_Q6_K_MMT, false, 1>},
+        {nullptr, nullptr, nullptr, k_mm<FTX_Q8_0, false, 2>, k_mm<FTX_Q8_0, false, 1>},
+        {nullptr, nullptr, nullptr, k_mm<FTX_Q4_0, false, 2>, k_mm<FTX_Q4_0, false, 1>},
+        {nullptr, nullptr, nullptr, k_mm<FTX_Q6_K, false, 2>, k_mm<FTX_Q6_K, false, 1>},
+        {nullptr, nullptr, nullptr, k_mm<FTX_F16, false, 2>, k_mm<FTX_F16, false, 1>},
+        {nullptr, nullptr, nullptr, k_mm<FTX_Q4_K_ROWS, false, 2>,
+         k_mm<FTX_Q4_K_ROWS, false, 1>}};
+    const int di = dt == FTX_Q4_K       ? 0
+                   : dt == FTX_Q8_0_MMT ? 1
+                   : dt == FTX_Q4_0_MMT ? 2
+                   : dt == FTX_Q6_K_MMT ? 3
+                   : dt == FTX_Q8_0     ? 4
+                   : dt == FTX_Q4_0     ? 5
+                   : dt == FTX_Q6_K     ? 6
+                   : dt == FTX_F16      ? 7
+                                        : 8;
     const int vi = xtab ? (ms == 4 ? 1 : 2) : (ms == 4 ? 0 : (ms == 2 ? 3 : 4));
     const K_t kern = kerns[di][vi];
     if (!kern) return hipErrorInvalidValue;
-    static bool lds_set[20] = {};
+    static bool lds_set[45] = {};
     const int ki = di * 5 + vi;
     if (!lds_set[ki]) {
         hipError_t e = hipFuncSetAttribute((const void*)kern,
@@ -1520,7 +1886,7 @@ static hipError_t mm_launch(hipStream_t st, const MmSeg* segs, int nseg, const M
     if (pend && epi != EPI_SWIGLU && !xtab && out.nseq == 1 && !fo) {
         // left for the consumer to add into (or store as) out
         pend->part = part;
-        pend->split_stride = act.Mp * cols;
+        pend->split_stride = prows * cols;
         pend->ldp = cols;
         pend->S = S;
         pend->N = cols;
@@ -1529,10 +1895,11 @@ static hipError_t mm_launch(hipStream_t st, const MmSeg* segs, int nseg, const M
     }
     MmReduceArgs r{};
     r.part = part;
-    r.split_stride = act.Mp * cols;
+    r.split_stride = prows * cols;
     r.ldp = cols;
     r.S = S;
     r.swiglu = epi == EPI_SWIGLU;
+    r.wide = op != nullptr;
     r.N = r.swiglu ? cols / 2 : cols;
     r.out = out_dev(out);
     r.xtab = xtab;
@@ -1551,6 +1918,61 @@ hipError_t launch_mm(hipStream_t st, const MmSeg* segs, int nseg, const MmAct& a
                      MmPend* pend) {
     return mm_launch(st, segs, nseg, act, M, epi, out, part, part_floats, cu_count, nullptr,
                      nullptr, 0, 0, nullptr, pend);
+}
+
+// ---- backend operations over stored rows
+bool mm_op_supported(int dt, int64_t M, int64_t K, int64_t N, int64_t row_bytes) {
+    const bool k32 = dt == FTX_Q8_0 || dt == FTX_Q4_0 || dt == FTX_F16;
+    const bool k256 = dt == FTX_Q4_K || dt == FTX_Q6_K;
+    // 32-bit offsets into the weights and the operand planes
+    return ((k32 && K % 32 == 0) || (k256 && K % 256 == 0)) && K > 0 && M > 0 && N > 0 &&
+           N * row_bytes < 0xF0000000ll && mm_pad_tokens(M) * ((K + 255) / 256 * 256) * 2 < 0xF0000000ll &&
+           M <= 65535;
+}
+// operand (with the row scales), then partials, in bytes
+static size_t mm_op_act_bytes(int64_t M, int64_t K) {
+    const int64_t Mp = mm_pad_tokens(M), Kp = (K + 255) / 256 * 256;
+    // hi and lo planes, Q4_K's limbs of the sums (2 KB per 16 x 256 elements),
+    // row scales
+    return ((size_t)(Mp * Kp * 4 + Mp * Kp / 2) + (size_t)M * 4 + 255) & ~(size_t)255;
+}
+static size_t mm_op_part_floats(int64_t M, int64_t K, int64_t cols, int epi, int cu_count) {
+    const int64_t units = epi == EPI_SWIGLU ? 2 * ((cols / 2 + MM_WROWS - 1) / MM_WROWS)
+                                            : (cols + MM_WROWS - 1) / MM_WROWS;
+    const int64_t mt = (M + 31) / 32;
+    const int S = mm_splits((units + MM_WAVES - 1) / MM_WAVES * mt, (K + 255) / 256, cu_count, MM_SPLIT_COST);
+    return S > 1 || epi == EPI_SWIGLU ? (size_t)S * (size_t)M * (size_t)cols : 0;
+}
+size_t mm_op_bytes(int64_t M, int64_t K, int64_t cols, int epi, int cu_count) {
+    return mm_op_act_bytes(M, K) + mm_op_part_floats(M, K, cols, epi, cu_count) * 4;
+}
+hipError_t launch_mm_op(hipStream_t st, const MmSeg* segs, int nseg, const float* x, int64_t ldx,
+                        int64_t K, int64_t M, int epi, float* y, int64_t ldy, void* ws, int cu_count) {
+    const int64_t Mp = mm_pad_tokens(M), Kp = (K + 255) / 256 * 256;
+    int64_t cols = 0;
+    for (int i = 0; i < nseg; ++i) cols += segs[i].N;
+    MmAct act = mm_act(ws, Mp, Kp);  // (its sums' place holds Q4_K's limbs)
+    float* rs = (float*)((uint8_t*)ws + Mp * Kp * 4 + Mp * Kp / 2);
+    MmSeg sg[2];
+    for (int i = 0; i < nseg && i < 2; ++i) {
+        sg[i] = segs[i];
+        if (sg[i].dt == FTX_Q4_K) sg[i].dt = FTX_Q4_K_ROWS;
+    }
+    float* part = (float*)((uint8_t*)ws + mm_op_act_bytes(M, K));
+    hipLaunchKernelGGL(k_mm_prep_op, dim3((unsigned)M), dim3(512), 0, st, x, ldx, K, Kp,
+                       segs[0].dt == FTX_Q4_0 ? 1 : 0, act.xh, act.xl,
+                       segs[0].dt == FTX_Q4_K ? (v8bf*)act.sh : nullptr, rs);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    MmOut o{};
+    o.nseq = 1;
+    o.base[0] = y;
+    o.row0[1] = M;
+    o.ld = ldy;
+    const MmOp op{rs, x, ldx, K};
+    if (nseg > 2) return hipErrorInvalidValue;
+    return mm_launch(st, sg, nseg, act, M, epi, o, part, mm_op_part_floats(M, K, cols, epi, cu_count),
+                     cu_count, nullptr, nullptr, 0, 0, nullptr, nullptr, &op);
 }
 
 hipError_t launch_mm_experts(hipStream_t st, const MmSeg* segs, int nseg, const int64_t* plane,
