@@ -196,3 +196,20 @@ def test_small_steps_of_stored_types(gctx, orc, dts, d, ff, M):
     assert rel_err_rows(got, want) < LOGIT_TOL
     for a, b in zip(kv, kvo):
         np.testing.assert_allclose(a.astype(np.float32), b.astype(np.float32), rtol=3e-3, atol=3e-3)
+
+
+@pytest.mark.parametrize("q,k,v", [(P.Q4_K, P.Q4_K, P.Q6_K), (P.Q6_K, P.Q8_0, P.Q4_K),
+                                   (P.Q4_K, P.Q4_0, P.Q6_K)])
+@pytest.mark.parametrize("M", [9, 33, 130])
+def test_projections_of_different_types(gctx, orc, q, k, v, M):
+    """q / k / v of different types in one projection of more than 8 tokens:
+    runs of one type over one operand (two and three launches, their split
+    partials side by side), and a Q4_0 between the others, whose operand
+    order they do not share; ffn_down Q6_K."""
+    dts = dict(tok_embd=P.Q8_0, output=P.Q6_K, q=q, k=k, v=v, o=P.Q6_K, gate=P.Q4_K, up=P.Q4_K,
+               down=P.Q6_K)
+    cfg = P.model_cfg(2, 1024, 8, 2, 128, 1024, 300, rope_theta=500000.0)
+    model = P.make_model(orc, cfg, dts, seed=q + 10 * k + M)
+    toks = np.random.default_rng(M + v).integers(0, 300, M).tolist()
+    (got, want, _, _), = run_batch(gctx, orc, model, [(toks, None, 30, 30 + M + 3)], 256)
+    assert rel_err_rows(got, want) < LOGIT_TOL

@@ -322,6 +322,8 @@ hipError_t launch_axpy(hipStream_t st, const uint8_t* W, int dt, int64_t row_byt
                        int64_t N, const float* h, int64_t ldh, int64_t M, float* y, int64_t ldy,
                        float* part, size_t part_floats, int cu_count, MmPend* pend = nullptr);
 bool mm_supported(int dt, int64_t K);
+// whether segments of two (tiled) types share one activation operand
+bool mm_together(int dt0, int dt1);
 // the one-pass GEMM's copy of Q8_0 / Q4_0 weights (per 16-row tile and
 // 256-element step, every lane's bytes contiguous): its internal dtype (or
 // -1), size, and the re-tiling of nplanes planes of `rows` rows each

@@ -1677,6 +1677,10 @@ hipError_t launch_mm_fold(hipStream_t st, const MmPend& fold, int64_t M, float* 
     return launch_reduce(st, r, M);
 }
 
+// weights whose operand takes each octet's even elements before its odd ones
+static bool mm_inter(int dt) { return dt == FTX_Q4_0_MMT || dt == FTX_Q4_0; }
+bool mm_together(int dt0, int dt1) { return mm_inter(dt0) == mm_inter(dt1); }
+
 bool mm_supported(int dt, int64_t K) {
     return (dt == FTX_Q4_K || dt == FTX_Q8_0_MMT || dt == FTX_Q4_0_MMT || dt == FTX_Q6_K_MMT) &&
            K % 256 == 0 && K >= 256;
@@ -1779,27 +1783,34 @@ static hipError_t mm_launch(hipStream_t st, const MmSeg* segs, int nseg, const M
     // fit the registers)
     const int ms = xtab ? (int)(trows / 16) : (M <= 16 ? 1 : (M <= 32 || op ? 2 : MM_MS));
     if (fo && (!xtab || epi != EPI_SWIGLU)) return hipErrorInvalidValue;
-    const int dt = segs[0].dt;
+    // segments of one type run in one launch; where the types differ (the
+    // "more bits" layers' Q6_K v beside Q4_K q and k) each run of one type is a
+    // launch of its own over the same operand, columns and splits
     MmArgs a{};
-    a.nseg = nseg;
-    int64_t units = 0, cols = 0;
+    int64_t wg = 0, cols = 0, gunits[3] = {};
+    int g0[4] = {}, ng = 0;  // first segment of each run
     for (int i = 0; i < nseg; ++i) {
-        if (segs[i].dt != dt || act.K % 256 || (op ? !mm_stored(dt) : !mm_supported(dt, act.K)))
+        const int dt = segs[i].dt;
+        if (i == 0 || dt != segs[i - 1].dt) g0[ng++] = i;
+        if (act.K % 256 || (op ? !mm_stored(dt) : !mm_supported(dt, act.K)) ||
+            (dt != segs[0].dt && (xtab || op || mm_inter(dt) != mm_inter(segs[0].dt))))
             return hipErrorInvalidValue;
         if (dt == FTX_Q4_K && segs[i].rpt != 16 && segs[i].rpt != 32) return hipErrorInvalidValue;
         MmSegDev& d = a.seg[i];
         d.W = segs[i].W;
         d.N = segs[i].N;
-        d.unit0 = units;
+        d.unit0 = gunits[ng - 1];
         d.col0 = cols;
         d.row_bytes = segs[i].row_bytes;
         d.rpt = segs[i].rpt;
-        units += (segs[i].N + MM_WROWS - 1) / MM_WROWS;
+        gunits[ng - 1] += (segs[i].N + MM_WROWS - 1) / MM_WROWS;
         cols += segs[i].N;
         a.plane[i] = plane ? plane[i] : 0;
     }
+    g0[ng] = nseg;
+    for (int g = 0; g < ng; ++g) wg += (gunits[g] + MM_WAVES - 1) / MM_WAVES;
+    if (epi == EPI_SWIGLU && ng > 1) return hipErrorInvalidValue;
     a.xtab = xtab;
-    a.units = units;
     a.K = act.K;
     a.nsb = (int)(act.K / 256);
     a.xh = act.xh;
@@ -1816,8 +1827,7 @@ static hipError_t mm_launch(hipStream_t st, const MmSeg* segs, int nseg, const M
     }
     // rows of a split's partials
     const int64_t prows = xtab ? act.Mp : M;
-    const int64_t wg = (units + MM_WAVES - 1) / MM_WAVES,
-                  mt = xtab ? ntile_max : (M + 16 * ms - 1) / (16 * ms);
+    const int64_t mt = xtab ? ntile_max : (M + 16 * ms - 1) / (16 * ms);
     int S = mm_splits(wg * mt, a.nsb, cu_count, MM_SPLIT_COST);
     // SwiGLU needs the gate and up sums together: always through the reduce
     const bool via_part = S > 1 || epi == EPI_SWIGLU || xtab;
@@ -1840,7 +1850,6 @@ static hipError_t mm_launch(hipStream_t st, const MmSeg* segs, int nseg, const M
     a.sb_per_split = (a.nsb + S - 1) / S;
     S = (a.nsb + a.sb_per_split - 1) / a.sb_per_split;
     a.ntt = (int)mt;
-    const dim3 grid((unsigned)(wg * mt), 1, (unsigned)S);
     const size_t lds = 2 * (size_t)ms * 16384;
     using K_t = void (*)(MmArgs);
     // [dtype][dense 64 | expert 64-row tiles | expert 16-row tiles | dense
@@ -1860,28 +1869,40 @@ static hipError_t mm_launch(hipStream_t st, const MmSeg* segs, int nseg, const M
         {nullptr, nullptr, nullptr, k_mm<FTX_F16, false, 2>, k_mm<FTX_F16, false, 1>},
         {nullptr, nullptr, nullptr, k_mm<FTX_Q4_K_ROWS, false, 2>,
          k_mm<FTX_Q4_K_ROWS, false, 1>}};
-    const int di = dt == FTX_Q4_K       ? 0
-                   : dt == FTX_Q8_0_MMT ? 1
-                   : dt == FTX_Q4_0_MMT ? 2
-                   : dt == FTX_Q6_K_MMT ? 3
-                   : dt == FTX_Q8_0     ? 4
-                   : dt == FTX_Q4_0     ? 5
-                   : dt == FTX_Q6_K     ? 6
-                   : dt == FTX_F16      ? 7
-                                        : 8;
-    const int vi = xtab ? (ms == 4 ? 1 : 2) : (ms == 4 ? 0 : (ms == 2 ? 3 : 4));
-    const K_t kern = kerns[di][vi];
-    if (!kern) return hipErrorInvalidValue;
-    static bool lds_set[45] = {};
-    const int ki = di * 5 + vi;
-    if (!lds_set[ki]) {
-        hipError_t e = hipFuncSetAttribute((const void*)kern,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        lds_set[ki] = true;
+    hipError_t e = hipSuccess;
+    for (int g = 0; g < ng && e == hipSuccess; ++g) {
+        const int dt = segs[g0[g]].dt;
+        const int di = dt == FTX_Q4_K       ? 0
+                       : dt == FTX_Q8_0_MMT ? 1
+                       : dt == FTX_Q4_0_MMT ? 2
+                       : dt == FTX_Q6_K_MMT ? 3
+                       : dt == FTX_Q8_0     ? 4
+                       : dt == FTX_Q4_0     ? 5
+                       : dt == FTX_Q6_K     ? 6
+                       : dt == FTX_F16      ? 7
+                                            : 8;
+        const int vi = xtab ? (ms == 4 ? 1 : 2) : (ms == 4 ? 0 : (ms == 2 ? 3 : 4));
+        const K_t kern = kerns[di][vi];
+        if (!kern) return hipErrorInvalidValue;
+        static bool lds_set[45] = {};
+        const int ki = di * 5 + vi;
+        if (!lds_set[ki]) {
+            e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)lds);
+            if (e != hipSuccess) return e;
+            lds_set[ki] = true;
+        }
+        MmArgs b = a;
+        b.nseg = g0[g + 1] - g0[g];
+        for (int i = 0; i < b.nseg; ++i) {
+            b.seg[i] = a.seg[g0[g] + i];
+            b.plane[i] = a.plane[g0[g] + i];
+        }
+        b.units = gunits[g];
+        const dim3 grid((unsigned)((gunits[g] + MM_WAVES - 1) / MM_WAVES * mt), 1, (unsigned)S);
+        ktimed_launch(kern, grid, dim3(64 * MM_WAVES), (uint32_t)lds, st, b);
+        e = hipGetLastError();
     }
-    ktimed_launch(kern, grid, dim3(64 * MM_WAVES), (uint32_t)lds, st, a);
-    hipError_t e = hipGetLastError();
     if (e != hipSuccess || !via_part) return e;
     if (pend && epi != EPI_SWIGLU && !xtab && out.nseq == 1 && !fo) {
         // left for the consumer to add into (or store as) out

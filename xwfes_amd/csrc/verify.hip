@@ -294,7 +294,7 @@ static int verify_large(ftx_ctx* ctx, ftx_model* m, const ftx_seq_args* sq, int6
         MmSeg sg[3];
         bool all = true;
         for (int i = 0; i < nseg; ++i) all = all && mm_seg(idx[i], ts[i], sg[i]);
-        for (int i = 1; all && i < nseg; ++i) all = sg[i].dt == sg[0].dt;
+        for (int i = 1; all && i < nseg; ++i) all = mm_together(sg[i].dt, sg[0].dt);
         if (all) {
             const MmAct act = mm_act(m->mm_act, mm_pad_tokens(Mr), K);
             if (act_ready) {
