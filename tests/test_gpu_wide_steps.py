@@ -213,3 +213,20 @@ def test_projections_of_different_types(gctx, orc, q, k, v, M):
     toks = np.random.default_rng(M + v).integers(0, 300, M).tolist()
     (got, want, _, _), = run_batch(gctx, orc, model, [(toks, None, 30, 30 + M + 3)], 256)
     assert rel_err_rows(got, want) < LOGIT_TOL
+
+
+@pytest.mark.parametrize("dt", [P.Q8_0, P.Q4_0])
+@pytest.mark.parametrize("d,ff,M", [(2048, 520, 1), (2304, 2080, 2), (4096, 2048, 3), (2048, 4128, 8)])
+def test_small_steps_over_tiles(gctx, orc, dt, d, ff, M):
+    """One to eight tokens of a Q8_0 / Q4_0 model on the re-tiled copies: one
+    step per wave, uneven steps and two per wave; a last 16-row tile of 8
+    rows (520 gate rows); the head's rows past the last whole tile."""
+    dts = dict(tok_embd=P.Q8_0, output=dt, q=dt, k=dt, v=dt, o=dt, gate=dt, up=dt, down=dt)
+    cfg = P.model_cfg(1, d, d // 128, max(d // 512, 1) if d != 2304 else 3, 128, ff, 203,
+                      rope_theta=500000.0)
+    model = P.make_model(orc, cfg, dts, seed=d + ff + M)
+    toks = np.random.default_rng(M).integers(0, 203, M).tolist()
+    (got, want, kv, kvo), = run_batch(gctx, orc, model, [(toks, None, 50, 70)], 16)
+    assert rel_err_rows(got, want) < LOGIT_TOL
+    for a, b in zip(kv, kvo):
+        np.testing.assert_allclose(a.astype(np.float32), b.astype(np.float32), rtol=3e-3, atol=3e-3)

@@ -304,6 +304,12 @@ hipError_t launch_mm_prep_fold(hipStream_t st, float* x, int64_t ldx, const floa
                                const MmPend& fold);
 // the partials `fold` added into y rows < M (a reduce launch)
 hipError_t launch_mm_fold(hipStream_t st, const MmPend& fold, int64_t M, float* y, int64_t ldy);
+// up to 8 tokens over the re-tiled Q8_0 / Q4_0 copies (segments with those
+// types and W), RMSNorm included when normw is given: EPI_STORE, EPI_ACCUM, or
+// EPI_SWIGLU over a gate and an up segment
+bool tile_supported(int dt, int64_t K, int64_t M);
+hipError_t launch_tile(hipStream_t st, const GemvSeg* segs, int nseg, const float* x, int64_t ldx,
+                       int64_t K, int64_t M, int epi, const float* normw, float eps);
 // a backend operation y[m][n] = sum_k x[m][k] W[n][k] (SwiGLU: two segments)
 // on the one-pass GEMM over rows as they are stored (segments with rpt 0 and
 // row_bytes), any fp32 x; ws of mm_op_bytes(), cols = the segments' rows

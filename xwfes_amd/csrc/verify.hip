@@ -1345,6 +1345,22 @@ int ftx_verify_step(ftx_ctx* ctx, ftx_model* m, ftx_kv* kv, const ftx_verify_arg
             TRACED(kind, bytes, chunks());
             return FTX_OK;
         }
+        // Q8_0 / Q4_0: the re-tiled copies where every segment has one type of
+        // them (its launch has the norm in it)
+        bool tl = epi != EPI_QKV;
+        for (int i = 0; tl && i < nseg; ++i) {
+            const size_t ti = (size_t)(tix0 + tix[i]);
+            tl = m->mmt[ti] && m->mmt_dt[ti] == m->mmt_dt[(size_t)(tix0 + tix[0])] &&
+                 tile_supported(m->mmt_dt[ti], K, M);
+        }
+        if (tl) {
+            for (int i = 0; i < nseg; ++i) {
+                segs[i].W = m->mmt[(size_t)(tix0 + tix[i])];
+                segs[i].dt = m->mmt_dt[(size_t)(tix0 + tix[i])];
+            }
+            TRACED(kind, bytes, launch_tile(st, segs, nseg, xin, ldx, K, M, epi, normw, eps));
+            return FTX_OK;
+        }
         // (the few-row kernel has the norm in it)
         const float* nw = normw && gemv_norm_ok(segs, nseg, K, M) ? normw : nullptr;
         const float* src = xin;
