@@ -56,11 +56,13 @@ def close(got, want, size):
 
 @pytest.mark.parametrize("dt", [P.Q4_0, P.Q8_0, P.Q4_K, P.Q6_K])
 @pytest.mark.parametrize("M,n_in,blocks", [(1, 1, 1), (3, 33, 2), (16, 257, 3), (17, 31, 5),
-                                           (33, 300, 1), (65, 96, 9), (130, 1408, 2)])
+                                           (33, 300, 1), (65, 96, 9), (130, 1408, 2),
+                                           (1, 1408, 16), (2, 131, 17), (5, 64, 33), (8, 577, 40)])
 def test_down_axpy_mfma(gctx, orc, dt, M, n_in, blocks):
-    """The column-axpy MFMA kernel at the edges of its token tiles (16, 32, 64),
-    32-row slices and 128-column groups, with one split and several; the
-    rows it adds to are kept."""
+    """The column-axpy kernels: the MFMA one at the edges of its token tiles (16,
+    32, 64), 32-row slices and 128-column groups, the few-token one (Q8_0,
+    Q4_0, up to 8) at those of its 512-column groups, waves' row runs and
+    4-row batches; with one split and several; the rows they add to are kept."""
     N = blocks * (256 if dt in (P.Q4_K, P.Q6_K) else 32)
     rng = np.random.default_rng(dt * 1000 + M + n_in)
     t, w = weight(gctx, orc, rng, dt, n_in, N)

@@ -394,7 +394,7 @@ int ftx_matmul(ftx_ctx* ctx, const float* x, int64_t M, int64_t K, const ftx_ten
 // caller, so that both entry points sum in one order.
 static size_t down_part_floats(ftx_ctx* ctx, int dt, int64_t M, int64_t n_in, int64_t N) {
     return axpy_supported(dt, N)
-               ? axpy_part_floats(M, n_in, N, NOALLOC_SCRATCH_FLOATS, ctx->cu_count)
+               ? axpy_part_floats(dt, M, n_in, N, NOALLOC_SCRATCH_FLOATS, ctx->cu_count)
                : down_scratch_floats(M, n_in, N);
 }
 static hipError_t down(ftx_ctx* ctx, const uint8_t* W, int dt, int64_t row_bytes, int64_t n_in,

@@ -323,7 +323,7 @@ hipError_t launch_mm_op(hipStream_t st, const MmSeg* segs, int nseg, const float
 // left in *pend for y's next reader; without room for them there is one split.
 bool axpy_supported(int dt, int64_t N);
 // the partials of the best split within `cap` floats
-size_t axpy_part_floats(int64_t M, int64_t n_in, int64_t N, size_t cap, int cu_count);
+size_t axpy_part_floats(int dt, int64_t M, int64_t n_in, int64_t N, size_t cap, int cu_count);
 hipError_t launch_axpy(hipStream_t st, const uint8_t* W, int dt, int64_t row_bytes, int64_t n_in,
                        int64_t N, const float* h, int64_t ldh, int64_t M, float* y, int64_t ldy,
                        float* part, size_t part_floats, int cu_count, MmPend* pend = nullptr);

@@ -30,10 +30,11 @@
 // work (about 100 VALU instructions per 32 x 32 weights), above that the limb
 // splits (52 VALU per 32 x 32 weights and 16 tokens) and MFMAs.
 // Measured, one launch (before: the generic kernel, or Q6_K's 8-token chunks):
-// Q8_0 14336 x 4096, 1 token 795 -> 25.6 us (2.4 TB/s); Q4_0, 24 tokens 2013 ->
-// 35.9 us; Q6_K, 256 tokens 531 -> 214 us (140 TFLOP/s); Q4_0 1408 x 512, 1
-// token 30.8 -> 5.8 us.  Error against 64 bits 0.8e-7 to 1.4e-7 (1000 to 14336
+// Q4_0 14336 x 4096, 24 tokens 2013 -> 35.9 us; Q6_K, 256 tokens 531 -> 214 us
+// (140 TFLOP/s); up to 8 tokens of Q8_0 / Q4_0 go to k_axpy_few below.  Error against 64 bits 0.8e-7 to 1.4e-7 (1000 to 14336
 // rows) where the fp32 sums of the generic kernel had 1.6e-7 to 5.7e-7.
+#include <algorithm>
+
 #include "ftx_internal.h"
 #include "quant_dev.h"
 
@@ -450,6 +451,125 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
     }
 }
 
+// ---------------------------------------------------------------- few tokens
+//
+// Up to 8 tokens of Q8_0 / Q4_0: with so few rows of A in use the MFMA form
+// spends its time on limbs and transposes, while the products themselves are
+// few.  Here a lane owns 8 neighbouring columns and walks rows: y[m][j] +=
+// (h[m][i] d) q, one multiplication per row and token for h d, a conversion
+// and M multiply-adds per weight, all fp32.  A wave covers 512 columns of a
+// contiguous run of rows (one load of 512 or 256 contiguous quant bytes a
+// row), four rows in flight ahead of the four computed; h comes through
+// scalar loads.  The 8 waves of a workgroup are added in LDS in wave order.
+// Measured, one token: Q8_0 14336 x 4096 25.6 (k_axpy) -> 15.6 us (4.0 TB/s)
+// with a sum of the partials of 4.4 us (6.2 before); Q4_0 1408 x 512 5.8 -> 4.1.
+constexpr int AF_WAVES = 8, AF_ROWS = 4;
+
+template <int DT, int MC>
+__global__ void __launch_bounds__(64 * AF_WAVES) k_axpy_few(AxArgs a) {
+    constexpr int QW = DT == FTX_Q8_0 ? 2 : 1, BB = DT == FTX_Q8_0 ? 34 : 18;
+    __shared__ __attribute__((aligned(16))) float red[AF_WAVES][512];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t j0 = (int64_t)blockIdx.x * 512;
+    const int ks = blockIdx.z;
+    // (columns past the row's end read its last block and are not stored)
+    const int64_t blk = min(j0 / 32 + lane / 4, a.N / 32 - 1);
+    const uint32_t soff = (uint32_t)(blk * BB), qoff = soff + 2 + (lane & 3) * 4 * QW;
+    // (slices_per_split counts rows here, an eighth of them per wave)
+    const int64_t i0 = (int64_t)ks * a.slices_per_split, i1 = min(i0 + (int64_t)a.slices_per_split, a.n_in);
+    const int64_t per = (i1 - i0 + AF_WAVES - 1) / AF_WAVES;
+    const int64_t r0 = i0 + w * per, r1 = min(r0 + per, i1);
+    float acc[MC][8];
+#pragma unroll
+    for (int m = 0; m < MC; ++m)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[m][e] = 0.f;
+    struct Rows {
+        uint32_t q[AF_ROWS][QW], d[AF_ROWS];
+    } cur, nxt;
+    auto load = [&](Rows& o, int64_t r) {
+#pragma unroll
+        for (int u = 0; u < AF_ROWS; ++u) {
+            const uint8_t* p = a.W + min(r + u, a.n_in - 1) * a.row_bytes;  // uniform
+            o.d[u] = ((const u16u*)(p + soff))->v;
+            if constexpr (DT == FTX_Q8_0) {
+                const u64u v = *(const u64u*)(p + qoff);
+                o.q[u][0] = v.v[0];
+                o.q[u][1] = v.v[1];
+            } else {
+                o.q[u][0] = ((const u32u*)(p + qoff))->v;
+            }
+        }
+    };
+    auto row = [&](const Rows& o, int u, int64_t r) {
+        float q[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            q[e] = DT == FTX_Q8_0 ? (float)(int8_t)(o.q[u][e / 4 % QW] >> (8 * (e & 3)))
+                                  : (float)((int)((o.q[u][0] >> (4 * e)) & 15u) - 8);
+        const float d = h2f((uint16_t)o.d[u]);
+#pragma unroll
+        for (int m = 0; m < MC; ++m) {
+            const float t = a.h[(int64_t)min(m, a.M - 1) * a.ldh + r] * d;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[m][e] = fmaf(t, q[e], acc[m][e]);
+        }
+    };
+    if (r0 < r1) {
+        load(cur, r0);
+        int64_t r = r0;
+        for (; r + AF_ROWS <= r1; r += AF_ROWS) {
+            load(nxt, r + AF_ROWS);
+#pragma unroll
+            for (int u = 0; u < AF_ROWS; ++u) row(cur, u, r + u);
+            cur = nxt;
+        }
+#pragma unroll
+        for (int u = 0; u < AF_ROWS; ++u)
+            if (r + u < r1) row(cur, u, r + u);  // uniform
+    }
+#pragma unroll
+    for (int m = 0; m < MC; ++m) {
+        if (m >= a.M) break;  // uniform
+        if (m) __syncthreads();
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            *(float4*)&red[w][8 * lane + 4 * h] =
+                float4{acc[m][4 * h], acc[m][4 * h + 1], acc[m][4 * h + 2], acc[m][4 * h + 3]};
+        __syncthreads();
+        float s = red[0][tid];
+#pragma unroll
+        for (int k = 1; k < AF_WAVES; ++k) s += red[k][tid];
+        if (j0 + tid < a.N) {
+            float* p = a.out + (int64_t)ks * a.split_stride + (int64_t)m * a.ldo + j0 + tid;
+            *p = a.accum ? *p + s : s;
+        }
+    }
+}
+
+// y[m][n] += sum_s part[s][m][n] of few rows: 64 columns per workgroup, its
+// four waves a quarter of the splits each (four partial sums, added in order)
+__global__ void __launch_bounds__(256) k_axpy_sum(const float* __restrict__ part, int S, int64_t stride,
+                                                  int64_t N, float* __restrict__ y, int64_t ldy) {
+    __shared__ float red[4][64];
+    const int c = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t n = (int64_t)blockIdx.x * 64 + c, m = blockIdx.y;
+    const float* p = part + m * N + min(n, N - 1);
+    const int per = (S + 3) / 4, s0 = w * per, s1 = min(s0 + per, S);
+    float v = 0.f;
+    for (int s = s0; s < s1; s += 8) {
+        float t[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) t[u] = p[(int64_t)min(s + u, S - 1) * stride];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v += s + u < s1 ? t[u] : 0.f;
+    }
+    red[w][c] = v;
+    __syncthreads();
+    if (w == 0 && n < N) y[m * ldy + n] += ((red[0][c] + red[1][c]) + red[2][c]) + red[3][c];
+}
+
 }  // namespace
 
 // whole blocks along a row (the K types have 256-column blocks)
@@ -463,6 +583,15 @@ bool axpy_supported(int dt, int64_t N) {
 // the split's) plus about two slices of start and reduction; the fewest slice
 // times, the fewest splits on ties, within `cap` partial floats (one split
 // writes y itself)
+// splits of the few-token kernel: workgroups of 512 columns, 8 waves each;
+// about 512 of them, at least 64 rows (8 a wave) per split, within `cap`
+static bool axpy_few(int dt, int64_t M) { return M <= 8 && (dt == FTX_Q8_0 || dt == FTX_Q4_0); }
+static int axpy_few_splits(int64_t M, int64_t n_in, int64_t N, size_t cap) {
+    const int64_t wg = (N + 511) / 512;
+    int64_t S = std::min(std::max<int64_t>(512 / wg, 1), std::max<int64_t>(n_in / 64, 1));
+    while (S > 1 && (size_t)(S * M * N) > cap) --S;
+    return (int)S;
+}
 static int axpy_ms(int64_t M) { return M <= 16 ? 1 : (M <= 32 ? 2 : 4); }
 static int axpy_splits(int64_t M, int64_t n_in, int64_t N, size_t cap, int cu_count) {
     const int ms = axpy_ms(M);
@@ -483,8 +612,9 @@ static int axpy_splits(int64_t M, int64_t n_in, int64_t N, size_t cap, int cu_co
     return best;
 }
 
-size_t axpy_part_floats(int64_t M, int64_t n_in, int64_t N, size_t cap, int cu_count) {
-    const int S = M > 0 ? axpy_splits(M, n_in, N, cap, cu_count) : 1;
+size_t axpy_part_floats(int dt, int64_t M, int64_t n_in, int64_t N, size_t cap, int cu_count) {
+    const int S = M <= 0 ? 1 : (axpy_few(dt, M) ? axpy_few_splits(M, n_in, N, cap)
+                                                 : axpy_splits(M, n_in, N, cap, cu_count));
     return S > 1 ? (size_t)S * (size_t)(M * N) : 0;
 }
 
@@ -494,8 +624,11 @@ hipError_t launch_axpy(hipStream_t st, const uint8_t* W, int dt, int64_t row_byt
     if (pend) *pend = MmPend{};
     if (M <= 0 || n_in <= 0) return hipSuccess;
     if (!axpy_supported(dt, N)) return hipErrorInvalidValue;
-    int S = axpy_splits(M, n_in, N, part ? part_floats : 0, cu_count);
-    const int64_t nsl = (n_in + 31) / 32;
+    const bool few = axpy_few(dt, M);
+    int S = few ? axpy_few_splits(M, n_in, N, part ? part_floats : 0)
+                : axpy_splits(M, n_in, N, part ? part_floats : 0, cu_count);
+    // rows (few) or 32-row slices
+    const int64_t nsl = few ? n_in : (n_in + 31) / 32;
     AxArgs a{};
     a.W = W;
     a.row_bytes = row_bytes;
@@ -513,6 +646,19 @@ hipError_t launch_axpy(hipStream_t st, const uint8_t* W, int dt, int64_t row_byt
     a.split_stride = S > 1 ? M * N : 0;
     a.accum = S == 1;
     using K_t = void (*)(AxArgs);
+    if (few) {
+        static const K_t fk[2][4] = {
+            {k_axpy_few<FTX_Q8_0, 1>, k_axpy_few<FTX_Q8_0, 2>, k_axpy_few<FTX_Q8_0, 4>, k_axpy_few<FTX_Q8_0, 8>},
+            {k_axpy_few<FTX_Q4_0, 1>, k_axpy_few<FTX_Q4_0, 2>, k_axpy_few<FTX_Q4_0, 4>, k_axpy_few<FTX_Q4_0, 8>}};
+        ktimed_launch(fk[dt == FTX_Q4_0][M == 1 ? 0 : (M == 2 ? 1 : (M <= 4 ? 2 : 3))],
+                      dim3((unsigned)((N + 511) / 512), 1, (unsigned)S), dim3(64 * AF_WAVES), 0, st, a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess || S == 1) return e;
+        // (many small partials: added here, not left in *pend)
+        hipLaunchKernelGGL(k_axpy_sum, dim3((unsigned)((N + 63) / 64), (unsigned)M), dim3(256), 0, st, part,
+                           S, M * N, N, y, ldy);
+        return hipGetLastError();
+    }
     static const K_t kerns[4][3] = {
         {k_axpy<FTX_Q4_0, 1>, k_axpy<FTX_Q4_0, 2>, k_axpy<FTX_Q4_0, 4>},
         {k_axpy<FTX_Q8_0, 1>, k_axpy<FTX_Q8_0, 2>, k_axpy<FTX_Q8_0, 4>},
