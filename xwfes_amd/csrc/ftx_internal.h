@@ -642,7 +642,8 @@ struct AcceptDev {
     const float* pd;         // device [M] or null
     int mode;
     float temp;
-    uint64_t* rng;           // device state of the acceptance stream
+    const uint64_t* rng;     // device state of the acceptance stream
+    uint64_t* rng_out;       // the state after the decisions
     uint64_t* sampler_rng;   // device state of the bonus sampler (ratio mode)
     int top_k;
     float top_p;
@@ -654,12 +655,15 @@ hipError_t launch_accept(hipStream_t st, const AcceptDev& a);
 // n acceptances (GREEDY / RATIO) in one launch, workgroup s taking d_arr[s]
 // (device memory)
 hipError_t launch_accept_multi(hipStream_t st, const AcceptDev* d_arr, int n);
-// the RESIDUAL mode over many workgroups (row statistics included); scratch
-// of accept_residual_scratch_bytes(); accept_residual_error copies the grid
-// barrier's time-out flag to the host int *err (enqueued on st)
+// the RESIDUAL mode over many workgroups: its row statistics (chunk maxima,
+// sub-chunk and chunk sums), then the walk; scratch of
+// accept_residual_scratch_bytes(), shared by the two launches.  The int after
+// *a.margin, zero before, is 1 after a barrier timed out.
 size_t accept_residual_scratch_bytes();
+hipError_t launch_residual_stats(hipStream_t st, const float* base_row, const float* rows,
+                                 int64_t nrows, int64_t V, float temp, const RowChunks& rc,
+                                 void* scratch);
 hipError_t launch_accept_residual(hipStream_t st, const AcceptDev& a, void* scratch);
-int accept_residual_error(const void* scratch, hipStream_t st, int* err);
 // argmax and its T = 1 softmax probability of one row: out = {token, prob
 // bits} (scratch: row_stats_scratch_bytes(1, V))
 hipError_t launch_argmax_prob(hipStream_t st, const float* row, int64_t V, void* scratch,

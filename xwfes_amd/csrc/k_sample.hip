@@ -150,6 +150,63 @@ __global__ void __launch_bounds__(256) k_row_sum(const float* __restrict__ base_
     }
 }
 
+// The same for the RESIDUAL mode, which reads the double sums only (no float
+// sums or sub-chunk maxima for a sampler): lanes side by side, a float4 each
+// at 4 t + 1024 k, so that a sub-chunk is half a wave's loads; the chunk's own
+// sum beside the sub-chunks' (csum, in csubf's place), from which the
+// acceptance kernel forms a row's statistics when it visits the row.  Also
+// clears the acceptance kernel's partial-sum words.  53 rows of 128256: 19.7
+// us by k_row_sum, 17.1 here.
+template <bool VEC>
+__global__ void __launch_bounds__(256) k_row_sum_res(const float* __restrict__ base_row,
+                                                     const float* __restrict__ rows, int64_t V,
+                                                     float temp, RowChunks rc,
+                                                     unsigned long long* __restrict__ words, int nwords) {
+#pragma clang fp contract(off)
+    __shared__ double sd[4];
+    const int64_t r = blockIdx.y;
+    const int c = blockIdx.x, t = threadIdx.x;
+    if (c == 0 && r == 0 && t < nwords) words[t] = 0;
+    const float* row = stat_row(base_row, rows, r, V);
+    const int64_t i0 = (int64_t)c * SCH + 4 * t;
+    float v[4][4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int64_t i = i0 + 1024 * k;
+        if (VEC && i + 4 <= V) {
+            const float4 q = *(const float4*)(row + i);
+            v[k][0] = q.x;
+            v[k][1] = q.y;
+            v[k][2] = q.z;
+            v[k][3] = q.w;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[k][e] = row[min(i + e, V - 1)];
+        }
+    }
+    float mx = -INFINITY;
+    for (int k = t & 63; k < rc.nch; k += 64) mx = fmaxf(mx, rc.cmax[r * rc.nch + k]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    double tot = 0.0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        double s = 0.0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (i0 + 1024 * k + e < V) s += texp(v[k][e], mx, temp);
+#pragma unroll
+        for (int o = 16; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+        const int64_t j = (int64_t)c * (SCH / SUB) + 8 * k + t / 32;
+        if ((t & 31) == 0 && j < rc.nsub) rc.csub[r * rc.nsub + j] = s;
+        tot += s;
+    }
+    tot += __shfl_xor(tot, 32, 64);
+    if ((t & 63) == 0) sd[t >> 6] = tot;
+    __syncthreads();
+    if (t == 0) rc.csubf[r * rc.nch + c] = ((sd[0] + sd[1]) + sd[2]) + sd[3];
+}
+
 // Inverse-CDF pick over p[0..V) (double weights) by one block: thread t sums
 // the contiguous chunk [t * chunk, (t + 1) * chunk) in index order (eight
 // loads issued together), a block scan, then the crossing chunk scanned in
@@ -605,6 +662,33 @@ __device__ void row_stat_wave(const AcceptDev& a, int64_t r, int l) {
     if (l == 0) a.stats[r] = RowStats{best, bi, sum};
 }
 
+// The same from the chunk sums of k_row_sum_res, in every lane of the wave.
+__device__ __forceinline__ RowStats row_stat_chunks(const RowChunks& rc, int64_t r, int l) {
+    float best = -INFINITY;
+    int32_t bi = 0x7FFFFFFF;
+    double sum = 0.0;
+    for (int c = l; c < rc.nch; c += 64) {
+        const float v = rc.cmax[r * rc.nch + c];
+        const int32_t iv = rc.carg[r * rc.nch + c];
+        sum += rc.csubf[r * rc.nch + c];
+        if (iv != 0x7FFFFFFF && (bi == 0x7FFFFFFF || better(v, iv, best, bi))) {
+            best = v;
+            bi = iv;
+        }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const float ov = __shfl_xor(best, o, 64);
+        const int32_t oi = __shfl_xor(bi, o, 64);
+        sum += __shfl_xor(sum, o, 64);
+        if (oi != 0x7FFFFFFF && (bi == 0x7FFFFFFF || better(ov, oi, best, bi))) {
+            best = ov;
+            bi = oi;
+        }
+    }
+    return RowStats{best, bi, sum};
+}
+
 // Decisions by one workgroup: GREEDY and RESIDUAL (one-block form) finish
 // here; RATIO walks the chain and draws the bonus with the sampler.
 __device__ void accept_wg(const AcceptDev& a) {
@@ -755,7 +839,7 @@ __device__ void accept_wg(const AcceptDev& a) {
     if (t == 0) {
         a.out[0] = nacc;
         a.out[1] = bonus;
-        *a.rng = rng;
+        *a.rng_out = rng;
         if (a.sampler_rng) *a.sampler_rng = srng;
         *a.margin = mg;
     }
@@ -789,55 +873,14 @@ __global__ void __launch_bounds__(NT) k_accept_multi(const AcceptDev* __restrict
 // the pick of the target (the crossing 128-element sub-chunk from the
 // statistics' sub-chunk sums, then the element).
 //
-// The grid barrier is a flag per workgroup: a workgroup publishes its
-// barrier count (release: its stores written back first), and one wave polls
-// every flag with one load per lane until all have reached that count
-// (acquire).  Measured on the device: 1.5-3 us for 16-32 workgroups, against
-// 2.7-4.1 us for one shared counter (its atomics serialise at the memory
-// side).  The waits are bounded: a barrier that does not complete in about
-// 0.3 s sets the error word and every workgroup returns.
+// A node's row statistics (maximum, sum) come from its 4096-element chunks'
+// when the walk reaches it, formed by every wave alike: no pass over the other
+// rows' and no barrier before the walk.
+// The reduction barrier's waits are bounded: a barrier that does not complete
+// in about 0.3 s sets the error word (after the margin in the small block) and
+// every workgroup returns.
 
 constexpr int RT = 256;  // threads per workgroup of the residual kernel
-
-struct GridBar {
-    int err, pad_[63];
-    unsigned flags[ACC_RES_WG];
-};
-
-__device__ bool grid_barrier(GridBar* gb, unsigned G, unsigned& gen) {
-    __shared__ int ok;
-    __syncthreads();
-    ++gen;
-    if (threadIdx.x == 0) {
-        ok = 1;
-        __threadfence();
-        __hip_atomic_store(&gb->flags[blockIdx.x], gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (threadIdx.x < 64) {
-        unsigned n = 0;
-        for (;;) {
-            int mine = 1;
-            for (unsigned w = threadIdx.x; w < G; w += 64)
-                mine &= (int)(__hip_atomic_load(&gb->flags[w], __ATOMIC_RELAXED,
-                                                __HIP_MEMORY_SCOPE_AGENT) -
-                                  gen <
-                              0x80000000u);
-            if (__all(mine)) break;
-            if (++n > (1u << 18) ||
-                __hip_atomic_load(&gb->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-                if (threadIdx.x == 0) {
-                    __hip_atomic_store(&gb->err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    ok = 0;
-                }
-                break;
-            }
-            __builtin_amdgcn_s_sleep(2);
-        }
-        if (threadIdx.x == 0) __threadfence();
-    }
-    __syncthreads();
-    return ok != 0;
-}
 
 // The reduction barrier of a pass: the partial sums are the flags.  Pass k
 // uses buffer k % 3 of G 64-bit words holding the bitwise complement of each
@@ -850,7 +893,7 @@ __device__ bool grid_barrier(GridBar* gb, unsigned G, unsigned& gen) {
 // 64-bit load per lane until none is zero (acquire), and forms the
 // sequential sum in slice order from the lanes' values.  vals and incl (LDS
 // [G]) receive the values and the running sums.
-__device__ bool part_barrier(GridBar* gb, unsigned long long* cur, unsigned long long* nxt,
+__device__ bool part_barrier(int* err, unsigned long long* cur, unsigned long long* nxt,
                              double loc, unsigned G,
                              double* vals, double* incl, double& tot) {
     __shared__ int ok;
@@ -877,9 +920,9 @@ __device__ bool part_barrier(GridBar* gb, unsigned long long* cur, unsigned long
             }
             if (__all(mine)) break;
             if (++n > (1u << 18) ||
-                __hip_atomic_load(&gb->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
                 if (l == 0) {
-                    __hip_atomic_store(&gb->err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     ok = 0;
                 }
                 break;
@@ -986,8 +1029,7 @@ __device__ int32_t range_pick(int64_t b, int64_t e, double target, Wf w,
     return r;
 }
 
-__global__ void __launch_bounds__(RT) k_accept_res(AcceptDev a, GridBar* gb,
-                                                   unsigned long long* part) {
+__global__ void __launch_bounds__(RT) k_accept_res(AcceptDev a, unsigned long long* part) {
 #pragma clang fp contract(off)
     constexpr int PU = 16;  // residual elements per thread with their loads in flight together
     __shared__ double sd[RT / 64];
@@ -995,11 +1037,7 @@ __global__ void __launch_bounds__(RT) k_accept_res(AcceptDev a, GridBar* gb,
     const unsigned G = gridDim.x;
     const int wg = blockIdx.x, t = threadIdx.x, lane = t & 63;
     const int64_t V = a.V, M = a.M;
-    unsigned gen = 0;
-    // row statistics: one wave per row, rows spread over the workgroups
-    for (int64_t r = (int64_t)wg * (RT / 64) + (t >> 6); r <= M; r += (int64_t)G * (RT / 64))
-        row_stat_wave(a, r, lane);
-    if (!grid_barrier(gb, G, gen)) return;
+    int* err = (int*)a.margin + 1;
     const int64_t slice = (V + G - 1) / G;
     const int64_t s0 = min(V, (int64_t)wg * slice), s1 = min(V, s0 + slice);
     uint64_t rng = *a.rng;
@@ -1009,7 +1047,7 @@ __global__ void __launch_bounds__(RT) k_accept_res(AcceptDev a, GridBar* gb,
     const double* Pc = a.p;  // the latest residual
 #define ROW(c) ((c) < 0 ? a.base_row : a.rows + (int64_t)(c) * V)
     for (int64_t step = 0; step <= M; ++step) {
-        const RowStats st = a.stats[cur + 1];
+        const RowStats st = row_stat_chunks(a.rc, cur + 1, lane);
         const float* lg = ROW(cur);
         double T = st.sum;
         bool have_res = false;
@@ -1071,7 +1109,7 @@ __global__ void __launch_bounds__(RT) k_accept_res(AcceptDev a, GridBar* gb,
                 ++pass;
                 Pc = Pn;
                 double tot;
-                if (!part_barrier(gb, partn, partx, loc, G, pvals, pincl, tot)) return;
+                if (!part_barrier(err, partn, partx, loc, G, pvals, pincl, tot)) return;
                 if (tot > 0) {
                     T = tot;
                     have_res = true;
@@ -1139,9 +1177,10 @@ __global__ void __launch_bounds__(RT) k_accept_res(AcceptDev a, GridBar* gb,
         break;
     }
 #undef ROW
+    // (not to *a.rng: a workgroup that starts late still reads it)
     if (wg == 0 && t == 0) {
         a.out[0] = nacc;
-        *a.rng = rng;
+        *a.rng_out = rng;
         *a.margin = mg;
     }
 }
@@ -1237,28 +1276,31 @@ hipError_t launch_accept_multi(hipStream_t st, const AcceptDev* d_arr, int n) {
     return hipGetLastError();
 }
 
-constexpr size_t ACC_RES_BAR = (sizeof(GridBar) + 255) & ~(size_t)255;
-size_t accept_residual_scratch_bytes() { return ACC_RES_BAR + 3 * ACC_RES_WG * sizeof(double); }
+size_t accept_residual_scratch_bytes() { return 3 * ACC_RES_WG * sizeof(double); }
 
 // RESIDUAL acceptance over ACC_RES_WG workgroups, launched cooperatively so
-// that all of them are resident for the grid barriers.  scratch: the
-// barrier flags and error word and the slices' partial-sum words (three
-// sets), all zeroed here; a.p holds two residual buffers of V doubles.
-hipError_t launch_accept_residual(hipStream_t st, const AcceptDev& a, void* scratch) {
-    GridBar* gb = (GridBar*)scratch;
-    unsigned long long* part = (unsigned long long*)((uint8_t*)scratch + ACC_RES_BAR);
-    // flags, error word and partial-sum words: zero
-    hipError_t e = hipMemsetAsync(gb, 0, accept_residual_scratch_bytes(), st);
+// that all of them are resident for the reduction barriers.  scratch: the
+// slices' partial-sum words (three sets), cleared by the statistics launch;
+// a.p holds two residual buffers of V doubles; a time-out is reported in the
+// word after *a.margin (the caller's, zero before).
+hipError_t launch_residual_stats(hipStream_t st, const float* base_row, const float* rows,
+                                 int64_t nrows, int64_t V, float temp, const RowChunks& rc,
+                                 void* scratch) {
+    const dim3 grid((unsigned)rc.nch, (unsigned)nrows);
+    hipLaunchKernelGGL(k_row_max, grid, dim3(256), 0, st, base_row, rows, V, rc);
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    AcceptDev ac = a;
-    void* args[] = {(void*)&ac, (void*)&gb, (void*)&part};
-    return hipLaunchCooperativeKernel((const void*)k_accept_res, dim3(ACC_RES_WG), dim3(RT), args,
-                                      0, st);
+    const bool vec = V % 4 == 0 && ((uintptr_t)base_row % 16) == 0 &&
+                     (nrows == 1 || ((uintptr_t)rows % 16) == 0);
+    hipLaunchKernelGGL(vec ? k_row_sum_res<true> : k_row_sum_res<false>, grid, dim3(256), 0, st,
+                       base_row, rows, V, temp, rc, (unsigned long long*)scratch, 3 * ACC_RES_WG);
+    return hipGetLastError();
 }
 
-int accept_residual_error(const void* scratch, hipStream_t st, int* err) {
-    return hipMemcpyAsync(err, (const uint8_t*)scratch + offsetof(GridBar, err), sizeof(int),
-                          hipMemcpyDeviceToHost, st) == hipSuccess
-               ? 0
-               : -1;
+hipError_t launch_accept_residual(hipStream_t st, const AcceptDev& a, void* scratch) {
+    unsigned long long* part = (unsigned long long*)scratch;
+    AcceptDev ac = a;
+    void* args[] = {(void*)&ac, (void*)&part};
+    return hipLaunchCooperativeKernel((const void*)k_accept_res, dim3(ACC_RES_WG), dim3(RT), args,
+                                      0, st);
 }

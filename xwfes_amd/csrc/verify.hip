@@ -1578,20 +1578,21 @@ AccPlan acc_plan(const ftx_accept_args* a) {
                           : 0;
     P.off_small = P.off_p + align256(pb);
     const size_t out_b = ((size_t)(M + 2) * 4 + 7) & ~(size_t)7;
-    P.head_b = 24 + out_b;  // rng | sampler rng | margin | pad | out
+    P.head_b = 32 + out_b;  // rng | sampler rng | margin | error | rng after | out
     P.small_b = P.head_b + (size_t)M * 12 + 64;
     P.off_rs = P.off_small + align256(P.small_b);
     P.bytes = P.off_rs + align256(row_stats_scratch_bytes(M + 1, V)) + 256;
     return P;
 }
 
-// the small block of a in host memory: rng | sampler rng | margin | pad |
+// the small block of a in host memory: rng | sampler rng | margin | error |
 // out | props | parents | pd
 void acc_fill_small(const ftx_accept_args* a, const AccPlan& P, uint8_t* pin) {
     const int64_t M = a->M;
     *(uint64_t*)pin = *a->rng;
     *(uint64_t*)(pin + 8) = a->sampler_rng ? *a->sampler_rng : 0;
     *(float*)(pin + 16) = INFINITY;
+    *(int32_t*)(pin + 20) = 0;
     int32_t* h_props = (int32_t*)(pin + P.head_b);
     int32_t* h_par = h_props + M;
     float* h_pd = (float*)(h_par + M);
@@ -1620,12 +1621,13 @@ AcceptDev acc_dev(const ftx_accept_args* a, const AccPlan& P, uint8_t* ws, uint8
     ad.pd = (const float*)(ad.parents + M);
     ad.mode = a->mode;
     ad.temp = a->temp;
-    ad.rng = (uint64_t*)d_small;
+    ad.rng = (const uint64_t*)d_small;
+    ad.rng_out = (uint64_t*)(d_small + 24);
     ad.sampler_rng = (uint64_t*)(d_small + 8);
     ad.top_k = a->top_k;
     ad.top_p = a->top_p;
     ad.p = (double*)(ws + P.off_p);
-    ad.out = (int32_t*)(d_small + 24);
+    ad.out = (int32_t*)(d_small + 32);
     ad.margin = (float*)(d_small + 16);
     return ad;
 }
@@ -1634,23 +1636,29 @@ void* acc_res_scratch(const ftx_accept_args* a, const AccPlan& P, uint8_t* ws) {
     return ws + P.off_p + align256(2 * (size_t)a->V * 8);
 }
 
-int acc_row_stats(ftx_ctx* ctx, const ftx_accept_args* a, const AcceptDev& ad) {
+int acc_row_stats(ftx_ctx* ctx, const ftx_accept_args* a, const AcceptDev& ad, void* res_scratch) {
     TraceScope ts(ctx);
-    FTX_HIP(ctx, launch_row_stats(ctx->stream, a->base_row, a->rows, a->M + 1, a->V, a->temp,
-                                  ad.with_sum, ad.rc));
+    if (a->mode == FTX_ACCEPT_RESIDUAL)
+        FTX_HIP(ctx, launch_residual_stats(ctx->stream, a->base_row, a->rows, a->M + 1, a->V, a->temp,
+                                           ad.rc, res_scratch));
+    else
+        FTX_HIP(ctx, launch_row_stats(ctx->stream, a->base_row, a->rows, a->M + 1, a->V, a->temp,
+                                      ad.with_sum, ad.rc));
     ts.end(TK_ROW_STATS, (double)(a->M + 1) * a->V * 4, ad.with_sum ? 2 : 1);
     return FTX_OK;
 }
 
 // the outputs of a from its small block's head, copied back to host memory
 int acc_results(ftx_ctx* ctx, const ftx_accept_args* a, const uint8_t* pin) {
-    const int32_t* h_out = (const int32_t*)(pin + 24);
+    if (*(const int32_t*)(pin + 20))
+        return ftx_fail(ctx, FTX_E_DEVICE, "acceptance: a grid barrier timed out");
+    const int32_t* h_out = (const int32_t*)(pin + 32);
     const int32_t na = h_out[0];
     if (na < 0 || na > a->M) return ftx_fail(ctx, FTX_E_DEVICE, "acceptance returned a bad count");
     *a->n_acc = na;
     *a->bonus = h_out[1];
     for (int32_t i = 0; i < na; ++i) a->accepted[i] = h_out[2 + i];
-    *a->rng = *(const uint64_t*)pin;
+    *a->rng = *(const uint64_t*)(pin + 24);
     if (a->sampler_rng) *a->sampler_rng = *(const uint64_t*)(pin + 8);
     if (a->margin) *a->margin = *(const float*)(pin + 16);
     return FTX_OK;
@@ -1680,10 +1688,9 @@ int ftx_accept(ftx_ctx* ctx, const ftx_accept_args* a) {
     uint8_t* d_small = ws + P.off_small;
     FTX_HIP(ctx, hipMemcpyAsync(d_small, pin, P.small_b, hipMemcpyHostToDevice, st));
     const AcceptDev ad = acc_dev(a, P, ws, d_small);
-    rc = acc_row_stats(ctx, a, ad);
-    if (rc) return rc;
-    int bar_err = 0;
     void* res_scratch = acc_res_scratch(a, P, ws);
+    rc = acc_row_stats(ctx, a, ad, res_scratch);
+    if (rc) return rc;
     {
         TraceScope ts(ctx);
         if (a->mode == FTX_ACCEPT_RESIDUAL)
@@ -1693,13 +1700,7 @@ int ftx_accept(ftx_ctx* ctx, const ftx_accept_args* a) {
         ts.end(TK_ACCEPT, (double)a->V * 4);
     }
     FTX_HIP(ctx, hipMemcpyAsync(pin, d_small, P.head_b, hipMemcpyDeviceToHost, st));
-    if (a->mode == FTX_ACCEPT_RESIDUAL && accept_residual_error(res_scratch, st, &bar_err)) {
-        (void)hipStreamSynchronize(st);  // the copy into the pinned block has landed
-        return ftx_fail(ctx, FTX_E_DEVICE, "acceptance: copy of the barrier state failed");
-    }
     FTX_HIP(ctx, hipStreamSynchronize(st));
-    if (bar_err)
-        return ftx_fail(ctx, FTX_E_DEVICE, "acceptance: a grid barrier timed out");
     return acc_results(ctx, a, pin);
 }
 
@@ -1743,10 +1744,9 @@ int ftx_accept_batch(ftx_ctx* ctx, const ftx_accept_args* args, int n) {
     }
     FTX_HIP(ctx, hipMemcpyAsync(d_small, pin, pin_total, hipMemcpyHostToDevice, st));
     for (int i = 0; i < n; ++i) {
-        rc = acc_row_stats(ctx, &args[i], ad[i]);
+        rc = acc_row_stats(ctx, &args[i], ad[i], acc_res_scratch(&args[i], P[i], ws + ws_off[i]));
         if (rc) return rc;
     }
-    int bar_err[FTX_MAX_SEQ] = {};
     for (int i = 0; i < n; ++i) {
         if (args[i].mode != FTX_ACCEPT_RESIDUAL) continue;
         TraceScope ts(ctx);
@@ -1759,15 +1759,8 @@ int ftx_accept_batch(ftx_ctx* ctx, const ftx_accept_args* args, int n) {
         ts.end(TK_ACCEPT, (double)args[0].V * 4 * nmulti);
     }
     FTX_HIP(ctx, hipMemcpyAsync(pin, d_small, adv_off, hipMemcpyDeviceToHost, st));
-    for (int i = 0; i < n; ++i)
-        if (args[i].mode == FTX_ACCEPT_RESIDUAL &&
-            accept_residual_error(acc_res_scratch(&args[i], P[i], ws + ws_off[i]), st, &bar_err[i])) {
-            (void)hipStreamSynchronize(st);  // the copy into the pinned block has landed
-            return ftx_fail(ctx, FTX_E_DEVICE, "acceptance: copy of the barrier state failed");
-        }
     FTX_HIP(ctx, hipStreamSynchronize(st));
     for (int i = 0; i < n; ++i) {
-        if (bar_err[i]) return ftx_fail(ctx, FTX_E_DEVICE, "acceptance: a grid barrier timed out");
         rc = acc_results(ctx, &args[i], pin + pin_off[i]);
         if (rc) return rc;
     }
