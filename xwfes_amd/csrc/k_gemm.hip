@@ -37,7 +37,7 @@
 // MFMA's rounding): 0.7e-7 to 0.9e-7 against 64 bits where the generic
 // kernel's fp32 sums had 0.8e-7 to 1.0e-7.  Measured (whole call): 48 tokens of
 // Q4_K 14336 x 4096 4.70 ms on the generic kernel -> 66 us; 16 tokens of Q8_0
-// 4096 x 4096 473 -> 50 us.
+// 4096 x 4096 473 -> 41 us.
 //
 // Column-axpy form (ffn_down in the reference orientation, n_ff rows of
 // n_embd columns, Q4_K blocks along the output): per 32-row slice the
@@ -493,13 +493,17 @@ template <>
 struct MmW<FTX_Q4_K_ROWS> : MmW<FTX_Q4_K> {};
 template <>
 struct MmW<FTX_Q8_0> {
-    v2i q[MM_NT][8];       // the lane's 8 quant bytes of each 32-block
-    uint32_t d[MM_NT][8];  // the fp16 block scales
+    // as loaded: the whole blocks 2 kq and 2 kq + 1 of the step (32 quant bytes
+    // each, then their scales); after mm_arrange, q[t][2 b], [2 b + 1] the
+    // lane's 8 quant bytes of block b, and d[t][g] the scales of blocks 2 g and
+    // 2 g + 1
+    uint32_t q[MM_NT][16];
+    uint32_t d[MM_NT][4];
 };
 template <>
 struct MmW<FTX_Q4_0> {
-    uint32_t q[MM_NT][8];
-    uint32_t d[MM_NT][8];
+    uint32_t q[MM_NT][8];  // (the same with 16 bytes a block, one word a lane and block)
+    uint32_t d[MM_NT][4];
 };
 template <>
 struct MmW<FTX_Q6_K> : MmW<FTX_Q6_K_MMT> {};
@@ -515,7 +519,6 @@ __host__ __device__ constexpr bool mm_q6k(int dt) { return dt == FTX_Q6_K_MMT ||
 
 // loads of any alignment (the hardware takes them as they come)
 struct __attribute__((packed)) mm_u16 { uint16_t v; };
-struct __attribute__((packed)) mm_u32 { uint32_t v; };
 struct __attribute__((packed)) mm_u64 { v2i v; };
 struct __attribute__((packed)) mm_u128 { v4i v; };
 
@@ -573,9 +576,7 @@ __device__ __forceinline__ void mm_ptrs(MmPtr& p, const MmSegDev& sg, int64_t rb
             p.tile[t] = 0;
             p.lh[t] = r;
             p.ld[t] = 0;
-            p.lq[t] = r + (DT == FTX_Q8_0 ? 2 + 8 * kq
-                           : DT == FTX_Q4_0 ? 2 + 4 * kq
-                           : DT == FTX_F16  ? 16 * kq
+            p.lq[t] = r + (DT == FTX_F16  ? 16 * kq
                            : DT == FTX_Q4_K_ROWS ? 16 + 8 * kq
                                             : 64 * (kq & 1) + 8 * (kq >> 1));
         } else if constexpr (DT == FTX_Q4_K) {
@@ -638,20 +639,33 @@ __device__ __forceinline__ void mm_load(MmW<DT>& o, const MmPtr& p, int sb) {
             }
             o.sc[t] = ((const mm_u128*)(p.base + (int64_t)p.nsb * 192 + (int64_t)sb * 16 + p.lh[t]))->v;
             o.d[t] = ((const mm_u16*)(p.base + (int64_t)p.nsb * 208 + (int64_t)sb * 2 + p.lh[t]))->v;
-        } else if constexpr (mm_stored(DT) && DT != FTX_Q4_K_ROWS) {
+        } else if constexpr (DT == FTX_Q8_0 || DT == FTX_Q4_0) {
+            // whole blocks per lane: 2 (Q4_0) or 4 (Q8_0) wide loads and two
+            // scales for the step instead of a narrow load and a scale per
+            // block (16 loads, each lane row touching every block's lines);
+            // mm_arrange then passes the words between the kq lanes.  24
+            // tokens of an expert chunk of Q4_0 14336 x 4096: 170 -> 132 us,
+            // 16 tokens of Q8_0 4096 x 4096 50 -> 41 us (whole calls)
+            constexpr int BB = DT == FTX_Q8_0 ? 34 : 18, NV = (BB - 2) / 16;
+            const int kq = (threadIdx.x >> 4) & 3;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                // (past the row's last block: that one again, against zeros)
+                const uint8_t* b = p.base + p.lh[t] + (uint32_t)(min(8 * sb + 2 * kq + h, p.nblk - 1) * BB);
+                o.d[t][h] = ((const mm_u16*)b)->v;
+#pragma unroll
+                for (int v = 0; v < NV; ++v) {
+                    const v4i x = ((const mm_u128*)(b + 2 + 16 * v))->v;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o.q[t][(4 * NV) * h + 4 * v + e] = (uint32_t)x[e];
+                }
+            }
+        } else if constexpr (DT == FTX_F16) {
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 // (past the row's last block: that one again, against zeros)
                 const int64_t blk = min(8 * sb + j, p.nblk - 1);  // uniform
-                if constexpr (DT == FTX_Q8_0) {
-                    o.q[t][j] = ((const mm_u64*)(p.base + blk * 34 + p.lq[t]))->v;
-                    o.d[t][j] = ((const mm_u16*)(p.base + blk * 34 + p.lh[t]))->v;
-                } else if constexpr (DT == FTX_Q4_0) {
-                    o.q[t][j] = ((const mm_u32*)(p.base + blk * 18 + p.lq[t]))->v;
-                    o.d[t][j] = ((const mm_u16*)(p.base + blk * 18 + p.lh[t]))->v;
-                } else {
-                    o.b[t][j] = __builtin_bit_cast(v8h, ((const mm_u128*)(p.base + blk * 64 + p.lq[t]))->v);
-                }
+                o.b[t][j] = __builtin_bit_cast(v8h, ((const mm_u128*)(p.base + blk * 64 + p.lq[t]))->v);
             }
         } else if constexpr (DT == FTX_Q4_K || DT == FTX_Q4_K_ROWS) {
 #pragma unroll
@@ -670,6 +684,62 @@ __device__ __forceinline__ void mm_load(MmW<DT>& o, const MmPtr& p, int sb) {
 #pragma unroll
             for (int v = 0; v < 2; ++v) o.q[t][v] = mm_ld16(p.rs, p.lq[t], so + 16 * v);
             o.d[t] = mm_ld16(p.rs, p.lh[t], so);
+        }
+    }
+}
+
+// a's upper 32 lanes with b's lower 32; a's odd 16-lane rows with b's even ones
+__device__ __forceinline__ void swap32(uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+__device__ __forceinline__ void swap16(uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+}
+// four registers by the four 16-lane rows, transposed: register g of row k
+// gets register k of row g
+__device__ __forceinline__ void rows4(uint32_t& a, uint32_t& b, uint32_t& c, uint32_t& d) {
+    swap32(a, c);
+    swap32(b, d);
+    swap16(a, b);
+    swap16(c, d);
+}
+
+// loaded blocks -> the lane's words of every block (see MmW)
+template <int DT>
+__device__ __forceinline__ void mm_arrange(MmW<DT>& o) {
+    if constexpr (DT == FTX_Q8_0 || DT == FTX_Q4_0) {
+#pragma unroll
+        for (int t = 0; t < MM_NT; ++t) {
+            constexpr int L = DT == FTX_Q8_0 ? 2 : 1;  // words per lane and block
+            uint32_t w[8 * L];
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int l = 0; l < L; ++l) {
+                    // word l of lane row k is word L k + l of its block
+                    uint32_t* q = &o.q[t][4 * L * h];
+                    uint32_t a = q[l], b = q[L + l], c = q[2 * L + l], d = q[3 * L + l];
+                    rows4(a, b, c, d);
+                    w[L * (0 + h) + l] = a;
+                    w[L * (2 + h) + l] = b;
+                    w[L * (4 + h) + l] = c;
+                    w[L * (6 + h) + l] = d;
+                }
+#pragma unroll
+            for (int i = 0; i < 8 * L; ++i) o.q[t][i] = w[i];
+            uint32_t a = o.d[t][0] | (o.d[t][1] << 16), c = a;
+            swap32(a, c);
+            uint32_t b = a, d = c;
+            swap16(a, b);
+            swap16(c, d);
+            o.d[t][0] = a;
+            o.d[t][1] = b;
+            o.d[t][2] = c;
+            o.d[t][3] = d;
         }
     }
 }
@@ -791,7 +861,7 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
 
     // one 256-element step from LDS buffer `buf` with weights `wc`; the
     // next step's copies and weights (into `wn`) are issued first
-    auto step = [&](int sb, int buf, const MmW<DT>& wc, MmW<DT>& wn) {
+    auto step = [&](int sb, int buf, MmW<DT>& wc, MmW<DT>& wn) {
         __builtin_amdgcn_s_waitcnt(0x0F70);  // this step's fragments and weights
         __syncthreads();                     // every wave is done with the other buffer
         // Q4_K: the step's sub-block sums, loaded before the next step's
@@ -819,6 +889,7 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
         // scheduler would otherwise sink the weight loads below the MFMAs
         // to save registers, and their latency would no longer be hidden)
         __builtin_amdgcn_sched_barrier(0);
+        mm_arrange<DT>(wc);
         v2h scp[MM_NT][4], scn[MM_NT][4];  // Q4_K: sc and -1024 sc per sub-block, fp16 pairs
         v4h mnh[MM_NT];                    // Q4_K: the 4 mins of the lane's K slots
         if constexpr (DT == FTX_Q4_K) {
@@ -933,11 +1004,11 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
                     bw[t] = v8h{h0[0], h0[1], h1[0], h1[1], h2[0], h2[1], h3[0], h3[1]};
                     bs[t] = bsk[t][j];
                 } else if constexpr (DT == FTX_Q8_0) {
-                    bw[t] = i8x8(wc.q[t][j]);
-                    bs[t] = h2f((uint16_t)wc.d[t][j]);
+                    bw[t] = i8x8(v2i{(int)wc.q[t][2 * j], (int)wc.q[t][2 * j + 1]});
+                    bs[t] = h2f((uint16_t)(wc.d[t][j >> 1] >> (16 * (j & 1))));
                 } else if constexpr (DT == FTX_Q4_0) {
                     bw[t] = nib8(wc.q[t][j], 8.f);
-                    bs[t] = h2f((uint16_t)wc.d[t][j]);
+                    bs[t] = h2f((uint16_t)(wc.d[t][j >> 1] >> (16 * (j & 1))));
                 } else if constexpr (DT == FTX_F16) {
                     bw[t] = wc.b[t][j];
                     bs[t] = 0.f;
