@@ -10,7 +10,11 @@
 // bf16 (q - 8, q or q - 32: at most 8 bits).  Three MFMAs per product; every
 // product is exact and the only rounding is that of the fp32 sums.
 //   Q4_0  d (q - 8)         Q8_0  d q            one A per 32 columns
-//   Q6_K  (d sc) (q - 32)                         one A per 16 columns
+//   Q6_K  d (sc (q - 32))                         one A per 256 columns: the
+//         integers (at most 4096) as two bf16 limbs, nearest and rest, five
+//         MFMAs (third limb x rest, 2^-26 of the product, is left out); with
+//         d sc in A, one per 16 columns, the splits took three quarters of
+//         the time
 //   Q4_K  (d sc) (q - 8) - (dmin m - 8 d sc)      one A per 32 columns; the min
 //         term is a product of its own, h (3 limbs) x its 3 limbs, with the
 //         four 32-column sub-blocks as B columns (centred on q = 8 the two
@@ -30,8 +34,9 @@
 // work (about 100 VALU instructions per 32 x 32 weights), above that the limb
 // splits (52 VALU per 32 x 32 weights and 16 tokens) and MFMAs.
 // Measured, one launch (before: the generic kernel, or Q6_K's 8-token chunks):
-// Q4_0 14336 x 4096, 24 tokens 2013 -> 35.9 us; Q6_K, 256 tokens 531 -> 214 us
-// (140 TFLOP/s); up to 8 tokens of Q8_0 / Q4_0 go to k_axpy_few below.  Error against 64 bits 0.8e-7 to 1.4e-7 (1000 to 14336
+// Q4_0 14336 x 4096, 24 tokens 2013 -> 35.9 us; Q6_K, 256 tokens 531 -> 141 us
+// (213 TFLOP/s; 219 with d sc in A and two workgroups a CU assumed by the split
+// rule); up to 8 tokens of Q8_0 / Q4_0 go to k_axpy_few below.  Error against 64 bits 0.8e-7 to 1.4e-7 (1000 to 14336
 // rows) where the fp32 sums of the generic kernel had 1.6e-7 to 5.7e-7.
 #include <algorithm>
 
@@ -117,6 +122,28 @@ __device__ __forceinline__ v8bf sbytes(uint32_t x, uint32_t y) {
     v.w = pack_hi((float)(int8_t)(y >> 16), (float)(int8_t)(y >> 24));
     return __builtin_bit_cast(v8bf, v);
 }
+// Q6_K: the integers enter as multiples of 2^-12 and d times 2^12, which
+// keeps the limbs of activations down to 1e-30 clear of the subnormal range
+constexpr float Q6_BS = 1.f / 4096;
+// a = hi + lo of integers up to 4096 (times Q6_BS): the nearest bf16 and the
+// rest (exact, at most 8 bits)
+__device__ __forceinline__ void split2(const float* a, v8bf* hl) {
+    typedef float v2f __attribute__((ext_vector_type(2)));
+    typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+    uint32_t p[2][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const v2f x = {a[2 * i], a[2 * i + 1]};
+        p[0][i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, v2bf));
+        p[1][i] = pack_hi(x[0] - __uint_as_float(p[0][i] << 16),
+                          x[1] - __uint_as_float(p[0][i] & 0xFFFF0000u));
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const uint4 v = {p[k][0], p[k][1], p[k][2], p[k][3]};
+        hl[k] = __builtin_bit_cast(v8bf, v);
+    }
+}
 // 4 bytes 0..127 minus `bias` (at most 120), as signed bytes
 __device__ __forceinline__ uint32_t minus4(uint32_t x, uint32_t bias) {
     return (x + (0x80u - bias) * 0x01010101u) ^ 0x80808080u;
@@ -127,8 +154,9 @@ struct AxCfg {
     // LDS tiles of 16 columns x 32 rows (nibble types hold two in one)
     static constexpr int TILES = (DT == FTX_Q8_0 || DT == FTX_Q6_K) ? 8 : 4;
     static constexpr int SWZ = DT == FTX_Q8_0 ? 7 : 3;
-    // scales per row: blocks, Q4_K's scales then mins, Q6_K's 16-column scales
-    static constexpr int NSC = (DT == FTX_Q4_K || DT == FTX_Q6_K) ? 8 : 4;
+    // scales per row: blocks, Q4_K's scales then mins, Q6_K's 16-column
+    // integer scales then d
+    static constexpr int NSC = DT == FTX_Q6_K ? 9 : (DT == FTX_Q4_K ? 8 : 4);
     static constexpr int WORDS = (DT == FTX_Q8_0 || DT == FTX_Q6_K) ? 2 : 1;  // per lane and row
 };
 
@@ -265,10 +293,10 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
                 scl[(4 + 2 * hf + i) * 32 + at] = dmin * (float)((mn >> sh) & 0xFF) - 8.f * ds;
             }
         } else if constexpr (DT == FTX_Q6_K) {
-            const float d = sgn * h2f((uint16_t)o.s[1]);
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                scl[(4 * hf + i) * 32 + at] = d * (float)(int8_t)(o.s[0] >> (8 * i));
+                scl[(4 * hf + i) * 32 + at] = Q6_BS * (float)(int8_t)(o.s[0] >> (8 * i));
+            scl[8 * 32 + at] = sgn / Q6_BS * h2f((uint16_t)o.s[1]);  // (both halves the same value)
         } else {
             scl[hf * 32 + at] = sgn * h2f((uint16_t)o.s[0]);
             scl[(2 + hf) * 32 + at] = sgn * h2f((uint16_t)o.s[1]);
@@ -276,11 +304,13 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
     };
     // h of the lane's token (past M: the last one's, never stored) in each
     // 16-token tile, rows 8 kq .. + 7 of the slice (zero past n_in)
-    const float* hrow[MS];
-#pragma unroll
-    for (int ms = 0; ms < MS; ++ms)
-        hrow[ms] = a.h + (int64_t)min(m0 + 16 * ms + c, a.M - 1) * a.ldh;
     auto load_h = [&](float (&hv)[MS][8], int64_t I) {
+        const float* hrow[MS];
+        int cc = c;  // (formed anew per slice: held, the pointers spill)
+        asm("" : "+v"(cc));
+#pragma unroll
+        for (int ms = 0; ms < MS; ++ms)
+            hrow[ms] = a.h + (int64_t)min(m0 + 16 * ms + cc, a.M - 1) * a.ldh;
         const int64_t i = 32 * I + 8 * kq;
         if (32 * I + 32 <= a.n_in) {  // uniform
 #pragma unroll
@@ -350,6 +380,36 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
                             accm[ms] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l[q], bm[p - q], accm[ms], 0, 0, 0);
                 }
             }
+            if constexpr (DT == FTX_Q6_K) {
+                float d[8];
+                scales8(8, kq, d);
+                v8bf l[MS][3];
+#pragma unroll
+                for (int ms = 0; ms < MS; ++ms) {
+                    float t[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) t[e] = hv[ms][e] * d[e];
+                    split3(t, l[ms]);
+                }
+#pragma unroll
+                for (int n = 0; n < 8; ++n) {  // 16 columns
+                    const uint2 v = cols[slot(n, c)];
+                    float t[8];
+                    scales8(n, kq, t);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        t[e] *= (float)(int8_t)((e < 4 ? v.x : v.y) >> (8 * (e & 3)));
+                    v8bf bw[2];
+                    split2(t, bw);
+#pragma unroll
+                    for (int ms = 0; ms < MS; ++ms) {
+                        acc[n][ms] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l[ms][1], bw[1], acc[n][ms], 0, 0, 0);
+                        acc[n][ms] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l[ms][0], bw[1], acc[n][ms], 0, 0, 0);
+                        acc[n][ms] = mfma3(l[ms], bw[0], acc[n][ms]);
+                    }
+                }
+            }
+            if constexpr (DT != FTX_Q6_K) {
 #pragma unroll
             for (int b = 0; b < 4; ++b) {  // 32 columns
                 v8bf bw[2];
@@ -366,31 +426,26 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
                         bw[p] = sbytes(minus4((v.x >> (4 * (b & 1))) & 0x0F0F0F0Fu, 8),
                                        minus4((v.y >> (4 * (b & 1))) & 0x0F0F0F0Fu, 8));
                     }
-                } else {
+                } else {  // Q8_0
 #pragma unroll
                     for (int p = 0; p < 2; ++p) {
                         const uint2 v = cols[slot(2 * b + p, c)];
                         bw[p] = sbytes(v.x, v.y);
                     }
                 }
-                float d[DT == FTX_Q6_K ? 2 : 1][8];
-#pragma unroll
-                for (int p = 0; p < (DT == FTX_Q6_K ? 2 : 1); ++p)
-                    scales8(DT == FTX_Q6_K ? 2 * b + p : b, kq, d[p]);
+                float d[8];
+                scales8(b, kq, d);
 #pragma unroll
                 for (int ms = 0; ms < MS; ++ms) {
                     v8bf l[3];
                     float t[8];
 #pragma unroll
-                    for (int p = 0; p < 2; ++p) {
-                        if (p == 0 || DT == FTX_Q6_K) {
+                    for (int e = 0; e < 8; ++e) t[e] = hv[ms][e] * d[e];
+                    split3(t, l);
 #pragma unroll
-                            for (int e = 0; e < 8; ++e) t[e] = hv[ms][e] * d[DT == FTX_Q6_K ? p : 0][e];
-                            split3(t, l);
-                        }
-                        acc[2 * b + p][ms] = mfma3(l, bw[p], acc[2 * b + p][ms]);
-                    }
+                    for (int p = 0; p < 2; ++p) acc[2 * b + p][ms] = mfma3(l, bw[p], acc[2 * b + p][ms]);
                 }
+            }
             }
             // (the reads above before the next slice's writes)
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -579,7 +634,7 @@ bool axpy_supported(int dt, int64_t N) {
 }
 
 // 16-token tiles per workgroup, and splits over the rows: workgroups run two
-// to a CU in rounds of 512, each as long as its waves' slices (every eighth of
+// to a CU in rounds of 512 (four tiles: 256 VGPRs, one to a CU), each as long as its waves' slices (every eighth of
 // the split's) plus about two slices of start and reduction; the fewest slice
 // times, the fewest splits on ties, within `cap` partial floats (one split
 // writes y itself)
@@ -596,7 +651,7 @@ static int axpy_ms(int64_t M) { return M <= 16 ? 1 : (M <= 32 ? 2 : 4); }
 static int axpy_splits(int64_t M, int64_t n_in, int64_t N, size_t cap, int cu_count) {
     const int ms = axpy_ms(M);
     const int64_t wg = (N + AX_COLS - 1) / AX_COLS * ((M + 16 * ms - 1) / (16 * ms));
-    const int64_t nsl = (n_in + 31) / 32, slots = 2 * (cu_count > 0 ? cu_count : 256);
+    const int64_t nsl = (n_in + 31) / 32, slots = (ms == 4 ? 1 : 2) * (cu_count > 0 ? cu_count : 256);
     int best = 1;
     int64_t best_cost = -1;
     for (int64_t S = 1; S <= 32 && S <= nsl; ++S) {
