@@ -259,17 +259,17 @@ hipError_t launch_part_reduce(hipStream_t st, const float* part, int S, int64_t 
 
 // Large-M GEMMs (k_gemm.hip): activations as fp16 hi / lo planes [Mp][K] and
 // their 32-element sums [Mp][K / 32] (Mp = tokens padded to 64), weights as
-// the tiled Q4_K copy or the planar Q8_0 / Q4_0 copy.
+// the re-tiled copies, or the rows as they are stored (launch_mm_op).
 struct MmAct {
     _Float16 *xh, *xl, *sh, *sl;
     int64_t Mp, K;
 };
 struct MmSeg {
     const uint8_t* W;
-    int dt;             // FTX_Q4_K (tiled), FTX_Q8_0_MMT or FTX_Q4_0_MMT (re-tiled copies)
+    int dt;             // FTX_Q4_K (tiled), FTX_Q6_K_MMT, FTX_Q8_0_MMT, FTX_Q4_0_MMT (re-tiled copies), or stored rows
     int64_t N;          // rows
     int rpt;            // Q4_K tile rows
-    int64_t row_bytes;  // planar rows
+    int64_t row_bytes;  // stored rows
 };
 // output rows of sequence s (row0[s] <= m < row0[s + 1]) go to base[s] +
 // (m - row0[s]) * ld

@@ -24,8 +24,8 @@
 // two 16-column MFMA tiles) and a 64-token tile (four 16-row MFMA tiles);
 // the activation tile is staged in LDS 256 contraction elements at a time
 // (double-buffered, one barrier per stage) and shared by the eight waves,
-// which read their weights straight from the tiled (Q4_K) or planar (Q8_0,
-// Q4_0) copies the model keeps.  Split-K across workgroups where the tiles
+// which read their weights straight from the re-tiled copies the model
+// keeps.  Split-K across workgroups where the tiles
 // alone do not fill the device; partial sums then go to a buffer that the
 // reduce launch adds in split order with the epilogue (store, accumulate,
 // SwiGLU).
@@ -397,11 +397,11 @@ __global__ void __launch_bounds__(512) k_mm_prep_op(const float* __restrict__ x,
 // ---------------------------------------------------------------- row-dot
 
 struct MmSegDev {
-    const uint8_t* W;   // tiled (Q4_K) or planar (Q8_0 / Q4_0) copy
+    const uint8_t* W;   // re-tiled copy, or the rows as they are stored
     int64_t N;          // weight rows
     int64_t unit0;      // first 64-row unit of the segment in the launch
     int64_t col0;       // first output column of the segment
-    int64_t row_bytes;  // planar rows
+    int64_t row_bytes;  // stored rows
     int rpt;            // Q4_K tile rows (16 or 32)
 };
 

@@ -207,71 +207,6 @@ __global__ void __launch_bounds__(256) k_row_sum_res(const float* __restrict__ b
     if (t == 0) rc.csubf[r * rc.nch + c] = ((sd[0] + sd[1]) + sd[2]) + sd[3];
 }
 
-// Inverse-CDF pick over p[0..V) (double weights) by one block: thread t sums
-// the contiguous chunk [t * chunk, (t + 1) * chunk) in index order (eight
-// loads issued together), a block scan, then the crossing chunk scanned in
-// order.  Falls back to the last positive weight when rounding leaves no
-// crossing.
-__device__ int32_t block_pick(const double* __restrict__ p, int64_t V, float u) {
-    __shared__ double incl[NT];
-    __shared__ int32_t lastpos[NT];
-    __shared__ int32_t pick;
-    const int t = threadIdx.x;
-    const int64_t chunk = (V + NT - 1) / NT;
-    const int64_t b = t * chunk, e = min(V, b + chunk);
-    double cs = 0.0;
-    int32_t lp = -1;
-    for (int64_t i0 = b; i0 < e; i0 += 8) {
-        double v[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = i0 + k < e ? p[i0 + k] : 0.0;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            if (i0 + k >= e) break;
-            cs += v[k];
-            if (v[k] > 0) lp = (int32_t)(i0 + k);
-        }
-    }
-    incl[t] = cs;
-    lastpos[t] = lp;
-    if (t == 0) pick = -1;
-    __syncthreads();
-    for (int o = 1; o < NT; o <<= 1) {
-        const double add = t >= o ? incl[t - o] : 0.0;
-        const int32_t lpo = t >= o ? lastpos[t - o] : -1;
-        __syncthreads();
-        incl[t] += add;
-        if (lastpos[t] < 0) lastpos[t] = lpo;
-        __syncthreads();
-    }
-    const double tot = incl[NT - 1];
-    const double target = (double)u * tot;
-    const double ex = t ? incl[t - 1] : 0.0;
-    if (incl[t] > target && ex <= target && b < e) {
-        double c = ex;
-        bool found = false;
-        for (int64_t i0 = b; i0 < e && !found; i0 += 8) {
-            double v[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) v[k] = i0 + k < e ? p[i0 + k] : 0.0;
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                if (found || i0 + k >= e) break;
-                c += v[k];
-                if (c > target) {
-                    pick = (int32_t)(i0 + k);
-                    found = true;
-                }
-            }
-        }
-    }
-    __syncthreads();
-    int32_t r = pick;
-    if (r < 0) r = lastpos[NT - 1] >= 0 ? lastpos[NT - 1] : 0;
-    __syncthreads();
-    return r;
-}
-
 constexpr int SMAXK = 64;     // largest top-k of the device sampler
 constexpr int SMAXSUB = 4096; // largest sub-chunk count it takes (V <= 524288)
 constexpr int SMAXEQ = 1024;  // probabilities equal to the k-th kept for the tie break
@@ -592,34 +527,6 @@ __device__ int32_t sampler_pick(const float* __restrict__ lg, int64_t V, float m
     return r;
 }
 
-__device__ double block_sum(double v, double* sd) {
-    const int t = threadIdx.x;
-    sd[t] = v;
-    __syncthreads();
-    for (int o = NT / 2; o > 0; o >>= 1) {
-        if (t < o) sd[t] += sd[t + o];
-        __syncthreads();
-    }
-    const double r = sd[0];
-    __syncthreads();
-    return r;
-}
-
-// p[i] = exp((double)((l_i - mx)/T)) / sum, the target distribution
-__device__ void target_dist(const float* __restrict__ lg, int64_t V, float temp, float mx,
-                            double* p, double* sd) {
-#pragma clang fp contract(off)
-    double s = 0.0;
-    for (int64_t i = threadIdx.x; i < V; i += NT) {
-        const double e = exp((double)((lg[i] - mx) / temp));
-        p[i] = e;
-        s += e;
-    }
-    s = block_sum(s, sd);
-    for (int64_t i = threadIdx.x; i < V; i += NT) p[i] /= s;
-    __syncthreads();
-}
-
 // Row r's statistics from its chunk results, by one wave (lane l): first-max
 // argmax over the chunks, the exp sum over the sub-chunks (lane-strided sums
 // in index order, then a fixed tree).
@@ -689,13 +596,12 @@ __device__ __forceinline__ RowStats row_stat_chunks(const RowChunks& rc, int64_t
     return RowStats{best, bi, sum};
 }
 
-// Decisions by one workgroup: GREEDY and RESIDUAL (one-block form) finish
-// here; RATIO walks the chain and draws the bonus with the sampler.
+// Decisions by one workgroup (GREEDY and RATIO; RESIDUAL: k_accept_res):
+// RATIO walks the chain and draws the bonus with the sampler.
 __device__ void accept_wg(const AcceptDev& a) {
 #pragma clang fp contract(off)
-    __shared__ double sd[NT];
     __shared__ uint64_t rng;
-    __shared__ int32_t cur, nacc, bonus, next;
+    __shared__ int32_t cur, nacc, bonus;
     __shared__ float mg;
     __shared__ uint64_t srng;
     const int t = threadIdx.x;
@@ -737,7 +643,7 @@ __device__ void accept_wg(const AcceptDev& a) {
             }
         }
         __syncthreads();
-    } else if (a.mode == FTX_ACCEPT_RATIO) {
+    } else {  // RATIO
         if (t == 0) {
             uint64_t s = rng;
             int32_t k = 0;
@@ -773,66 +679,6 @@ __device__ void accept_wg(const AcceptDev& a) {
                                        STAT(c).amax, &srng);
         if (t == 0) bonus = b;
         __syncthreads();
-    } else {  // RESIDUAL
-        for (;;) {
-            const int32_t c = cur;
-            target_dist(ROW(c), V, a.temp, STAT(c).mx, a.p, sd);
-            if (t == 0) next = -2;
-            __syncthreads();
-            for (int64_t ch = 0; ch < a.M; ++ch) {
-                if (a.parents[ch] != c) continue;
-                __shared__ int32_t acc_flag;
-                if (t == 0) {
-                    const float* qc = a.q + ch * V;
-                    const int32_t tok = a.props[ch];
-                    const float pt = (float)a.p[tok];
-                    const float ratio = fminf(1.f, pt / fmaxf(qc[tok], 1e-9f));
-                    uint64_t s = rng;
-                    const float u = splitmix_float(s);
-                    rng = s;
-                    mg = fminf(mg, fabsf(u - ratio));
-                    acc_flag = u <= ratio;
-                    if (acc_flag) next = (int32_t)ch;
-                }
-                __syncthreads();
-                if (acc_flag) break;
-                // p <- norm(max(0, p - q_ch))
-                const float* qc = a.q + ch * V;
-                double s = 0.0;
-                for (int64_t i = t; i < V; i += NT) {
-                    const double r = a.p[i] - (double)qc[i];
-                    const double v = r > 0 ? r : 0;
-                    a.p[i] = v;
-                    s += v;
-                }
-                s = block_sum(s, sd);
-                if (s > 0) {
-                    for (int64_t i = t; i < V; i += NT) a.p[i] /= s;
-                    __syncthreads();
-                } else {
-                    target_dist(ROW(c), V, a.temp, STAT(c).mx, a.p, sd);
-                }
-            }
-            __syncthreads();
-            if (next < -1) {
-                __shared__ float ub2;
-                if (t == 0) {
-                    uint64_t s = rng;
-                    ub2 = splitmix_float(s);
-                    rng = s;
-                }
-                __syncthreads();
-                const int32_t b = block_pick(a.p, V, ub2);
-                if (t == 0) bonus = b;
-                __syncthreads();
-                break;
-            }
-            if (t == 0) {
-                a.out[2 + nacc++] = next;
-                cur = next;
-            }
-            __syncthreads();
-        }
     }
 #undef ROW
 #undef STAT

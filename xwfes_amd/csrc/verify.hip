@@ -60,7 +60,7 @@ struct ftx_model {
     bool has_ext = false;
     std::vector<float*> attn_bias;  // [qdim + 2 kdim] q | k | v bias per layer, or null
     std::vector<float*> qnorm, knorm;  // [hd] per layer, or null
-    // MoE layers: planar copies of the gate and up expert planes, the
+    // MoE layers: re-tiled copies of the gate and up expert planes, the
     // re-tiled down planes, the router bias as F32; shared buffers for the
     // routing tables, the gathered operand, the down operand, split partials,
     // and tmpo for shared experts
@@ -179,8 +179,8 @@ static bool dalloc(T** p, size_t n) {
 
 // The verify step for more than 8 tokens or for several sequences: every
 // projection over the tokens of all sequences at once, through the one-pass
-// GEMMs of k_gemm.hip where the weights allow (tiled Q4_K, planar Q8_0 /
-// Q4_0 copies) and the generic kernels otherwise; RoPE, the KV write and
+// GEMMs of k_gemm.hip where the weights allow (the re-tiled
+// copies) and the generic kernels otherwise; RoPE, the KV write and
 // attention per sequence against its own cache (Engine::forward,
 // src/engine.cpp:461-596, per sequence).  The caller has checked the
 // arguments.
@@ -1314,36 +1314,6 @@ int ftx_verify_step(ftx_ctx* ctx, ftx_model* m, ftx_kv* kv, const ftx_verify_arg
             TRACED(TK_DOWN, Md * D * f4 * (2.0 + fold_S),
                    launch_part_reduce(st, m->downpart, fold_S, D, M, m->x, D));
             fold_S = 0;
-        }
-        // more than 8 tokens on tiled K-quant weights (not the fused qkv
-        // epilogue): the row-dot MFMA kernel on 8-row chunks, each with its
-        // own activation prep
-        bool tiled_all = epi != EPI_QKV && M > 8 && mv_all(ts, nseg, K, 8) &&
-                         (epi != EPI_SWIGLU || mv_swiglu_supported(K));
-        for (int i = 0; tiled_all && i < nseg; ++i) tiled_all = m->mvt[tix0 + tix[i]] != nullptr;
-        if (tiled_all) {
-            auto chunks = [&]() -> hipError_t {
-                // one prep for every chunk's operand, then a launch per chunk
-                hipError_t e = launch_xq_prep(st, xin, ldx, normw, nullptr, 0, D, K, M, m->xq);
-                if (e != hipSuccess) return e;
-                for (int64_t c0 = 0; c0 < M; c0 += 8) {
-                    const int64_t mc = M - c0 < 8 ? M - c0 : 8;
-                    GemvSeg cs[3];
-                    for (int i = 0; i < nseg; ++i) {
-                        cs[i] = segs[i];
-                        cs[i].W = m->mvt[tix0 + tix[i]];
-                        cs[i].tiled = 1;
-                        cs[i].rpt = m->mvt_rpt[tix0 + tix[i]];
-                        if (cs[i].y) cs[i].y += c0 * cs[i].ldy;
-                    }
-                    e = launch_mv(st, cs, nseg, m->xq + (c0 / 8) * (int64_t)xq_chunk_bytes(K), K,
-                                  mc, epi, ctx->cu_count, normw != nullptr, eps, nullptr);
-                    if (e != hipSuccess) return e;
-                }
-                return hipSuccess;
-            };
-            TRACED(kind, bytes, chunks());
-            return FTX_OK;
         }
         // Q8_0 / Q4_0: the re-tiled copies where every segment has one type of
         // them (its launch has the norm in it)
