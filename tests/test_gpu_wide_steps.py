@@ -45,10 +45,9 @@ def weight(gctx, orc, rng, dt, rows, cols):
 
 
 def close(got, want, size):
-    """|got - want| against `size`, the sum of the products' magnitudes: an
-    activation split in two fp16 halves is off by at most 2^-23 of itself
-    (three bf16 limbs: exact), and sums of blocks in fp32, in chains of some
-    20 additions at most, by 20 x 2^-24 of it at worst: 2^-19 together, 2^-20
+    """|got - want| against `size`, the sum of the products' magnitudes: the
+    operands are exact (three bf16 limbs), and sums of blocks in fp32, in chains
+    of some 20 additions at most, are off by 20 x 2^-24 of it at worst; 2^-20
     asked for.  A misplaced operand moves a sum by about size / sqrt(terms)."""
     err = np.abs(got - want) / np.maximum(size, 1e-300)
     assert err.max() < 2.0 ** -20, err.max()
@@ -131,6 +130,40 @@ def test_matmul_many_rows(gctx, orc, dt, M, K, N):
     t.free()
     assert not got[4].any()
     close(got, x.astype(np.float64) @ w.T, np.abs(x.astype(np.float64)) @ np.abs(w).T)
+
+
+def outlier(gctx, orc, dt, M, size, down):
+    """One activation `size` times the rest of its row, against a weight of zero
+    (down: against zeros in every other column): the outputs it adds nothing
+    to, held to the magnitudes of the other products alone."""
+    rng = np.random.default_rng(dt + M)
+    K, N, k0 = 1024, 512, 300
+    w = (rng.standard_normal((K, N) if down else (N, K)) * 0.02).astype(np.float32)
+    if dt == P.Q4_K:
+        w = np.abs(w)  # a minimum of zero, so that zero is one of the block's values
+    if down:
+        w[k0, ::2] = 0
+    else:
+        w[:, k0] = 0
+    raw = orc.quantize(w, dt)
+    v = orc.dequant(raw, dt, w.shape[1], rows=w.shape[0]).reshape(w.shape).astype(np.float64)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[:, k0] = size
+    t = gctx.upload(raw, dt, w.shape[::-1])
+    got = gctx.down_axpy(x, t) if down else gctx.matmul(x, t)
+    t.free()
+    v = v if down else v.T
+    zero = v[k0] == 0
+    assert zero.sum() >= N // 2
+    rest = x.astype(np.float64)
+    rest[:, k0] = 0
+    close(got[:, zero], (rest @ v)[:, zero], (np.abs(rest) @ np.abs(v))[:, zero])
+
+
+@pytest.mark.parametrize("dt", [P.Q4_0, P.Q8_0, P.Q6_K, P.F16])
+@pytest.mark.parametrize("M,size", [(12, 1e8), (40, 1e20)])
+def test_matmul_keeps_small_activations_beside_an_outlier(gctx, orc, dt, M, size):
+    outlier(gctx, orc, dt, M, size, False)
 
 
 @pytest.mark.parametrize("dt,M", [(P.Q8_0, 4), (P.Q8_0, 12), (P.Q4_0, 12), (P.Q4_K, 12), (P.Q6_K, 12),

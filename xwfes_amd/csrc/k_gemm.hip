@@ -31,13 +31,14 @@
 // SwiGLU).
 //
 // The backend's single operations (launch_mm_op: ftx_matmul, ftx_expert_chunk)
-// run the same kernel over rows as they are stored and any fp32 activations
-// (scaled per row by a power of two, k_mm_prep_op); their sums are kept
+// run the same kernel over rows as they are stored and any fp32 activations, on
+// v_mfma_f32_16x16x32_bf16: activations as three bf16 limbs and weights'
+// integers as one or two, all exact (k_mm_prep_op); their sums are kept
 // tighter than the steps' (64-bit additions, alternating signs against the
-// MFMA's rounding): 0.7e-7 to 0.9e-7 against 64 bits where the generic
-// kernel's fp32 sums had 0.8e-7 to 1.0e-7.  Measured (whole call): 48 tokens of
-// Q4_K 14336 x 4096 4.70 ms on the generic kernel -> 66 us; 16 tokens of Q8_0
-// 4096 x 4096 473 -> 41 us.
+// MFMA's rounding): 0.6e-7 against 64 bits where the generic kernel's fp32 sums
+// had 0.9e-7.  Measured (whole call): 48 tokens of Q4_K 14336 x 4096 4.70 ms on
+// the generic kernel, 71 us here (66 with two fp16 halves, a third less operand
+// to copy); 16 tokens of Q8_0 4096 x 4096 473 -> 41 us.
 //
 // Column-axpy form (ffn_down in the reference orientation, n_ff rows of
 // n_embd columns, Q4_K blocks along the output): per 32-row slice the
@@ -49,8 +50,6 @@
 #include "quant_dev.h"
 
 namespace {
-
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 constexpr int MM_TOK = 64;              // tokens per workgroup tile
 constexpr int MM_MS = MM_TOK / 16;      // 16-token MFMA tiles
@@ -318,14 +317,17 @@ __global__ void __launch_bounds__(1024) k_mm_prep_row(float* __restrict__ x, int
 }
 
 // The operand of a backend operation: rows of any fp32 values (rows m < M;
-// elements past K up to the contraction's padded length Kp are zeros).  Row m
-// is scaled by the power of two that brings its largest finite value into
-// [2^9, 2^10), so that the hi and lo halves carry 22 bits of every element
-// down to 2^-13 of that value (and 2^-35 of it below) and the 32-element sums
-// stay finite; rscale[m] undoes it.  Workgroup = row m.
+// elements past K up to the contraction's padded length Kp are zeros), exactly:
+// three bf16 limbs by truncation (split3), planes [3][Mp / 16][Kp / 32][64][8].
+// Two fp16 halves (22 bits down to 2^-13 of a row's largest value) lost the rest
+// of a row with one outlier wherever the outlier meets a zero weight: 2.8e-7 at
+// 1e4 times the rest, 1.7e-5 at 1e6, against 0.9e-7 of the fp32 product chain.
+// Row m is scaled by the power of two that brings its largest finite value into
+// [1, 2), which keeps products and limbs inside the fp32 range; rscale[m] undoes
+// it.  Odd 32-element blocks enter negated (k_mm).  Workgroup = row m.
 __global__ void __launch_bounds__(512) k_mm_prep_op(const float* __restrict__ x, int64_t ldx,
                                                     int64_t K, int64_t Kp, int inter,
-                                                    _Float16* __restrict__ xh, _Float16* __restrict__ xl,
+                                                    __bf16* __restrict__ xb, int64_t plane,
                                                     v8bf* __restrict__ xs, float* __restrict__ rscale) {
 #pragma clang fp contract(off)
     struct __attribute__((packed, aligned(4))) f4 { float v[4]; };
@@ -347,9 +349,9 @@ __global__ void __launch_bounds__(512) k_mm_prep_op(const float* __restrict__ x,
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 8; ++i) mx = fmaxf(mx, red[i]);
-    // 2^e with mx 2^e in [2^9, 2^10); both factors normal
-    int e = mx > 0.f ? 9 - ilogbf(mx) : 0;
-    e = min(max(e, -118), 126);
+    // 2^e with mx 2^e in [1, 2); both factors normal
+    int e = mx > 0.f ? -ilogbf(mx) : 0;
+    e = min(max(e, -126), 126);
     const float s = ldexpf(1.f, e);
     if (t == 0) rscale[m] = ldexpf(1.f, -e);
     for (int64_t k = 4 * t; k < Kp; k += 2048) {
@@ -359,20 +361,24 @@ __global__ void __launch_bounds__(512) k_mm_prep_op(const float* __restrict__ x,
 #pragma unroll
             for (int i = 0; i < 4; ++i) o[i] = u.v[i] * s;
         }
-        _Float16 hv[4], lv[4];
+        const uint32_t neg = (k & 32) ? 0x80008000u : 0u;
+        float r[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) split_hl(o[i], hv[i], lv[i]);
-        if (!inter) {
-            const int64_t at = frag_at(m, k, Kp, false);
-            *(v4h*)(xh + at) = v4h{hv[0], hv[1], hv[2], hv[3]};
-            *(v4h*)(xl + at) = v4h{lv[0], lv[1], lv[2], lv[3]};
-        } else {
+        for (int i = 0; i < 4; ++i) r[i] = o[i];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int64_t at = frag_at(m, k + i, Kp, true);
-                xh[at] = hv[i];
-                xl[at] = lv[i];
+        for (int p = 0; p < 3; ++p) {
+            const uint32_t w0 = pack_hi(r[0], r[1]) ^ neg, w1 = pack_hi(r[2], r[3]) ^ neg;
+            __bf16* d = xb + p * plane;
+            if (!inter) {
+                *(uint2*)(d + frag_at(m, k, Kp, false)) = uint2{w0, w1};
+            } else {
+                // octet order: elements k, k + 2 side by side, k + 1, k + 3 four on
+                const int64_t at = frag_at(m, k, Kp, true);
+                *(uint32_t*)(d + at) = perm(w1, w0, 0x05040100u);
+                *(uint32_t*)(d + at + 4) = perm(w1, w0, 0x07060302u);
             }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) r[i] = r[i] - trunc_bf(r[i]);
         }
         float q = (o[0] + o[1]) + (o[2] + o[3]);
         q += __shfl_xor(q, 1, 64);
@@ -382,8 +388,7 @@ __global__ void __launch_bounds__(512) k_mm_prep_op(const float* __restrict__ x,
             // Q4_K's min operand: lane (token, kq) of fragment (16-token tile,
             // super-block, MFMA), element j = sub-block j's limb
             const int j = (int)(k / 32 % 8);
-            const float h = __uint_as_float(__float_as_uint(q) & 0xFFFF0000u), r = q - h;
-            const float md = __uint_as_float(__float_as_uint(r) & 0xFFFF0000u), l = r - md;
+            const float h = trunc_bf(q), u = q - h, md = trunc_bf(u), l = u - md;
             __bf16* f = (__bf16*)(xs + ((int64_t)(m >> 4) * (Kp / 256) + k / 256) * 128 + (m & 15)) + j;
             f[0 * 128] = f[1 * 128] = (__bf16)h;
             f[2 * 128] = f[3 * 128] = (__bf16)md;
@@ -509,13 +514,13 @@ template <>
 struct MmW<FTX_Q6_K> : MmW<FTX_Q6_K_MMT> {};
 template <>
 struct MmW<FTX_F16> {
-    v8h b[MM_NT][8];       // the operand itself
+    v8h b[MM_NT][8];       // 8 elements of every block
 };
 __host__ __device__ constexpr bool mm_stored(int dt) {
     return dt == FTX_Q8_0 || dt == FTX_Q4_0 || dt == FTX_Q6_K || dt == FTX_F16 || dt == FTX_Q4_K_ROWS;
 }
-// Q6_K operands (tiled or stored): the same registers
-__host__ __device__ constexpr bool mm_q6k(int dt) { return dt == FTX_Q6_K_MMT || dt == FTX_Q6_K; }
+// activation planes: three bf16 limbs (the backend's operations) or fp16 hi, lo
+__host__ __device__ constexpr int mm_planes(int dt) { return mm_stored(dt) ? 3 : 2; }
 
 // loads of any alignment (the hardware takes them as they come)
 struct __attribute__((packed)) mm_u16 { uint16_t v; };
@@ -758,6 +763,25 @@ __device__ __forceinline__ void bytes4_h(uint32_t w, v2h& lo, v2h& hi) {
 
 typedef __attribute__((address_space(3))) void lds_void;
 
+// Q6_K operands (tiled or stored), elements 32 j + 8 kq .. + 7 of the step
+// (half h = j / 4, 32-group g = j % 4 of it): their 6-bit quants, a byte each;
+// low nibbles from ql run 2 h + (g & 1) (high half of the byte for g >= 2),
+// two high bits from qh run h
+template <typename W>
+__device__ __forceinline__ void q6k_bytes(const W& wc, int t, int j, uint32_t& b0, uint32_t& b1) {
+    const int h = j >> 2, g = j & 3, run = 2 * h + (g & 1);
+    const v4i qv = wc.q[t][run >> 1], hv = wc.q[t][2];
+    const uint32_t w0 = (uint32_t)qv[2 * (run & 1)], w1 = (uint32_t)qv[2 * (run & 1) + 1];
+    const uint32_t h0 = (uint32_t)hv[2 * h], h1 = (uint32_t)hv[2 * h + 1];
+    b0 = ((w0 >> (4 * (g >> 1))) & 0x0F0F0F0Fu) | (((h0 >> (2 * g)) & 0x03030303u) << 4);
+    b1 = ((w1 >> (4 * (g >> 1))) & 0x0F0F0F0Fu) | (((h1 >> (2 * g)) & 0x03030303u) << 4);
+}
+// and the scale of their sub-block 2 j + kq / 2
+template <typename W>
+__device__ __forceinline__ int q6k_scale(const W& wc, int t, int j, int kq) {
+    return (int)(int8_t)(((uint32_t)wc.sc[t][j >> 1]) >> (8 * (2 * (j & 1) + (kq >> 1))));
+}
+
 template <bool D>
 struct MmAcc {
     typedef v4f T;
@@ -823,22 +847,30 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
     MmPtr wp;
     mm_ptrs<DT>(wp, sg, rbase, a.nsb, col, kq, a.nblk);
 
-    // the step's 16 MS fragments: block b = (hl, ms, j) = 8 (MS hl + ms) + j
-    // -> LDS offset b KB; wave w copies blocks BPW w .. BPW w + BPW - 1 (one
-    // (hl, ms) per wave: BPW divides 8)
-    constexpr int BPW = 16 * MS / MM_WAVES;
-    constexpr int BUF = MS * 16384;
+    // the step's 8 NP MS fragments: block b = (plane, ms, j) = 8 (MS plane +
+    // ms) + j -> LDS offset b KB; wave w copies blocks BPW w .. BPW w + BPW - 1
+    // (two planes: one (plane, ms) per wave, BPW divides 8)
+    constexpr int NP = mm_planes(DT), BPW = 8 * NP * MS / MM_WAVES;
+    constexpr int BUF = NP * MS * 8192;
     const int b0 = BPW * w, hl0 = b0 / (8 * MS), ms0 = (b0 / 8) % MS, j0 = b0 % 8;
-    const __amdgpu_buffer_rsrc_t xrs = mm_rsrc(hl0 ? a.xl : a.xh);
+    const __amdgpu_buffer_rsrc_t xrs = mm_rsrc(NP == 2 && hl0 ? a.xl : a.xh);
     const uint32_t xoff = (uint32_t)((mt0 + ms0) * nks * 64 * 8 * 2);  // bytes, uniform
     const uint32_t glane = (uint32_t)lane * 16;
     auto stage = [&](int sb, int buf) {
         if (XT && ms0 >= nsub) return;  // this wave's blocks belong to an unused token tile
-        const uint32_t so = xoff + (uint32_t)(sb * 8 + j0) * 1024;
 #pragma unroll
-        for (int i = 0; i < BPW; ++i)
+        for (int i = 0; i < BPW; ++i) {
+            uint32_t so;
+            if constexpr (NP == 2) {
+                so = xoff + (uint32_t)(sb * 8 + j0 + i) * 1024;
+            } else {
+                const int g = (b0 + i) / 8;  // (planes side by side: a.plane[0] bytes apart)
+                so = (uint32_t)(g / MS) * (uint32_t)a.plane[0] +
+                     (uint32_t)((mt0 + g % MS) * nks + sb * 8 + (b0 + i) % 8) * 1024;
+            }
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                xrs, (lds_void*)(mm_lds + buf * BUF + (b0 + i) * 1024), 16, glane, so + i * 1024, 0, 0);
+                xrs, (lds_void*)(mm_lds + buf * BUF + (b0 + i) * 1024), 16, glane, so, 0, 0);
+        }
     };
     auto frag = [&](int buf, int hl, int ms, int j) -> v8h {
         return *(const v8h*)(mm_lds + buf * BUF + ((hl * MS + ms) * 8 + j) * 1024 + lane * 16);
@@ -932,10 +964,11 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     const int h = 8 * (j & 3);
-                    bsk[t][j] = d * (float)((sc[j >> 2] >> h) & 0xFF);
-                    const float g = dmin * (float)((mn[j >> 2] >> h) & 0xFF) - 8.f * bsk[t][j];
-                    const float gh = __uint_as_float(__float_as_uint(g) & 0xFFFF0000u), r = g - gh;
-                    const float gm = __uint_as_float(__float_as_uint(r) & 0xFFFF0000u), gl = r - gm;
+                    const float ds = d * (float)((sc[j >> 2] >> h) & 0xFF);
+                    const float g = dmin * (float)((mn[j >> 2] >> h) & 0xFF) - 8.f * ds;
+                    bsk[t][j] = ds;
+                    const float gh = trunc_bf(g), r = g - gh;
+                    const float gm = trunc_bf(r), gl = r - gm;
                     g0[j] = (__bf16)((kq & 1) ? gm : gh);
                     g1[j] = (__bf16)(kq == 0 ? gl : (kq == 1 ? gh : 0.f));
                 }
@@ -957,6 +990,84 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
         v4f tmp[MM_NT][MS];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {  // 32-element K-step (sub-block / block) of the step
+            if constexpr (mm_stored(DT)) {
+                // the backend's operations: a fresh sum per 32 elements, the
+                // small limbs first (their terms are then rounded at their own
+                // size), added in fp32 with the block scale, four blocks to one
+                // 64-bit addition.  The MFMA rounds its sums down (toward
+                // minus infinity): every other block's activations are negated
+                // and its sum subtracted, and the shares cancel instead of
+                // adding up.
+                constexpr int NL = DT == FTX_Q6_K || DT == FTX_F16 ? 2 : 1;  // limbs of a weight
+                v8bf xl[3][MS];
+#pragma unroll
+                for (int ms = 0; ms < MS; ++ms)
+#pragma unroll
+                    for (int p = 0; p < 3; ++p) xl[p][ms] = __builtin_bit_cast(v8bf, frag(buf, p, ms, j));
+                v8bf bw[MM_NT][NL];
+                float f[MM_NT];
+#pragma unroll
+                for (int t = 0; t < MM_NT; ++t) {
+                    if constexpr (DT == FTX_Q4_K_ROWS) {
+                        const v2i wv = wc.qs[t][j >> 1];
+                        const uint32_t x0 = ((uint32_t)wv.x >> (4 * (j & 1))) & 0x0F0F0F0Fu;
+                        const uint32_t x1 = ((uint32_t)wv.y >> (4 * (j & 1))) & 0x0F0F0F0Fu;
+                        bw[t][0] = sbytes(minus4(x0, 8), minus4(x1, 8));
+                        f[t] = bsk[t][j];
+                    } else if constexpr (DT == FTX_Q8_0) {
+                        bw[t][0] = sbytes(wc.q[t][2 * j], wc.q[t][2 * j + 1]);
+                        f[t] = h2f((uint16_t)(wc.d[t][j >> 1] >> (16 * (j & 1))));
+                    } else if constexpr (DT == FTX_Q4_0) {
+                        const uint32_t v = wc.q[t][j];
+                        bw[t][0] = sbytes(minus4(v & 0x0F0F0F0Fu, 8), minus4((v >> 4) & 0x0F0F0F0Fu, 8));
+                        f[t] = h2f((uint16_t)(wc.d[t][j >> 1] >> (16 * (j & 1))));
+                    } else if constexpr (DT == FTX_F16) {
+                        float v[8];
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) v[i] = (float)wc.b[t][j][i];
+                        split2(v, bw[t]);
+                        f[t] = 1.f;
+                    } else {  // Q6_K: sc (q - 32), at most 4096
+                        uint32_t b0_, b1_;
+                        q6k_bytes(wc, t, j, b0_, b1_);
+                        const uint32_t q[2] = {minus4(b0_, 32), minus4(b1_, 32)};
+                        const float sc = (float)q6k_scale(wc, t, j, kq);
+                        float v[8];
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) v[i] = sc * (float)(int8_t)(q[i >> 2] >> (8 * (i & 3)));
+                        split2(v, bw[t]);
+                        f[t] = dq6[t];
+                    }
+                }
+                v4f p[MM_NT][MS];
+                bool first = true;
+#pragma unroll
+                for (int l = 2; l >= 0; --l)
+#pragma unroll
+                    for (int b = NL - 1; b >= 0; --b) {
+#pragma unroll
+                        for (int t = 0; t < MM_NT; ++t)
+#pragma unroll
+                            for (int ms = 0; ms < MS; ++ms)
+                                p[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                    xl[l][ms], bw[t][b], first ? zero4 : p[t][ms], 0, 0, 0);
+                        first = false;
+                    }
+#pragma unroll
+                for (int t = 0; t < MM_NT; ++t) {
+                    const float fj = (j & 1) ? -f[t] : f[t];
+#pragma unroll
+                    for (int ms = 0; ms < MS; ++ms) {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            tmp[t][ms][r] = j % 4 == 0 ? fj * p[t][ms][r] : fmaf(fj, p[t][ms][r], tmp[t][ms][r]);
+                        if (j % 4 == 3)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) acc[t][ms][r] += (double)tmp[t][ms][r];
+                    }
+                }
+                continue;
+            } else {
             // every fragment read of the K-step first, then the weight
             // operands, then the MFMAs
             v8h ah[MS], al[MS];
@@ -991,46 +1102,15 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
                     for (int i = 0; i < 4; ++i) q[i] = __builtin_elementwise_fma(q[i], sc, sn);
                     bw[t] = v8h{q[0][0], q[0][1], q[1][0], q[1][1], q[2][0], q[2][1], q[3][0], q[3][1]};
                     bs[t] = 0.f;
-                } else if constexpr (DT == FTX_Q4_K_ROWS) {
-                    // (the nibbles of 8 consecutive bytes: bytes4_h's pairs)
-                    const v2i wv = wc.qs[t][j >> 1];
-                    const uint32_t x0 = ((uint32_t)wv.x >> (4 * (j & 1))) & 0x0F0F0F0Fu;
-                    const uint32_t x1 = ((uint32_t)wv.y >> (4 * (j & 1))) & 0x0F0F0F0Fu;
-                    const v2h o8 = {(_Float16)(-1032.f), (_Float16)(-1032.f)};
-                    const v2h h0 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(x0, 0x64646464u, 0x00050004u)) + o8;
-                    const v2h h1 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(x0, 0x64646464u, 0x00070006u)) + o8;
-                    const v2h h2 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(x1, 0x64646464u, 0x00050004u)) + o8;
-                    const v2h h3 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(x1, 0x64646464u, 0x00070006u)) + o8;
-                    bw[t] = v8h{h0[0], h0[1], h1[0], h1[1], h2[0], h2[1], h3[0], h3[1]};
-                    bs[t] = bsk[t][j];
-                } else if constexpr (DT == FTX_Q8_0) {
-                    bw[t] = i8x8(v2i{(int)wc.q[t][2 * j], (int)wc.q[t][2 * j + 1]});
-                    bs[t] = h2f((uint16_t)(wc.d[t][j >> 1] >> (16 * (j & 1))));
-                } else if constexpr (DT == FTX_Q4_0) {
-                    bw[t] = nib8(wc.q[t][j], 8.f);
-                    bs[t] = h2f((uint16_t)(wc.d[t][j >> 1] >> (16 * (j & 1))));
-                } else if constexpr (DT == FTX_F16) {
-                    bw[t] = wc.b[t][j];
-                    bs[t] = 0.f;
                 } else if constexpr (DT == FTX_Q8_0_MMT) {
                     const v4i qv = wc.q[t][j >> 1];
                     bw[t] = i8x8((j & 1) ? v2i{qv[2], qv[3]} : v2i{qv[0], qv[1]});
                     bs[t] = scale8(wc.d[t], j);
-                } else if constexpr (mm_q6k(DT)) {
-                    // elements 32 j + 8 kq .. + 7: half h, 32-group g of it;
-                    // low nibbles from ql run 2 h + (g & 1) (high half of
-                    // the byte for g >= 2), two high bits from qh run h
-                    const int h = j >> 2, g = j & 3, run = 2 * h + (g & 1);
-                    const v4i qv = wc.q[t][run >> 1], hv = wc.q[t][2];
-                    const uint32_t w0 = (uint32_t)qv[2 * (run & 1)], w1 = (uint32_t)qv[2 * (run & 1) + 1];
-                    const uint32_t h0 = (uint32_t)hv[2 * h], h1 = (uint32_t)hv[2 * h + 1];
-                    const uint32_t b0 = ((w0 >> (4 * (g >> 1))) & 0x0F0F0F0Fu) |
-                                        (((h0 >> (2 * g)) & 0x03030303u) << 4);
-                    const uint32_t b1 = ((w1 >> (4 * (g >> 1))) & 0x0F0F0F0Fu) |
-                                        (((h1 >> (2 * g)) & 0x03030303u) << 4);
-                    // the scale of sub-block 2 j + kq / 2, split 16 sh + sl
-                    const int sc = (int)(int8_t)(((uint32_t)wc.sc[t][j >> 1]) >>
-                                                 (8 * (2 * (j & 1) + (kq >> 1))));
+                } else if constexpr (DT == FTX_Q6_K_MMT) {
+                    uint32_t b0, b1;
+                    q6k_bytes(wc, t, j, b0, b1);
+                    // the scale split 16 sh + sl
+                    const int sc = q6k_scale(wc, t, j, kq);
                     const int sl = sc & 15, sh = sc >> 4;
                     const _Float16 fl = (_Float16)(float)sl, fh = (_Float16)(float)sh;
                     const _Float16 ol = (_Float16)(float)(-1056 * sl), oh = (_Float16)(float)(-1056 * sh);
@@ -1056,55 +1136,7 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
                     bs[t] = scale8(wc.d[t], j);
                 }
             }
-            if constexpr (mm_stored(DT)) {
-                // the backend's operations: a fresh sum per 32 elements, the lo
-                // half first (its small terms are then rounded at their own
-                // size), added in fp32 with the block scale, four blocks to one
-                // 64-bit addition.  The MFMA rounds its sums down (toward
-                // minus infinity), so every other block is formed negated and
-                // subtracted: the shares cancel instead of adding up.
-                if (j & 1) {
-#pragma unroll
-                    for (int t = 0; t < MM_NT; ++t) {
-                        bw[t] = -bw[t];
-                        if constexpr (DT == FTX_Q6_K) bw2[t] = -bw2[t];
-                    }
-                }
-                v4f p[MM_NT][MS];
-#pragma unroll
-                for (int t = 0; t < MM_NT; ++t)
-#pragma unroll
-                    for (int ms = 0; ms < MS; ++ms)
-                        p[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[ms], bw[t], zero4, 0, 0, 0);
-                if constexpr (DT == FTX_Q6_K) {
-#pragma unroll
-                    for (int t = 0; t < MM_NT; ++t)
-#pragma unroll
-                        for (int ms = 0; ms < MS; ++ms) {
-                            p[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[ms], bw2[t], p[t][ms], 0, 0, 0);
-                            p[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[ms], bw2[t], p[t][ms], 0, 0, 0);
-                        }
-                }
-#pragma unroll
-                for (int t = 0; t < MM_NT; ++t)
-#pragma unroll
-                    for (int ms = 0; ms < MS; ++ms)
-                        p[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[ms], bw[t], p[t][ms], 0, 0, 0);
-#pragma unroll
-                for (int t = 0; t < MM_NT; ++t) {
-                    const float f0 = DT == FTX_F16 ? 1.f : (DT == FTX_Q6_K ? dq6[t] : bs[t]);
-                    const float f = (j & 1) ? -f0 : f0;
-#pragma unroll
-                    for (int ms = 0; ms < MS; ++ms) {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            tmp[t][ms][r] = j % 4 == 0 ? f * p[t][ms][r] : fmaf(f, p[t][ms][r], tmp[t][ms][r]);
-                        if (j % 4 == 3)
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) acc[t][ms][r] += (double)tmp[t][ms][r];
-                    }
-                }
-            } else if constexpr (DT == FTX_Q4_K || DT == FTX_Q6_K_MMT) {
+            if constexpr (DT == FTX_Q4_K || DT == FTX_Q6_K_MMT) {
                 // hi parts of every tile first, then lo: no MFMA waits on the
                 // one before it
 #pragma unroll
@@ -1161,6 +1193,7 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
 #pragma unroll
                         for (int r = 0; r < 4; ++r) acc[t][ms][r] += bs[t] * p[t][ms][r];
                     }
+            }
             }
         }
         if constexpr (DT == FTX_Q6_K_MMT) {
@@ -2059,6 +2092,7 @@ static hipError_t mm_launch(hipStream_t st, const MmSeg* segs, int nseg, const M
         a.rscale = op->rscale;
         a.x = op->x;
         a.ldx = op->ldx;
+        a.plane[0] = act.Mp * act.K * 2;
         a.nblk = (int)(op->K / 32);
     }
     // rows of a split's partials
@@ -2086,7 +2120,7 @@ static hipError_t mm_launch(hipStream_t st, const MmSeg* segs, int nseg, const M
     a.sb_per_split = (a.nsb + S - 1) / S;
     S = (a.nsb + a.sb_per_split - 1) / a.sb_per_split;
     a.ntt = (int)mt;
-    const size_t lds = 2 * (size_t)ms * 16384;
+    const size_t lds = 2 * (size_t)ms * (op ? 3 : 2) * 8192;
     using K_t = void (*)(MmArgs);
     // [dtype][dense 64 | expert 64-row tiles | expert 16-row tiles | dense
     // 32 | dense 16] (Q6_K and stored rows: dense only)
@@ -2233,15 +2267,15 @@ bool mm_op_supported(int dt, int64_t M, int64_t K, int64_t N, int64_t row_bytes)
     const bool k256 = dt == FTX_Q4_K || dt == FTX_Q6_K;
     // 32-bit offsets into the weights and the operand planes
     return ((k32 && K % 32 == 0) || (k256 && K % 256 == 0)) && K > 0 && M > 0 && N > 0 &&
-           N * row_bytes < 0xF0000000ll && mm_pad_tokens(M) * ((K + 255) / 256 * 256) * 2 < 0xF0000000ll &&
+           N * row_bytes < 0xF0000000ll && mm_pad_tokens(M) * ((K + 255) / 256 * 256) * 6 < 0xF0000000ll &&
            M <= 65535;
 }
 // operand (with the row scales), then partials, in bytes
 static size_t mm_op_act_bytes(int64_t M, int64_t K) {
     const int64_t Mp = mm_pad_tokens(M), Kp = (K + 255) / 256 * 256;
-    // hi and lo planes, Q4_K's limbs of the sums (2 KB per 16 x 256 elements),
-    // row scales
-    return ((size_t)(Mp * Kp * 4 + Mp * Kp / 2) + (size_t)M * 4 + 255) & ~(size_t)255;
+    // three planes, Q4_K's limbs of the sums (2 KB per 16 x 256 elements), row
+    // scales
+    return ((size_t)(Mp * Kp * 6 + Mp * Kp / 2) + (size_t)M * 4 + 255) & ~(size_t)255;
 }
 static size_t mm_op_part_floats(int64_t M, int64_t K, int64_t cols, int epi, int cu_count) {
     const int64_t units = epi == EPI_SWIGLU ? 2 * ((cols / 2 + MM_WROWS - 1) / MM_WROWS)
@@ -2258,8 +2292,14 @@ hipError_t launch_mm_op(hipStream_t st, const MmSeg* segs, int nseg, const float
     const int64_t Mp = mm_pad_tokens(M), Kp = (K + 255) / 256 * 256;
     int64_t cols = 0;
     for (int i = 0; i < nseg; ++i) cols += segs[i].N;
-    MmAct act = mm_act(ws, Mp, Kp);  // (its sums' place holds Q4_K's limbs)
-    float* rs = (float*)((uint8_t*)ws + Mp * Kp * 4 + Mp * Kp / 2);
+    __bf16* xb = (__bf16*)ws;
+    v8bf* xs = (v8bf*)(xb + 3 * Mp * Kp);
+    float* rs = (float*)((uint8_t*)xs + Mp * Kp / 2);
+    MmAct act{};
+    act.xh = (_Float16*)xb;  // (the three bf16 planes)
+    act.sh = (_Float16*)xs;  // (Q4_K's limbs of the sums)
+    act.Mp = Mp;
+    act.K = Kp;
     MmSeg sg[2];
     for (int i = 0; i < nseg && i < 2; ++i) {
         sg[i] = segs[i];
@@ -2267,8 +2307,8 @@ hipError_t launch_mm_op(hipStream_t st, const MmSeg* segs, int nseg, const float
     }
     float* part = (float*)((uint8_t*)ws + mm_op_act_bytes(M, K));
     hipLaunchKernelGGL(k_mm_prep_op, dim3((unsigned)M), dim3(512), 0, st, x, ldx, K, Kp,
-                       segs[0].dt == FTX_Q4_0 ? 1 : 0, act.xh, act.xl,
-                       segs[0].dt == FTX_Q4_K ? (v8bf*)act.sh : nullptr, rs);
+                       segs[0].dt == FTX_Q4_0 ? 1 : 0, xb, Mp * Kp,
+                       segs[0].dt == FTX_Q4_K ? xs : nullptr, rs);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     MmOut o{};

@@ -1,6 +1,7 @@
-// mm_dev.h -- operand helpers shared by the fp16-MFMA kernels (k_gemm.hip,
-// k_moe.hip): vector types, exact integer -> fp16 conversions and the fp16
-// hi + lo split of an fp32 value.
+// mm_dev.h -- operand helpers shared by the fp16- and bf16-MFMA kernels
+// (k_gemm.hip, k_moe.hip, k_axpy.hip): vector types, exact integer -> fp16 and
+// bf16 conversions, the fp16 hi + lo split of an fp32 value and its exact
+// split into three bf16 limbs.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -11,6 +12,7 @@ namespace {
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
@@ -93,6 +95,71 @@ __device__ __forceinline__ void split_hl2(float v0, float v1, v2h& h, v2h& l) {
     asm volatile("v_fma_mixhi_f16 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
                  : "+v"(lw) : "v"(hw), "v"(v1));
     l = __builtin_bit_cast(v2h, lw);
+}
+
+// ---- bf16 operands
+__device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) {
+    return __builtin_amdgcn_perm(hi, lo, sel);
+}
+// the high halves of two floats (bf16 by truncation)
+__device__ __forceinline__ uint32_t pack_hi(float a, float b) {
+    return perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+__device__ __forceinline__ float trunc_bf(float a) {
+    return __uint_as_float(__float_as_uint(a) & 0xFFFF0000u);
+}
+
+// a = l[0] + l[1] + l[2] exactly
+__device__ __forceinline__ void split3(const float* a, v8bf* l) {
+#pragma clang fp contract(off)
+    uint32_t p[3][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float a0 = a[2 * i], a1 = a[2 * i + 1];
+        const float b0 = a0 - trunc_bf(a0), b1 = a1 - trunc_bf(a1);
+        const float c0 = b0 - trunc_bf(b0), c1 = b1 - trunc_bf(b1);
+        p[0][i] = pack_hi(a0, a1);
+        p[1][i] = pack_hi(b0, b1);
+        p[2][i] = pack_hi(c0, c1);
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const uint4 v = {p[k][0], p[k][1], p[k][2], p[k][3]};
+        l[k] = __builtin_bit_cast(v8bf, v);
+    }
+}
+
+// 8 signed bytes -> bf16, exact
+__device__ __forceinline__ v8bf sbytes(uint32_t x, uint32_t y) {
+    uint4 v;
+    v.x = pack_hi((float)(int8_t)x, (float)(int8_t)(x >> 8));
+    v.y = pack_hi((float)(int8_t)(x >> 16), (float)(int8_t)(x >> 24));
+    v.z = pack_hi((float)(int8_t)y, (float)(int8_t)(y >> 8));
+    v.w = pack_hi((float)(int8_t)(y >> 16), (float)(int8_t)(y >> 24));
+    return __builtin_bit_cast(v8bf, v);
+}
+// a = hl[0] + hl[1], the nearest bf16 and the rest: exact for integers of at
+// most 16 bits and fp16 values (times any power of two)
+__device__ __forceinline__ void split2(const float* a, v8bf* hl) {
+    typedef float v2f __attribute__((ext_vector_type(2)));
+    typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+    uint32_t p[2][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const v2f x = {a[2 * i], a[2 * i + 1]};
+        p[0][i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, v2bf));
+        p[1][i] = pack_hi(x[0] - __uint_as_float(p[0][i] << 16),
+                          x[1] - __uint_as_float(p[0][i] & 0xFFFF0000u));
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const uint4 v = {p[k][0], p[k][1], p[k][2], p[k][3]};
+        hl[k] = __builtin_bit_cast(v8bf, v);
+    }
+}
+// 4 bytes 0..127 minus `bias` (at most 120), as signed bytes
+__device__ __forceinline__ uint32_t minus4(uint32_t x, uint32_t bias) {
+    return (x + (0x80u - bias) * 0x01010101u) ^ 0x80808080u;
 }
 
 }  // namespace
