@@ -166,6 +166,15 @@ def test_matmul_keeps_small_activations_beside_an_outlier(gctx, orc, dt, M, size
     outlier(gctx, orc, dt, M, size, False)
 
 
+@pytest.mark.parametrize("down,dt,M", [(False, P.Q4_K, 12), (False, P.Q4_K, 40), (True, P.Q4_K, 4),
+                                       (True, P.Q4_K, 40), (True, P.Q4_0, 40), (True, P.Q8_0, 4),
+                                       (True, P.Q8_0, 20), (True, P.Q6_K, 20)])
+def test_zero_weights_of_a_block_stay_zero(gctx, orc, down, dt, M):
+    """Q4_K's zeros are the difference of a scaled integer and a minimum; the
+    column-axpy form of every block type."""
+    outlier(gctx, orc, dt, M, 1e8, down)
+
+
 @pytest.mark.parametrize("dt,M", [(P.Q8_0, 4), (P.Q8_0, 12), (P.Q4_0, 12), (P.Q4_K, 12), (P.Q6_K, 12),
                                   (P.F16, 12)])
 def test_matmul_special_values(gctx, orc, dt, M):

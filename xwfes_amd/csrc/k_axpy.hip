@@ -15,11 +15,12 @@
 //         MFMAs (third limb x rest, 2^-26 of the product, is left out); with
 //         d sc in A, one per 16 columns, the splits took three quarters of
 //         the time
-//   Q4_K  (d sc) (q - 8) - (dmin m - 8 d sc)      one A per 32 columns; the min
+//   Q4_K  (d sc) (q - c) - (dmin m - c d sc)      one A per 32 columns; the min
 //         term is a product of its own, h (3 limbs) x its 3 limbs, with the
-//         four 32-column sub-blocks as B columns (centred on q = 8 the two
-//         sums are the size of the result: with q and dmin m their difference
-//         loses a bit and a half)
+//         four 32-column sub-blocks as B columns; c is the integer nearest to
+//         dmin m / (d sc) (q4k_c), so that neither sum is larger than the
+//         weights call for (a fixed c = 8 left a zero weight as the difference
+//         of two terms)
 //
 // The MFMA wants 8 contraction values (rows) of one column in a lane, the
 // tensor has a row's columns side by side.  A wave loads 8 rows x 4 or 8
@@ -93,6 +94,8 @@ struct AxCfg {
     // scales per row: blocks, Q4_K's scales then mins, Q6_K's 16-column
     // integer scales then d
     static constexpr int NSC = DT == FTX_Q6_K ? 9 : (DT == FTX_Q4_K ? 8 : 4);
+    // Q4_K: 128 - c of every row and sub-block, a byte each, after the scales
+    static constexpr int CEN = DT == FTX_Q4_K ? 128 : 0;
     static constexpr int WORDS = (DT == FTX_Q8_0 || DT == FTX_Q6_K) ? 2 : 1;  // per lane and row
 };
 
@@ -110,7 +113,7 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
     using C = AxCfg<DT>;
     // per wave: columns, then scales; at the end the waves' sums of one
     // 16-token tile
-    constexpr int WB = C::TILES * 512 + C::NSC * 128;
+    constexpr int WB = C::TILES * 512 + C::NSC * 128 + C::CEN;
     __shared__ __attribute__((aligned(16))) uint8_t lds[65536];
     static_assert(WB * AX_WAVES <= 65536, "");
     const int tid = threadIdx.x, lane = tid & 63;
@@ -127,6 +130,7 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
     const float sgn = (w & 1) ? -1.f : 1.f;
     uint2* cols = (uint2*)(lds + w * WB);
     float* scl = (float*)(lds + w * WB + C::TILES * 512);  // [NSC][kq][8]
+    uint8_t* cen = (uint8_t*)(scl + C::NSC * 32);          // Q4_K: [4][kq][8]
 
     // the lane's byte offset in a row and its scale fields' (blocks past the
     // row's end read the last one; their columns are not stored)
@@ -226,7 +230,9 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
                 const int sh = 16 * hf + 8 * i;
                 const float ds = d * (float)((sc >> sh) & 0xFF);
                 scl[(2 * hf + i) * 32 + at] = ds;
-                scl[(4 + 2 * hf + i) * 32 + at] = dmin * (float)((mn >> sh) & 0xFF) - 8.f * ds;
+                const float dm = dmin * (float)((mn >> sh) & 0xFF), ctr = q4k_c(ds, dm);
+                scl[(4 + 2 * hf + i) * 32 + at] = q4k_g(ds, dm, ctr);
+                cen[(2 * hf + i) * 32 + at] = (uint8_t)(128.f - ctr);
             }
         } else if constexpr (DT == FTX_Q6_K) {
 #pragma unroll
@@ -298,7 +304,7 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
             load(raw, min(I + AX_WAVES, I1 - 1));
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             if constexpr (DT == FTX_Q4_K) {
-                // B column b < 4: dmin m - 8 d sc of sub-block b
+                // B column b < 4: dmin m - c d sc of sub-block b
                 float dm[8];
                 scales8(4 + (c & 3), kq, dm);
 #pragma unroll
@@ -356,11 +362,12 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
                         bw[p] = sbytes(minus4((v.x >> (4 * p)) & 0x0F0F0F0Fu, 8),
                                        minus4((v.y >> (4 * p)) & 0x0F0F0F0Fu, 8));
                 } else if constexpr (DT == FTX_Q4_K) {
+                    const uint2 cb = *(const uint2*)&cen[b * 32 + kq * 8];  // of the 8 rows
 #pragma unroll
                     for (int p = 0; p < 2; ++p) {
                         const uint2 v = cols[slot(2 * (b >> 1) + p, c)];
-                        bw[p] = sbytes(minus4((v.x >> (4 * (b & 1))) & 0x0F0F0F0Fu, 8),
-                                       minus4((v.y >> (4 * (b & 1))) & 0x0F0F0F0Fu, 8));
+                        bw[p] = sbytes((((v.x >> (4 * (b & 1))) & 0x0F0F0F0Fu) + cb.x) ^ 0x80808080u,
+                                       (((v.y >> (4 * (b & 1))) & 0x0F0F0F0Fu) + cb.y) ^ 0x80808080u);
                     }
                 } else {  // Q8_0
 #pragma unroll

@@ -37,7 +37,7 @@
 // tighter than the steps' (64-bit additions, alternating signs against the
 // MFMA's rounding): 0.6e-7 against 64 bits where the generic kernel's fp32 sums
 // had 0.9e-7.  Measured (whole call): 48 tokens of Q4_K 14336 x 4096 4.70 ms on
-// the generic kernel, 71 us here (66 with two fp16 halves, a third less operand
+// the generic kernel, 73 us here (66 with two fp16 halves, a third less operand
 // to copy); 16 tokens of Q8_0 4096 x 4096 473 -> 41 us.
 //
 // Column-axpy form (ffn_down in the reference orientation, n_ff rows of
@@ -946,11 +946,16 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
                 for (int i = 0; i < 4; ++i) scn[t][i] = scp[t][i] * v2h{(_Float16)(-1024.f), (_Float16)(-1024.f)};
             }
         }
-        // stored Q4_K: w = d sc (q - 8) - g, g = dmin m - 8 d sc; the g of the
-        // eight sub-blocks against the 32-element sums is two MFMAs of three
-        // bf16 limbs each (K slot 8 kq + j: sub-block j; first the limb pairs
-        // hh, hm, mh, mm of kq = 0 .. 3, then hl, lh)
+        // stored Q4_K: w = d sc (q - c) - g, g = dmin m - c d sc with c the
+        // integer nearest to dmin m / (d sc), so that neither term exceeds the
+        // weight by more than half a step (a fixed c = 8 left a weight of zero
+        // as the difference of two terms: 5.6e-5 where such a weight meets an
+        // activation 1e4 times the rest).  The g of the eight sub-blocks
+        // against the 32-element sums is two MFMAs of three bf16 limbs each (K
+        // slot 8 kq + j: sub-block j; first the limb pairs hh, hm, mh, mm of
+        // kq = 0 .. 3, then hl, lh)
         float bsk[DT == FTX_Q4_K_ROWS ? MM_NT : 1][8];
+        uint32_t cen[DT == FTX_Q4_K_ROWS ? MM_NT : 1][2];  // 128 - c, a byte each
         if constexpr (DT == FTX_Q4_K_ROWS) {
             const v8bf* xs = (const v8bf*)a.sh;
 #pragma unroll
@@ -965,7 +970,10 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
                 for (int j = 0; j < 8; ++j) {
                     const int h = 8 * (j & 3);
                     const float ds = d * (float)((sc[j >> 2] >> h) & 0xFF);
-                    const float g = dmin * (float)((mn[j >> 2] >> h) & 0xFF) - 8.f * ds;
+                    const float dm = dmin * (float)((mn[j >> 2] >> h) & 0xFF), c = q4k_c(ds, dm);
+                    const float g = q4k_g(ds, dm, c);
+                    const uint32_t cb = (128u - (uint32_t)c) << h;
+                    cen[t][j >> 2] = (j & 3) ? cen[t][j >> 2] | cb : cb;
                     bsk[t][j] = ds;
                     const float gh = trunc_bf(g), r = g - gh;
                     const float gm = trunc_bf(r), gl = r - gm;
@@ -1012,7 +1020,8 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
                         const v2i wv = wc.qs[t][j >> 1];
                         const uint32_t x0 = ((uint32_t)wv.x >> (4 * (j & 1))) & 0x0F0F0F0Fu;
                         const uint32_t x1 = ((uint32_t)wv.y >> (4 * (j & 1))) & 0x0F0F0F0Fu;
-                        bw[t][0] = sbytes(minus4(x0, 8), minus4(x1, 8));
+                        const uint32_t cb = perm(0, cen[t][j >> 2], 0x01010101u * (j & 3));
+                        bw[t][0] = sbytes((x0 + cb) ^ 0x80808080u, (x1 + cb) ^ 0x80808080u);
                         f[t] = bsk[t][j];
                     } else if constexpr (DT == FTX_Q8_0) {
                         bw[t][0] = sbytes(wc.q[t][2 * j], wc.q[t][2 * j + 1]);

@@ -162,4 +162,12 @@ __device__ __forceinline__ uint32_t minus4(uint32_t x, uint32_t bias) {
     return (x + (0x80u - bias) * 0x01010101u) ^ 0x80808080u;
 }
 
+// Q4_K: w = ds q - dm as ds (q - c) - g, g = dm - c ds, with c the integer of
+// 0 .. 15 nearest to dm / ds (|g| <= |ds| / 2 while dm / ds lies in the range),
+// so that both terms are of the weight's own size: c, and g from it
+__device__ __forceinline__ float q4k_c(float ds, float dm) {
+    return fminf(fmaxf(rintf(dm * __builtin_amdgcn_rcpf(ds)), 0.f), 15.f);
+}
+__device__ __forceinline__ float q4k_g(float ds, float dm, float c) { return fmaf(-c, ds, dm); }
+
 }  // namespace
