@@ -274,3 +274,79 @@ def test_small_steps_over_tiles(gctx, orc, dt, d, ff, M):
     assert rel_err_rows(got, want) < LOGIT_TOL
     for a, b in zip(kv, kvo):
         np.testing.assert_allclose(a.astype(np.float32), b.astype(np.float32), rtol=3e-3, atol=3e-3)
+
+
+# ---- scales and activations at the ends of their ranges
+
+
+def close_or_special(got, want, size):
+    """Finite results as close(), the others (infinite, NaN) the same."""
+    fin = np.isfinite(want)
+    assert np.array_equal(got[~fin], want[~fin].astype(np.float32), equal_nan=True)
+    close(got[fin], want[fin], np.broadcast_to(size, want.shape)[fin])
+
+
+@pytest.mark.parametrize("dt,at", [(P.Q4_0, 0), (P.Q8_0, 0), (P.Q4_K, 0), (P.Q4_K, 2), (P.Q6_K, 208)])
+@pytest.mark.parametrize("M", [1, 6, 12])
+@pytest.mark.parametrize("down", [False, True])
+def test_infinite_and_nan_scales(gctx, orc, dt, at, M, down):
+    """A block whose fp16 scale field is infinite or NaN: the products of its
+    zero quants are NaN, and so are sums over both signs; the other rows (or
+    columns) are untouched.  (Up to 8 rows of the K types' matmul: only the
+    rows that hold no such block are looked at.)"""
+    rng = np.random.default_rng(7 * dt + at + M)
+    K, N = 768, 512
+    shape = (K, N) if down else (N, K)
+    be, bb = (256, {P.Q4_K: 144, P.Q6_K: 210}[dt]) if dt in (P.Q4_K, P.Q6_K) else (32, {P.Q4_0: 18, P.Q8_0: 34}[dt])
+    w32 = (rng.standard_normal(shape) * 0.02).astype(np.float32)
+    raw = orc.quantize(w32, dt).reshape(shape[0], shape[1] // be, bb).copy()
+    for row, bits in ((5, 0x7C00), (9, 0x7E00)):
+        raw[row, 0, at:at + 2] = np.array([bits], np.uint16).view(np.uint8)
+    raw = raw.ravel()
+    w = orc.dequant(raw, dt, shape[1], rows=shape[0]).reshape(shape)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    if down:
+        x[:, [5, 9]] = rng.standard_normal((M, 2)) * (rng.random((M, 2)) < 0.8)
+    t = gctx.upload(raw, dt, shape[::-1])
+    got = gctx.down_axpy(x, t) if down else gctx.matmul(x, t)
+    t.free()
+    wk = w if down else w.T
+    with np.errstate(invalid="ignore"):
+        prod = x[:, :, None] * wk[None]
+        want, size = prod.astype(np.float64).sum(1), np.abs(prod).astype(np.float64).sum(1)
+    if not down and M <= 8 and dt in (P.Q4_K, P.Q6_K):
+        assert np.isfinite(got[:, np.isfinite(want[0])]).all()
+        return
+    close_or_special(got, want, size)
+
+
+@pytest.mark.parametrize("dt,d", [(P.Q8_0, 2048), (P.Q4_0, 2048), (P.Q8_0, 512)])
+@pytest.mark.parametrize("M", [1, 5])
+def test_small_step_with_an_infinite_head_scale(gctx, orc, dt, d, M):
+    """Head rows of one block with an infinite scale: their logits as the
+    oracle's (NaN: products of both signs), the others close; over the re-tiled
+    copies and over the stored rows."""
+    cfg = P.model_cfg(1, d, d // 128, d // 256, 128, 512, 203, rope_theta=10000.0)
+    dts = dict(tok_embd=P.Q8_0, output=dt, q=dt, k=dt, v=dt, o=dt, gate=dt, up=dt, down=dt)
+    model = P.make_model(orc, cfg, dts, seed=d + M + dt)
+    bb = 34 if dt == P.Q8_0 else 18
+    rows = model["output"]["raw"].reshape(203, d // 32, bb)
+    bad = np.arange(203) % 4 == 1
+    rows[bad, 3, :2] = np.array([0x7C00], np.uint16).view(np.uint8)
+    toks = np.random.default_rng(M).integers(0, 203, M).tolist()
+    (got, want, _, _), = run_batch(gctx, orc, model, [(toks, None, 20, 40)], 8)
+    assert np.array_equal(got[:, bad], want[:, bad], equal_nan=True) and np.isnan(want[:, bad]).any()
+    assert rel_err_rows(got[:, ~bad], want[:, ~bad]) < LOGIT_TOL
+
+
+@pytest.mark.parametrize("dt,d", [(P.Q8_0, 2048), (P.Q4_0, 2048)])
+def test_small_step_of_a_huge_residual(gctx, orc, dt, d):
+    """Rows so large that their squares overflow: the norm's factor is zero and
+    every normalised product with it, as in the oracle."""
+    cfg = P.model_cfg(1, d, d // 128, d // 256, 128, 512, 203, rope_theta=10000.0)
+    dts = dict(tok_embd=P.F32, output=dt, q=dt, k=dt, v=dt, o=dt, gate=dt, up=dt, down=dt)
+    model = P.make_model(orc, cfg, dts, seed=d + dt)
+    emb = model["tok_embd"]["raw"].view(np.float32)
+    emb[:] = np.where(np.random.default_rng(3).random(emb.shape) < 0.5, -3e38, 3e38)
+    (got, want, _, _), = run_batch(gctx, orc, model, [([5, 6, 9], None, 0, 16)], 8)
+    assert not want.any() and not got.any()

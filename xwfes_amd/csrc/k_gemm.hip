@@ -439,8 +439,10 @@ struct MmArgs {
     int M;
     MmOutDev out;
     // the backend's single operations (null otherwise): row m of the operand
-    // is row m of x times 1 / rscale[m], a power of two; a sum that comes out
-    // as NaN is formed again from x itself (k_mm_prep_op)
+    // is row m of x times 1 / rscale[m], a power of two; a sum that does not
+    // come out finite is formed again from x itself, product by product (an
+    // infinite or NaN activation breaks the limbs; an infinite block scale times
+    // the block's sum is not the sum of its products, some of them NaN)
     const float* rscale;
     const float* x;
     int64_t ldx;
@@ -1266,7 +1268,7 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
                 float v = (float)acc[t][ms][r];
                 if constexpr (mm_stored(DT)) {
                     v *= a.rscale[m];
-                    if (v != v)
+                    if (!is_finite(v))
                         v = mm_redo(a, sg.W + n * sg.row_bytes, DT == FTX_Q4_K_ROWS ? FTX_Q4_K : DT, m,
                                     (int64_t)sb0 * 256, min((int64_t)sb1 * 256, (int64_t)a.nblk * 32));
                 }
@@ -1300,6 +1302,23 @@ struct MtArgs {
     const float* normw;  // or null
     float eps;
 };
+
+// row col of a tile times the (normalised) row m of x, product by product
+template <int DT>
+__device__ float tile_redo(const MtArgs& a, const uint8_t* tile, int col, int m, float inv) {
+    constexpr int STEP = (int)mmt_step_bytes(DT), LB = (int)mmt_lane_bytes(DT);
+    const float* x = a.x + (int64_t)m * a.ldx;
+    float v = 0.f;
+    for (int k = 0; k < a.nsb * 256; ++k) {
+        const int j = (k >> 5) & 7, e = k & 7;
+        const uint8_t* p = tile + (int64_t)(k >> 8) * STEP;
+        const float d = h2f(ld16(p + 64 * LB + col * 16 + 2 * j));
+        const uint8_t* l = p + (col + 16 * ((k >> 3) & 3)) * LB + (LB >> 3) * j;
+        const int q = DT == FTX_Q8_0_MMT ? (int)(int8_t)l[e] : (int)((l[e >> 1] >> (4 * (e & 1))) & 15) - 8;
+        v += (a.normw ? x[k] * inv * a.normw[k] : x[k]) * (d * (float)q);
+    }
+    return v;
+}
 
 template <int DT, int MC, bool PAIR>
 __global__ void __launch_bounds__(64 * MT_WAVES) k_tile(MtArgs a) {
@@ -1433,9 +1452,16 @@ __global__ void __launch_bounds__(64 * MT_WAVES) k_tile(MtArgs a) {
     if (n >= a.seg[si].N) return;
     float* yp = a.y[si] + m * a.ldy[si] + n;
     g *= inv;
+    // (an infinite block scale, or activations whose unnormalised products leave
+    // the fp32 range)
+    if (!is_finite(g)) g = tile_redo<DT>(a, base[0], col, m, inv);
+    if constexpr (PAIR) {
+        up *= inv;
+        if (!is_finite(up)) up = tile_redo<DT>(a, base[1], col, m, inv);
+    }
     // src/engine.cpp:271-273: g / (1 + exp(-g)) * u
     if constexpr (PAIR)
-        *yp = g / (1.f + expf(-g)) * (up * inv);
+        *yp = g / (1.f + expf(-g)) * up;
     else
         *yp = a.epi == EPI_ACCUM ? *yp + g : g;
 }

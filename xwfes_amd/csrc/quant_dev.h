@@ -23,6 +23,8 @@ __device__ __forceinline__ float h2f(uint16_t h) {
     return (float)__builtin_bit_cast(_Float16, h);
 }
 
+__device__ __forceinline__ bool is_finite(float v) { return fabsf(v) <= 3.402823466e38f; }
+
 __device__ __forceinline__ float bf2f(uint16_t b) {
     return __uint_as_float((uint32_t)b << 16);
 }
