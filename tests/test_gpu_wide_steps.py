@@ -320,6 +320,28 @@ def test_infinite_and_nan_scales(gctx, orc, dt, at, M, down):
     close_or_special(got, want, size)
 
 
+@pytest.mark.parametrize("dt", [P.Q4_0, P.Q8_0])
+@pytest.mark.parametrize("M", [1, 4, 20])
+def test_down_axpy_large_products(gctx, orc, dt, M):
+    """h d beyond the fp32 range where the quant is zero adds nothing."""
+    rng = np.random.default_rng(dt + M)
+    n_in, N = 40, 512
+    w = (rng.standard_normal((n_in, N)) * 500).astype(np.float32)
+    w[7, ::2] = 0
+    raw = orc.quantize(w, dt)
+    v = orc.dequant(raw, dt, N, rows=n_in).reshape(n_in, N)
+    x = rng.standard_normal((M, n_in)).astype(np.float32)
+    x[0, 7] = 3e38
+    t = gctx.upload(raw, dt, (N, n_in))
+    got = gctx.down_axpy(x, t)
+    t.free()
+    with np.errstate(over="ignore"):
+        prod = x[:, :, None] * v[None]
+        want, size = prod.astype(np.float64).sum(1), np.abs(prod).astype(np.float64).sum(1)
+    assert np.isfinite(want[0]).sum() >= N // 2 and np.isinf(want[0]).any()
+    close_or_special(got, want, size)
+
+
 @pytest.mark.parametrize("dt,d", [(P.Q8_0, 2048), (P.Q4_0, 2048), (P.Q8_0, 512)])
 @pytest.mark.parametrize("M", [1, 5])
 def test_small_step_with_an_infinite_head_scale(gctx, orc, dt, d, M):

@@ -107,6 +107,22 @@ struct AxRaw {
     uint32_t s[DT == FTX_Q4_K ? 4 : 2];
 };
 
+// rows i0 .. i1 - 1 of token m and column col, product by product: for sums
+// that do not come out finite (an infinite or NaN operand breaks the limbs,
+// and h d may leave the fp32 range where h (d q) does not)
+__device__ float ax_redo(const AxArgs& a, int dt, int m, int64_t col, int64_t i0, int64_t i1) {
+    const float* hr = a.h + (int64_t)m * a.ldh;
+    float v = 0.f;
+    for (int64_t i = i0; i < i1; ++i) {
+        float q[8], x = 0.f;
+        dq8(a.W + i * a.row_bytes, dt, col & ~(int64_t)7, a.N, q);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x = (int)(col & 7) == e ? q[e] : x;
+        v += hr[i] * x;
+    }
+    return v;
+}
+
 template <int DT, int MS>
 __global__ void __launch_bounds__(64 * AX_WAVES)
     __attribute__((amdgpu_waves_per_eu(MS == 1 ? 4 : 2, MS == 1 ? 4 : 2))) k_axpy(AxArgs a) {
@@ -430,19 +446,7 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
             const int m = m0 + 16 * ms + 4 * kq + r;
             if (m >= a.M) continue;
             float v = s[r];
-            if (v != v) {
-                // an infinite or NaN operand breaks the limbs: this sum again,
-                // one product after the other
-                const float* hr = a.h + (int64_t)m * a.ldh;
-                v = 0.f;
-                for (int64_t i = 32 * I0; i < min(32 * I1, a.n_in); ++i) {
-                    float q[8], x = 0.f;
-                    dq8(a.W + i * a.row_bytes, DT, col & ~(int64_t)7, a.N, q);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) x = (int)(col & 7) == e ? q[e] : x;
-                    v += hr[i] * x;
-                }
-            }
+            if (!is_finite(v)) v = ax_redo(a, DT, m, col, 32 * I0, min(32 * I1, a.n_in));
             float* p = a.out + (int64_t)ks * a.split_stride + (int64_t)m * a.ldo + col;
             *p = a.accum ? *p + v : v;
         }
@@ -540,6 +544,7 @@ __global__ void __launch_bounds__(64 * AF_WAVES) k_axpy_few(AxArgs a) {
 #pragma unroll
         for (int k = 1; k < AF_WAVES; ++k) s += red[k][tid];
         if (j0 + tid < a.N) {
+            if (!is_finite(s)) s = ax_redo(a, DT, m, j0 + tid, i0, i1);
             float* p = a.out + (int64_t)ks * a.split_stride + (int64_t)m * a.ldo + j0 + tid;
             *p = a.accum ? *p + s : s;
         }
