@@ -361,7 +361,7 @@ def test_small_step_with_an_infinite_head_scale(gctx, orc, dt, d, M):
     assert rel_err_rows(got[:, ~bad], want[:, ~bad]) < LOGIT_TOL
 
 
-@pytest.mark.parametrize("dt,d", [(P.Q8_0, 2048), (P.Q4_0, 2048)])
+@pytest.mark.parametrize("dt,d", [(P.Q8_0, 2048), (P.Q4_0, 2048), (P.Q8_0, 512), (P.F16, 512)])
 def test_small_step_of_a_huge_residual(gctx, orc, dt, d):
     """Rows so large that their squares overflow: the norm's factor is zero and
     every normalised product with it, as in the oracle."""

@@ -318,7 +318,23 @@ __global__ void __launch_bounds__(256) k_rows(Segs segs, const float* __restrict
         sq = __shfl(sq, m * (64 / MC), 64);
     }
     const int idx = lane / PER, r = idx / MC, m = idx % MC;
-    float o = normw ? v * (1.f / sqrtf(sq / (float)K + eps)) : v;
+    const float inv = normw ? 1.f / sqrtf(sq / (float)K + eps) : 1.f;
+    float o = normw ? v * inv : v;
+    if (normw && !is_finite(o) && lane % PER == 0 && m < M) {
+        // (activations whose unnormalised products leave the fp32 range: this
+        // sum again from the normalised ones)
+        const int64_t n = min(r0 + r % R, total - 1);
+        const int si = PAIR ? r / R : (n < segs.start[1] ? 0 : (n < segs.start[2] ? 1 : 2));
+        const uint8_t* row = segs.s[si].W + (n - (PAIR ? 0 : segs.start[si])) * segs.s[si].row_bytes;
+        const float* xm = x + (int64_t)m * ldx;
+        o = 0.f;
+        for (int k = 0; k < K; k += 8) {
+            float w[8];
+            dq8(row, DT, k, K, w);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) o += xm[k + i] * inv * normw[k + i] * w[i];
+        }
+    }
     float up = 0.f;
     if constexpr (PAIR) up = __shfl(o, (lane + 32) & 63, 64);  // the up rows' lanes are the upper half
     if (lane % PER || m >= M) return;
