@@ -34,6 +34,44 @@ def test_attention_of_more_than_512_query_rows(gctx, orc, hd, heads, kvh, M, npa
         np.testing.assert_allclose(a.astype(np.float32), b.astype(np.float32), rtol=3e-3, atol=3e-3)
 
 
+def attention_model(orc, hd, heads, kvh, seed, q_std=None, k_std=None):
+    """One layer of Q8_0 weights; q_std / k_std: the spread of the q / k
+    weights in place of the builder's."""
+    d = heads * hd
+    cfg = P.model_cfg(1, d, heads, kvh, hd, 512, 300, rope_theta=500000.0)
+    dts = dict(tok_embd=P.Q8_0, output=P.Q8_0, q=P.Q8_0, k=P.Q8_0, v=P.Q8_0, o=P.Q8_0,
+               gate=P.Q8_0, up=P.Q8_0, down=P.Q4_K)
+    model = P.make_model(orc, cfg, dts, seed=seed)
+    rng = np.random.default_rng(seed)
+    for role, rows, std in (("q", heads * hd, q_std), ("k", kvh * hd, k_std)):
+        if std:
+            w = (rng.standard_normal((rows, d)) * std).astype(np.float32)
+            model["blk.0.%s" % role]["raw"][:] = orc.quantize(w, P.Q8_0).ravel()
+    return model
+
+
+@pytest.mark.parametrize("hd,heads,kvh,M,npast", [(128, 8, 2, 129, 70), (64, 16, 4, 200, 0)])
+def test_attention_of_queries_beyond_the_fp16_range(gctx, orc, hd, heads, kvh, M, npast):
+    """Query elements of some 1e5 (above fp16's largest value) against keys
+    that bring the scores back to ordinary size."""
+    model = attention_model(orc, hd, heads, kvh, hd + M, q_std=5000.0, k_std=1e-5)
+    toks = np.random.default_rng(M).integers(0, 300, M).tolist()
+    (got, want, _, _), = run_batch(gctx, orc, model, [(toks, None, npast, npast + M)], 256)
+    assert rel_err_rows(got, want) < LOGIT_TOL
+
+
+def test_attention_of_a_long_chain_beside_a_short_one(gctx, orc):
+    """Sequences of more than 512 and of at most 16 query rows per kv head in
+    one step: no attention launch takes both."""
+    model = attention_model(orc, 128, 8, 2, 77)
+    rng = np.random.default_rng(78)
+    seqs = [(rng.integers(0, 300, 130).tolist(), None, 20, 160), (rng.integers(0, 300, 3).tolist(), None, 50, 60)]
+    for (got, want, kv, kvo) in run_batch(gctx, orc, model, seqs, 256):
+        assert rel_err_rows(got, want) < LOGIT_TOL
+        for a, b in zip(kv, kvo):
+            np.testing.assert_allclose(a.astype(np.float32), b.astype(np.float32), rtol=3e-3, atol=3e-3)
+
+
 # ---- the backend's single operations ----
 
 

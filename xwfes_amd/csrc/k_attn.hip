@@ -23,6 +23,8 @@
 #include "mm_dev.h"
 #include "xq_dev.h"
 
+#include <type_traits>
+
 namespace {
 
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
@@ -478,6 +480,19 @@ __device__ __forceinline__ void attn_mfma_wg_mc(const AttnMArgs& a, int grp, int
 // Measured: 8 waves (two per SIMD) beat 16 (four per SIMD) and 32 rows per
 // wave on the 52-node tree and the 70B batch; the workgroup's MFMAs and
 // softmax arithmetic do not overlap, so its time is their sum.
+//
+// WIDE (more than 512 query rows per kv head: prefill chains): the query comes
+// from its fp32 row, scaled by the power of two that brings its largest value
+// into [2^14, 2^15) (undone in the exponent's factor: no value is too large for
+// fp16, and the halves hold 22 bits of every element down to 2^-17 of it); each
+// chunk's P . V is a sum of its own, added in fp32 (the MFMA rounds its sums
+// down, and a long context adds that up), the running sum in 64 bits, and the
+// exponents' offset is carried as it was rounded (formed anew from the maximum it
+// is off by an ulp of the score, a factor between chunks and partials).  Error
+// against 64 bits, 256 tokens, hd 128, context 444 / 4000: 2.1e-7 / 2.6e-7, with
+// scores six times as large 5.1e-7 / 6.6e-7 (the other form 3.1e-7 / 8.2e-7 and
+// 8.0e-7 / 2.4e-6, the generic kernel's fp32 dots and 64-bit softmax sum 4.9e-7 /
+// 9.1e-7 and 1.2e-6 / 1.7e-6), at the same time.
 constexpr int FA_WAVES = 8;
 constexpr int FA_CHK = 64;  // slots per chunk
 typedef __attribute__((address_space(3))) void lds_void;
@@ -487,7 +502,7 @@ __host__ __device__ constexpr size_t fa_lds_bytes() {
     return 2 * (size_t)(HD / 8 + HD / 8) * 1024;  // two buffers of K and V^T blocks
 }
 
-template <int HD>
+template <int HD, bool WIDE>
 __device__ __forceinline__ void attn_fa_wg(const AttnMArgs& a, int grp, int kvh, int qsplit,
                                            int ngrp) {
     constexpr int NDC = HD / 32;     // 32-dim steps of the score contraction
@@ -543,7 +558,35 @@ __device__ __forceinline__ void attn_fa_wg(const AttnMArgs& a, int grp, int kvh,
     // results stay in their own O^T columns and are never stored)
     v8h qf[NDC][2];
     const int rq0 = min(rbase + col, qrows - 1), node = rq0 / gqa;
-    {
+    float c2 = 1.4426950408889634f / sqrtf((float)HD);  // (of the lane's row)
+    if constexpr (WIDE) {
+        const float* qr = a.qkv + node * a.ldq + (kvh * gqa + rq0 % gqa) * HD + 8 * kq;
+        float qv[NDC][8], mx = 0.f;
+#pragma unroll
+        for (int dc = 0; dc < NDC; ++dc) {
+            *(float4*)&qv[dc][0] = *(const float4*)(qr + 32 * dc);
+            *(float4*)&qv[dc][4] = *(const float4*)(qr + 32 * dc + 4);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float b = fabsf(qv[dc][i]);
+                mx = b <= 3.402823466e38f ? fmaxf(mx, b) : mx;
+            }
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const int e = mx > 0.f ? min(max(14 - ilogbf(mx), -113), 126) : 0;
+        const float qscale = ldexpf(1.f, e);
+        c2 *= ldexpf(1.f, -e);
+#pragma unroll
+        for (int dc = 0; dc < NDC; ++dc)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                _Float16 h, l;
+                split_hl(qv[dc][i] * qscale, h, l);
+                qf[dc][0][i] = h;
+                qf[dc][1][i] = l;
+            }
+    } else {
         const int64_t qo = ((int64_t)node * a.n_head + kvh * gqa + rq0 % gqa) * HD + 8 * kq;
 #pragma unroll
         for (int dc = 0; dc < NDC; ++dc) {
@@ -551,8 +594,9 @@ __device__ __forceinline__ void attn_fa_wg(const AttnMArgs& a, int grp, int kvh,
             qf[dc][1] = wlive ? *(const v8h*)(a.ql16 + qo + 32 * dc) : v8h{};
         }
     }
-    const float c2 = 1.4426950408889634f / sqrtf((float)HD);
-    float mrun = -INFINITY, lrun = 0.f;  // running maximum of the raw scores, running sum
+    float mrun = -INFINITY;  // running maximum of the raw scores
+    float mcrun = -INFINITY;  // WIDE: the last chunk's exponent offset, as it was rounded
+    std::conditional_t<WIDE, double, float> lrun = 0;  // running sum
     v4f o[NDT];
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) o[dt] = v4f{0.f, 0.f, 0.f, 0.f};
@@ -585,10 +629,23 @@ __device__ __forceinline__ void attn_fa_wg(const AttnMArgs& a, int grp, int kvh,
 #pragma unroll
             for (int dc = 0; dc < NDC; ++dc) {
                 const v8h kf = *(const v8h*)(bufp + (st * NDC + dc) * 1024 + lane * 16);
+                if constexpr (WIDE) {
+                    // the lo products first, at their own size
+                    s[st] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                        kf, qf[dc][1], dc == 0 ? v4f{0.f, 0.f, 0.f, 0.f} : s[st], 0, 0, 0);
+                    continue;
+                }
                 s[st] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                     kf, qf[dc][0], dc == 0 ? v4f{0.f, 0.f, 0.f, 0.f} : s[st], 0, 0, 0);
                 s[st] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[dc][1], s[st], 0, 0, 0);
             }
+        if constexpr (WIDE)
+#pragma unroll
+            for (int st = 0; st < 4; ++st)
+#pragma unroll
+                for (int dc = 0; dc < NDC; ++dc)
+                    s[st] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                        *(const v8h*)(bufp + (st * NDC + dc) * 1024 + lane * 16), qf[dc][0], s[st], 0, 0, 0);
         if (tree) {
             // slot 8 kq + e of run sp: allowed iff before the draft, or a
             // draft slot j < M whose ancestor bit is set
@@ -614,7 +671,9 @@ __device__ __forceinline__ void attn_fa_wg(const AttnMArgs& a, int grp, int kvh,
         const float mn = fmaxf(mrun, mx);
         // every score so far masked: p = 0, nothing to rescale
         const float mc = mn == -INFINITY ? 0.f : mn * c2;
-        const float al = __builtin_amdgcn_exp2f(mrun * c2 - mc);  // 0 while mrun = -inf
+        // 0 while mrun = -inf
+        const float al = __builtin_amdgcn_exp2f(WIDE ? mcrun - mc : mrun * c2 - mc);
+        mcrun = mc;
         float sum = 0.f;
         v8h ph[2], pl[2];
 #pragma unroll
@@ -637,6 +696,24 @@ __device__ __forceinline__ void attn_fa_wg(const AttnMArgs& a, int grp, int kvh,
         sum += __shfl_xor(sum, 32, 64);
         lrun = al * lrun + sum;
         mrun = mn;
+        if constexpr (WIDE) {
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt) {
+                v4f t = {0.f, 0.f, 0.f, 0.f};
+                v8h vf[2];
+#pragma unroll
+                for (int sp = 0; sp < 2; ++sp) {
+                    vf[sp] = *(const v8h*)(bufp + (KB + 2 * dt + sp) * 1024 + lane * 16);
+                    t = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[sp], pl[sp], t, 0, 0, 0);
+                }
+#pragma unroll
+                for (int sp = 0; sp < 2; ++sp)
+                    t = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[sp], ph[sp], t, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[dt][r] = __builtin_fmaf(o[dt][r], al, t[r]);
+            }
+            continue;
+        }
         if (__builtin_amdgcn_ballot_w64(al != 1.f))  // a maximum moved (wave-uniform)
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt) o[dt] *= al;
@@ -656,27 +733,42 @@ __device__ __forceinline__ void attn_fa_wg(const AttnMArgs& a, int grp, int kvh,
     // lane (col, kq) of tile dt holds dims 16 dt + 4 kq + r of row col
     const int64_t qrow = (int64_t)(rq / gqa) * a.n_head + kvh * gqa + rq % gqa;
     float* po = a.pout + (qrow * ngrp + grp) * HD + 4 * kq;
+    if constexpr (WIDE) {
+        // the partial relative to e^pm, pm the offset in natural-log units as
+        // it is stored: 2^(mcrun - pm log2 e), log2 e in two parts
+        const float pm = mrun == -INFINITY ? -INFINITY : mcrun * 0.6931471805599453f;
+        const float f = mrun == -INFINITY ? 1.f
+                                          : __builtin_amdgcn_exp2f(__builtin_fmaf(-pm, 1.44269502f, mcrun) -
+                                                                   pm * 1.92596303e-8f);
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) *(v4f*)(po + 16 * dt) = o[dt] * f;
+        if (kq == 0) {
+            a.pmax[qrow * ngrp + grp] = pm;
+            a.psum[qrow * ngrp + grp] = (float)(lrun * f);
+        }
+        return;
+    }
 #pragma unroll
     for (int dt = 0; dt < NDT; ++dt) *(v4f*)(po + 16 * dt) = o[dt];
     if (kq == 0) {
         a.pmax[qrow * ngrp + grp] = mrun == -INFINITY ? -INFINITY : mrun * (c2 * 0.6931471805599453f);
-        a.psum[qrow * ngrp + grp] = lrun;
+        a.psum[qrow * ngrp + grp] = (float)lrun;
     }
 }
 
-template <int HD>
+template <int HD, bool WIDE>
 __global__ void __launch_bounds__(64 * FA_WAVES) k_attn_fa(AttnMArgs a) {
-    attn_fa_wg<HD>(a, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x);
+    attn_fa_wg<HD, WIDE>(a, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x);
 }
 
 // several sequences: grid.z runs over every sequence's query splits
 // (sequence s owns splits qt0[s] .. qt0[s + 1] - 1)
-template <int HD>
+template <int HD, bool WIDE>
 __global__ void __launch_bounds__(64 * FA_WAVES) k_attn_fa_batch(AttnMBatch b) {
     int s = 0;
     while (s + 1 < b.nseq && (int)blockIdx.z >= b.qt0[s + 1]) ++s;
     const AttnMArgs a = b.s[s];  // loaded once
-    attn_fa_wg<HD>(a, blockIdx.x, blockIdx.y, (int)blockIdx.z - b.qt0[s], b.nch[s]);
+    attn_fa_wg<HD, WIDE>(a, blockIdx.x, blockIdx.y, (int)blockIdx.z - b.qt0[s], b.nch[s]);
 }
 
 template <int HD, int CHK, int NWV>
@@ -936,6 +1028,16 @@ static int attn_chunks_per_wg(int64_t wgs) {
 // rows per kv head (measured: the 8-token chain of 32 rows per kv head at
 // context 2048 gains a little, the trees and batches most)
 static bool attn_fa_rows(int64_t qrows) { return qrows > 16; }
+// and its WIDE form those above 512, which no other kernel here takes
+static bool attn_wide_rows(int64_t qrows) { return qrows > 512; }
+bool attn_batch_supported(const int64_t* Ms, int nseq, int64_t n_head, int64_t n_kv) {
+    bool fa = true, wide = false;
+    for (int s = 0; s < nseq; ++s) {
+        fa = fa && attn_fa_rows(Ms[s] * (n_head / n_kv));
+        wide = wide || attn_wide_rows(Ms[s] * (n_head / n_kv));
+    }
+    return fa || !wide;
+}
 static int attn_fa_splits(int64_t qrows) { return (int)((qrows + 16 * FA_WAVES - 1) / (16 * FA_WAVES)); }
 
 // 64-slot chunks per workgroup (and per partial) for the many-row kernel:
@@ -963,7 +1065,7 @@ static int attn_fa_chunks_per_wg(const int64_t* nchk, const int* splits, int nse
     return best;
 }
 
-template <int HD, typename A>
+template <int HD, bool WIDE, typename A>
 static hipError_t launch_fa(void (*kern)(A), const dim3& grid, hipStream_t st, const A& args) {
     static bool lds_set = false;
     if (!lds_set) {
@@ -998,10 +1100,13 @@ hipError_t launch_attn_mfma(hipStream_t st, AttnMArgs a, float* part, int8_t* xq
         a.pout = part + 2 * qi * ngrp;
         const dim3 grid((unsigned)ngrp, (unsigned)a.n_kv, (unsigned)qs);
         hipError_t e;
+        const bool wide = attn_wide_rows(qrows);
         if (a.hd == 128)
-            e = launch_fa<128>(k_attn_fa<128>, grid, st, a);
+            e = wide ? launch_fa<128, true>(k_attn_fa<128, true>, grid, st, a)
+                     : launch_fa<128, false>(k_attn_fa<128, false>, grid, st, a);
         else
-            e = launch_fa<64>(k_attn_fa<64>, grid, st, a);
+            e = wide ? launch_fa<64, true>(k_attn_fa<64, true>, grid, st, a)
+                     : launch_fa<64, false>(k_attn_fa<64, false>, grid, st, a);
         if (e != hipSuccess) return e;
         if (xq) {
             const int64_t K = (int64_t)a.n_head * a.hd;
@@ -1058,8 +1163,13 @@ hipError_t launch_attn_mfma_batch(hipStream_t st, const AttnMArgs* as, const flo
     b.nseq = nseq;
     int hd = as[0].hd, nkv = as[0].n_kv, maxch = 0, qt = 0, qi = 0;
     // the many-row kernel when every sequence has the rows for it
-    bool fa = true;
-    for (int s = 0; s < nseq; ++s) fa = fa && attn_fa_rows((int64_t)as[s].M * (as[s].n_head / nkv));
+    bool fa = true, wide = false;
+    for (int s = 0; s < nseq; ++s) {
+        const int64_t r = (int64_t)as[s].M * (as[s].n_head / nkv);
+        fa = fa && attn_fa_rows(r);
+        wide = wide || attn_wide_rows(r);
+    }
+    if (wide && !fa) return hipErrorInvalidValue;  // attn_batch_supported
     int64_t wgs = 0;  // the one-block grid's live workgroups
     int64_t nblk[FTX_MAX_SEQ], nchk[FTX_MAX_SEQ];
     int splits[FTX_MAX_SEQ];
@@ -1101,9 +1211,11 @@ hipError_t launch_attn_mfma_batch(hipStream_t st, const AttnMArgs* as, const flo
     if (fa) {
         hipError_t e;
         if (hd == 128)
-            e = launch_fa<128>(k_attn_fa_batch<128>, grid, st, b);
+            e = wide ? launch_fa<128, true>(k_attn_fa_batch<128, true>, grid, st, b)
+                     : launch_fa<128, false>(k_attn_fa_batch<128, false>, grid, st, b);
         else if (hd == 64)
-            e = launch_fa<64>(k_attn_fa_batch<64>, grid, st, b);
+            e = wide ? launch_fa<64, true>(k_attn_fa_batch<64, true>, grid, st, b)
+                     : launch_fa<64, false>(k_attn_fa_batch<64, false>, grid, st, b);
         else
             return hipErrorInvalidValue;
         if (e != hipSuccess) return e;

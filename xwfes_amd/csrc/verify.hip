@@ -454,7 +454,9 @@ static int verify_large(ftx_ctx* ctx, ftx_model* m, const ftx_seq_args* sq, int6
         // RoPE, the KV write and attention: one launch each over all
         // sequences when every sequence takes the MFMA attention, else per
         // sequence
-        bool all_mattn = nseq > 1;
+        int64_t Ms[FTX_MAX_SEQ];
+        for (int64_t s = 0; s < nseq; ++s) Ms[s] = sq[s].M;
+        bool all_mattn = nseq > 1 && attn_batch_supported(Ms, (int)nseq, d.n_head, d.n_head_kv);
         for (int64_t s = 0; s < nseq && all_mattn; ++s)
             all_mattn = attn_mfma_supported(hd, sq[s].kv->kv_f16, sq[s].M, d.n_head, d.n_head_kv,
                                             sq[s].kv->cap_alloc);
@@ -478,7 +480,6 @@ static int verify_large(ftx_ctx* ctx, ftx_model* m, const ftx_seq_args* sq, int6
             RopeArgs ras[FTX_MAX_SEQ];
             AttnMArgs ams[FTX_MAX_SEQ];
             const float* parts[FTX_MAX_SEQ];
-            int64_t Ms[FTX_MAX_SEQ];
             double rope_b = 0.0, attn_b = 0.0;
             for (int64_t s = 0; s < nseq; ++s) {
                 ftx_kv* kv = sq[s].kv;
@@ -503,7 +504,6 @@ static int verify_large(ftx_ctx* ctx, ftx_model* m, const ftx_seq_args* sq, int6
                 }
                 ra.cs = d_cs + r0 * hd2 * 2;
                 ras[s] = ra;
-                Ms[s] = M;
                 AttnMArgs am{};
                 am.qkv = m->qkv + r0 * m->ldq;
                 am.ldq = m->ldq;
