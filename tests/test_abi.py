@@ -48,3 +48,17 @@ def test_dtype_ids_match_reference_and_oracle():
     assert (ftx.F32, ftx.F16, ftx.Q4_0, ftx.Q4_1, ftx.Q8_0, ftx.BF16) == (0, 1, 2, 3, 8, 30)
     assert (ftx.Q4_K, ftx.Q6_K) == (P.Q4_K, P.Q6_K)
     assert ftx.BLOCK == P.BLOCK
+
+
+@pytest.mark.parametrize("M", [9, 64, 2000, 65535])
+@pytest.mark.parametrize("K,cols,swiglu", [(4096, 2 * 14336, True), (4096, 14336, False),
+                                           (32, 524288, True), (262144, 64, False)])
+def test_scratch_of_the_single_operations_is_bounded(M, K, cols, swiglu):
+    """The one-pass GEMM's scratch for ftx_matmul and an expert's gate / up
+    (operand, split partials): 256 MiB, and what up to 64 rows and the splits
+    of a small launch (some 1024 tiles of 32 x 256) take."""
+    f = ftx.load()._Z11mm_op_byteslllii
+    f.restype, f.argtypes = C.c_size_t, [C.c_long] * 3 + [C.c_int] * 2
+    rows = min(M, 64)
+    small = rows * (6.5 * max(K, 256) + 4 * cols) + 1024 * 32 * 256 * 4 * 2
+    assert f(M, K, cols, 2 if swiglu else 0, 256) <= (256 << 20) + small

@@ -288,6 +288,31 @@ def test_expert_chunk_shapes(gctx, orc, dt, M, K, IC):
     close(got, out + h @ wd, np.abs(out) + ah @ np.abs(wd))
 
 
+def test_expert_chunk_in_several_launches(gctx, orc):
+    """So many gate / up rows that the tokens go through the GEMM 64 at a time,
+    the last launch with fewer."""
+    rng = np.random.default_rng(91)
+    M, K, IC, dt = 150, 32, 262144, P.Q8_0
+    (g, wg), (u, wu), (d, wd) = (weight(gctx, orc, rng, dt, IC, K) for _ in range(3))
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    got = rng.standard_normal((M, K)).astype(np.float32)
+    out = got.astype(np.float64)
+    j = ftx.ExpertJob(x.ctypes.data, got.ctypes.data, g.ptr, u.ptr, d.ptr, dt, 0, M, K, IC, g.nbytes // IC,
+                      d.nbytes // IC)
+    gctx.check(gctx.lib.ftx_expert_chunk(gctx.h, ctypes.byref(j)))
+    for t in (g, u, d):
+        t.free()
+    size = np.abs(out)
+    for m in range(M):
+        xg, xu = wg @ x[m].astype(np.float64), wu @ x[m].astype(np.float64)
+        h = xg / (1 + np.exp(-xg)) * xu
+        out[m] += h @ wd
+        size[m] += np.abs(h) @ np.abs(wd)
+    # 262144 products of a row: the splits' and waves' fp32 chains of some 64
+    # additions at most, 64 x 2^-24
+    assert (np.abs(got - out) / size).max() < 2.0 ** -18
+
+
 @pytest.mark.parametrize("dts,d,ff", [("q8_0", 512, 1408), ("q4_0", 256, 544), ("f16", 128, 200),
                                       ("mixed", 384, 512)])
 @pytest.mark.parametrize("M", [1, 3, 8])

@@ -363,10 +363,14 @@ int ftx_matmul(ftx_ctx* ctx, const float* x, int64_t M, int64_t K, const ftx_ten
     Staged s{};
     float* extra;
     const bool mv = mv_supported(W->dtype, K, M);
-    const bool mm = !mv && op_mm(W->dtype, M, K, N, W->row_bytes);
+    bool mm = !mv && op_mm(W->dtype, M, K, N, W->row_bytes);
     const size_t xqf = (xq_bytes(K) + 255) / 4;
     const size_t ef = mv ? xqf : (mm ? mm_op_bytes(M, K, N, EPI_STORE, ctx->cu_count) / 4 + 64 : 0);
     int rc = stage_xy(ctx, x, (size_t)(M * K), y, (size_t)(M * N), false, ef, s, &extra);
+    if (rc == FTX_E_NOMEM && mm) {
+        mm = false;  // (the generic kernels take no scratch)
+        rc = stage_xy(ctx, x, (size_t)(M * K), y, (size_t)(M * N), false, 0, s, &extra);
+    }
     if (rc) return rc;
     GemvSeg seg{W->data, W->dtype, W->row_bytes, N, s.y, N};
     if (mm) {
@@ -415,8 +419,12 @@ int ftx_down_axpy(ftx_ctx* ctx, const float* x, int64_t M, int64_t n_in, const f
     if (M == 0) return FTX_OK;
     Staged s{};
     float* part;
-    const size_t pf = down_part_floats(ctx, W->dtype, M, n_in, N);
+    size_t pf = down_part_floats(ctx, W->dtype, M, n_in, N);
     int rc = stage_xy(ctx, x, (size_t)(M * n_in), y, (size_t)(M * N), true, pf, s, &part);
+    if (rc == FTX_E_NOMEM && pf && axpy_supported(W->dtype, N)) {
+        pf = 0;  // one split
+        rc = stage_xy(ctx, x, (size_t)(M * n_in), y, (size_t)(M * N), true, pf, s, &part);
+    }
     if (rc) return rc;
     FTX_HIP(ctx, down(ctx, W->data, W->dtype, W->row_bytes, n_in, N, s.x, M, s.y, part, pf));
     if (s.y_host)
@@ -470,15 +478,23 @@ int ftx_expert_chunk(ftx_ctx* ctx, const ftx_expert_job* j) {
     const int64_t M = j->M, K = j->K, IC = j->IC;
     Staged s{};
     float* extra;
-    const size_t pf = down_part_floats(ctx, j->dt, M, IC, K);
+    size_t pf = down_part_floats(ctx, j->dt, M, IC, K);
     // h, then one block for the gate / up launch and after it the down one
-    const bool mm = op_mm(j->dt, M, K, 2 * IC, rb);
+    bool mm = op_mm(j->dt, M, K, 2 * IC, rb);
     const size_t gf = mm ? mm_op_bytes(M, K, 2 * IC, EPI_SWIGLU, ctx->cu_count) / 4 + 64 : 0;
     int rc = stage_xy(ctx, j->x, (size_t)(M * K), j->out, (size_t)(M * K), true,
                       (pf > gf ? pf : gf) + (size_t)(M * IC) + 64, s, &extra);
+    if (rc == FTX_E_NOMEM && (mm || axpy_supported(j->dt, K))) {
+        // without the block: gate / up on the kernels that take none, one
+        // split of the down
+        mm = false;
+        if (axpy_supported(j->dt, K)) pf = 0;
+        rc = stage_xy(ctx, j->x, (size_t)(M * K), j->out, (size_t)(M * K), true,
+                      pf + (size_t)(M * IC) + 64, s, &extra);
+    }
     if (rc) return rc;
     float* h = extra;
-    float* part = extra + (((size_t)(M * IC) + 63) & ~(size_t)63);
+    float* part = pf || mm ? extra + (((size_t)(M * IC) + 63) & ~(size_t)63) : nullptr;
     if (mm) {
         const MmSeg ms[2] = {{(const uint8_t*)j->gate, j->dt, IC, 0, rb},
                              {(const uint8_t*)j->up, j->dt, IC, 0, rb}};

@@ -2297,13 +2297,22 @@ hipError_t launch_tile(hipStream_t st, const GemvSeg* segs, int nseg, const floa
 }
 
 // ---- backend operations over stored rows
+constexpr int64_t MM_OP_ROWS = 64;
 bool mm_op_supported(int dt, int64_t M, int64_t K, int64_t N, int64_t row_bytes) {
     const bool k32 = dt == FTX_Q8_0 || dt == FTX_Q4_0 || dt == FTX_F16;
     const bool k256 = dt == FTX_Q4_K || dt == FTX_Q6_K;
-    // 32-bit offsets into the weights and the operand planes
+    // 32-bit offsets into the weights and the operand planes (of MM_OP_ROWS rows
+    // at least)
     return ((k32 && K % 32 == 0) || (k256 && K % 256 == 0)) && K > 0 && M > 0 && N > 0 &&
-           N * row_bytes < 0xF0000000ll && mm_pad_tokens(M) * ((K + 255) / 256 * 256) * 6 < 0xF0000000ll &&
+           N * row_bytes < 0xF0000000ll && MM_OP_ROWS * ((K + 255) / 256 * 256) * 6 < 0xF0000000ll &&
            M <= 65535;
+}
+// rows of one launch: all, or as many as keep its operand and a SwiGLU's gate
+// and up sums within 256 MiB (an operation of any M then has bounded scratch,
+// and a launch of that size fills the chip many times over)
+static int64_t mm_op_rows(int64_t M, int64_t K, int64_t cols, int epi) {
+    const int64_t row = (K + 255) / 256 * 256 * 13 / 2 + (epi == EPI_SWIGLU ? 4 * cols : 0);
+    return std::min(M, std::max<int64_t>(MM_OP_ROWS, (int64_t(256) << 20) / row / 64 * 64));
 }
 // operand (with the row scales), then partials, in bytes
 static size_t mm_op_act_bytes(int64_t M, int64_t K) {
@@ -2320,13 +2329,25 @@ static size_t mm_op_part_floats(int64_t M, int64_t K, int64_t cols, int epi, int
     return S > 1 || epi == EPI_SWIGLU ? (size_t)S * (size_t)M * (size_t)cols : 0;
 }
 size_t mm_op_bytes(int64_t M, int64_t K, int64_t cols, int epi, int cu_count) {
-    return mm_op_act_bytes(M, K) + mm_op_part_floats(M, K, cols, epi, cu_count) * 4;
+    // (the last launch's fewer rows may take more splits)
+    const int64_t rows = mm_op_rows(M, K, cols, epi), last = (M - 1) % rows + 1;
+    return mm_op_act_bytes(rows, K) + std::max(mm_op_part_floats(rows, K, cols, epi, cu_count),
+                                               mm_op_part_floats(last, K, cols, epi, cu_count)) * 4;
 }
 hipError_t launch_mm_op(hipStream_t st, const MmSeg* segs, int nseg, const float* x, int64_t ldx,
                         int64_t K, int64_t M, int epi, float* y, int64_t ldy, void* ws, int cu_count) {
-    const int64_t Mp = mm_pad_tokens(M), Kp = (K + 255) / 256 * 256;
     int64_t cols = 0;
     for (int i = 0; i < nseg; ++i) cols += segs[i].N;
+    const int64_t rows = mm_op_rows(M, K, cols, epi);
+    if (rows < M) {
+        for (int64_t m0 = 0; m0 < M; m0 += rows) {
+            const hipError_t e = launch_mm_op(st, segs, nseg, x + m0 * ldx, ldx, K, std::min(rows, M - m0),
+                                              epi, y + m0 * ldy, ldy, ws, cu_count);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
+    const int64_t Mp = mm_pad_tokens(M), Kp = (K + 255) / 256 * 256;
     __bf16* xb = (__bf16*)ws;
     v8bf* xs = (v8bf*)(xb + 3 * Mp * Kp);
     float* rs = (float*)((uint8_t*)xs + Mp * Kp / 2);
