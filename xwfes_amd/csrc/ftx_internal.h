@@ -203,9 +203,7 @@ hipError_t launch_down(hipStream_t st, const uint8_t* W, int dt, int64_t row_byt
 // (written back) and takes an RMSNorm weight; a normed operand is consumed
 // with launch_mv(..., normed = 1, eps).
 size_t xq_bytes(int64_t K);
-// stride of the per-8-row-chunk operands when a prep covers more than 8 rows
-size_t xq_chunk_bytes(int64_t K);
-// layout16: the operand layout of the 16x16x32 row-dot GEMV (launch_rd)
+// up to 8 rows; layout16: the operand layout of the 16x16x32 row-dot GEMV (launch_rd)
 // instead of launch_mv's
 hipError_t launch_xq_prep(hipStream_t st, float* x, int64_t ldx, const float* normw,
                           const float* part, int S, int64_t ldpart, int64_t K, int64_t M,
@@ -415,13 +413,12 @@ bool down_mfma_supported(int dt, int64_t n_in, int64_t N, int64_t M);
 size_t down_tiled_bytes(int dt, int64_t n_in, int64_t N);
 hipError_t launch_down_tile(hipStream_t st, const uint8_t* src, int64_t src_row_bytes, int dt,
                             int64_t n_in, int64_t N, uint8_t* dst);
-// split partials of launch_down_mfma for up to Mmax rows in 8-row chunks
-size_t down_mfma_part_floats(int dt, int64_t n_in, int64_t N, int64_t Mmax, int cu_count);
-// splits == null: the split partials are added into y here; otherwise the
-// partials are left in part[S][8][N] for the caller to fold and *splits = S
+// up to 8 rows: the split partials are left in part[S][8][N]
+// (down_mfma_part_floats) for the caller to fold, *splits = S
+size_t down_mfma_part_floats(int dt, int64_t n_in, int64_t N, int cu_count);
 hipError_t launch_down_mfma(hipStream_t st, int dt, const uint8_t* tiled, int64_t n_in, int64_t N,
-                            const float* h, int64_t ldh, int64_t M, float* y, int64_t ldy,
-                            float* part, int cu_count, int* splits);
+                            const float* h, int64_t ldh, int64_t M, float* part, int cu_count,
+                            int* splits);
 
 // quantise rows (synthetic model builder)
 hipError_t launch_quantize(hipStream_t st, const float* src, int dt, int64_t ncols,

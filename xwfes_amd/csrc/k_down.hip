@@ -485,14 +485,13 @@ static int64_t down_mfma_splits(int dt, int64_t n_in, int64_t N, int cu_count,
     return (nslices + spp - 1) / spp;
 }
 
-size_t down_mfma_part_floats(int dt, int64_t n_in, int64_t N, int64_t Mmax, int cu_count) {
-    const int64_t S = down_mfma_splits(dt, n_in, N, cu_count);
-    return (size_t)(((Mmax + 7) / 8) * S * 8 * N);
+size_t down_mfma_part_floats(int dt, int64_t n_in, int64_t N, int cu_count) {
+    return (size_t)(down_mfma_splits(dt, n_in, N, cu_count) * 8 * N);
 }
 
 hipError_t launch_down_mfma(hipStream_t st, int dt, const uint8_t* tiled, int64_t n_in, int64_t N,
-                            const float* h, int64_t ldh, int64_t M, float* y, int64_t ldy,
-                            float* part, int cu_count, int* splits) {
+                            const float* h, int64_t ldh, int64_t M, float* part, int cu_count,
+                            int* splits) {
     DownArgs a{};
     uint8_t *qs, *qh, *hdr, *d6;
     down_planes(dt, n_in, N, (uint8_t*)tiled, &qs, &qh, &hdr, &d6);
@@ -519,11 +518,6 @@ hipError_t launch_down_mfma(hipStream_t st, int dt, const uint8_t* tiled, int64_
         ktimed_launch(k_down_mfma<FTX_Q4_K>, grid, dim3(64 * DOWN_WAVES), 0, st, a);
     else
         ktimed_launch(k_down_mfma<FTX_Q6_K>, grid, dim3(64 * DOWN_WAVES), 0, st, a);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    if (splits) {
-        *splits = (int)S;
-        return hipSuccess;
-    }
-    return launch_part_reduce(st, part, (int)S, N, M, y, ldy);
+    *splits = (int)S;
+    return hipGetLastError();
 }

@@ -75,20 +75,13 @@ __global__ void __launch_bounds__(256) k_xq_prep(float* __restrict__ x, int64_t 
                                                  int8_t* __restrict__ xs32,
                                                  int8_t* __restrict__ xs16,
                                                  float* __restrict__ scale,
-                                                 float* __restrict__ ssq, int64_t cstride) {
+                                                 float* __restrict__ ssq) {
 #pragma clang fp contract(off)
     __shared__ float vs[256];
     const int64_t sb = blockIdx.x;
-    // row m of 8-row chunk c: the chunk's operand lies cstride bytes after
-    // the previous one's
-    const int c = blockIdx.y >> 3, m = blockIdx.y & 7, t = threadIdx.x;
-    const bool live = c * 8 + m < M;  // block-uniform
-    float* row = x + (int64_t)(c * 8 + m) * ldx;
-    frag += c * cstride;
-    xs32 += c * cstride;
-    xs16 += c * cstride;
-    scale = (float*)((int8_t*)scale + c * cstride);
-    ssq = (float*)((int8_t*)ssq + c * cstride);
+    const int m = blockIdx.y, t = threadIdx.x;
+    const bool live = m < M;  // block-uniform
+    float* row = x + (int64_t)m * ldx;
     const int l = t & 63;
     const int64_t k0 = sb * 256 + 4 * l;
     // the norm weights of lane l's four elements are loaded first, so that
@@ -640,11 +633,9 @@ __global__ void __launch_bounds__(256) k_part_reduce(const float* __restrict__ p
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int m = blockIdx.y;
     if (t >= N) return;
-    // rows past 8 read the partials of their own 8-row chunk, chunks S * 8 * N apart
-    const float* pc = part + (int64_t)(m >> 3) * S * 8 * N;
     float v = 0.f;
 #pragma unroll 8
-    for (int s = 0; s < S; ++s) v += pc[((int64_t)s * 8 + (m & 7)) * N + t];
+    for (int s = 0; s < S; ++s) v += part[((int64_t)s * 8 + m) * N + t];
     y[(int64_t)m * ldy + t] += v;
 }
 
@@ -652,7 +643,6 @@ __global__ void __launch_bounds__(256) k_part_reduce(const float* __restrict__ p
 
 // fragments K*16 | xs32 K | xs16 2K | scales (K/256)*8 floats | ssq (K/256)*8 floats
 size_t xq_bytes(int64_t K) { return (size_t)(K * 16 + K + K * 2 + K / 8 + K / 8 + 64); }
-size_t xq_chunk_bytes(int64_t K) { return (xq_bytes(K) + 255) / 256 * 256; }
 
 static float* xq_scale(int8_t* xq, int64_t K) { return xq_ptrs(xq, K).scale; }
 static float* xq_ssq(int8_t* xq, int64_t K) { return xq_ptrs(xq, K).ssq; }
@@ -660,16 +650,13 @@ static float* xq_ssq(int8_t* xq, int64_t K) { return xq_ptrs(xq, K).ssq; }
 hipError_t launch_xq_prep(hipStream_t st, float* x, int64_t ldx, const float* normw,
                           const float* part, int S, int64_t ldpart, int64_t K, int64_t M,
                           int8_t* xq, int layout16) {
-    if (K % 512 || K > 16384 || M < 1 || (part && M > 8)) return hipErrorInvalidValue;
+    if (K % 512 || K > 16384 || M < 1 || M > 8) return hipErrorInvalidValue;
     int8_t* frag = xq;
     int8_t* xs32 = xq + K * 16;
     int8_t* xs16 = xs32 + K;
-    // one operand per 8-row chunk, xq_chunk_bytes(K) apart
-    const int64_t chunks = (M + 7) / 8;
-    hipLaunchKernelGGL(layout16 ? k_xq_prep<true> : k_xq_prep<false>,
-                       dim3((unsigned)(K / 256), (unsigned)(8 * chunks)), dim3(256), 0, st, x, ldx,
-                       normw, part, S, ldpart, K, (int)M, frag, xs32, xs16, xq_scale(xq, K),
-                       xq_ssq(xq, K), (int64_t)xq_chunk_bytes(K));
+    hipLaunchKernelGGL(layout16 ? k_xq_prep<true> : k_xq_prep<false>, dim3((unsigned)(K / 256), 8),
+                       dim3(256), 0, st, x, ldx, normw, part, S, ldpart, K, (int)M, frag, xs32, xs16,
+                       xq_scale(xq, K), xq_ssq(xq, K));
     return hipGetLastError();
 }
 
@@ -680,8 +667,7 @@ bool mv_supported(int dt, int64_t K, int64_t M) {
            K <= 16384;
 }
 
-// y[m*ldy + n] += sum_s part[c][s][m % 8][n] for n < N, m < M, c = m / 8
-// (the split partials of 8-row chunks, one after another)
+// y[m*ldy + n] += sum_s part[s][m][n] for n < N, m < M <= 8 (rows of 8 per split)
 hipError_t launch_part_reduce(hipStream_t st, const float* part, int S, int64_t N, int64_t M,
                               float* y, int64_t ldy) {
     hipLaunchKernelGGL(k_part_reduce, dim3((unsigned)((N + 255) / 256), (unsigned)M), dim3(256), 0,

@@ -321,37 +321,30 @@ static int verify_large(ftx_ctx* ctx, ftx_model* m, const ftx_seq_args* sq, int6
             const int fr = flush_x();
             if (fr) return fr;
         }
-        // tiled K-quants the one-pass kernels do not take (Q6_K): the
-        // row-dot MFMA kernel on 8-row chunks (one activation prep for all)
-        bool tiled_all = mv_all(ts, nseg, K, 8) && (epi != EPI_SWIGLU || mv_swiglu_supported(K));
+        // tiled K-quants without a one-pass copy (Q6_K of models of at most 8
+        // tokens): the row-dot MFMA kernels
+        bool tiled_all = mv_all(ts, nseg, K, Mr) && (epi != EPI_SWIGLU || mv_swiglu_supported(K));
         for (int i = 0; tiled_all && i < nseg; ++i) tiled_all = m->mvt[idx[i]] != nullptr;
         if (tiled_all) {
             int rpts[3] = {0, 0, 0};
-            for (int i = 0; i < nseg; ++i) rpts[i] = m->mvt_rpt[idx[i]];
-            const bool rd = rd_use(ts, rpts, nseg, K, 8, epi, ctx->cu_count);
-            auto chunks = [&]() -> hipError_t {
-                hipError_t e = launch_xq_prep(st, (float*)xin, ldx, normw, nullptr, 0, D, K, Mr, m->xq,
-                                              rd);
+            GemvSeg cs[3];
+            for (int i = 0; i < nseg; ++i) {
+                rpts[i] = m->mvt_rpt[idx[i]];
+                cs[i] = gs[i];
+                cs[i].W = m->mvt[idx[i]];
+                cs[i].tiled = 1;
+                cs[i].rpt = rpts[i];
+            }
+            const bool rd = rd_use(ts, rpts, nseg, K, Mr, epi, ctx->cu_count);
+            auto gemv = [&]() -> hipError_t {
+                const hipError_t e = launch_xq_prep(st, (float*)xin, ldx, normw, nullptr, 0, D, K, Mr,
+                                                    m->xq, rd);
                 if (e != hipSuccess) return e;
-                for (int64_t c0 = 0; c0 < Mr; c0 += 8) {
-                    const int64_t mc = Mr - c0 < 8 ? Mr - c0 : 8;
-                    GemvSeg cs[3];
-                    for (int i = 0; i < nseg; ++i) {
-                        cs[i] = gs[i];
-                        cs[i].W = m->mvt[idx[i]];
-                        cs[i].tiled = 1;
-                        cs[i].rpt = m->mvt_rpt[idx[i]];
-                        if (cs[i].y) cs[i].y += c0 * cs[i].ldy;
-                    }
-                    const int8_t* xc = m->xq + (c0 / 8) * (int64_t)xq_chunk_bytes(K);
-                    e = rd ? launch_rd(st, cs, nseg, xc, K, mc, epi, normw != nullptr, eps)
-                           : launch_mv(st, cs, nseg, xc, K, mc, epi, ctx->cu_count, normw != nullptr,
-                                       eps, nullptr);
-                    if (e != hipSuccess) return e;
-                }
-                return hipSuccess;
+                return rd ? launch_rd(st, cs, nseg, m->xq, K, Mr, epi, normw != nullptr, eps)
+                          : launch_mv(st, cs, nseg, m->xq, K, Mr, epi, ctx->cu_count, normw != nullptr,
+                                      eps, nullptr);
             };
-            TRACED_L(kind, bytes, chunks());
+            TRACED_L(kind, bytes, gemv());
             return FTX_OK;
         }
         // (the few-row kernel has the norm in it)
@@ -625,7 +618,7 @@ static int verify_large(ftx_ctx* ctx, ftx_model* m, const ftx_seq_args* sq, int6
             auto small = [&]() -> hipError_t {
                 int S = 0;
                 hipError_t e = launch_down_mfma(st, dn->dtype, m->down_tiled[l], F, D, m->h, F, Mt,
-                                                m->x, D, m->downpart, ctx->cu_count, &S);
+                                                m->downpart, ctx->cu_count, &S);
                 return e != hipSuccess ? e
                                        : launch_part_reduce(st, m->downpart, S, D, Mt, m->x, D);
             };
@@ -827,7 +820,7 @@ int ftx_model_create(ftx_ctx* ctx, const ftx_model_desc* d, ftx_model** out) {
     }
     if (ok) {
         const int64_t Kmax = std::max(D, qdim);
-        ok = dalloc(&m->xq, (size_t)((Mmax + 7) / 8) * xq_chunk_bytes(Kmax)) &&
+        ok = dalloc(&m->xq, xq_bytes(Kmax)) &&
              dalloc(&m->qhl, (size_t)(2 * Mmax * qdim));
     }
     // re-tiled ffn_down copies (same bytes, MFMA-friendly order)
@@ -850,7 +843,7 @@ int ftx_model_create(ftx_ctx* ctx, const ftx_model_desc* d, ftx_model** out) {
     if (ok && any_tiled) {
         size_t pf = 0;
         for (int dt : {FTX_Q4_K, FTX_Q6_K})
-            pf = std::max(pf, down_mfma_part_floats(dt, d->n_ff, D, 8, ctx->cu_count));
+            pf = std::max(pf, down_mfma_part_floats(dt, d->n_ff, D, ctx->cu_count));
         ok = dalloc(&m->downpart, pf);
     }
     // row-dot projections and the LM head: tiled copies for the MFMA kernel
@@ -1441,7 +1434,7 @@ int ftx_verify_step(ftx_ctx* ctx, ftx_model* m, ftx_kv* kv, const ftx_verify_arg
         if (m->down_tiled[l] && down_mfma_supported(T[FTX_T_DOWN]->dtype, F, D, M)) {
             TRACED_IDEM(TK_DOWN, down_b,
                         launch_down_mfma(st, T[FTX_T_DOWN]->dtype, m->down_tiled[l], F, D, m->h,
-                                         F, M, m->x, D, m->downpart, ctx->cu_count, &fold_S));
+                                         F, M, m->downpart, ctx->cu_count, &fold_S));
         } else if (axpy_supported(T[FTX_T_DOWN]->dtype, D)) {
             TRACED(TK_DOWN, down_b,
                    launch_axpy(st, T[FTX_T_DOWN]->data, T[FTX_T_DOWN]->dtype,
