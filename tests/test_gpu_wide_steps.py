@@ -72,35 +72,6 @@ def test_attention_of_a_long_chain_beside_a_short_one(gctx, orc):
             np.testing.assert_allclose(a.astype(np.float32), b.astype(np.float32), rtol=3e-3, atol=3e-3)
 
 
-@pytest.mark.parametrize("hd,M,cap,npast", [
-    (64, 1, 66000, 70), (64, 1, 66000, 65900), (64, 2, 66000, 65900), (64, 8, 66000, 1000),
-    (64, 9, 66000, 65900), (64, 65, 66000, 300), (64, 65, 140000, 66100), (128, 3, 131300, 500),
-    (128, 66, 131300, 2000)])
-def test_attention_over_large_caches(gctx, orc, hd, M, cap, npast):
-    """Caches of more than 1024 attention blocks (65536 slots of head size 64,
-    131072 of 128), short and long contexts, 8 to 560 query rows per kv head:
-    the fused o operand (up to 8 tokens), the combine's rows above."""
-    heads = 8
-    d = heads * hd
-    cfg = P.model_cfg(1, d, heads, 1, hd, 512, 300, rope_theta=500000.0)
-    dts = dict(tok_embd=P.Q8_0, output=P.Q8_0, q=P.Q4_K, k=P.Q4_K, v=P.Q4_K, o=P.Q4_K,
-               gate=P.Q4_K, up=P.Q4_K, down=P.Q4_K)
-    model = P.make_model(orc, cfg, dts, seed=hd + M)
-    toks = np.random.default_rng(M).integers(0, 300, M).tolist()
-    (got, want, _, _), = run_batch(gctx, orc, model, [(toks, None, npast, cap)], max(M, 8))
-    assert rel_err_rows(got, want) < LOGIT_TOL
-
-
-def test_attention_of_a_batch_over_a_large_cache(gctx, orc):
-    """Two sequences of different cache sizes in one launch, few rows and many."""
-    model = attention_model(orc, 64, 8, 1, 79)
-    rng = np.random.default_rng(80)
-    for M in (1, 12):
-        seqs = [(rng.integers(0, 300, M).tolist(), None, 65700, 66000), (rng.integers(0, 300, M).tolist(), None, 50, 90)]
-        for (got, want, _, _) in run_batch(gctx, orc, model, seqs, 32):
-            assert rel_err_rows(got, want) < LOGIT_TOL
-
-
 # ---- the backend's single operations ----
 
 

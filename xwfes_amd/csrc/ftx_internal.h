@@ -568,7 +568,8 @@ struct AttnMArgs {
     int pslots = 0;      // slots per partial (set by the launcher)
     MmFragDst frag;      // frag.xh set: the fp32 combine writes this operand instead of out
 };
-bool attn_mfma_supported(int64_t hd, int kv_f16, int64_t M);
+bool attn_mfma_supported(int64_t hd, int kv_f16, int64_t M, int64_t n_head, int64_t n_kv,
+                         int64_t cap_alloc);
 // whether sequences of Ms[s] tokens share one launch (launch_attn_mfma_batch)
 bool attn_batch_supported(const int64_t* Ms, int nseq, int64_t n_head, int64_t n_kv);
 size_t attn_part_floats(int64_t M, int64_t n_head, int64_t hd, int64_t cap_alloc);

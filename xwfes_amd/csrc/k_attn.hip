@@ -23,7 +23,6 @@
 #include "mm_dev.h"
 #include "xq_dev.h"
 
-#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -809,7 +808,7 @@ __device__ __forceinline__ void attn_combine_row(const AttnMArgs& a, int64_t qi,
     // first CPF partials are read from their lanes (v_readlane), later ones
     // (more than CPF partials) through the wave's own LDS copy.
     constexpr int CPF = 8;
-    __shared__ float wsh[2][1024];  // weights of the partials (at most 1024) per wave
+    __shared__ float wsh[2][1024];  // chunk weights (nch <= 1024) per wave
     const int d = threadIdx.x, wv = d >> 6, lane = d & 63;
     const int64_t npast = a.npast;
     const int ch = a.pslots;  // slots per partial
@@ -897,7 +896,7 @@ template <int HD, bool L16>
 __global__ void __launch_bounds__(256) k_attn_combine_xq(AttnMArgs a, int nch, XqPtrs o) {
     constexpr int HPB = 256 / HD;
     constexpr int CPF = 8;  // chunk partials per thread held in registers
-    __shared__ float wsh[HPB][1024];  // weights of the partials (at most 1024)
+    __shared__ float wsh[HPB][1024];  // chunk weights (nch <= 1024)
     __shared__ float sden[HPB];
     __shared__ float4 red[4][64];
     const int64_t sb = blockIdx.x;
@@ -997,17 +996,16 @@ bool attn_combine_xq_supported(int64_t hd, int64_t n_head) {
 }
 
 // Any number of query rows: past 16 rows per kv head the many-row kernel takes
-// them 128 at a time.  Measured (256 tokens, 32 query heads on 8 kv heads of 128,
-// context 0-444): 2.05 ms per layer on the generic kernel, 14.5 + 8.5 us
-// (combine) here.  Any cache: attn_min_blocks.
-bool attn_mfma_supported(int64_t hd, int kv_f16, int64_t M) {
-    return kv_f16 && (hd == 64 || hd == 128) && M >= 1;
+// them 128 at a time.  Above 512 rows (256-token prefill chains) a cache of
+// more than 1024 chunks, whose weights the combine could not hold in LDS,
+// stays on the generic kernel.  Measured (256 tokens, 32 query heads on 8 kv
+// heads of 128, context 0-444): 2.05 ms per layer on the generic kernel, 14.5
+// + 8.5 us (combine) here.
+bool attn_mfma_supported(int64_t hd, int kv_f16, int64_t M, int64_t n_head, int64_t n_kv,
+                         int64_t cap_alloc) {
+    return kv_f16 && (hd == 64 || hd == 128) && M >= 1 &&
+           (M * (n_head / n_kv) <= 512 || cap_alloc / chunk_slots((int)hd) <= 1024);
 }
-
-// The combine holds a row's partial weights in LDS, 1024 of them: caches of more
-// blocks (65536 slots of head size 64, 131072 of 128) take this many blocks per
-// partial at least.
-static int attn_min_blocks(int64_t cap, int ch) { return (int)((cap / ch + 1023) / 1024); }
 
 size_t attn_part_floats(int64_t M, int64_t n_head, int64_t hd, int64_t cap_alloc) {
     const int64_t nch = (cap_alloc + chunk_slots((int)hd) - 1) / chunk_slots((int)hd);
@@ -1047,16 +1045,15 @@ static int attn_fa_splits(int64_t qrows) { return (int)((qrows + 16 * FA_WAVES -
 // chunks per workgroup the live workgroups run in rounds of 256, a round
 // costing about 3 + g chunk times (measured: ~3 us of start and ~1-2 us per
 // chunk, the chunk's MFMAs and softmax); the cheapest g in [gmin, 32], the
-// largest on ties (fewer partials for the combine).  gmin = the chunks of the
-// attn_min_blocks() blocks, so the partials fit the buffer sized per block and
-// the combine's LDS.
+// largest on ties (fewer partials for the combine).  gmin = the chunks of
+// one chunk_slots(hd) block, so the partials fit the buffer sized per block.
 // Whole chunks rather than whole blocks let the 52-node tree at context
 // 4096 take 224 workgroups of 5 chunks instead of 176 of 6.
 static int attn_fa_chunks_per_wg(const int64_t* nchk, const int* splits, int nseq, int n_kv,
                                  int gmin) {
     int best = gmin;
     int64_t best_cost = -1;
-    for (int g = gmin; g <= std::max(32, gmin); ++g) {
+    for (int g = gmin; g <= 32; ++g) {
         int64_t wgs = 0;
         for (int s = 0; s < nseq; ++s) wgs += (nchk[s] + g - 1) / g * n_kv * splits[s];
         const int64_t cost = (wgs + 255) / 256 * (3 + (int64_t)g);
@@ -1086,7 +1083,8 @@ hipError_t launch_attn_mfma(hipStream_t st, AttnMArgs a, float* part, int8_t* xq
     // whole chunks of the allocation: every slot a chunk reads is allocated
     const int ch = chunk_slots(a.hd);
     if (a.cap % ch) return hipErrorInvalidValue;
-    const int nch = (int)(a.cap / ch), nb = attn_min_blocks(a.cap, ch);
+    const int nch = (int)(a.cap / ch);
+    if (nch > 1024) return hipErrorInvalidValue;  // combine weights live in LDS
     const int64_t qi = (int64_t)a.M * a.n_head;
     const int64_t qrows = (int64_t)a.M * (a.n_head / a.n_kv);
     if (attn_fa_rows(qrows)) {
@@ -1094,8 +1092,7 @@ hipError_t launch_attn_mfma(hipStream_t st, AttnMArgs a, float* part, int8_t* xq
         const int64_t nchk = (a.npast + a.M + FA_CHK - 1) / FA_CHK;
         // the combine that writes the GEMV operand takes one block per
         // partial (the 8-token chain: 136 workgroups of two chunks)
-        const int gmin = nb * ch / FA_CHK;
-        const int g = xq ? gmin : attn_fa_chunks_per_wg(&nchk, &qs, 1, a.n_kv, gmin);
+        const int g = xq ? ch / FA_CHK : attn_fa_chunks_per_wg(&nchk, &qs, 1, a.n_kv, ch / FA_CHK);
         a.pslots = g * FA_CHK;
         const int ngrp = (int)((a.cap + a.pslots - 1) / a.pslots);  // the partials' stride
         a.pmax = part;
@@ -1125,7 +1122,7 @@ hipError_t launch_attn_mfma(hipStream_t st, AttnMArgs a, float* part, int8_t* xq
     // one workgroup per (chunk or group of chunks, kv head, tile of 32 query rows)
     const int qtiles = (int)((a.M * (a.n_head / a.n_kv) + 31) / 32);
     const int64_t nvalid = (a.npast + a.M + ch - 1) / ch;
-    a.nc = std::max(nb, xq ? 1 : attn_chunks_per_wg(nvalid * a.n_kv * qtiles));
+    a.nc = xq ? 1 : attn_chunks_per_wg(nvalid * a.n_kv * qtiles);
     a.pslots = a.nc * ch;
     const int ngrp = (nch + a.nc - 1) / a.nc;  // the partials' stride
     a.pmax = part;
@@ -1175,10 +1172,9 @@ hipError_t launch_attn_mfma_batch(hipStream_t st, const AttnMArgs* as, const flo
     if (wide && !fa) return hipErrorInvalidValue;  // attn_batch_supported
     int64_t wgs = 0;  // the one-block grid's live workgroups
     int64_t nblk[FTX_MAX_SEQ], nchk[FTX_MAX_SEQ];
-    int splits[FTX_MAX_SEQ], nb = 1;
+    int splits[FTX_MAX_SEQ];
     for (int s = 0; s < nseq; ++s) {
         const int ch = chunk_slots(as[s].hd);
-        nb = std::max(nb, attn_min_blocks(as[s].cap, ch));
         if (as[s].hd != hd || as[s].n_kv != nkv || as[s].cap % ch) return hipErrorInvalidValue;
         const int64_t r = (int64_t)as[s].M * (as[s].n_head / nkv);
         nblk[s] = (as[s].npast + as[s].M + ch - 1) / ch;
@@ -1187,11 +1183,12 @@ hipError_t launch_attn_mfma_batch(hipStream_t st, const AttnMArgs* as, const flo
         wgs += nblk[s] * nkv * splits[s];
     }
     // many-row: g chunks per partial; otherwise nc blocks
-    const int g = fa ? attn_fa_chunks_per_wg(nchk, splits, nseq, nkv, nb * chunk_slots(hd) / FA_CHK) : 0;
-    const int nc = fa ? 1 : std::max(nb, attn_chunks_per_wg(wgs));
+    const int g = fa ? attn_fa_chunks_per_wg(nchk, splits, nseq, nkv, chunk_slots(hd) / FA_CHK) : 0;
+    const int nc = fa ? 1 : attn_chunks_per_wg(wgs);
     for (int s = 0; s < nseq; ++s) {
         AttnMArgs a = as[s];
         const int ch = chunk_slots(a.hd);
+        if (a.cap / ch > 1024) return hipErrorInvalidValue;  // combine weights live in LDS
         a.nc = nc;
         a.pslots = fa ? g * FA_CHK : nc * ch;
         const int nch = (int)((a.cap + a.pslots - 1) / a.pslots);  // the partials' stride

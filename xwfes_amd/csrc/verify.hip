@@ -451,7 +451,8 @@ static int verify_large(ftx_ctx* ctx, ftx_model* m, const ftx_seq_args* sq, int6
         for (int64_t s = 0; s < nseq; ++s) Ms[s] = sq[s].M;
         bool all_mattn = nseq > 1 && attn_batch_supported(Ms, (int)nseq, d.n_head, d.n_head_kv);
         for (int64_t s = 0; s < nseq && all_mattn; ++s)
-            all_mattn = attn_mfma_supported(hd, sq[s].kv->kv_f16, sq[s].M);
+            all_mattn = attn_mfma_supported(hd, sq[s].kv->kv_f16, sq[s].M, d.n_head, d.n_head_kv,
+                                            sq[s].kv->cap_alloc);
         // the attention combine writes the o projection's one-pass GEMM
         // operand when every sequence takes the MFMA attention (its prep is
         // then skipped)
@@ -460,7 +461,8 @@ static int verify_large(ftx_ctx* ctx, ftx_model* m, const ftx_seq_args* sq, int6
             MmSeg oseg;
             bool of = mm_seg((size_t)(lt + FTX_T_O), T[FTX_T_O], oseg);
             for (int64_t s = 0; s < nseq && of; ++s)
-                of = attn_mfma_supported(hd, sq[s].kv->kv_f16, sq[s].M);
+                of = attn_mfma_supported(hd, sq[s].kv->kv_f16, sq[s].M, d.n_head, d.n_head_kv,
+                                            sq[s].kv->cap_alloc);
             if (of) {
                 const MmAct oact = mm_act(m->mm_act, mm_pad_tokens(Mt), m->qdim);
                 ofd = MmFragDst{oact.xh, oact.xl, oact.sh, oact.sl, 0, m->qdim,
@@ -527,7 +529,8 @@ static int verify_large(ftx_ctx* ctx, ftx_model* m, const ftx_seq_args* sq, int6
             const size_t kvel = kv->kv_f16 ? 2 : 4;
             uint8_t* kl = (uint8_t*)kv->k + (size_t)(l * kv->cap_alloc * kv->kdim) * kvel;
             uint8_t* vl = (uint8_t*)kv->v + (size_t)(l * kv->cap_alloc * kv->kdim) * kvel;
-            const bool mattn = attn_mfma_supported(hd, kv->kv_f16, M);
+            const bool mattn = attn_mfma_supported(hd, kv->kv_f16, M, d.n_head, d.n_head_kv,
+                                                   kv->cap_alloc);
             RopeArgs ra{m->qkv + r0 * m->ldq, m->ldq,  d.n_head,   d.n_head_kv, hd,
                         d_depth + r0,         d_np + s, d.rope_theta, d.rope_neox, kl,
                         vl,                   kv->kv_f16, kv->cap_alloc};
@@ -1351,7 +1354,8 @@ int ftx_verify_step(ftx_ctx* ctx, ftx_model* m, ftx_kv* kv, const ftx_verify_arg
                           seg(T[FTX_T_V], m->qkv + m->qdim + m->kdim, m->ldq)};
         uint8_t* kl = (uint8_t*)kv->k + (size_t)(l * kv->cap_alloc * kv->kdim) * kvel;
         uint8_t* vl = (uint8_t*)kv->v + (size_t)(l * kv->cap_alloc * kv->kdim) * kvel;
-        const bool mattn = attn_mfma_supported(d.head_dim, kv->kv_f16, M);
+        const bool mattn = attn_mfma_supported(d.head_dim, kv->kv_f16, M, d.n_head, d.n_head_kv,
+                                               kv->cap_alloc);
         // RoPE and the KV write ride on the projection's epilogue when the
         // MFMA kernels take both (interleaved pairs are adjacent outputs)
         const bool fuse = mattn && !d.rope_neox && mv_all(tqkv, 3, D, M);
