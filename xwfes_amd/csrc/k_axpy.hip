@@ -581,11 +581,6 @@ bool axpy_supported(int dt, int64_t N) {
                      ((dt == FTX_Q4_K || dt == FTX_Q6_K) && N % 256 == 0));
 }
 
-// 16-token tiles per workgroup, and splits over the rows: workgroups run two
-// to a CU in rounds of 512 (four tiles: 256 VGPRs, one to a CU), each as long as its waves' slices (every eighth of
-// the split's) plus about two slices of start and reduction; the fewest slice
-// times, the fewest splits on ties, within `cap` partial floats (one split
-// writes y itself)
 // splits of the few-token kernel: workgroups of 512 columns, 8 waves each;
 // about 512 of them, at least 64 rows (8 a wave) per split, within `cap`
 static bool axpy_few(int dt, int64_t M) { return M <= 8 && (dt == FTX_Q8_0 || dt == FTX_Q4_0); }
@@ -595,11 +590,18 @@ static int axpy_few_splits(int64_t M, int64_t n_in, int64_t N, size_t cap) {
     while (S > 1 && (size_t)(S * M * N) > cap) --S;
     return (int)S;
 }
+// 16-token tiles per workgroup, and splits over the rows: one-tile workgroups run
+// two to a CU, those of two and four tiles (164 to 256 VGPRs) one, in rounds, each
+// as long as its waves' slices (every eighth of the split's) plus about two
+// slices of start and reduction; the fewest slice times, the fewest splits on
+// ties, within `cap` partial floats (one split writes y itself).  (Two to a CU
+// assumed for two tiles as well: twice the splits in two rounds, 24 tokens of
+// Q4_0 14336 x 4096 79 us a call against 70 us, 4096 x 4096 60 against 53.)
 static int axpy_ms(int64_t M) { return M <= 16 ? 1 : (M <= 32 ? 2 : 4); }
 static int axpy_splits(int64_t M, int64_t n_in, int64_t N, size_t cap, int cu_count) {
     const int ms = axpy_ms(M);
     const int64_t wg = (N + AX_COLS - 1) / AX_COLS * ((M + 16 * ms - 1) / (16 * ms));
-    const int64_t nsl = (n_in + 31) / 32, slots = (ms == 4 ? 1 : 2) * (cu_count > 0 ? cu_count : 256);
+    const int64_t nsl = (n_in + 31) / 32, slots = (ms == 1 ? 2 : 1) * (cu_count > 0 ? cu_count : 256);
     int best = 1;
     int64_t best_cost = -1;
     for (int64_t S = 1; S <= 32 && S <= nsl; ++S) {
