@@ -72,6 +72,17 @@ def test_attention_of_a_long_chain_beside_a_short_one(gctx, orc):
             np.testing.assert_allclose(a.astype(np.float32), b.astype(np.float32), rtol=3e-3, atol=3e-3)
 
 
+@pytest.mark.parametrize("hd,M,cap,npast", [(64, 65, 66000, 300), (128, 66, 131300, 2000)])
+def test_many_rows_over_a_large_cache(gctx, orc, hd, M, cap, npast):
+    """More than 512 query rows per kv head over a cache of more than 1024
+    attention blocks, whose weights the combine could not hold: the generic
+    kernel (steps of fewer rows are refused, test_trace_disarmed_after_failed_launch)."""
+    model = attention_model(orc, hd, 8, 1, hd + M)
+    toks = np.random.default_rng(M).integers(0, 300, M).tolist()
+    (got, want, _, _), = run_batch(gctx, orc, model, [(toks, None, npast, cap)], M)
+    assert rel_err_rows(got, want) < LOGIT_TOL
+
+
 # ---- the backend's single operations ----
 
 
