@@ -152,7 +152,9 @@ int ftx_down_axpy(ftx_ctx* ctx, const float* x, int64_t M, int64_t n_in, const f
  * that forbid hipMalloc).  x and y must be device memory; the split partials
  * go to a file-scope device array of the library (16 MiB per GPU, held until
  * the process ends) instead of the context's workspace, so nothing is
- * allocated.  Shapes whose partials exceed that array return FTX_E_RANGE.
+ * allocated.  Shapes whose partials would exceed that array (reckoned for any
+ * weight type; a quarter of a million tokens x columns and more may) return
+ * FTX_E_RANGE.
  * The result is stream-ordered: the call returns once its two kernels are
  * enqueued on the context's stream (ftx_sync, or any later synchronising
  * call, waits for them), so it may be recorded into a HIP graph.  Every call

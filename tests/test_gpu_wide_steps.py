@@ -446,3 +446,52 @@ def test_small_step_of_a_huge_residual(gctx, orc, dt, d):
     emb[:] = np.where(np.random.default_rng(3).random(emb.shape) < 0.5, -3e38, 3e38)
     (got, want, _, _), = run_batch(gctx, orc, model, [([5, 6, 9], None, 0, 16)], 8)
     assert not want.any() and not got.any()
+
+
+# ---- residual acceptance: its own row statistics
+
+
+@pytest.mark.parametrize("V", [1, 3, 127, 4095, 4096, 4097, 8194, 20480, 33001])
+@pytest.mark.parametrize("off", [0, 4])
+def test_residual_statistics_at_chunk_edges(gctx, orc, V, off):
+    """Rows that end inside, at and past a 4096-element chunk and a 128-element
+    sub-chunk, of any alignment; logits of any size, masked ones (-inf, the
+    type's lowest value) among them, a row whose last element is its maximum."""
+    rng = np.random.default_rng(V + off)
+    M = 6
+    rows = (rng.standard_normal((M + 1, V)) * np.array([1, 3, 0.1, 1, 20, 1, 1])[:, None]).astype(np.float32)
+    rows[1, V // 3:V // 2] = -np.inf
+    rows[3, 2 * V // 3:] = np.finfo(np.float32).min
+    rows[2, V - 1] = 9
+    rows[4] += 1e4
+    q = rng.dirichlet(np.ones(V) * 0.5, size=M).astype(np.float32)
+    b, qb = gctx.buffer((M + 1) * V * 4 + 16), gctx.buffer(M * V * 4)
+    b.write(rows, off)
+    qb.write(q)
+    for seed in range(1, 9):
+        parents = [-1, -1, 0, 0, 1, 3] if seed % 2 else list(range(-1, M - 1))
+        # every other token the target's favourite, the others the draft's
+        props = [int(np.argmax(rows[parents[i] + 1] if (i + seed) % 2 else q[i])) for i in range(M)]
+        g = gctx.accept(b.ptr + off, b.ptr + off + V * 4, M, V, props, ftx.ACCEPT_RESIDUAL, temp=0.8,
+                        rng=seed, parents=parents, q_ptr=qb.ptr)
+        o = orc.verify_accept(rows[0], rows[1:], props, P.ACCEPT_RESIDUAL, temp=0.8, seed=seed,
+                              parents=parents, q=q)
+        assert (g["accepted"], g["bonus"], g["rng"]) == (o["accepted"], o["bonus"], o["rng"]), seed
+        # a ratio of sums of V terms in 64 bits, rounded to fp32
+        assert abs(g["margin"] - o["margin"]) < 1e-6, seed
+    for x in (b, qb):
+        x.free()
+
+
+@pytest.mark.parametrize("d,down,M", [(16384, P.Q8_0, 12), (16640, P.Q8_0, 12), (16640, P.Q6_K, 9), (288, P.Q8_0, 20)])
+def test_down_partials_of_wide_and_ragged_rows(gctx, orc, d, down, M):
+    """ffn_down on the stored rows of models at both sides of 16384 columns, and
+    of rows that are no whole 256: its partials left to the next norm, or added
+    at once."""
+    dts = dict(tok_embd=P.Q8_0, output=P.Q8_0, q=P.Q8_0, k=P.Q8_0, v=P.Q8_0, o=P.Q8_0, gate=P.Q8_0,
+               up=P.Q8_0, down=down)
+    cfg = P.model_cfg(2, d, 2, 1, 64, 1024, 60, rope_theta=10000.0)
+    model = P.make_model(orc, cfg, dts, seed=d + down)
+    toks = np.random.default_rng(M).integers(0, 60, M).tolist()
+    (got, want, _, _), = run_batch(gctx, orc, model, [(toks, None, 5, 40)], 32)
+    assert rel_err_rows(got, want) < LOGIT_TOL

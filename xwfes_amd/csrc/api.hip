@@ -447,6 +447,8 @@ int ftx_down_axpy_noalloc(ftx_ctx* ctx, const float* x, int64_t M, int64_t n_in,
         return ftx_fail(ctx, FTX_E_INVALID, "down_axpy_noalloc: x and y must be device memory");
     const int64_t N = W->ne[0];
     if (M == 0) return FTX_OK;
+    // (one rule for every type: the generic kernel's partials.  The block types'
+    // kernel fits its splits to the array and would need less.)
     const size_t pf = down_scratch_floats(M, n_in, N);
     if (pf > NOALLOC_SCRATCH_FLOATS)
         return ftx_fail(ctx, FTX_E_RANGE,

@@ -619,7 +619,8 @@ struct RowChunks {
     float* cmax;     // [nrows][nch]
     int32_t* carg;   // [nrows][nch]
     double* csub;    // [nrows][nsub] sum of exp((double)((l - max)/T))
-    double* csubf;   // [nrows][nsub] sum of the float expf((l - max)/T) (the sampler's)
+    double* csubf;   // [nrows][nsub] sum of the float expf((l - max)/T) (the sampler's);
+                     // RESIDUAL, which has no sampler: [nrows][nch] the chunks' double sums
     float* submax;   // [nrows][nsub] sub-chunk maxima
     int nch, nsub;
 };

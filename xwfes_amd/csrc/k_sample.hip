@@ -166,7 +166,7 @@ __global__ void __launch_bounds__(256) k_row_sum_res(const float* __restrict__ b
     __shared__ double sd[4];
     const int64_t r = blockIdx.y;
     const int c = blockIdx.x, t = threadIdx.x;
-    if (c == 0 && r == 0 && t < nwords) words[t] = 0;
+    if (c == 0 && r == 0 && t < nwords) words[t] = 0;  // (at most 256)
     const float* row = stat_row(base_row, rows, r, V);
     const int64_t i0 = (int64_t)c * SCH + 4 * t;
     float v[4][4];
@@ -1122,6 +1122,7 @@ hipError_t launch_accept_multi(hipStream_t st, const AcceptDev* d_arr, int n) {
     return hipGetLastError();
 }
 
+static_assert(3 * ACC_RES_WG <= 256, "k_row_sum_res clears a word per thread of one workgroup");
 size_t accept_residual_scratch_bytes() { return 3 * ACC_RES_WG * sizeof(double); }
 
 // RESIDUAL acceptance over ACC_RES_WG workgroups, launched cooperatively so
