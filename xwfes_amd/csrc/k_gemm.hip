@@ -1077,134 +1077,133 @@ __global__ void __launch_bounds__(64 * MM_WAVES)
                             for (int r = 0; r < 4; ++r) acc[t][ms][r] += (double)tmp[t][ms][r];
                     }
                 }
-                continue;
             } else {
-            // every fragment read of the K-step first, then the weight
-            // operands, then the MFMAs
-            v8h ah[MS], al[MS];
+                // every fragment read of the K-step first, then the weight
+                // operands, then the MFMAs
+                v8h ah[MS], al[MS];
 #pragma unroll
-            for (int ms = 0; ms < MS; ++ms) {
-                if (XT && ms >= nsub) break;
-                ah[ms] = frag(buf, 0, ms, j);
-                al[ms] = frag(buf, 1, ms, j);
-            }
-            v8h bw[MM_NT], bw2[MM_NT];
-            float bs[MM_NT];
+                for (int ms = 0; ms < MS; ++ms) {
+                    if (XT && ms >= nsub) break;
+                    ah[ms] = frag(buf, 0, ms, j);
+                    al[ms] = frag(buf, 1, ms, j);
+                }
+                v8h bw[MM_NT], bw2[MM_NT];
+                float bs[MM_NT];
 #pragma unroll
-            for (int t = 0; t < MM_NT; ++t) {
-                if constexpr (DT == FTX_Q4_K) {
-                    // (1024 + q) * sc - 1024 sc = sc q, one rounding of an exact
-                    // integer <= 945
-                    const v2i wv = wc.qs[t][j >> 1];
-                    const uint32_t x0 = (j & 1) ? ((uint32_t)wv.x >> 4) & 0x0F0F0F0Fu
-                                                : (uint32_t)wv.x & 0x0F0F0F0Fu;
-                    const uint32_t x1 = (j & 1) ? ((uint32_t)wv.y >> 4) & 0x0F0F0F0Fu
-                                                : (uint32_t)wv.y & 0x0F0F0F0Fu;
-                    const v2h sc = (j & 1) ? v2h{scp[t][j >> 1][1], scp[t][j >> 1][1]}
-                                           : v2h{scp[t][j >> 1][0], scp[t][j >> 1][0]};
-                    const v2h sn = (j & 1) ? v2h{scn[t][j >> 1][1], scn[t][j >> 1][1]}
-                                           : v2h{scn[t][j >> 1][0], scn[t][j >> 1][0]};
-                    v2h q[4];
-                    q[0] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(x0, 0x64646464u, 0x00050004u));
-                    q[1] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(x0, 0x64646464u, 0x00070006u));
-                    q[2] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(x1, 0x64646464u, 0x00050004u));
-                    q[3] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(x1, 0x64646464u, 0x00070006u));
+                for (int t = 0; t < MM_NT; ++t) {
+                    if constexpr (DT == FTX_Q4_K) {
+                        // (1024 + q) * sc - 1024 sc = sc q, one rounding of an exact
+                        // integer <= 945
+                        const v2i wv = wc.qs[t][j >> 1];
+                        const uint32_t x0 = (j & 1) ? ((uint32_t)wv.x >> 4) & 0x0F0F0F0Fu
+                                                    : (uint32_t)wv.x & 0x0F0F0F0Fu;
+                        const uint32_t x1 = (j & 1) ? ((uint32_t)wv.y >> 4) & 0x0F0F0F0Fu
+                                                    : (uint32_t)wv.y & 0x0F0F0F0Fu;
+                        const v2h sc = (j & 1) ? v2h{scp[t][j >> 1][1], scp[t][j >> 1][1]}
+                                               : v2h{scp[t][j >> 1][0], scp[t][j >> 1][0]};
+                        const v2h sn = (j & 1) ? v2h{scn[t][j >> 1][1], scn[t][j >> 1][1]}
+                                               : v2h{scn[t][j >> 1][0], scn[t][j >> 1][0]};
+                        v2h q[4];
+                        q[0] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(x0, 0x64646464u, 0x00050004u));
+                        q[1] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(x0, 0x64646464u, 0x00070006u));
+                        q[2] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(x1, 0x64646464u, 0x00050004u));
+                        q[3] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(x1, 0x64646464u, 0x00070006u));
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) q[i] = __builtin_elementwise_fma(q[i], sc, sn);
-                    bw[t] = v8h{q[0][0], q[0][1], q[1][0], q[1][1], q[2][0], q[2][1], q[3][0], q[3][1]};
-                    bs[t] = 0.f;
-                } else if constexpr (DT == FTX_Q8_0_MMT) {
-                    const v4i qv = wc.q[t][j >> 1];
-                    bw[t] = i8x8((j & 1) ? v2i{qv[2], qv[3]} : v2i{qv[0], qv[1]});
-                    bs[t] = scale8(wc.d[t], j);
-                } else if constexpr (DT == FTX_Q6_K_MMT) {
-                    uint32_t b0, b1;
-                    q6k_bytes(wc, t, j, b0, b1);
-                    // the scale split 16 sh + sl
-                    const int sc = q6k_scale(wc, t, j, kq);
-                    const int sl = sc & 15, sh = sc >> 4;
-                    const _Float16 fl = (_Float16)(float)sl, fh = (_Float16)(float)sh;
-                    const _Float16 ol = (_Float16)(float)(-1056 * sl), oh = (_Float16)(float)(-1056 * sh);
-                    const v2h l1 = {fl, fl}, l0 = {ol, ol}, m1 = {fh, fh}, m0 = {oh, oh};
-                    const v2h s16 = {(_Float16)16.f, (_Float16)16.f};
-                    v2h q[4];
-                    q[0] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(b0, 0x64646464u, 0x00050004u));
-                    q[1] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(b0, 0x64646464u, 0x00070006u));
-                    q[2] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(b1, 0x64646464u, 0x00050004u));
-                    q[3] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(b1, 0x64646464u, 0x00070006u));
-                    v2h r1[4], r2[4];
+                        for (int i = 0; i < 4; ++i) q[i] = __builtin_elementwise_fma(q[i], sc, sn);
+                        bw[t] = v8h{q[0][0], q[0][1], q[1][0], q[1][1], q[2][0], q[2][1], q[3][0], q[3][1]};
+                        bs[t] = 0.f;
+                    } else if constexpr (DT == FTX_Q8_0_MMT) {
+                        const v4i qv = wc.q[t][j >> 1];
+                        bw[t] = i8x8((j & 1) ? v2i{qv[2], qv[3]} : v2i{qv[0], qv[1]});
+                        bs[t] = scale8(wc.d[t], j);
+                    } else if constexpr (DT == FTX_Q6_K_MMT) {
+                        uint32_t b0, b1;
+                        q6k_bytes(wc, t, j, b0, b1);
+                        // the scale split 16 sh + sl
+                        const int sc = q6k_scale(wc, t, j, kq);
+                        const int sl = sc & 15, sh = sc >> 4;
+                        const _Float16 fl = (_Float16)(float)sl, fh = (_Float16)(float)sh;
+                        const _Float16 ol = (_Float16)(float)(-1056 * sl), oh = (_Float16)(float)(-1056 * sh);
+                        const v2h l1 = {fl, fl}, l0 = {ol, ol}, m1 = {fh, fh}, m0 = {oh, oh};
+                        const v2h s16 = {(_Float16)16.f, (_Float16)16.f};
+                        v2h q[4];
+                        q[0] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(b0, 0x64646464u, 0x00050004u));
+                        q[1] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(b0, 0x64646464u, 0x00070006u));
+                        q[2] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(b1, 0x64646464u, 0x00050004u));
+                        q[3] = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(b1, 0x64646464u, 0x00070006u));
+                        v2h r1[4], r2[4];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        // (1024 + q) x - 1056 x = x (q - 32), exact
-                        r1[i] = __builtin_elementwise_fma(q[i], l1, l0);
-                        r2[i] = __builtin_elementwise_fma(q[i], m1, m0) * s16;
+                        for (int i = 0; i < 4; ++i) {
+                            // (1024 + q) x - 1056 x = x (q - 32), exact
+                            r1[i] = __builtin_elementwise_fma(q[i], l1, l0);
+                            r2[i] = __builtin_elementwise_fma(q[i], m1, m0) * s16;
+                        }
+                        bw[t] = v8h{r1[0][0], r1[0][1], r1[1][0], r1[1][1], r1[2][0], r1[2][1], r1[3][0], r1[3][1]};
+                        bw2[t] = v8h{r2[0][0], r2[0][1], r2[1][0], r2[1][1], r2[2][0], r2[2][1], r2[3][0], r2[3][1]};
+                        bs[t] = 0.f;
+                    } else {
+                        bw[t] = nib8((uint32_t)wc.q[t][j >> 2][j & 3], 8.f);
+                        bs[t] = scale8(wc.d[t], j);
                     }
-                    bw[t] = v8h{r1[0][0], r1[0][1], r1[1][0], r1[1][1], r1[2][0], r1[2][1], r1[3][0], r1[3][1]};
-                    bw2[t] = v8h{r2[0][0], r2[0][1], r2[1][0], r2[1][1], r2[2][0], r2[2][1], r2[3][0], r2[3][1]};
-                    bs[t] = 0.f;
+                }
+                if constexpr (DT == FTX_Q4_K || DT == FTX_Q6_K_MMT) {
+                    // hi parts of every tile first, then lo: no MFMA waits on the
+                    // one before it
+#pragma unroll
+                    for (int t = 0; t < MM_NT; ++t)
+#pragma unroll
+                        for (int ms = 0; ms < MS; ++ms) {
+                            if (XT && ms >= nsub) break;
+                            tmp[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                ah[ms], bw[t], j == 0 ? zero4 : tmp[t][ms], 0, 0, 0);
+                        }
+#pragma unroll
+                    for (int t = 0; t < MM_NT; ++t)
+#pragma unroll
+                        for (int ms = 0; ms < MS; ++ms) {
+                            if (XT && ms >= nsub) break;
+                            tmp[t][ms] =
+                                __builtin_amdgcn_mfma_f32_16x16x32_f16(al[ms], bw[t], tmp[t][ms], 0, 0, 0);
+                        }
+                    if constexpr (DT == FTX_Q6_K_MMT) {
+#pragma unroll
+                        for (int t = 0; t < MM_NT; ++t)
+#pragma unroll
+                            for (int ms = 0; ms < MS; ++ms)
+                                tmp[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[ms], bw2[t],
+                                                                                    tmp[t][ms], 0, 0, 0);
+#pragma unroll
+                        for (int t = 0; t < MM_NT; ++t)
+#pragma unroll
+                            for (int ms = 0; ms < MS; ++ms)
+                                tmp[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[ms], bw2[t],
+                                                                                    tmp[t][ms], 0, 0, 0);
+                    }
                 } else {
-                    bw[t] = nib8((uint32_t)wc.q[t][j >> 2][j & 3], 8.f);
-                    bs[t] = scale8(wc.d[t], j);
-                }
-            }
-            if constexpr (DT == FTX_Q4_K || DT == FTX_Q6_K_MMT) {
-                // hi parts of every tile first, then lo: no MFMA waits on the
-                // one before it
-#pragma unroll
-                for (int t = 0; t < MM_NT; ++t)
-#pragma unroll
-                    for (int ms = 0; ms < MS; ++ms) {
-                        if (XT && ms >= nsub) break;
-                        tmp[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                            ah[ms], bw[t], j == 0 ? zero4 : tmp[t][ms], 0, 0, 0);
-                    }
-#pragma unroll
-                for (int t = 0; t < MM_NT; ++t)
-#pragma unroll
-                    for (int ms = 0; ms < MS; ++ms) {
-                        if (XT && ms >= nsub) break;
-                        tmp[t][ms] =
-                            __builtin_amdgcn_mfma_f32_16x16x32_f16(al[ms], bw[t], tmp[t][ms], 0, 0, 0);
-                    }
-                if constexpr (DT == FTX_Q6_K_MMT) {
+                    v4f p[MM_NT][MS];
 #pragma unroll
                     for (int t = 0; t < MM_NT; ++t)
 #pragma unroll
-                        for (int ms = 0; ms < MS; ++ms)
-                            tmp[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[ms], bw2[t],
-                                                                                tmp[t][ms], 0, 0, 0);
+                        for (int ms = 0; ms < MS; ++ms) {
+                            if (XT && ms >= nsub) break;
+                            p[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[ms], bw[t], zero4, 0, 0, 0);
+                        }
 #pragma unroll
                     for (int t = 0; t < MM_NT; ++t)
 #pragma unroll
-                        for (int ms = 0; ms < MS; ++ms)
-                            tmp[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[ms], bw2[t],
-                                                                                tmp[t][ms], 0, 0, 0);
+                        for (int ms = 0; ms < MS; ++ms) {
+                            if (XT && ms >= nsub) break;
+                            p[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[ms], bw[t], p[t][ms], 0, 0, 0);
+                        }
+#pragma unroll
+                    for (int t = 0; t < MM_NT; ++t)
+#pragma unroll
+                        for (int ms = 0; ms < MS; ++ms) {
+                            if (XT && ms >= nsub) break;
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) acc[t][ms][r] += bs[t] * p[t][ms][r];
+                        }
                 }
-            } else {
-                v4f p[MM_NT][MS];
-#pragma unroll
-                for (int t = 0; t < MM_NT; ++t)
-#pragma unroll
-                    for (int ms = 0; ms < MS; ++ms) {
-                        if (XT && ms >= nsub) break;
-                        p[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[ms], bw[t], zero4, 0, 0, 0);
-                    }
-#pragma unroll
-                for (int t = 0; t < MM_NT; ++t)
-#pragma unroll
-                    for (int ms = 0; ms < MS; ++ms) {
-                        if (XT && ms >= nsub) break;
-                        p[t][ms] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[ms], bw[t], p[t][ms], 0, 0, 0);
-                    }
-#pragma unroll
-                for (int t = 0; t < MM_NT; ++t)
-#pragma unroll
-                    for (int ms = 0; ms < MS; ++ms) {
-                        if (XT && ms >= nsub) break;
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) acc[t][ms][r] += bs[t] * p[t][ms][r];
-                    }
-            }
             }
         }
         if constexpr (DT == FTX_Q6_K_MMT) {
