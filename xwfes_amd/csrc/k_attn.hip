@@ -999,8 +999,8 @@ bool attn_combine_xq_supported(int64_t hd, int64_t n_head) {
 // them 128 at a time.  Above 512 rows (256-token prefill chains) a cache of
 // more than 1024 chunks, whose weights the combine could not hold in LDS,
 // stays on the generic kernel.  Measured (256 tokens, 32 query heads on 8 kv
-// heads of 128, context 0-444): 2.05 ms per layer on the generic kernel, 14.5
-// + 8.5 us (combine) here.
+// heads of 128, context 0-444): 2.05 ms per layer on the generic kernel, 15.6
+// + 8.3 us (combine) here.
 bool attn_mfma_supported(int64_t hd, int kv_f16, int64_t M, int64_t n_head, int64_t n_kv,
                          int64_t cap_alloc) {
     return kv_f16 && (hd == 64 || hd == 128) && M >= 1 &&

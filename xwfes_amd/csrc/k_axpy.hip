@@ -36,7 +36,7 @@
 // splits (52 VALU per 32 x 32 weights and 16 tokens; Q6_K an eighth of that) and
 // MFMAs.
 // Measured, one launch (before: the generic kernel, or Q6_K's 8-token chunks):
-// Q4_0 14336 x 4096, 24 tokens 2013 -> 35.9 us; Q6_K, 256 tokens 531 -> 141 us
+// Q4_0 14336 x 4096, 24 tokens 2013 -> 29.7 us; Q6_K, 256 tokens 531 -> 141 us
 // (213 TFLOP/s; 219 with d sc in A and two workgroups a CU assumed by the
 // split rule); up to 8 tokens of Q8_0 / Q4_0 go to k_axpy_few below.  Error
 // against 64 bits 0.8e-7 to 1.4e-7 (1000 to 14336 rows) where the fp32 sums of
