@@ -416,6 +416,22 @@ def test_down_axpy_large_products(gctx, orc, dt, M):
     close_or_special(got, want, size)
 
 
+@pytest.mark.parametrize("dt", [P.Q4_0, P.Q8_0, P.Q4_K, P.Q6_K])
+@pytest.mark.parametrize("M", [4, 20, 40])
+def test_down_axpy_tiny_products(gctx, orc, dt, M):
+    """Activations whose products with the weights lie just above the smallest
+    normal fp32 number keep their precision."""
+    rng = np.random.default_rng(dt + M)
+    n_in, N = 200, 512
+    t, w = weight(gctx, orc, rng, dt, n_in, N)
+    x = (rng.standard_normal((M, n_in)) * 3e-34).astype(np.float32)
+    got = gctx.down_axpy(x, t)
+    t.free()
+    size = np.abs(x.astype(np.float64)) @ np.abs(w)
+    # (the sums are kept to 2^-149 at worst)
+    assert (np.abs(got - x.astype(np.float64) @ w) < 2.0 ** -20 * size + 2.0 ** -149).all()
+
+
 @pytest.mark.parametrize("dt,d", [(P.Q8_0, 2048), (P.Q4_0, 2048), (P.Q8_0, 512)])
 @pytest.mark.parametrize("M", [1, 5])
 def test_small_step_with_an_infinite_head_scale(gctx, orc, dt, d, M):

@@ -82,9 +82,12 @@ __device__ __forceinline__ void tr4(uint32_t r0, uint32_t r1, uint32_t r2, uint3
     c[3] = perm(e, b, 0x07060302u);
 }
 
-// Q6_K: the integers enter as multiples of 2^-12 and d times 2^12, which
-// keeps the limbs of activations down to 1e-30 clear of the subnormal range
-constexpr float Q6_BS = 1.f / 4096;
+// The scales (Q4_K: the activations) enter times 2^24, undone on the sums: the
+// limbs of products h d down to the smallest normal number stay clear of the
+// subnormal range, which the MFMA does not keep (third limbs of 1e-30, second
+// limbs of 1e-34 were lost).  Products that this takes out of the fp32 range
+// are formed again (ax_redo).
+constexpr float AX_UP = 16777216.f, AX_DOWN = 1.f / 16777216.f;
 
 template <int DT>
 struct AxCfg {
@@ -253,11 +256,11 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
         } else if constexpr (DT == FTX_Q6_K) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                scl[(4 * hf + i) * 32 + at] = Q6_BS * (float)(int8_t)(o.s[0] >> (8 * i));
-            scl[8 * 32 + at] = sgn / Q6_BS * h2f((uint16_t)o.s[1]);  // (both halves the same value)
+                scl[(4 * hf + i) * 32 + at] = (float)(int8_t)(o.s[0] >> (8 * i));
+            scl[8 * 32 + at] = sgn * AX_UP * h2f((uint16_t)o.s[1]);  // (both halves the same value)
         } else {
-            scl[hf * 32 + at] = sgn * h2f((uint16_t)o.s[0]);
-            scl[(2 + hf) * 32 + at] = sgn * h2f((uint16_t)o.s[1]);
+            scl[hf * 32 + at] = sgn * AX_UP * h2f((uint16_t)o.s[0]);
+            scl[(2 + hf) * 32 + at] = sgn * AX_UP * h2f((uint16_t)o.s[1]);
         }
     };
     // h of the lane's token (past M: the last one's, never stored) in each
@@ -289,6 +292,11 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
                     hv[ms][e] = i + e < a.n_in ? v : 0.f;
                 }
         }
+        if constexpr (DT == FTX_Q4_K)
+#pragma unroll
+            for (int ms = 0; ms < MS; ++ms)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) hv[ms][e] *= AX_UP;
     };
     v4f acc[8][MS], accm[DT == FTX_Q4_K ? MS : 1];
 #pragma unroll
@@ -445,7 +453,7 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
         for (int r = 0; r < 4; ++r) {
             const int m = m0 + 16 * ms + 4 * kq + r;
             if (m >= a.M) continue;
-            float v = s[r];
+            float v = s[r] * AX_DOWN;
             if (!is_finite(v)) v = ax_redo(a, DT, m, col, 32 * I0, min(32 * I1, a.n_in));
             float* p = a.out + (int64_t)ks * a.split_stride + (int64_t)m * a.ldo + col;
             *p = a.accum ? *p + v : v;
@@ -510,7 +518,7 @@ __global__ void __launch_bounds__(64 * AF_WAVES) k_axpy_few(AxArgs a) {
         for (int e = 0; e < 8; ++e)
             q[e] = DT == FTX_Q8_0 ? (float)(int8_t)(o.q[u][e / 4 % QW] >> (8 * (e & 3)))
                                   : (float)((int)((o.q[u][0] >> (4 * e)) & 15u) - 8);
-        const float d = h2f((uint16_t)o.d[u]);
+        const float d = AX_UP * h2f((uint16_t)o.d[u]);
 #pragma unroll
         for (int m = 0; m < MC; ++m) {
             const float t = a.h[(int64_t)min(m, a.M - 1) * a.ldh + r] * d;
@@ -543,6 +551,7 @@ __global__ void __launch_bounds__(64 * AF_WAVES) k_axpy_few(AxArgs a) {
         float s = red[0][tid];
 #pragma unroll
         for (int k = 1; k < AF_WAVES; ++k) s += red[k][tid];
+        s *= AX_DOWN;
         if (j0 + tid < a.N) {
             if (!is_finite(s)) s = ax_redo(a, DT, m, j0 + tid, i0, i1);
             float* p = a.out + (int64_t)ks * a.split_stride + (int64_t)m * a.ldo + j0 + tid;
