@@ -300,8 +300,10 @@ struct MmPend {
 hipError_t launch_mm_prep_fold(hipStream_t st, float* x, int64_t ldx, const float* normw,
                                float eps, int64_t M, const MmAct& act, int weight_dt,
                                const MmPend& fold);
-// the partials `fold` added into y rows < M (a reduce launch)
-hipError_t launch_mm_fold(hipStream_t st, const MmPend& fold, int64_t M, float* y, int64_t ldy);
+// the partials `fold` added into y rows < M (a reduce launch); wide: their sum
+// in 64 bits
+hipError_t launch_mm_fold(hipStream_t st, const MmPend& fold, int64_t M, float* y, int64_t ldy,
+                          int wide = 0);
 // up to 8 tokens over the re-tiled Q8_0 / Q4_0 copies (segments with those
 // types and W), RMSNorm included when normw is given: EPI_STORE, EPI_ACCUM, or
 // EPI_SWIGLU over a gate and an up segment

@@ -39,8 +39,9 @@
 // Q4_0 14336 x 4096, 24 tokens 2013 -> 29.7 us; Q6_K, 256 tokens 531 -> 141 us
 // (213 TFLOP/s; 219 with d sc in A and two workgroups a CU assumed by the
 // split rule); up to 8 tokens of Q8_0 / Q4_0 go to k_axpy_few below.  Error
-// against 64 bits 0.8e-7 to 1.4e-7 (1000 to 14336 rows) where the fp32 sums of
-// the generic kernel had 1.6e-7 to 5.7e-7.
+// against 64 bits 0.5e-7 to 1.5e-7 (1408 to 14336 rows; Q6_K, 64 tokens of 14336
+// rows 2.0e-7) where the fp32 sums of the generic kernel had 1.6e-7 to 5.7e-7:
+// the waves and the splits are added in 64 bits.
 #include <algorithm>
 
 #include "ftx_internal.h"
@@ -48,6 +49,8 @@
 #include "quant_dev.h"
 
 namespace {
+
+typedef double v4d __attribute__((ext_vector_type(4)));
 
 constexpr int AX_WAVES = 8;
 constexpr int AX_COLS = 128;  // columns per workgroup
@@ -298,17 +301,29 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
 #pragma unroll
                 for (int e = 0; e < 8; ++e) hv[ms][e] *= AX_UP;
     };
-    v4f acc[8][MS], accm[DT == FTX_Q4_K ? MS : 1];
+    // (two tiles, whose registers allow it: the first limbs' products in a
+    // sum of their own, so that a slice rounds that once and not three times: 24
+    // tokens of 14336 rows of Q4_0 / Q6_K 1.4e-7 / 2.0e-7 -> 0.6e-7 / 1.0e-7
+    // against 64 bits, at the same time)
+    constexpr bool LO = MS == 2;
+    v4f acc[8][MS], acl[LO ? 8 : 1][LO ? MS : 1], accm[DT == FTX_Q4_K ? MS : 1];
 #pragma unroll
     for (int n = 0; n < 8; ++n)
 #pragma unroll
-        for (int ms = 0; ms < MS; ++ms) acc[n][ms] = v4f{0.f, 0.f, 0.f, 0.f};
+        for (int ms = 0; ms < MS; ++ms) {
+            acc[n][ms] = v4f{0.f, 0.f, 0.f, 0.f};
+            if constexpr (LO) acl[n][ms] = v4f{0.f, 0.f, 0.f, 0.f};
+        }
 #pragma unroll
     for (int ms = 0; ms < (DT == FTX_Q4_K ? MS : 1); ++ms) accm[ms] = v4f{0.f, 0.f, 0.f, 0.f};
-    auto mfma3 = [&](const v8bf* l, const v8bf& b, v4f acc_) {
-        acc_ = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l[2], b, acc_, 0, 0, 0);
-        acc_ = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l[1], b, acc_, 0, 0, 0);
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(l[0], b, acc_, 0, 0, 0);
+    auto low = [&](int n, int ms) -> v4f& {
+        if constexpr (LO) return acl[n][ms];
+        else return acc[n][ms];
+    };
+    auto mfma3 = [&](const v8bf* l, const v8bf& b, int n, int ms) {
+        low(n, ms) = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l[2], b, low(n, ms), 0, 0, 0);
+        low(n, ms) = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l[1], b, low(n, ms), 0, 0, 0);
+        acc[n][ms] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l[0], b, acc[n][ms], 0, 0, 0);
     };
     auto scales8 = [&](int s, int q, float* d) {
         const float4 u = *(const float4*)&scl[s * 32 + q * 8], v = *(const float4*)&scl[s * 32 + q * 8 + 4];
@@ -369,9 +384,9 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
                     split2(t, bw);
 #pragma unroll
                     for (int ms = 0; ms < MS; ++ms) {
-                        acc[n][ms] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l[ms][1], bw[1], acc[n][ms], 0, 0, 0);
-                        acc[n][ms] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l[ms][0], bw[1], acc[n][ms], 0, 0, 0);
-                        acc[n][ms] = mfma3(l[ms], bw[0], acc[n][ms]);
+                        low(n, ms) = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l[ms][1], bw[1], low(n, ms), 0, 0, 0);
+                        low(n, ms) = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l[ms][0], bw[1], low(n, ms), 0, 0, 0);
+                        mfma3(l[ms], bw[0], n, ms);
                     }
                 }
             }
@@ -410,7 +425,7 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
                     for (int e = 0; e < 8; ++e) t[e] = hv[ms][e] * d[e];
                     split3(t, l);
 #pragma unroll
-                    for (int p = 0; p < 2; ++p) acc[2 * b + p][ms] = mfma3(l, bw[p], acc[2 * b + p][ms]);
+                    for (int p = 0; p < 2; ++p) mfma3(l, bw[p], 2 * b + p, ms);
                 }
             }
             }
@@ -418,6 +433,11 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
     }
+    if constexpr (LO)
+#pragma unroll
+        for (int n = 0; n < 8; ++n)
+#pragma unroll
+            for (int ms = 0; ms < MS; ++ms) acc[n][ms] += acl[n][ms];
     if constexpr (DT == FTX_Q4_K) {
         // the min sums: lane (c, kq) of tile n holds tokens 4 kq + r; those of
         // sub-block n / 2 are in lane 16 kq + n / 2
@@ -442,10 +462,10 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
 #pragma unroll
         for (int n = 0; n < 8; ++n) red[(w * 8 + n) * 64 + lane] = acc[n][ms];
         __syncthreads();
-        v4f s = red[w * 64 + lane];
+        v4d s = {0., 0., 0., 0.};
 #pragma unroll
-        for (int k = 1; k < AX_WAVES; ++k) {
-            const v4f v = red[(k * 8 + w) * 64 + lane];
+        for (int k = 0; k < AX_WAVES; ++k) {
+            const v4d v = __builtin_convertvector(red[(k * 8 + w) * 64 + lane], v4d);
             s = (k & 1) ? s - v : s + v;
         }
         if (col >= a.N) continue;
@@ -453,7 +473,7 @@ __global__ void __launch_bounds__(64 * AX_WAVES)
         for (int r = 0; r < 4; ++r) {
             const int m = m0 + 16 * ms + 4 * kq + r;
             if (m >= a.M) continue;
-            float v = s[r] * AX_DOWN;
+            float v = (float)s[r] * AX_DOWN;
             if (!is_finite(v)) v = ax_redo(a, DT, m, col, 32 * I0, min(32 * I1, a.n_in));
             float* p = a.out + (int64_t)ks * a.split_stride + (int64_t)m * a.ldo + col;
             *p = a.accum ? *p + v : v;
@@ -694,5 +714,5 @@ hipError_t launch_axpy(hipStream_t st, const uint8_t* W, int dt, int64_t row_byt
         *pend = p;  // added into y by the next kernel that reads it
         return hipSuccess;
     }
-    return launch_mm_fold(st, p, M, y, ldy);
+    return launch_mm_fold(st, p, M, y, ldy, 1);
 }

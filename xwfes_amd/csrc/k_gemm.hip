@@ -1962,7 +1962,8 @@ static hipError_t launch_reduce(hipStream_t st, const MmReduceArgs& r, int64_t r
     return hipGetLastError();
 }
 
-hipError_t launch_mm_fold(hipStream_t st, const MmPend& fold, int64_t M, float* y, int64_t ldy) {
+hipError_t launch_mm_fold(hipStream_t st, const MmPend& fold, int64_t M, float* y, int64_t ldy,
+                          int wide) {
     if (fold.S < 1) return hipSuccess;
     MmReduceArgs r{};
     r.part = fold.part;
@@ -1977,6 +1978,7 @@ hipError_t launch_mm_fold(hipStream_t st, const MmPend& fold, int64_t M, float* 
     r.out.row0[1] = M;
     r.out.ld = ldy;
     r.out.accum = fold.accum;
+    r.wide = wide;
     return launch_reduce(st, r, M);
 }
 
