@@ -4,6 +4,7 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <cstring>
 #include <string>
@@ -61,6 +62,18 @@ inline void ktimed_launch(F kernel, const dim3& grid, const dim3& block, uint32_
     } else {
         hipLaunchKernelGGL(kernel, grid, block, shm, st, args...);
     }
+}
+
+// A kernel's dynamic LDS limit raised to `bytes`, once per device (`devs`: a bit
+// for each that has it, a static of the launch site for that kernel)
+inline hipError_t lds_limit(const void* kern, size_t bytes, std::atomic<uint64_t>& devs) {
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    const uint64_t bit = 1ull << (dev & 63);
+    if (e != hipSuccess || (devs.load(std::memory_order_relaxed) & bit)) return e;
+    e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e == hipSuccess) devs.fetch_or(bit, std::memory_order_relaxed);
+    return e;
 }
 
 struct ftx_ctx {

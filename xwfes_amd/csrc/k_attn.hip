@@ -1067,14 +1067,9 @@ static int attn_fa_chunks_per_wg(const int64_t* nchk, const int* splits, int nse
 
 template <int HD, bool WIDE, typename A>
 static hipError_t launch_fa(void (*kern)(A), const dim3& grid, hipStream_t st, const A& args) {
-    static bool lds_set = false;
-    if (!lds_set) {
-        hipError_t e = hipFuncSetAttribute((const void*)kern,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)fa_lds_bytes<HD>());
-        if (e != hipSuccess) return e;
-        lds_set = true;
-    }
+    static std::atomic<uint64_t> lds_set{0};
+    const hipError_t e = lds_limit((const void*)kern, fa_lds_bytes<HD>(), lds_set);
+    if (e != hipSuccess) return e;
     ktimed_launch(kern, grid, dim3(64 * FA_WAVES), (uint32_t)fa_lds_bytes<HD>(), st, args);
     return hipGetLastError();
 }

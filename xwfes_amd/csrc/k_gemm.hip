@@ -2190,14 +2190,9 @@ static hipError_t mm_launch(hipStream_t st, const MmSeg* segs, int nseg, const M
         const int vi = xtab ? (ms == 4 ? 1 : 2) : (ms == 4 ? 0 : (ms == 2 ? 3 : 4));
         const K_t kern = kerns[di][vi];
         if (!kern) return hipErrorInvalidValue;
-        static bool lds_set[45] = {};
-        const int ki = di * 5 + vi;
-        if (!lds_set[ki]) {
-            e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)lds);
-            if (e != hipSuccess) return e;
-            lds_set[ki] = true;
-        }
+        static std::atomic<uint64_t> lds_set[45];
+        e = lds_limit((const void*)kern, lds, lds_set[di * 5 + vi]);
+        if (e != hipSuccess) return e;
         MmArgs b = a;
         b.nseg = g0[g + 1] - g0[g];
         for (int i = 0; i < b.nseg; ++i) {

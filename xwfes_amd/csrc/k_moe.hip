@@ -844,12 +844,9 @@ hipError_t launch_moe_down(hipStream_t st, const uint8_t* tiled, int dt, int64_t
     const bool small = trows == 16;
     const size_t lds = 2 * (size_t)(small ? MOE_BUF<1> : MOE_BUF<4>);
     const void* kern = small ? (const void*)k_moe_down<1> : (const void*)k_moe_down<4>;
-    static bool lds_set[2] = {};
-    if (!lds_set[small]) {
-        hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        lds_set[small] = true;
-    }
+    static std::atomic<uint64_t> lds_set[2];
+    const hipError_t le = lds_limit(kern, lds, lds_set[small]);
+    if (le != hipSuccess) return le;
     const dim3 grid((unsigned)(K / 256), (unsigned)ntile_max, (unsigned)S);
     if (small)
         ktimed_launch(k_moe_down<1>, grid, dim3(256), (uint32_t)lds, st, a);
