@@ -62,10 +62,11 @@ def test_attention_of_queries_beyond_the_fp16_range(gctx, orc, hd, heads, kvh, M
 
 def test_attention_of_a_long_chain_beside_a_short_one(gctx, orc):
     """Sequences of more than 512 and of at most 16 query rows per kv head in
-    one step: no attention launch takes both."""
-    model = attention_model(orc, 128, 8, 2, 77)
+    one step, in turn: no attention launch takes both."""
+    model = attention_model(orc, 128, 16, 2, 77)
     rng = np.random.default_rng(78)
-    seqs = [(rng.integers(0, 300, 130).tolist(), None, 20, 160), (rng.integers(0, 300, 3).tolist(), None, 50, 60)]
+    seqs = [(rng.integers(0, 300, M).tolist(), None, npast, npast + M + 7)
+            for M, npast in ((3, 50), (70, 20), (1, 90), (80, 0), (9, 33))]
     for (got, want, kv, kvo) in run_batch(gctx, orc, model, seqs, 256):
         assert rel_err_rows(got, want) < LOGIT_TOL
         for a, b in zip(kv, kvo):

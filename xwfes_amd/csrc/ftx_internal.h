@@ -585,8 +585,6 @@ struct AttnMArgs {
 };
 bool attn_mfma_supported(int64_t hd, int kv_f16, int64_t M, int64_t n_head, int64_t n_kv,
                          int64_t cap_alloc);
-// whether sequences of Ms[s] tokens share one launch (launch_attn_mfma_batch)
-bool attn_batch_supported(const int64_t* Ms, int nseq, int64_t n_head, int64_t n_kv);
 size_t attn_part_floats(int64_t M, int64_t n_head, int64_t hd, int64_t cap_alloc);
 // xq != null: the chunk combine writes the output projection's activation
 // operand (xq_dev.h layout, K = n_head * hd) instead of a.out

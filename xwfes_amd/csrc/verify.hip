@@ -449,7 +449,7 @@ static int verify_large(ftx_ctx* ctx, ftx_model* m, const ftx_seq_args* sq, int6
         // sequence
         int64_t Ms[FTX_MAX_SEQ];
         for (int64_t s = 0; s < nseq; ++s) Ms[s] = sq[s].M;
-        bool all_mattn = nseq > 1 && attn_batch_supported(Ms, (int)nseq, d.n_head, d.n_head_kv);
+        bool all_mattn = nseq > 1;
         for (int64_t s = 0; s < nseq && all_mattn; ++s)
             all_mattn = attn_mfma_supported(hd, sq[s].kv->kv_f16, sq[s].M, d.n_head, d.n_head_kv,
                                             sq[s].kv->cap_alloc);
