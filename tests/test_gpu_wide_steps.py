@@ -60,6 +60,19 @@ def test_attention_of_queries_beyond_the_fp16_range(gctx, orc, hd, heads, kvh, M
     assert rel_err_rows(got, want) < LOGIT_TOL
 
 
+def test_attention_past_a_masked_chunk(gctx, orc):
+    """A draft of two roots: the second chain's first 64-slot chunk is all
+    masked, and what it sees in the next may score far below 2^-128 of one."""
+    model = attention_model(orc, 128, 8, 2, 91, q_std=0.5, k_std=0.5)
+    par = [i - 1 for i in range(200)]
+    par[100] = -1
+    toks = np.random.default_rng(92).integers(0, 300, 200).tolist()
+    (got, want, _, _), = run_batch(gctx, orc, model, [(toks, par, 0, 202)], 256)
+    assert np.isfinite(want).all() and np.isfinite(got).all()
+    err = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+    assert np.median(err) < LOGIT_TOL
+
+
 def test_attention_of_a_long_chain_beside_a_short_one(gctx, orc):
     """Sequences of more than 512 and of at most 16 query rows per kv head in
     one step, in turn: no attention launch takes both."""

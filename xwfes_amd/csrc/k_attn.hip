@@ -595,7 +595,7 @@ __device__ __forceinline__ void attn_fa_wg(const AttnMArgs& a, int grp, int kvh,
         }
     }
     float mrun = -INFINITY;  // running maximum of the raw scores
-    float mcrun = -INFINITY;  // WIDE: the last chunk's exponent offset, as it was rounded
+    float mcrun = -INFINITY;  // WIDE: the last chunk's exponent offset, as it was rounded, or -inf
     std::conditional_t<WIDE, double, float> lrun = 0;  // running sum
     v4f o[NDT];
 #pragma unroll
@@ -673,7 +673,7 @@ __device__ __forceinline__ void attn_fa_wg(const AttnMArgs& a, int grp, int kvh,
         const float mc = mn == -INFINITY ? 0.f : mn * c2;
         // 0 while mrun = -inf
         const float al = __builtin_amdgcn_exp2f(WIDE ? mcrun - mc : mrun * c2 - mc);
-        mcrun = mc;
+        mcrun = mn == -INFINITY ? -INFINITY : mc;
         float sum = 0.f;
         v8h ph[2], pl[2];
 #pragma unroll
@@ -736,7 +736,7 @@ __device__ __forceinline__ void attn_fa_wg(const AttnMArgs& a, int grp, int kvh,
     if constexpr (WIDE) {
         // the partial relative to e^pm, pm the offset in natural-log units as
         // it is stored: 2^(mcrun - pm log2 e), log2 e in two parts
-        const float pm = mrun == -INFINITY ? -INFINITY : mcrun * 0.6931471805599453f;
+        const float pm = mcrun * 0.6931471805599453f;
         const float f = mrun == -INFINITY ? 1.f
                                           : __builtin_amdgcn_exp2f(__builtin_fmaf(-pm, 1.44269502f, mcrun) -
                                                                    pm * 1.92596303e-8f);
