@@ -60,6 +60,21 @@ def test_attention_of_queries_beyond_the_fp16_range(gctx, orc, hd, heads, kvh, M
     assert rel_err_rows(got, want) < LOGIT_TOL
 
 
+@pytest.mark.parametrize("hd,heads,kvh,M,npast", [(128, 8, 2, 129, 70), (64, 16, 4, 200, 0)])
+def test_attention_of_huge_scores(gctx, orc, hd, heads, kvh, M, npast):
+    """Scores of some 1e10, whose fp32 neighbours are 1024 apart: one key takes
+    all, and no exponent may leave its range.  Rows of a head whose two best
+    keys lie within 1e-4 of each other (the fp16 rounding of a key) may take
+    either: 7e-4 of them (density of the gap at 0 of some hundred normal
+    scores, 7 of their size), 1e-2 of the rows of 8 or 16 heads."""
+    model = attention_model(orc, hd, heads, kvh, hd + M, q_std=1.5e6, k_std=10.0)
+    toks = np.random.default_rng(M).integers(0, 300, M).tolist()
+    (got, want, _, _), = run_batch(gctx, orc, model, [(toks, None, npast, npast + M)], 256)
+    assert np.isfinite(want).all() and np.isfinite(got).all()
+    err = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+    assert (err > LOGIT_TOL).mean() < 0.03
+
+
 def test_attention_past_a_masked_chunk(gctx, orc):
     """A draft of two roots: the second chain's first 64-slot chunk is all
     masked, and what it sees in the next may score far below 2^-128 of one."""

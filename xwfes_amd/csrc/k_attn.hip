@@ -495,6 +495,10 @@ __device__ __forceinline__ void attn_mfma_wg_mc(const AttnMArgs& a, int grp, int
 // 9.1e-7 and 1.2e-6 / 1.7e-6), at the same time.
 constexpr int FA_WAVES = 8;
 constexpr int FA_CHK = 64;  // slots per chunk
+// WIDE: exponents (in powers of two) from which an fp32 value is half of one or
+// more off: a row there takes them from its scores' differences instead, or a
+// probability of one would be formed as up to 2^(|exponent| 2^-24)
+constexpr float FA_BIG = 8388608.f;
 typedef __attribute__((address_space(3))) void lds_void;
 
 template <int HD>
@@ -670,10 +674,22 @@ __device__ __forceinline__ void attn_fa_wg(const AttnMArgs& a, int grp, int kvh,
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
         const float mn = fmaxf(mrun, mx);
         // every score so far masked: p = 0, nothing to rescale
-        const float mc = mn == -INFINITY ? 0.f : mn * c2;
+        float mc = mn == -INFINITY ? 0.f : mn * c2;
         // 0 while mrun = -inf
-        const float al = __builtin_amdgcn_exp2f(WIDE ? mcrun - mc : mrun * c2 - mc);
+        float al = __builtin_amdgcn_exp2f(WIDE ? mcrun - mc : mrun * c2 - mc);
         mcrun = mn == -INFINITY ? -INFINITY : mc;
+        if constexpr (WIDE)
+            if (__builtin_amdgcn_ballot_w64(fabsf(mc) > FA_BIG)) {  // (rare)
+                // exponents from the scores' differences, no product's rounding in them
+                if (fabsf(mc) > FA_BIG) {
+                    al = __builtin_amdgcn_exp2f((mrun - mn) * c2);
+#pragma unroll
+                    for (int st = 0; st < 4; ++st)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) s[st][r] -= mn;
+                    mc = 0.f;
+                }
+            }
         float sum = 0.f;
         v8h ph[2], pl[2];
 #pragma unroll
@@ -737,9 +753,10 @@ __device__ __forceinline__ void attn_fa_wg(const AttnMArgs& a, int grp, int kvh,
         // the partial relative to e^pm, pm the offset in natural-log units as
         // it is stored: 2^(mcrun - pm log2 e), log2 e in two parts
         const float pm = mcrun * 0.6931471805599453f;
-        const float f = mrun == -INFINITY ? 1.f
-                                          : __builtin_amdgcn_exp2f(__builtin_fmaf(-pm, 1.44269502f, mcrun) -
-                                                                   pm * 1.92596303e-8f);
+        const float f = fabsf(mcrun) <= FA_BIG
+                            ? __builtin_amdgcn_exp2f(__builtin_fmaf(-pm, 1.44269502f, mcrun) -
+                                                     pm * 1.92596303e-8f)
+                            : 1.f;
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt) *(v4f*)(po + 16 * dt) = o[dt] * f;
         if (kq == 0) {
